@@ -30,17 +30,11 @@ def main():
     ln2 = Decimal(2).ln()
     ln10 = Decimal(10).ln()
     lines = ["// Generated by gen_crmath_tables.py -- do not edit.", ""]
-    # 2^(j/64), j = 0..63, as hi + lo
-    lines.append("static constexpr double kExp2TabHi[64] = {")
-    his, los = [], []
+    # 2^(j/64), j = 0..63, as (hi, lo) pairs, so that one 16-byte load fetches an entry
+    lines.append("alignas(16) static constexpr double kExp2Tab[64][2] = {")
     for j in range(64):
         hi, lo = split((ln2 * j / 64).exp())
-        his.append(hi)
-        los.append(lo)
-    lines += ["    " + ", ".join(h.hex() for h in his[i:i + 4]) + "," for i in range(0, 64, 4)]
-    lines.append("};")
-    lines.append("static constexpr double kExp2TabLo[64] = {")
-    lines += ["    " + ", ".join(h.hex() for h in los[i:i + 4]) + "," for i in range(0, 64, 4)]
+        lines.append(f"    {{{hi.hex()}, {lo.hex()}}},")
     lines.append("};")
     # Cody-Waite split of ln2/64: c1 has 32 significant bits (n*c1 exact for |n| < 2^21)
     l64 = ln2 / 64
@@ -53,8 +47,10 @@ def main():
     lh = trunc_bits(float(ln2), 40)
     ll = float(ln2 - Decimal(lh))
     ih, il = split(1 / ln10)
+    th, tl = split(ln10)
     for name, v in (("kInvLn2x64", inv), ("kLn2o64C1", c1), ("kLn2o64C2", c2), ("kLn2o64C3", c3),
-                    ("kLn2Hi", lh), ("kLn2Lo", ll), ("kInvLn10Hi", ih), ("kInvLn10Lo", il)):
+                    ("kLn2Hi", lh), ("kLn2Lo", ll), ("kInvLn10Hi", ih), ("kInvLn10Lo", il),
+                    ("kLn10Hi", th), ("kLn10Lo", tl)):
         lines.append(f"static constexpr double {name} = {v.hex()};")
     with open(os.path.join(HERE, "tempo_crmath_tables.inc"), "w") as f:
         f.write("\n".join(lines) + "\n")

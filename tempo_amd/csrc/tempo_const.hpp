@@ -42,6 +42,28 @@ constexpr double kKap0 = 490.6, kKap1 = 17.46, kLam0 = 20.78, kLam1 = 3.29;
 constexpr int kIdxBg1 = 6;  // graupel density index when hail-aware is off (500 kg/m3)
 constexpr int kNrhg = 9;
 
+// exponents of the size-distribution integrals that the fixed parameters
+// alone determine (initialize_parameters, src/module_mp_tempo_params.F90:
+// 411-722: cre, the density-independent cge, 1/bm_r = 1/bm_i = 1/bm_g).  Known
+// to the compiler, so that whole powers become products in the FP64 step and
+// the FP32 power folds what depends on the exponent alone.
+constexpr double kCre[13] = {kBmR + 1.0,
+                             kMuR + 1.0,
+                             kBmR + kMuR + 1.0,
+                             kBmR * 2.0 + kMuR + 1.0,
+                             kMuR + kBvR + 1.0,
+                             kBmR + kMuR + kBvR + 1.0,
+                             kBmR * 0.5 + kMuR + kBvR + 1.0,
+                             kBmR + kMuR + kBvR + 3.0,
+                             kMuR + kBvR + 3.0,
+                             kMuR + 2.0,
+                             0.5 * (kBvR + 5.0 + 2.0 * kMuR),
+                             kBmR * 0.5 + kMuR + 1.0,
+                             kBmR * 2.0 + kMuR + kBvR + 1.0};
+constexpr double kCge0 = kBmG + 1.0, kCge1 = kMuG + 1.0, kCge3 = kBmG * 2. + kMuG + 1.0, kCge9 = kMuG + 2.0;
+constexpr double kOneThird = 1.0 / kBmR;
+static_assert(kBmR == 3.0 && kBmI == 3.0 && kBmG == 3.0, "one exponent for the inverse mass-diameter relations");
+
 // lookup-table dimensions (src/module_mp_tempo_params.F90:170-191)
 constexpr int kNbins = 100, kNtbI = 64, kNtbI1 = 55, kNtbC = 37, kNtbT = 9, kNtbR = 37, kNtbR1 = 37;
 constexpr int kNtbS = 37, kNtbG = 37, kNtbG1 = 37, kNtbT1 = 45, kNtbIn = 55;

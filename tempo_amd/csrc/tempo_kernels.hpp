@@ -408,8 +408,8 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>
                 (L.l_qc ? PF_QC : 0u);
   if (L.rr > R(kR1)) {  // rain_fallspeed (:1771-1774)
     const R lamr = R(1.0) / L.ilamr;
-    vtrr = L.rhof * R(kAvR) * C.crg[5] * C.org3 * mpow(lamr, C.cre[2]) * mpow(lamr + R(kFvR), -C.cre[5]);
-    vtnr = L.rhof * R(kAvR) * C.crg[6] / C.crg[11] * mpow(lamr, C.cre[11]) * mpow(lamr + R(kFvR), -C.cre[6]);
+    vtrr = L.rhof * R(kAvR) * C.crg[5] * C.org3 * mpow(lamr, R(kCre[2])) * mpow(lamr + R(kFvR), -R(kCre[5]));
+    vtnr = L.rhof * R(kAvR) * C.crg[6] / C.crg[11] * mpow(lamr, R(kCre[11])) * mpow(lamr + R(kFvR), -R(kCre[6]));
   }
   if (L.rg > R(kR1)) {  // graupel_fallspeed (:1815-1832)
     R afall, bfall;
@@ -798,8 +798,8 @@ __device__ void semi_rain_refresh(const StepArgs<R>& a, int c, int nzc, W_t<R>* 
     sd[SD_NR * plane + s] = W(L.nr);
     if (L.rr > R(kR1)) {  // rain_fallspeed (:1771-1774)
       const R rhof = sr[SR_RHOF * plane + s], lamr = R(1.0) / L.ilamr;
-      v1 = rhof * R(kAvR) * C.crg[5] * C.org3 * mpow(lamr, C.cre[2]) * mpow(lamr + R(kFvR), -C.cre[5]);
-      v2 = rhof * R(kAvR) * C.crg[6] / C.crg[11] * mpow(lamr, C.cre[11]) * mpow(lamr + R(kFvR), -C.cre[6]);
+      v1 = rhof * R(kAvR) * C.crg[5] * C.org3 * mpow(lamr, R(kCre[2])) * mpow(lamr + R(kFvR), -R(kCre[5]));
+      v2 = rhof * R(kAvR) * C.crg[6] / C.crg[11] * mpow(lamr, R(kCre[11])) * mpow(lamr + R(kFvR), -R(kCre[6]));
     }
     vt1[s] = W(v1);
     vt2[s] = W(v2);
@@ -1107,8 +1107,8 @@ __global__ void __launch_bounds__(256) k_melt_refl(StepArgs<R> a) {
   R ze_r = R(1.e-22), ze_s = R(1.e-22), ze_g = R(1.e-22);
   if (L.l_qr) {
     const R lamr = R(1.0) / L.ilamr;
-    const R n0_r = L.nr * C.org2 * mpow(lamr, C.cre[1]);
-    ze_r = n0_r * C.crg[3] * mpow(L.ilamr, C.cre[3]);
+    const R n0_r = L.nr * C.org2 * mpow(lamr, R(kCre[1]));
+    ze_r = n0_r * C.crg[3] * mpow(L.ilamr, R(kCre[3]));
   }
   if (L.l_qs)
     ze_s = R(S_t<R>(radar::melting_snow<kCR>(*a.radar, double(value(L.rs)), double(value(L.smob)),
@@ -1116,7 +1116,7 @@ __global__ void __launch_bounds__(256) k_melt_refl(StepArgs<R> a) {
   if (L.l_qg) {
     const int idx = L.idx_bg;
     ze_g = R(S_t<R>(radar::melting_graupel<kCR>(*a.radar, double(C.am_g[idx - 1]), double(C.ogg2),
-                                                double(C.cge[1][0]), double(value(L.rg)), double(value(L.ng)),
+                                                kCge1, double(value(L.rg)), double(value(L.ng)),
                                                 double(value(L.ilamg)), idx, double(value(L.rr)))));
   }
   const size_t d3 = size_t(c % a.ni) + size_t(k) * a.dldk + size_t(c / a.ni) * a.dldj;
@@ -1280,7 +1280,7 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, const Scr<R>
     R hail = R(0.0);
     if (L.rg / L.rho >= R(1.e-6) && rho_g<R>(L.idx_bg) >= R(350.0)) {
       const R lamg = R(1.0) / L.ilamg;
-      const R n0_g = L.ng * C.ogg2 * mpow(lamg, C.cge[1][0]);
+      const R n0_g = L.ng * C.ogg2 * mpow(lamg, R(kCge1));
       R sum_nh = R(0), sum_t = R(0);
       const R thr = R(0.0005);
       int n;
@@ -1309,16 +1309,16 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, const Scr<R>
       R ze_r = R(1.e-22), ze_s = R(1.e-22), ze_g = R(1.e-22);
       if (L.l_qr) {
         const R lamr = R(1.0) / L.ilamr;
-        const R n0_r = L.nr * C.org2 * mpow(lamr, C.cre[1]);
-        ze_r = n0_r * C.crg[3] * mpow(L.ilamr, C.cre[3]);
+        const R n0_r = L.nr * C.org2 * mpow(lamr, R(kCre[1]));
+        ze_r = n0_r * C.crg[3] * mpow(L.ilamr, R(kCre[3]));
       }
       const R k6 = R(0.176 / 0.93) * (R(6.0) / R(kPi)) * (R(6.0) / R(kPi));
       if (L.l_qs) ze_s = k6 * (R(kAmS) / R(900.0)) * (R(kAmS) / R(900.0)) * L.smoz;
       if (L.l_qg) {
         const int idx = L.idx_bg;
-        const R n0_g = L.ng * C.ogg2 * mpow(R(1.0) / L.ilamg, C.cge[1][0]);
+        const R n0_g = L.ng * C.ogg2 * mpow(R(1.0) / L.ilamg, R(kCge1));
         ze_g = k6 * (C.am_g[idx - 1] / R(900.0)) * (C.am_g[idx - 1] / R(900.0)) * n0_g * C.cgg[3][0] *
-               mpow(L.ilamg, C.cge[3][0]);
+               mpow(L.ilamg, R(kCge3));
       }
       dbz = mx(R(-35.0), R(10.0) * mlog10((ze_r + ze_s + ze_g) * R(1.e18)));
     }

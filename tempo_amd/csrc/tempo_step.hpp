@@ -574,7 +574,7 @@ __device__ __forceinline__ void cloud_check(const Const<S_t<R>>& C, Lvl<R>& L, R
       if (L.nc <= R(kNtCMin)) { hit = true; L.nc = R(kNtCMin); }
       if (L.nc > R(kNtCMax)) { hit = true; L.nc = R(kNtCMax); }
       nu = get_nuc(L.nc);
-      lamc = mpow(L.nc * C.am_r * C.ccg[1][nu] * C.ocg1[nu] / L.rc, C.obmr);
+      lamc = mpow(L.nc * C.am_r * C.ccg[1][nu] * C.ocg1[nu] / L.rc, R(kOneThird));
       const R xdc = (R(kBmR) + R(nu) + R(1.0)) / lamc;
       if (xdc < R(kD0C)) {
         lamc = C.cce[1][nu] / R(kD0C);
@@ -591,7 +591,7 @@ __device__ __forceinline__ void cloud_check(const Const<S_t<R>>& C, Lvl<R>& L, R
       L.nc = ncv;
     }
     nu = get_nuc(L.nc);
-    lamc = mpow(L.nc * C.am_r * C.ccg[1][nu] * C.ocg1[nu] / L.rc, C.obmr);
+    lamc = mpow(L.nc * C.am_r * C.ccg[1][nu] * C.ocg1[nu] / L.rc, R(kOneThird));
     L.ilamc = R(1.0) / lamc;
     L.mvd_c = mx(mn((R(3.0) + R(nu) + R(0.672)) * L.ilamc, R(kD0R)), R(kD0C));
   } else {
@@ -626,7 +626,7 @@ __device__ __forceinline__ void rain_check(const Const<S_t<R>>& C, Lvl<R>& L, R&
       lamr = c3 / L.mvd_r;
       L.nr = C.crg[1] * C.org3 * L.rr * mpow(lamr, R(kBmR)) / C.am_r;
     }
-    lamr = mpow(C.am_r * C.crg[2] * C.org2 * L.nr / L.rr, C.obmr);
+    lamr = mpow(C.am_r * C.crg[2] * C.org2 * L.nr / L.rr, R(kOneThird));
     L.mvd_r = c3 / lamr;
     if (L.mvd_r > R(kD0RMax)) {
       hit = true;
@@ -670,7 +670,7 @@ __device__ __forceinline__ void ice_check(const Const<S_t<R>>& C, Lvl<R>& L, R& 
       lami = C.cie[1] / R(5.e-6);
       L.ni = mn(R(kMaxNi), C.cig[0] * C.oig2 * L.ri / C.am_i * mpow(lami, R(kBmI)));
     }
-    lami = mpow(C.am_i * C.cig[1] * C.oig1 * L.ni / L.ri, C.obmi);
+    lami = mpow(C.am_i * C.cig[1] * C.oig1 * L.ni / L.ri, R(kOneThird));
     const R xdi = (R(kBmI) + R(kMuI) + R(1.0)) / lami;
     if (xdi < R(5.e-6)) {
       hit = true;
@@ -737,7 +737,7 @@ __device__ __forceinline__ void graupel_check(const Const<S_t<R>>& C, Lvl<R>& L,
         lamg = c3 / L.mvd_g;
         L.ng = C.cgg[1][0] * C.ogg3 * L.rg * mpow(lamg, R(kBmG)) / C.am_g[L.idx_bg - 1];
       }
-      lamg = mpow(C.am_g[L.idx_bg - 1] * C.cgg[2][0] * C.ogg2 * L.ng / L.rg, C.obmg);
+      lamg = mpow(C.am_g[L.idx_bg - 1] * C.cgg[2][0] * C.ogg2 * L.ng / L.rg, R(kOneThird));
       L.mvd_g = c3 / lamg;
       if (L.mvd_g > R(25.4e-3)) {
         hit = true;
@@ -760,7 +760,7 @@ __device__ __forceinline__ void graupel_check(const Const<S_t<R>>& C, Lvl<R>& L,
       const R zans1 = R(3.4) + R(2.0 / 7.0) * (ygra1 + R(8.0));
       const R n0_exp = mx(R(kGonvMin), mn(mpow(R(10.0), zans1), R(kGonvMax)));
       const R lam_exp = mpow(n0_exp * C.am_g[L.idx_bg - 1] * C.cgg[0][0] / L.rg, C.oge1);
-      lamg = lam_exp * mpow(C.cgg[2][0] * C.ogg2 * C.ogg1, C.obmg);
+      lamg = lam_exp * mpow(C.cgg[2][0] * C.ogg2 * C.ogg1, R(kOneThird));
       L.ng = C.cgg[1][0] * C.ogg3 * L.rg * mpow(lamg, R(kBmG)) / C.am_g[L.idx_bg - 1];
       L.rb = R(kM3ToL) * L.rg / rho_g<R>(L.idx_bg);
     }
@@ -869,7 +869,7 @@ __device__ void rain_index(const Const<S_t<R>>& C, R rr, R ilamr, int& ir, int& 
   ir = decade_index(rr, C.nir2, kNtbR);
   const R lamr = R(1.) / ilamr;
   const R lam_exp = lamr * mpow(C.crg[2] * C.org2 * C.org1, R(kBmR));
-  const R n0_exp = C.org1 * rr / C.am_r * mpow(lam_exp, C.cre[0]);
+  const R n0_exp = C.org1 * rr / C.am_r * mpow(lam_exp, R(kCre[0]));
   ir1 = decade_index(n0_exp, C.nir3, kNtbR1);
 }
 
@@ -878,7 +878,7 @@ __device__ void graupel_index(const Const<S_t<R>>& C, R rg, R ilamg, int idx, in
   ig = decade_index(rg, C.nig2, kNtbG);
   const R lamg = R(1.) / ilamg;
   const R lam_exp = lamg * mpow(C.cgg[2][0] * C.ogg2 * C.ogg1, R(kBmG));
-  const R n0_exp = C.ogg1 * rg / C.am_g[idx - 1] * mpow(lam_exp, C.cge[0][0]);
+  const R n0_exp = C.ogg1 * rg / C.am_g[idx - 1] * mpow(lam_exp, R(kCge0));
   ig1 = decade_index(n0_exp, C.nig3, kNtbG1);
 }
 
@@ -900,8 +900,8 @@ __device__ __forceinline__ void warm_rain(const Const<S_t<R>>& C, const Tables<S
   if (L.l_qc && L.rc > R(0.01e-3)) {
     const int nu = get_nuc(L.nc);
     const R lamc = R(1.0) / L.ilamc;
-    const R xdc = mx(R(kD0C) * R(1.e6), (mpow(L.rc / (C.am_r * L.nc), C.obmr)) * R(1.e6));
-    const R dc_g = (mpow(C.ccg[2][nu] * C.ocg2[nu], C.obmr) / lamc) * R(1.e6);
+    const R xdc = mx(R(kD0C) * R(1.e6), (mpow(L.rc / (C.am_r * L.nc), R(kOneThird))) * R(1.e6));
+    const R dc_g = (mpow(C.ccg[2][nu] * C.ocg2[nu], R(kOneThird)) / lamc) * R(1.e6);
     const R dc_b = mpow(xdc * xdc * xdc * dc_g * dc_g * dc_g - xdc * xdc * xdc * xdc * xdc * xdc, R(1.0 / 6.0));
     const R z0 = R(6.25e-6) * xdc * dc_b * dc_b * dc_b - R(0.4);
     const R zeta1 = R(0.5) * (z0 + mabs(z0));
@@ -920,8 +920,8 @@ __device__ __forceinline__ void warm_rain(const Const<S_t<R>>& C, const Tables<S
     idx = min(idx, kNbins);
     const int jc = int(L.mvd_c * R(1.e6));
     const R ef_rw = T.efrw[(idx - 1) + kNbins * (jc - 1)];
-    const R n0_r = L.nr * C.org2 * mpow(lamr, C.cre[1]);
-    const R f = mpow(lamr + R(kFvR), -C.cre[8]);
+    const R n0_r = L.nr * C.org2 * mpow(lamr, R(kCre[1]));
+    const R f = mpow(lamr + R(kFvR), -R(kCre[8]));
     t.prr_rcw = L.rhof * C.t1_qr_qc * ef_rw * L.rc * n0_r * f;
     t.prr_rcw = mn(L.rc * odt, t.prr_rcw);
     t.pnc_rcw = L.rhof * C.t1_qr_qc * ef_rw * L.nc * n0_r * f;
@@ -1123,14 +1123,14 @@ __device__ __forceinline__ void ice_processes(const Const<S_t<R>>& C, const Tabl
     }
     if (L.rr >= R(1.e-6) && L.mvd_r > R(4.0) * xdi) {
       const R lamr = R(1.0) / L.ilamr;
-      const R n0_r = L.nr * C.org2 * mpow(lamr, C.cre[1]);
-      const R f9 = mpow(lamr + R(kFvR), -C.cre[8]);
+      const R n0_r = L.nr * C.org2 * mpow(lamr, R(kCre[1]));
+      const R f9 = mpow(lamr + R(kFvR), -R(kCre[8]));
       t.pri_rci = L.rhof * C.t1_qr_qi * R(kEfRI) * L.ri * n0_r * f9;
       t.pnr_rci = L.rhof * C.t1_qr_qi * R(kEfRI) * L.ni * n0_r * f9;
       t.pnr_rci = mn(L.nr * odt, t.pnr_rci);
       t.png_rci = t.pnr_rci * mx(mn((mpow(R(10.0), R(-0.1) * w) + R(0.1)), R(1.0)), R(0.1));
       t.pni_rci = t.pri_rci * oxmi;
-      t.prr_rci = L.rhof * C.t2_qr_qi * R(kEfRI) * L.ni * n0_r * mpow(lamr + R(kFvR), -C.cre[7]);
+      t.prr_rci = L.rhof * C.t2_qr_qi * R(kEfRI) * L.ni * n0_r * mpow(lamr + R(kFvR), -R(kCre[7]));
       t.prr_rci = mn(L.rr * odt, t.prr_rci);
       t.prg_rci = t.pri_rci + t.prr_rci;
       t.pbg_rci = t.prg_rci / R(kRhoI);
@@ -1147,10 +1147,10 @@ __device__ __forceinline__ void ice_processes(const Const<S_t<R>>& C, const Tabl
   }
   if (L.l_qg && L.ssati < R(-kEps)) {
     const int idx = L.idx_bg;
-    const R n0_g = L.ng * C.ogg2 * mpow(R(1.0) / L.ilamg, C.cge[1][0]);
+    const R n0_g = L.ng * C.ogg2 * mpow(R(1.0) / L.ilamg, R(kCge1));
     const R t2_qg_sd = R(0.28) * C.sc3 * msqrt(C.av_g[idx - 1]) * C.cgg[10][idx - 1];
     t.prg_gde = R(kCCube) * t1s * L.diffu * L.ssati * rvs * n0_g *
-                (C.t1_qg_sd * mpow(L.ilamg, C.cge[9][0]) + t2_qg_sd * L.vsc2 * L.rhof2 * mpow(L.ilamg, C.cge[10][idx - 1]));
+                (C.t1_qg_sd * mpow(L.ilamg, R(kCge9)) + t2_qg_sd * L.vsc2 * L.rhof2 * mpow(L.ilamg, C.cge[10][idx - 1]));
     if (t.prg_gde < R(0.0)) {
       t.prg_gde = mx(mx(-L.rg * odt, t.prg_gde), rate_max);
       t.png_gde = t.prg_gde * L.ng / L.rg;
@@ -1213,7 +1213,7 @@ __device__ __forceinline__ R riming(const Const<S_t<R>>& C, const Tables<S_t<R>>
         ef_gw = R(0.77);
       if (L.temp > R(kT0)) ef_gw = ef_gw * R(0.1);
       const R t1_qg_qc = R(kPi) * R(.25) * C.av_g[idx - 1] * C.cgg[8][idx - 1];
-      const R n0_g = L.ng * C.ogg2 * mpow(R(1.0) / L.ilamg, C.cge[1][0]);
+      const R n0_g = L.ng * C.ogg2 * mpow(R(1.0) / L.ilamg, R(kCge1));
       const R f9 = mpow(L.ilamg, C.cge[8][idx - 1]);
       t.prg_gcw = L.rhof * t1_qg_qc * ef_gw * L.rc * n0_g * f9;
       t.pnc_gcw = L.rhof * t1_qg_qc * ef_gw * L.nc * n0_g * f9;
@@ -1261,14 +1261,14 @@ __device__ __forceinline__ void melting(const Const<S_t<R>>& C, const Lvl<R>& L,
   }
   if (L.l_qg) {
     const int idx = L.idx_bg;
-    const R n0_g = L.ng * C.ogg2 * mpow(R(1.0) / L.ilamg, C.cge[1][0]);
+    const R n0_g = L.ng * C.ogg2 * mpow(R(1.0) / L.ilamg, R(kCge1));
     R n0_melt = n0_g;
     if ((L.rg * L.ng) < R(1.e-4)) {
       const R lamg = R(1.) / L.ilamg;
-      n0_melt = (R(1.e-4) / L.rg) * C.ogg2 * mpow(lamg, C.cge[1][0]);
+      n0_melt = (R(1.e-4) / L.rg) * C.ogg2 * mpow(lamg, R(kCge1));
     }
     const R t2_qg_me = R(kPi) * R(4.0) * R(kCCube) * C.olfus * R(0.28) * C.sc3 * msqrt(C.av_g[idx - 1]) * C.cgg[10][idx - 1];
-    const R f10 = mpow(L.ilamg, C.cge[9][0]), f11 = mpow(L.ilamg, C.cge[10][idx - 1]);
+    const R f10 = mpow(L.ilamg, R(kCge9)), f11 = mpow(L.ilamg, C.cge[10][idx - 1]);
     t.prr_gml = drive * n0_melt * (C.t1_qg_me * f10 + t2_qg_me * L.rhof2 * L.vsc2 * f11);
     t.prr_gml = mn(L.rg * odt, mx(R(0.0), t.prr_gml));
     if (t.prr_gml > R(0.0)) {
@@ -1329,8 +1329,8 @@ __device__ __forceinline__ void aerosol_scavenging(const Const<S_t<R>>& C, const
   if (L.l_qr && L.mvd_r > R(kD0R)) {
     R ef = aero_eff(C, L.mvd_r, wf, L.visco, L.rho, L.temp, 'r');
     const R lamr = R(1.0) / L.ilamr;
-    const R n0_r = L.nr * C.org2 * mpow(lamr, C.cre[1]);
-    const R f9 = mpow(lamr + R(kFvR), -C.cre[8]);
+    const R n0_r = L.nr * C.org2 * mpow(lamr, R(kCre[1]));
+    const R f9 = mpow(lamr + R(kFvR), -R(kCre[8]));
     t.pna_rca = L.rhof * C.t1_qr_qc * ef * L.nwfa * n0_r * f9;
     t.pna_rca = mn(L.nwfa * odt, t.pna_rca);
     ef = aero_eff(C, L.mvd_r, iff, L.visco, L.rho, L.temp, 'r');
@@ -1351,7 +1351,7 @@ __device__ __forceinline__ void aerosol_scavenging(const Const<S_t<R>>& C, const
     const R xdg = (R(kBmG) + R(kMuG) + R(1.0)) * L.ilamg;
     R ef = aero_eff(C, xdg, wf, L.visco, L.rho, L.temp, 'g');
     const R t1_qg_qc = R(kPi) * R(.25) * C.av_g[idx - 1] * C.cgg[8][idx - 1];
-    const R n0_g = L.ng * C.ogg2 * mpow(R(1.0) / L.ilamg, C.cge[1][0]);
+    const R n0_g = L.ng * C.ogg2 * mpow(R(1.0) / L.ilamg, R(kCge1));
     const R f9 = mpow(L.ilamg, C.cge[8][idx - 1]);
     t.pna_gca = L.rhof * t1_qg_qc * ef * L.nwfa * n0_g * f9;
     t.pna_gca = mn(L.nwfa * odt, t.pna_gca);
@@ -1559,10 +1559,10 @@ __device__ __forceinline__ void rain_evaporation(const Const<S_t<R>>& C, const L
     t.prv_rev = L.rr * orho * odt;
   } else {
     const R lamr = R(1.0) / L.ilamr;
-    const R n0_r = L.nr * C.org2 * mpow(lamr, C.cre[1]);
+    const R n0_r = L.nr * C.org2 * mpow(lamr, R(kCre[1]));
     t.prv_rev = t1_evap * L.diffu * (-L.ssatw) * n0_r * rvs *
-                (C.t1_qr_ev * mpow(L.ilamr, C.cre[9]) +
-                 C.t2_qr_ev * L.vsc2 * L.rhof2 * (mpow(lamr + R(0.5) * R(kFvR), -C.cre[10])));
+                (C.t1_qr_ev * mpow(L.ilamr, R(kCre[9])) +
+                 C.t2_qr_ev * L.vsc2 * L.rhof2 * (mpow(lamr + R(0.5) * R(kFvR), -R(kCre[10]))));
     const R rate_max = mn((L.rr * orho * odt), (L.qvs - L.qv) * odt);
     t.prv_rev = mn(rate_max, t.prv_rev * orho);
     if (t.prr_gml > R(0.0)) {
