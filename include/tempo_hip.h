@@ -141,8 +141,8 @@ int tempo_hip_run(tempo_hip_ctx *ctx, const tempo_hip_fields *f, const tempo_hip
  * scratch comes from a static device array of 256 MiB per GPU instead of
  * the context's buffers; batches needing more are rejected with
  * TEMPO_HIP_E_ARG (per point, levels rounded up to 16 and columns to 8:
- * 188 bytes in FP32 -- 348 where the lane-per-column sedimentation runs --
- * and 348 in FP64, plus 88 per column; about 14,800 FP32 columns of 90
+ * 188 bytes in FP32 -- 348 above 128 levels and where the lane-per-column
+ * sedimentation runs -- and 348 in FP64, plus 88 per column; about 14,800 FP32 columns of 90
  * levels).  Results equal tempo_hip_run's bit for bit.
  * Every call on one GPU shares that array: calls that overlap on a GPU
  * (several streams or host threads) race, and must be serialised by the
@@ -302,11 +302,11 @@ int tempo_hip_substeps(tempo_hip_ctx *ctx, int *host_out, size_t n);
 /* Launch-shape tuning of subsequent runs in one precision (no counterpart in
  * the reference; set by tempo_amd/autotune.py).  Keys and values:
  *   TEMPO_HIP_TUNE_SED_WAVE  1: sedimentation with one wavefront per column
- *                               (default; used when nz <= 128), 0: one lane
+ *                               (default; used when nz <= 256), 0: one lane
  *                               per column, 2: the wavefront kernel issuing
  *                               every load pass of its LDS staging, also
  *                               those past the column group's end (a check
- *                               form of the staging)
+ *                               form of the staging; nz <= 128, else as 1)
  *   TEMPO_HIP_TUNE_BLOCK_A   threads per block of the level-local physics
  *   TEMPO_HIP_TUNE_BLOCK_C   ... and of the final update: 64, 128 or 256
  *   TEMPO_HIP_TUNE_FUSED     1: the whole step as one persistent launch that

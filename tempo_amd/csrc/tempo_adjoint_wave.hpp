@@ -515,8 +515,7 @@ hipError_t adjoint_passes(const StepArgs<D>& a, const AdjArgs& g, Dual<double>* 
     if ((e = cp(snap.sd_a, a.sd, sd_bytes)) != hipSuccess) return e;
   }
   if (wave_b)
-    hipLaunchKernelGGL(k_phase_b_wave<D>, dim3(unsigned((a.ncol + kSedCols - 1) / kSedCols)), dim3(64 * kSedCols),
-                       sed_lds_bytes(a.nz), s, a);
+    launch_phase_b_wave(a, s);
   else
     hipLaunchKernelGGL(k_phase_b<D>, dim3(unsigned((a.ncol + 127) / 128)), dim3(128), 0, s, a, vtbuf);
   double* post = static_cast<double*>(snap.sd_b);

@@ -529,16 +529,18 @@ int ensure_scratch(tempo_hip_ctx* x, size_t ncol, size_t nz, size_t br = 8, size
   return TEMPO_HIP_OK;
 }
 
-// the scratch sizes of one step of a in the context's configuration
+// the scratch sizes of one step of a in the context's configuration, on
+// more than wave_levels levels with the wide copy of the lane-per-column
+// sedimentation
 template <class R>
-ScratchSizes step_scratch(const tempo_hip_ctx* x, const StepArgs<R>& a) {
+ScratchSizes step_scratch(const tempo_hip_ctx* x, const StepArgs<R>& a, int wave_levels = kSedMaxLevels) {
   using S = S_t<R>;
   using W = W_t<R>;
   using D = Sd_t<R>;
   // the wide copy is needed where the one-lane-per-column sedimentation runs
   // on narrow planes
   const LaunchCfg& lc = x->launch[sizeof(S) == 8 ? 1 : 0];
-  const bool lane_sed = !lc.sed_wave || a.nz > kSedLevels || x->cfg.semi_sedi_flag;
+  const bool lane_sed = !lc.sed_wave || a.nz > wave_levels || x->cfg.semi_sedi_flag;
   const size_t vt_planes = 3 + (sizeof(D) < sizeof(W) && lane_sed ? SD_N : 0);
   return ScratchSizes(size_t(a.ncol), size_t(a.nz), sizeof(R), sizeof(W), sizeof(D), vt_planes,
                       x->cfg.semi_sedi_flag != 0);
@@ -1757,7 +1759,9 @@ int run_with_scratch(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hi
   std::memset(&p64, 0, sizeof(p64));
   p32.ncol = p64.ncol = dm->ni * dm->nj;
   p32.nz = p64.nz = dm->nz;
-  const ScratchSizes z = r64 ? step_scratch(x, p64) : step_scratch(x, p32);
+  // the batches accepted are those of the stated bytes per point, which count
+  // the wide copy above kSedLevels levels
+  const ScratchSizes z = r64 ? step_scratch(x, p64, kSedLevels) : step_scratch(x, p32, kSedLevels);
   if (z.total() > bytes)
     return fail(TEMPO_HIP_E_ARG, std::to_string(p32.ncol) + " columns of " + std::to_string(p32.nz) +
                                      " levels need " + std::to_string(z.total()) + " bytes of scratch, more than the " +

@@ -132,7 +132,7 @@ __device__ __forceinline__ const StepArgs<R>& fresh(const StepArgs<R>& a) {
 template <class R>
 __global__ void __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(FusedWaves<R>::n)))
 k_step_fused(StepArgs<R> a) {
-  extern __shared__ double tile_mem[];  // sed_lds_bytes(nz)
+  extern __shared__ double tile_mem[];  // sed_lds_bytes<SedStage<R>>(nz)
   __shared__ int item_s;
   __shared__ int nzc_s[kSedCols];
   const int tid = int(threadIdx.x), w = tid >> 6;
@@ -182,7 +182,7 @@ int fused_grid(int ncol, int nz) {
   int& n = per_cu[sizeof(S_t<R>) == 8 ? 1 : 0][nz];
   if (n == 0) {
     int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_step_fused<R>, kFusedThreads, sed_lds_bytes(nz)) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_step_fused<R>, kFusedThreads, sed_lds_bytes<SedStage<R>>(nz)) !=
             hipSuccess ||
         blocks < 1)
       blocks = 1;
@@ -200,7 +200,7 @@ hipError_t launch_step_fused_impl(const StepArgs<R>& a, int grid, hipStream_t s,
   if (ev) (void)hipEventRecord(ev[0], s);
   hipLaunchKernelGGL(k_fused_reset<R>, dim3(1), dim3(64), 0, s, a.queue);
   if (ev) (void)hipEventRecord(ev[1], s);
-  hipLaunchKernelGGL(k_step_fused<R>, dim3(unsigned(grid)), dim3(kFusedThreads), sed_lds_bytes(a.nz), s, a);
+  hipLaunchKernelGGL(k_step_fused<R>, dim3(unsigned(grid)), dim3(kFusedThreads), sed_lds_bytes<SedStage<R>>(a.nz), s, a);
   if (ev) {
     (void)hipEventRecord(ev[2], s);
     (void)hipEventRecord(ev[3], s);

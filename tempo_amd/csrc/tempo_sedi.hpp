@@ -1,7 +1,8 @@
 // Phase B on CDNA4: one wavefront per column, levels across lanes.
 //
-// Level k of a column lives in lane k % 64 of register chunk k / 64
-// (kChunks chunks, so nz <= 64 * kChunks).  The column couplings of the
+// Level k of a column lives in lane k % 64 of register chunk k / 64; the
+// kernel is compiled for 1 to kSedMaxChunks chunks and a launch takes the
+// fewest that hold its levels; columns of more levels run one lane each.  The column couplings of the
 // reference's sedimentation (src/module_mp_tempo_main.F90:590-727) become
 // wavefront primitives:
 //   top-down fill of a fall-speed profile (:1768-1789 and species variants)
@@ -31,12 +32,29 @@ namespace tempo {
 
 constexpr int kSedCols = kScrW;           // columns (wavefronts) per block: one scratch column group
 constexpr int kSedSlots = 8;              // LDS planes staged at once
-constexpr int kSedChunks = 2;             // register chunks of 64 levels
+constexpr int kSedMaxChunks = 4;          // register chunks of 64 levels of the largest form
+constexpr int kSedMaxLevels = 64 * kSedMaxChunks;
+constexpr int kSedChunks = 2;             // chunks of the adjoint's and the fused step's column kernels
 constexpr int kSedLevels = 64 * kSedChunks;
-// LDS row of one column: nz + 1 doubles (odd, so that the 8 columns of a
-// level fall in different banks); the block's LDS is sized at launch
-__host__ __device__ constexpr int sed_row(int nz) { return nz + 1; }
-__host__ __device__ constexpr size_t sed_lds_bytes(int nz) { return size_t(kSedSlots) * kSedCols * sed_row(nz) * sizeof(double); }
+
+// Staged values are kept as the scratch holds them: 4 bytes in the FP32
+// step (the sedimentation widens them in registers, and rounds the
+// tendencies once on the way back, as a store from FP64 would), 8 bytes
+// otherwise.  Half the LDS lets twice the blocks share a CU; at 160 levels,
+// where eight FP64 planes take 82 KB, it decides between one block and four.
+template <class R>
+using SedStage = typename std::conditional<std::is_same<Sd_t<R>, float>::value, float, double>::type;
+// LDS row of one column, in stage elements: at least nz, and an odd multiple
+// of 8 (4-byte elements) or 4 (8-byte), so that the 8 columns x 8 (4) levels
+// that a wavefront (half one) writes at a time fall in 64 different banks
+template <class E>
+__host__ __device__ constexpr int sed_row(int nz) {
+  return ((nz + int(32 / sizeof(E)) - 1) / int(32 / sizeof(E)) | 1) * int(32 / sizeof(E));
+}
+template <class E>
+__host__ __device__ constexpr size_t sed_lds_bytes(int nz) {
+  return size_t(kSedSlots) * kSedCols * sed_row<E>(nz) * sizeof(E);
+}
 
 namespace wv {
 __device__ __forceinline__ int lane() { return int(threadIdx.x & 63u); }
@@ -49,22 +67,22 @@ __device__ __forceinline__ unsigned uor(unsigned v) {
   return v;
 }
 // value of x at level k (k uniform or per lane), chunks held in x[]
-template <class T>
-__device__ __forceinline__ T at_level(const T (&x)[kSedChunks], int k) {
+template <class T, int CH>
+__device__ __forceinline__ T at_level(const T (&x)[CH], int k) {
   T v = T(0);
 #pragma unroll
-  for (int j = 0; j < kSedChunks; ++j) {
+  for (int j = 0; j < CH; ++j) {
     const T t = __shfl(x[j], k & 63, 64);
     if ((k >> 6) == j) v = t;
   }
   return v;
 }
 // value of x at level k+1 for every lane's level k in chunk j (0 above the top chunk)
-template <class T>
-__device__ __forceinline__ T above(const T (&x)[kSedChunks], int j) {
+template <class T, int CH>
+__device__ __forceinline__ T above(const T (&x)[CH], int j) {
   const T up = __shfl_down(x[j], 1, 64);
   T nxt = T(0);
-  if (j + 1 < kSedChunks) nxt = __shfl(x[j + 1 < kSedChunks ? j + 1 : j], 0, 64);
+  if (j + 1 < CH) nxt = __shfl(x[j + 1 < CH ? j + 1 : j], 0, 64);
   return lane() == 63 ? nxt : up;
 }
 }  // namespace wv
@@ -84,21 +102,21 @@ __device__ __forceinline__ double sval(const Dual<T>& x) {
 // kEveryPass: issue every load pass, also those past the group's end (all
 // lanes then load the group's last element and write nothing) -- a check
 // form of the staging, selected with sed_wave = 2; results are identical.
-template <bool kEveryPass = false>
+template <class E, int CH, bool kEveryPass = false>
 struct SedTile {
-  double* lds;  // kSedSlots x kSedCols x row
+  E* lds;       // kSedSlots x kSedCols x row
   int c0, ncol, nz;
   int nzs;      // level stride of a scratch column group
-  int row;      // LDS row of one column (sed_row(nz))
+  int row;      // LDS row of one column (sed_row<E>(nz))
   size_t sbase; // scratch offset of the group's first element
 
-  __device__ double* slot(int s) const { return lds + s * (kSedCols * row); }
+  __device__ E* slot(int s) const { return lds + s * (kSedCols * row); }
   // Several scratch planes of one stage (the block's column group of each is
   // one contiguous run).  Every global load of the stage is issued into
   // registers before the first LDS write, so the stage waits for one memory
   // latency instead of one per plane and pass (a load-convert-write loop per
   // plane waits for each load before its write).  The block has
-  // 64 * kSedCols threads and nz <= kSedLevels, so kSedChunks passes cover
+  // 64 * kSedCols threads and nz <= 64 * CH, so CH passes cover
   // the column group; a pass runs only when the group reaches it (a
   // block-uniform test), and its elements past the group's end load the last
   // one (the index is clamped, not branched on per lane, so that the loads
@@ -106,12 +124,12 @@ struct SedTile {
   template <class TA, int NA, class TB, int NB>
   __device__ void load_many(const int (&sa)[NA], const TA* const (&pa)[NA], const int (&sb)[NB],
                             const TB* const (&pb)[NB]) const {
-    TA va[kSedChunks][NA];
-    TB vb[kSedChunks][NB];
+    TA va[CH][NA];
+    TB vb[CH][NB];
     const int n = kSedCols * nz;
     const size_t base = sbase;
 #pragma unroll
-    for (int it = 0; it < kSedChunks; ++it) {
+    for (int it = 0; it < CH; ++it) {
       if (!kEveryPass && it * 64 * kSedCols >= n) break;
       const int e = min(int(threadIdx.x) + it * 64 * kSedCols, n - 1);
 #pragma unroll
@@ -120,14 +138,14 @@ struct SedTile {
       for (int p = 0; p < NB; ++p) vb[it][p] = pb[p][base + e];
     }
 #pragma unroll
-    for (int it = 0; it < kSedChunks; ++it) {
+    for (int it = 0; it < CH; ++it) {
       const int e = int(threadIdx.x) + it * 64 * kSedCols;
       if (e < n) {
         const int cc = e % kSedCols, k = e / kSedCols;
 #pragma unroll
-        for (int p = 0; p < NA; ++p) slot(sa[p])[cc * row + k] = sval(va[it][p]);
+        for (int p = 0; p < NA; ++p) slot(sa[p])[cc * row + k] = E(sval(va[it][p]));
 #pragma unroll
-        for (int p = 0; p < NB; ++p) slot(sb[p])[cc * row + k] = sval(vb[it][p]);
+        for (int p = 0; p < NB; ++p) slot(sb[p])[cc * row + k] = E(sval(vb[it][p]));
       }
     }
   }
@@ -135,14 +153,14 @@ struct SedTile {
   // from the state (slot 1), density (slot 2) and rain mass (slot 3)
   template <class R, class H, class M>
   __device__ void load_head(const StepArgs<R>& a, const unsigned* pf, const H* rho, const M* rr) const {
-    unsigned vf[kSedChunks];
-    R vz[kSedChunks];
-    H vh[kSedChunks];
-    M vr[kSedChunks];
+    unsigned vf[CH];
+    R vz[CH];
+    H vh[CH];
+    M vr[CH];
     const int n = kSedCols * nz;
     const size_t base = sbase;
 #pragma unroll
-    for (int it = 0; it < kSedChunks; ++it) {
+    for (int it = 0; it < CH; ++it) {
       if (!kEveryPass && it * 64 * kSedCols >= n) break;
       const int e = min(int(threadIdx.x) + it * 64 * kSedCols, n - 1);
       const int cc = e % kSedCols, k = e / kSedCols, c = min(c0 + cc, ncol - 1);
@@ -152,20 +170,20 @@ struct SedTile {
       vz[it] = a.f[F_DZ][TEMPO_IDX_STATE(a, c, k)];
     }
 #pragma unroll
-    for (int it = 0; it < kSedChunks; ++it) {
+    for (int it = 0; it < CH; ++it) {
       const int e = int(threadIdx.x) + it * 64 * kSedCols;
       if (e < n) {
         const int cc = e % kSedCols, k = e / kSedCols, x = cc * row + k;
-        slot(0)[x] = double(vf[it]);
-        slot(1)[x] = c0 + cc < ncol ? sval(vz[it]) : 0.0;
-        slot(2)[x] = sval(vh[it]);
-        slot(3)[x] = sval(vr[it]);
+        slot(0)[x] = E(vf[it]);
+        slot(1)[x] = c0 + cc < ncol ? E(sval(vz[it])) : E(0);
+        slot(2)[x] = E(sval(vh[it]));
+        slot(3)[x] = E(sval(vr[it]));
       }
     }
   }
   template <class T>
   __device__ void store(int s, T* plane) const {
-    const double* d = slot(s);
+    const E* d = slot(s);
     T* dst = plane + sbase;
     for (int e = threadIdx.x; e < kSedCols * nz; e += blockDim.x) {
       const int cc = e % kSedCols, k = e / kSedCols;
@@ -174,49 +192,50 @@ struct SedTile {
   }
   // this wavefront's column <-> registers
   template <class T>
-  __device__ void get(int s, int w, T (&x)[kSedChunks]) const {
-    const double* d = slot(s);
+  __device__ void get(int s, int w, T (&x)[CH]) const {
+    const E* d = slot(s);
 #pragma unroll
-    for (int j = 0; j < kSedChunks; ++j) {
+    for (int j = 0; j < CH; ++j) {
       const int k = j * 64 + wv::lane();
       x[j] = (k < nz) ? T(d[w * row + k]) : T(0);
     }
   }
   template <class T>
-  __device__ void put(int s, int w, const T (&x)[kSedChunks]) const {
-    double* d = slot(s);
+  __device__ void put(int s, int w, const T (&x)[CH]) const {
+    E* d = slot(s);
 #pragma unroll
-    for (int j = 0; j < kSedChunks; ++j) {
+    for (int j = 0; j < CH; ++j) {
       const int k = j * 64 + wv::lane();
-      if (k < nz) d[w * row + k] = double(x[j]);
+      if (k < nz) d[w * row + k] = E(x[j]);
     }
   }
 };
 
 // Per-column level geometry held by every lane.
+template <int CH>
 struct SedCol {
   int nzc;                          // active levels
-  double odz[kSedChunks], orho[kSedChunks];
+  double odz[CH], orho[CH];
 };
 
 // top-down fill (:1768-1789): out(k) = raw(k') at the lowest k' >= k whose
 // mass exceeds r1 (0 when none); CFL substeps and ktop from the filled
 // speeds in the working precision.
-template <class R>
-__device__ __forceinline__ void wave_fill(const double (&mass)[kSedChunks], const R (&raw1)[kSedChunks],
-                                          const R (&raw2)[kSedChunks], bool two, bool use_max,
-                                          const R (&dz)[kSedChunks], int nzc, double dt, double (&out1)[kSedChunks],
-                                          double (&out2)[kSedChunks], int& substeps, int& ktop) {
+template <class R, int CH>
+__device__ __forceinline__ void wave_fill(const double (&mass)[CH], const R (&raw1)[CH],
+                                          const R (&raw2)[CH], bool two, bool use_max,
+                                          const R (&dz)[CH], int nzc, double dt, double (&out1)[CH],
+                                          double (&out2)[CH], int& substeps, int& ktop) {
 #pragma clang fp contract(off)  // as the lane-per-column kernel: every operation rounded on its own
-  unsigned long long m[kSedChunks];
+  unsigned long long m[CH];
 #pragma unroll
-  for (int j = 0; j < kSedChunks; ++j) {
+  for (int j = 0; j < CH; ++j) {
     const int k = j * 64 + wv::lane();
     m[j] = __ballot(k < nzc && mass[j] > kR1);
   }
   int st = 1, kt = 1;
 #pragma unroll
-  for (int j = 0; j < kSedChunks; ++j) {
+  for (int j = 0; j < CH; ++j) {
     const int l = wv::lane(), k = j * 64 + l;
     int src = -1;
     const unsigned long long mm = m[j] & (~0ull << l);
@@ -224,7 +243,7 @@ __device__ __forceinline__ void wave_fill(const double (&mass)[kSedChunks], cons
       src = j * 64 + __ffsll((long long)mm) - 1;
     } else {
 #pragma unroll
-      for (int j2 = j + 1; j2 < kSedChunks; ++j2)
+      for (int j2 = j + 1; j2 < CH; ++j2)
         if (src < 0 && m[j2]) src = j2 * 64 + __ffsll((long long)m[j2]) - 1;
     }
     const R r1 = wv::at_level(raw1, src < 0 ? 0 : src);
@@ -250,17 +269,18 @@ __device__ __forceinline__ void wave_fill(const double (&mass)[kSedChunks], cons
 
 // one flux-form substep of one field (:1516-1559); returns the surface
 // precipitation increment (0 when the caller does not accumulate it)
-__device__ __forceinline__ double wave_sediment(const SedCol& g, double (&xr)[kSedChunks],
-                                                const double (&vt)[kSedChunks], double (&xten)[kSedChunks],
+template <int CH>
+__device__ __forceinline__ double wave_sediment(const SedCol<CH>& g, double (&xr)[CH],
+                                                const double (&vt)[CH], double (&xten)[CH],
                                                 double limit, int steps, int ktop, double dt, bool precip) {
 #pragma clang fp contract(off)  // as the lane-per-column kernel: every operation rounded on its own
   const double ost = 1.0 / double(steps);
-  double sed[kSedChunks];
+  double sed[CH];
 #pragma unroll
-  for (int j = 0; j < kSedChunks; ++j) sed[j] = vt[j] * xr[j];
+  for (int j = 0; j < CH; ++j) sed[j] = vt[j] * xr[j];
   const double s0 = __shfl(sed[0], 0, 64);
 #pragma unroll
-  for (int j = 0; j < kSedChunks; ++j) {
+  for (int j = 0; j < CH; ++j) {
     const double up = wv::above(sed, j);
     const int k = j * 64 + wv::lane();
     if (k < g.nzc && (k == g.nzc - 1 || k <= ktop - 1)) {
@@ -280,25 +300,26 @@ __device__ __forceinline__ double wave_sediment(const SedCol& g, double (&xr)[kS
 // tile_mem sed_lds_bytes(nz) of LDS.  For a dual working type it runs on the
 // values (V, the scalar type) and writes tendencies with zero tangents: the
 // tangent-free forward of an adjoint.
-template <class R, bool kEveryPass = false>
-__device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>& scr, int c0, double* tile_mem) {
+template <class R, int CH = kSedChunks, bool kEveryPass = false>
+__device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>& scr, int c0, void* tile_mem) {
   __shared__ unsigned blk_any;
   const int w = int(threadIdx.x >> 6);
   const int c = c0 + w;
   const bool col_ok = c < a.ncol;
   const size_t plane = scr.plane;
-  const SedTile<kEveryPass> T{tile_mem, c0, a.ncol, a.nz, scr.nzs, sed_row(a.nz), scr.at(c0, 0)};
+  using E = SedStage<R>;
+  const SedTile<E, CH, kEveryPass> T{static_cast<E*>(tile_mem), c0, a.ncol, a.nz, scr.nzs, sed_row<E>(a.nz), scr.at(c0, 0)};
   const double dt = a.dt;
   Sd_t<R>* sd = scr.sd;
   const R* sr = scr.sr;
   using V = typename Num<R>::S;
 
-  SedCol g;
+  SedCol<CH> g;
   g.nzc = col_ok ? (a.nlev ? min(max(a.nlev[c], 1), a.nz) : a.nz) : 0;
   if (a.sig && col_ok) {  // signature run: this kernel's decisions are per column (tempo_hip_substeps)
     const size_t n3 = size_t(a.ncol) * size_t(a.nz);
 #pragma unroll
-    for (int j = 0; j < kSedChunks; ++j) {
+    for (int j = 0; j < CH; ++j) {
       const int k = j * 64 + wv::lane();
       if (k < g.nzc) a.sig[4 * n3 + size_t(k) * a.ncol + c] = a.sig[5 * n3 + size_t(k) * a.ncol + c] = 0u;
     }
@@ -310,16 +331,16 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
   if (threadIdx.x == 0) blk_any = 0;
   T.load_head(a, scr.pf, sr + SR_RHO * plane, sd + SD_RR * plane);
   __syncthreads();
-  unsigned pfl[kSedChunks];
-  V dz[kSedChunks], rho[kSedChunks];
-  double rr[kSedChunks], vr[kSedChunks];
+  unsigned pfl[CH];
+  V dz[CH], rho[CH];
+  double rr[CH], vr[CH];
   T.get(0, w, pfl);
   T.get(1, w, dz);
   T.get(2, w, rho);
   T.get(3, w, rr);
   unsigned any = 0;
 #pragma unroll
-  for (int j = 0; j < kSedChunks; ++j) {
+  for (int j = 0; j < CH; ++j) {
     if (j * 64 + wv::lane() < g.nzc) any |= pfl[j];
     g.odz[j] = 1.0 / double(dz[j]);
     g.orho[j] = 1.0 / double(rho[j]);
@@ -335,8 +356,8 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
 
   // ---- rain (:603-630) ----
   if (bany & PF_QR) {
-    double xn[kSedChunks], tr[kSedChunks], tn[kSedChunks], v2[kSedChunks];
-    V raw1[kSedChunks], raw2[kSedChunks];
+    double xn[CH], tr[CH], tn[CH], v2[CH];
+    V raw1[CH], raw2[CH];
     T.load_many({0, 1, 2}, {sd + SD_NR * plane, sd + SD_QRTEN * plane, sd + SD_NRTEN * plane}, {4, 5},
                 {sr + SR_VTRR * plane, sr + SR_VTNR * plane});
     __syncthreads();
@@ -365,9 +386,9 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
 
   // ---- graupel (:632-660) ----
   if (bany & PF_QG) {
-    double xg[kSedChunks], xn[kSedChunks], xb[kSedChunks], tg[kSedChunks], tn[kSedChunks], tb[kSedChunks];
-    double v1[kSedChunks], v2[kSedChunks];
-    V raw1[kSedChunks], raw2[kSedChunks];
+    double xg[CH], xn[CH], xb[CH], tg[CH], tn[CH], tb[CH];
+    double v1[CH], v2[CH];
+    V raw1[CH], raw2[CH];
     T.load_many({0, 1, 2, 4, 5, 6},
                 {sd + SD_RG * plane, sd + SD_NG * plane, sd + SD_RB * plane, sd + SD_QGTEN * plane,
                  sd + SD_NGTEN * plane, sd + SD_QBTEN * plane},
@@ -406,8 +427,8 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
   // ---- snow (:662-697): mixes in the filled rain speed where snow melts,
   // with the rain mass after rain sedimentation ----
   if (bany & PF_QS) {
-    double xs[kSedChunks], ts[kSedChunks], v1[kSedChunks];
-    V raw[kSedChunks];
+    double xs[CH], ts[CH], v1[CH];
+    V raw[CH];
     T.load_many({0, 1}, {sd + SD_RS * plane, sd + SD_QSTEN * plane}, {2}, {sr + SR_VTS * plane});
     __syncthreads();
     T.get(0, w, xs);
@@ -415,9 +436,9 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
     T.get(2, w, raw);
     if (any & PF_QS) {
 #pragma clang fp contract(off)  // the snow-rain speed mix, as the lane-per-column kernel
-      V vraw[kSedChunks];
+      V vraw[CH];
 #pragma unroll
-      for (int j = 0; j < kSedChunks; ++j) {
+      for (int j = 0; j < CH; ++j) {
         V v = raw[j];
         if (pfl[j] & PF_SNOWMIX) {
           const V sr_ = V(xs[j] / (xs[j] + rr[j]));
@@ -425,7 +446,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
         }
         vraw[j] = v;
       }
-      double unused[kSedChunks];
+      double unused[CH];
       int steps, ktop;
       wave_fill(xs, vraw, vraw, false, false, dz, g.nzc, dt, v1, unused, steps, ktop);
       for (int n = 0; n < steps; ++n) pr[2] += wave_sediment(g, xs, v1, ts, kR1, steps, ktop, dt, true);
@@ -440,8 +461,8 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
 
   // ---- ice (:699-715): one call with steps = substeps ----
   if (bany & PF_QI) {
-    double xi[kSedChunks], xn[kSedChunks], ti[kSedChunks], tn[kSedChunks], v1[kSedChunks], v2[kSedChunks];
-    V raw1[kSedChunks], raw2[kSedChunks];
+    double xi[CH], xn[CH], ti[CH], tn[CH], v1[CH], v2[CH];
+    V raw1[CH], raw2[CH];
     T.load_many({0, 1, 2, 4}, {sd + SD_RI * plane, sd + SD_NI * plane, sd + SD_QITEN * plane, sd + SD_NITEN * plane},
                 {5, 6}, {sr + SR_VTRI * plane, sr + SR_VTNI * plane});
     __syncthreads();
@@ -469,8 +490,8 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
 
   // ---- cloud (:717-727, cloud_fallspeed :1945-1977): below 500 m only ----
   if (bany & PF_QC) {
-    double xc[kSedChunks], xn[kSedChunks], tc[kSedChunks], tn[kSedChunks], v1[kSedChunks], v2[kSedChunks];
-    V raw1[kSedChunks], raw2[kSedChunks];
+    double xc[CH], xn[CH], tc[CH], tn[CH], v1[CH], v2[CH];
+    V raw1[CH], raw2[CH];
     T.load_many({0, 1, 2, 4}, {sd + SD_RC * plane, sd + SD_NC * plane, sd + SD_QCTEN * plane, sd + SD_NCTEN * plane},
                 {5, 6}, {sr + SR_VTRC * plane, sr + SR_VTNC * plane});
     __syncthreads();
@@ -489,7 +510,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
         if (hgt > V(500.0)) break;
       }
 #pragma unroll
-      for (int j = 0; j < kSedChunks; ++j) {
+      for (int j = 0; j < CH; ++j) {
         const int k = j * 64 + wv::lane();
         v1[j] = (k < kt) ? double(raw1[j]) : 0.0;
         v2[j] = (k < kt) ? double(raw2[j]) : 0.0;
@@ -528,10 +549,35 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
   if (a.d2[D2_HAIL_COL]) a.d2[D2_HAIL_COL][d2] = R(0);
 }
 
-template <class R, bool kEveryPass = false>
-__global__ void __launch_bounds__(64 * kSedCols) __attribute__((amdgpu_waves_per_eu(6))) k_phase_b_wave(StepArgs<R> a) {
-  extern __shared__ double tile_mem[];  // sed_lds_bytes(nz)
-  phase_b_group<R, kEveryPass>(a, batch_scr(a), int(blockIdx.x) * kSedCols, tile_mem);
+// waves per SIMD by chunks: one chunk fits 8 without spills, two are held to
+// 6 (56 B of spills; measured faster than 4 without), three and four take
+// what their registers allow.  Against one lane per column the wavefront
+// form takes, for the whole step, 0.41 instead of 2.93 ms at 8,191 x 160
+// (FP32; one lane per column is 128 wavefronts on 256 CUs).  Two chunks with
+// 4-byte instead of 8-byte staging: 131,072 uneven columns of 30-128 levels
+// 4.70 -> 4.42 ms a step.
+constexpr int sed_waves(int chunks) { return chunks <= 1 ? 8 : chunks == 2 ? 6 : chunks == 3 ? 4 : 3; }
+template <class R, int CH, bool kEveryPass = false>
+__global__ void __launch_bounds__(64 * kSedCols) __attribute__((amdgpu_waves_per_eu(sed_waves(CH)))) k_phase_b_wave(StepArgs<R> a) {
+  extern __shared__ double tile_mem[];  // sed_lds_bytes<SedStage<R>>(nz)
+  phase_b_group<R, CH, kEveryPass>(a, batch_scr(a), int(blockIdx.x) * kSedCols, tile_mem);
+}
+
+// nz <= kSedMaxLevels (dual working types: kSedLevels)
+template <class R>
+void launch_phase_b_wave(const StepArgs<R>& a, hipStream_t s) {
+  const dim3 g(unsigned((a.ncol + kSedCols - 1) / kSedCols)), b(64 * kSedCols);
+  const size_t lds = sed_lds_bytes<SedStage<R>>(a.nz);
+  if (a.nz <= 64)
+    hipLaunchKernelGGL((k_phase_b_wave<R, 1>), g, b, lds, s, a);
+  else if (a.nz <= 128)
+    hipLaunchKernelGGL((k_phase_b_wave<R, 2>), g, b, lds, s, a);
+  else if constexpr (!IsDual<R>::value) {
+    if (a.nz <= 192)
+      hipLaunchKernelGGL((k_phase_b_wave<R, 3>), g, b, lds, s, a);
+    else
+      hipLaunchKernelGGL((k_phase_b_wave<R, 4>), g, b, lds, s, a);
+  }
 }
 
 // ------------------------------------------------------------- launch ----
@@ -552,11 +598,10 @@ hipError_t launch_step_impl(const StepArgs<T>& a, const StepArgs<RA>& ga, const 
     hipLaunchKernelGGL(k_phase_a<RA>, level_grid(a, lc.block_a), dim3(unsigned(lc.block_a)), 0, s, ga);
   if (ev) (void)hipEventRecord(ev[2], s);
   if (lc.sed_wave == 2 && a.nz <= kSedLevels && !a.fl.semi_sedi)
-    hipLaunchKernelGGL((k_phase_b_wave<T, true>), dim3(unsigned((a.ncol + kSedCols - 1) / kSedCols)),
-                       dim3(64 * kSedCols), sed_lds_bytes(a.nz), s, a);
-  else if (lc.sed_wave && a.nz <= kSedLevels && !a.fl.semi_sedi)
-    hipLaunchKernelGGL(k_phase_b_wave<T>, dim3(unsigned((a.ncol + kSedCols - 1) / kSedCols)), dim3(64 * kSedCols),
-                       sed_lds_bytes(a.nz), s, a);
+    hipLaunchKernelGGL((k_phase_b_wave<T, kSedChunks, true>), dim3(unsigned((a.ncol + kSedCols - 1) / kSedCols)),
+                       dim3(64 * kSedCols), sed_lds_bytes<SedStage<T>>(a.nz), s, a);
+  else if (lc.sed_wave && a.nz <= kSedMaxLevels && !a.fl.semi_sedi)
+    launch_phase_b_wave(a, s);
   else
     hipLaunchKernelGGL(k_phase_b<T>, dim3(unsigned((a.ncol + 127) / 128)), dim3(128), 0, s, a, vtbuf);
   if (a.fl.refl_from_melting && a.fl.refl10cm && a.d3[D3_REFL]) {

@@ -1198,3 +1198,36 @@ def test_gpu_surface_emissions_matches_reference_fixture(hip):
     with pytest.raises(hip.TempoError) as e:
         ctx.surface_emissions(torch.zeros((4, 5), device="cuda"), torch.zeros(5, device="cuda"), dt, k=4)
     assert e.value.code == hip.E_ARG
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "fp64"])
+@pytest.mark.parametrize("nz", [2, 3, 63, 64, 65, 127, 129, 160, 191, 192, 193, 255, 256, 257])
+def test_gpu_sedimentation_level_counts(hip, dtype, nz):
+    """the wavefront sedimentation compiled for 1 to 4 chunks of 64 levels
+    against one lane per column, bit for bit, at the chunk edges: 45 columns
+    (the last group of 8 cut short) of uneven depth, the multistep columns
+    interpolated onto nz levels"""
+    import torch
+    from tempo_amd import generator as gen
+    ctx = context(hip, dict(aerosolaware=True, hailaware=True))
+    prec = hip.FP32 if dtype == "fp32" else hip.FP64
+    st, m = gen.generate("multistep", ncol=45, col0=4321)
+    x_old, x_new = np.arange(90, dtype=np.float64), np.linspace(0.0, 60.0, nz)
+    st = {k: np.ascontiguousarray(np.stack([np.interp(x_new, x_old, v[:, c]) for c in range(45)], axis=1))
+          for k, v in st.items()}
+    st["dz"] = st["dz"] * min(1.0, 90.0 / nz) * 0.5
+    nlev = np.maximum(2, nz - np.arange(45) % max(1, nz // 2)).astype(np.int32)
+    got = {}
+    try:
+        for wave in (1, 0):
+            ctx.tune(prec, hip.TUNE_SED_WAVE, wave)
+            dev = {k: torch.tensor(v, dtype=torch.float32 if dtype == "fp32" else torch.float64, device="cuda")
+                   for k, v in st.items()}
+            d = ctx.run(dev, m["dt"], 2, nlev=torch.tensor(nlev, device="cuda"))
+            got[wave] = {**{k: v.cpu().numpy() for k, v in dev.items()}, **{k: v.cpu().numpy() for k, v in d.items()},
+                         "substeps": ctx.substeps(45)}
+    finally:
+        ctx.tune(prec, hip.TUNE_SED_WAVE, 1)
+    for k, v in got[1].items():
+        assert np.array_equal(v, got[0][k], equal_nan=True), (k, nz)
+    assert got[1]["substeps"].max() > 1 or nz < 64
