@@ -250,6 +250,31 @@ struct SigScope<Sig<T>> {
   }
 };
 
+// rain_fallspeed (:1771-1774) and graupel_fallspeed (:1815-1832) of one level:
+// mass- and number-weighted speeds
+template <class R>
+__device__ __forceinline__ void rain_fallspeed(const Const<S_t<R>>& C, R rhof, R lamr, R& v1, R& v2) {
+  v1 = rhof * R(kAvR) * C.crg[5] * C.org3 * mpow(lamr, R(kCre[2])) * mpow(lamr + R(kFvR), -R(kCre[5]));
+  v2 = rhof * R(kAvR) * C.crg[6] / C.crg[11] * mpow(lamr, R(kCre[11])) * mpow(lamr + R(kFvR), -R(kCre[6]));
+}
+template <class R>
+__device__ __forceinline__ void graupel_fallspeed(const Const<S_t<R>>& C, const Lvl<R>& L, R rhof, R visco, bool has_qb,
+                                                  R& v1, R& v2) {
+  R afall, bfall;
+  if (has_qb) {
+    const R dens_g = mx(rho_g<R>(1), mn(R(kM3ToL) * L.rg / L.rb, rho_g<R>(kNrhg)));
+    afall = R(kACoeff) * mpow((R(4.0) * dens_g * R(kGravity)) / (R(3.0) * L.rho), R(kBCoeff));
+    afall = afall * mpow(visco, R(1.0) - R(2.0) * R(kBCoeff));
+    bfall = R(3.0) * R(kBCoeff) - R(1.0);
+  } else {
+    afall = R(kAvGOld);
+    bfall = R(kBvGOld);
+  }
+  const int idx = L.idx_bg;
+  v1 = rhof * afall * C.cgg[5][idx - 1] * C.ogg3 * mpow(L.ilamg, bfall);
+  v2 = rhof * afall * C.cgg[6][idx - 1] / C.cgg[11][idx - 1] * mpow(L.ilamg, bfall);
+}
+
 // the level-local physics of point (c, k), from the initial checks to the
 // fall speeds (src/module_mp_tempo_main.F90:320-588); scratch in scr
 template <class R>
@@ -406,26 +431,8 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>
   R vtrr = R(0), vtnr = R(0), vtrg = R(0), vtng = R(0), vts = R(0), vtri = R(0), vtni = R(0), vtrc = R(0), vtnc = R(0);
   unsigned pf = (L.l_qr ? PF_QR : 0u) | (L.l_qg ? PF_QG : 0u) | (L.l_qs ? PF_QS : 0u) | (L.l_qi ? PF_QI : 0u) |
                 (L.l_qc ? PF_QC : 0u);
-  if (L.rr > R(kR1)) {  // rain_fallspeed (:1771-1774)
-    const R lamr = R(1.0) / L.ilamr;
-    vtrr = L.rhof * R(kAvR) * C.crg[5] * C.org3 * mpow(lamr, R(kCre[2])) * mpow(lamr + R(kFvR), -R(kCre[5]));
-    vtnr = L.rhof * R(kAvR) * C.crg[6] / C.crg[11] * mpow(lamr, R(kCre[11])) * mpow(lamr + R(kFvR), -R(kCre[6]));
-  }
-  if (L.rg > R(kR1)) {  // graupel_fallspeed (:1815-1832)
-    R afall, bfall;
-    if (a.f[F_QB]) {
-      const R dens_g = mx(rho_g<R>(1), mn(R(kM3ToL) * L.rg / L.rb, rho_g<R>(kNrhg)));
-      afall = R(kACoeff) * mpow((R(4.0) * dens_g * R(kGravity)) / (R(3.0) * L.rho), R(kBCoeff));
-      afall = afall * mpow(L.visco, R(1.0) - R(2.0) * R(kBCoeff));
-      bfall = R(3.0) * R(kBCoeff) - R(1.0);
-    } else {
-      afall = R(kAvGOld);
-      bfall = R(kBvGOld);
-    }
-    const int idx = L.idx_bg;
-    vtrg = L.rhof * afall * C.cgg[5][idx - 1] * C.ogg3 * mpow(L.ilamg, bfall);
-    vtng = L.rhof * afall * C.cgg[6][idx - 1] / C.cgg[11][idx - 1] * mpow(L.ilamg, bfall);
-  }
+  if (L.rr > R(kR1)) rain_fallspeed(C, L.rhof, R(1.0) / L.ilamr, vtrr, vtnr);
+  if (L.rg > R(kR1)) graupel_fallspeed(C, L, L.rhof, L.visco, a.f[F_QB] != nullptr, vtrg, vtng);
   if (L.rs > R(kR1)) {  // snow_fallspeed (:1873-1891)
     const R xds = L.smoc / L.smob;
     const R mrat = R(1.0) / xds;
@@ -797,9 +804,7 @@ __device__ void semi_rain_refresh(const StepArgs<R>& a, int c, int nzc, W_t<R>* 
     sd[SD_RR * plane + s] = W(L.rr);
     sd[SD_NR * plane + s] = W(L.nr);
     if (L.rr > R(kR1)) {  // rain_fallspeed (:1771-1774)
-      const R rhof = sr[SR_RHOF * plane + s], lamr = R(1.0) / L.ilamr;
-      v1 = rhof * R(kAvR) * C.crg[5] * C.org3 * mpow(lamr, R(kCre[2])) * mpow(lamr + R(kFvR), -R(kCre[5]));
-      v2 = rhof * R(kAvR) * C.crg[6] / C.crg[11] * mpow(lamr, R(kCre[11])) * mpow(lamr + R(kFvR), -R(kCre[6]));
+      rain_fallspeed(C, sr[SR_RHOF * plane + s], R(1.0) / L.ilamr, v1, v2);
     }
     vt1[s] = W(v1);
     vt2[s] = W(v2);
@@ -838,20 +843,7 @@ __device__ void semi_graupel_refresh(const StepArgs<R>& a, int c, int nzc, W_t<R
     sd[SD_NG * plane + s] = W(L.ng);
     sd[SD_RB * plane + s] = W(L.rb);
     if (L.rg > R(kR1)) {  // graupel_fallspeed (:1815-1832)
-      const R rhof = sr[SR_RHOF * plane + s];
-      R afall, bfall;
-      if (a.f[F_QB]) {
-        const R dens_g = mx(rho_g<R>(1), mn(R(kM3ToL) * L.rg / L.rb, rho_g<R>(kNrhg)));
-        afall = R(kACoeff) * mpow((R(4.0) * dens_g * R(kGravity)) / (R(3.0) * L.rho), R(kBCoeff));
-        afall = afall * mpow(sr[SR_VISCO * plane + s], R(1.0) - R(2.0) * R(kBCoeff));
-        bfall = R(3.0) * R(kBCoeff) - R(1.0);
-      } else {
-        afall = R(kAvGOld);
-        bfall = R(kBvGOld);
-      }
-      const int idx = L.idx_bg;
-      v1 = rhof * afall * C.cgg[5][idx - 1] * C.ogg3 * mpow(L.ilamg, bfall);
-      v2 = rhof * afall * C.cgg[6][idx - 1] / C.cgg[11][idx - 1] * mpow(L.ilamg, bfall);
+      graupel_fallspeed(C, L, sr[SR_RHOF * plane + s], sr[SR_VISCO * plane + s], a.f[F_QB] != nullptr, v1, v2);
     }
     vt1[s] = W(v1);
     vt2[s] = W(v2);

@@ -295,12 +295,337 @@ __device__ __forceinline__ double wave_sediment(const SedCol<CH>& g, double (&xr
   return x0 > kLowLimitPrecip ? s0 * dt * ost : 0.0;
 }
 
+// ---- semi-Lagrangian sedimentation on the wavefront --------------------
+// semi_sediment (tempo_kernels.hpp) recast with levels across lanes.  What is
+// serial there and how it runs here, with the same roundings:
+//   heights: summed in level order once per column (they depend on the layer
+//     depths alone);
+//   the top-down limit of the interface speeds: w(k) is a function of its own
+//     unlimited value and of w(k+1), so all levels are updated together from
+//     the level above until no level changes (after n rounds the top n levels
+//     are final; the chains are short);
+//   source cells kb, kt: the limit leaves every departure cell at least 95 %
+//     of its layer, so the departure points increase with height and each
+//     level finds its cells by bisection instead of following the level below;
+//   the surface flux and the decision hash: in level order, on values that
+//     every lane reads.
+// Arrays that are read at other levels live in LDS rows of the column (kSemiRows
+// of nz + 2 doubles): a column's work needs about 30 loads from them per
+// level, which in global memory, one lane per column, took 2.43 ms for
+// 10,007 columns of 59 levels (157 wavefronts on 256 CUs); here 0.15 ms.
+constexpr int kSemiLevels = 128;  // the tile's and these rows' LDS: 119 KB in FP64 at 128 levels
+enum SemiRow { SW_ZI, SW_ZA, SW_DZA, SW_QA, SW_QMI, SW_QPI, kSemiRows };
+__host__ __device__ constexpr int semi_row(int nz) { return nz + 2; }
+__host__ __device__ constexpr size_t semi_lds_bytes(int nz) {
+  return size_t(kSedCols) * kSemiRows * semi_row(nz) * sizeof(double);
+}
+
+template <int CH>
+struct SemiCol {
+  double* row;  // this column's LDS rows
+  int len;      // semi_row(nz)
+  int nz;       // active levels
+  double dt;
+  double dz[CH], orho[CH];
+  __device__ __forceinline__ double& at(int q, int k) const { return row[q * len + k]; }
+  // the wavefront's LDS writes before its later reads
+  static __device__ __forceinline__ void settle() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  // layer interfaces, summed upwards in level order (every lane the same sum)
+  __device__ __forceinline__ void heights() const {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      const int k = j * 64 + wv::lane();
+      if (k < nz) at(SW_ZA, k) = dz[j];
+    }
+    settle();
+    double z = 0.0;
+    at(SW_ZI, 0) = z;
+    for (int k = 0; k < nz; ++k) {
+      z = z + at(SW_ZA, k);
+      at(SW_ZI, k + 1) = z;
+    }
+    settle();
+  }
+};
+
+// value of x at level k + 1, k - 1, k - 2 of every lane's level k (0 outside)
+template <int CH>
+__device__ __forceinline__ double wave_up(const double (&x)[CH], int j) { return wv::above(x, j); }
+template <int CH>
+__device__ __forceinline__ double wave_down(const double (&x)[CH], int j, int d) {
+  double v = __shfl_up(x[j], d, 64);
+  if (wv::lane() < d) v = 0.0;
+  if (j > 0) {
+    const double p = __shfl(x[j > 0 ? j - 1 : 0], 64 - d + wv::lane(), 64);
+    if (wv::lane() < d) v = p;
+  }
+  return v;
+}
+
+// one substep of one field (semi_sediment), xr, vt, xten in registers; hash:
+// the column's decisions, folded in level order
+template <int CH>
+__device__ __forceinline__ void wave_semi_sediment(const SemiCol<CH>& g, double (&xr)[CH], double (&xten)[CH],
+                                                   const double (&vt)[CH], int steps, double limit, double* precip,
+                                                   unsigned& hash) {
+#pragma clang fp contract(off)  // as semi_sediment: every operation rounded on its own
+  const int nz = g.nz;
+  const double dt = g.dt, odt = 1.0 / dt, ost = 1.0 / double(steps), nst = double(steps), con1 = 0.05;
+  const double fa1 = 9.0 / 16.0, fa2 = 1.0 / 16.0;
+  // interface speeds; level nz has none above it: 0
+  double w[CH], w0[CH];
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    const int k = j * 64 + wv::lane();
+    // (every lane takes part in the shuffles; the speeds are 0 above the column)
+    const double v = vt[j], up = wave_up(vt, j), dn = wave_down(vt, j, 1), dn2 = wave_down(vt, j, 2);
+    double x = 0.0;
+    if (k == 0)
+      x = v;
+    else if (k == 1 || k == nz - 1)
+      x = 0.5 * (v + dn);
+    else if (k < nz - 1)
+      x = fa1 * (v + dn) - fa2 * (up + dn2);
+    if (k >= 1 && k < nz && v == 0.0) x = dn;
+    w0[j] = w[j] = k < nz ? x : 0.0;
+  }
+  for (int round = 0; round < nz; ++round) {
+    bool moved = false;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      const int k = j * 64 + wv::lane();
+      const double up = wave_up(w, j);  // 0 at the top interface, the initial value of level nz
+      const double decfl = (up - w0[j]) * dt * ost / g.dz[j];
+      const double x = k < nz && decfl > con1 ? up - con1 * g.dz[j] * odt * nst : w0[j];
+      moved = moved || !(x == w[j]);
+      w[j] = x;
+    }
+    if (!__any(moved)) break;
+  }
+  // departure points, cells and their contents
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    const int k = j * 64 + wv::lane();
+    if (k <= nz) g.at(SW_ZA, k) = g.at(SW_ZI, k) - w[j] * dt * ost;
+    if (k == 0) g.at(SW_ZA, nz + 1) = g.at(SW_ZI, nz);
+  }
+  if (nz == 64 * CH && wv::lane() == 0) g.at(SW_ZA, nz) = g.at(SW_ZI, nz) - 0.0 * dt * ost;
+  SemiCol<CH>::settle();
+  double qa[CH], dza[CH];
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    const int k = j * 64 + wv::lane();
+    if (k < nz) {
+      dza[j] = g.at(SW_ZA, k + 1) - g.at(SW_ZA, k);
+      qa[j] = xr[j] * g.dz[j] / dza[j];
+      g.at(SW_DZA, k) = dza[j];
+      g.at(SW_QA, k) = qa[j];
+    } else {
+      dza[j] = qa[j] = 0.0;
+    }
+  }
+  if (wv::lane() == 0) {
+    g.at(SW_DZA, nz) = g.at(SW_ZA, nz + 1) - g.at(SW_ZA, nz);
+    g.at(SW_QA, nz) = 0.0;
+    g.at(SW_QMI, nz) = g.at(SW_QPI, nz) = 0.0;
+  }
+  SemiCol<CH>::settle();
+  // monotone interface values
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    const int k = j * 64 + wv::lane();
+    if (k >= nz) continue;
+    double qp = qa[j], qm = qa[j];
+    if (k > 0) {
+      const double dip = (g.at(SW_QA, k + 1) - qa[j]) / (g.at(SW_DZA, k + 1) + dza[j]);
+      const double dim = (qa[j] - g.at(SW_QA, k - 1)) / (g.at(SW_DZA, k - 1) + dza[j]);
+      if (!(dip * dim <= 0.0)) {
+        const double a = qa[j] + 0.5 * (dip + dim) * dza[j];
+        const double b = 2.0 * qa[j] - a;
+        if (!(a > 0.0 || b < 0.0)) {
+          qp = a;
+          qm = b;
+        }
+      }
+    }
+    g.at(SW_QPI, k) = qp;
+    g.at(SW_QMI, k) = qm;
+  }
+  SemiCol<CH>::settle();
+  // remap onto the model levels (1-based kb, kt; level k here is k + 1 there)
+  const double zatop = g.at(SW_ZA, nz);
+  unsigned out[CH];
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    const int k = j * 64 + wv::lane();
+    out[j] = 0u;
+    if (k >= nz) continue;
+    const double zlo = g.at(SW_ZI, k), zhi = g.at(SW_ZI, k + 1);
+    if (zlo >= zatop) continue;
+    // kb: the first of za(1..nz) at or above zlo; kt: the first of
+    // za(0..nz+1) at or above zhi
+    int a = 1, b = nz, c = 0, d = nz + 1;
+    while (__any(a < b || c < d)) {
+      const int ab = (a + b) >> 1, cd = (c + d) >> 1;
+      const double x = g.at(SW_ZA, ab), y = g.at(SW_ZA, cd);
+      if (a < b) {
+        if (zlo <= x) b = ab;
+        else a = ab + 1;
+      }
+      if (c < d) {
+        if (zhi <= y) d = cd;
+        else c = cd + 1;
+      }
+    }
+    const int kb = a, kt = c;
+    out[j] = (unsigned(kb) << 16) ^ unsigned(kt);
+    double x = xr[j];
+    if (kt == kb) {
+      const double da = g.at(SW_DZA, kb - 1), za = g.at(SW_ZA, kb - 1), qm = g.at(SW_QMI, kb - 1);
+      const double tl = (zlo - za) / da, th = (zhi - za) / da;
+      const double tl2 = tl * tl, th2 = th * th;
+      const double qqd = 0.5 * (g.at(SW_QPI, kb - 1) - qm);
+      const double qqh = qqd * th2 + qm * th;
+      const double qql = qqd * tl2 + qm * tl;
+      x = (qqh - qql) / (th - tl);
+    } else if (kt > kb) {
+      const double da = g.at(SW_DZA, kb - 1), qm = g.at(SW_QMI, kb - 1);
+      const double tl = (zlo - g.at(SW_ZA, kb - 1)) / da;
+      const double tl2 = tl * tl;
+      double qqd = 0.5 * (g.at(SW_QPI, kb - 1) - qm);
+      const double qql = qqd * tl2 + qm * tl;
+      const double dql = g.at(SW_QA, kb - 1) - qql;
+      double zsum = (1.0 - tl) * da;
+      double qsum = dql * da;
+      for (int m = kb; m < kt - 1; ++m) {
+        zsum = zsum + g.at(SW_DZA, m);
+        qsum = qsum + g.at(SW_QA, m) * g.at(SW_DZA, m);
+      }
+      const double dt_ = g.at(SW_DZA, kt - 1), qt = g.at(SW_QMI, kt - 1);
+      const double th = (zhi - g.at(SW_ZA, kt - 1)) / dt_;
+      const double th2 = th * th;
+      qqd = 0.5 * (g.at(SW_QPI, kt - 1) - qt);
+      const double dqh = qqd * th2 + qt * th;
+      zsum = zsum + th * dt_;
+      qsum = qsum + dqh * dt_;
+      x = qsum / zsum;
+    }
+    x = x > limit ? x : limit;
+    xten[j] = xten[j] + (x - xr[j]) * g.orho[j] * odt;
+    xr[j] = x;
+  }
+  // the decisions: every remapped level's cells, then the first level left out
+  bool ended = false;
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    const int n = min(64, nz - j * 64);
+    for (int l = 0; l < n && !ended; ++l) {
+      const unsigned v = unsigned(__builtin_amdgcn_readlane(int(out[j]), l));
+      if (v == 0u) {  // kb >= 1: a remapped level's word is not 0
+        hash = decision(hash, 0x100u + unsigned(j * 64 + l + 1));
+        ended = true;
+      } else {
+        hash = decision(hash, v);
+      }
+    }
+  }
+  // surface flux: the cells that leave the column
+  if (!precip) return;
+  double p = *precip;
+  for (int k = 0; k < nz; ++k) {
+    const double z0 = g.at(SW_ZA, k), z1 = g.at(SW_ZA, k + 1);
+    if (!(z0 < 0.0)) break;  // the departure points increase with height
+    if (z1 <= 0.0) {
+      p = p + g.at(SW_QA, k) * g.at(SW_DZA, k);
+      hash = decision(hash, 0x200u + unsigned(k));
+    } else if (z1 > 0.0) {
+      hash = decision(hash, 0x300u + unsigned(k));
+      const double th = (0.0 - z0) / g.at(SW_DZA, k);
+      const double th2 = th * th;
+      const double qqd = 0.5 * (g.at(SW_QPI, k) - g.at(SW_QMI, k));
+      const double qqh = qqd * th2 + g.at(SW_QMI, k) * th;
+      p = p + qqh * g.at(SW_DZA, k);
+      break;
+    }
+  }
+  *precip = p;
+}
+
+// top-down fill of refreshed fall speeds: the value of the lowest level at or
+// above each whose mass exceeds r1, 0 above the topmost one
+template <class R, int CH>
+__device__ __forceinline__ void wave_refill(const double (&mass)[CH], int nzc, const R (&raw1)[CH], const R (&raw2)[CH],
+                                            double (&out1)[CH], double (&out2)[CH]) {
+  unsigned long long m[CH];
+#pragma unroll
+  for (int j = 0; j < CH; ++j) m[j] = __ballot(j * 64 + wv::lane() < nzc && mass[j] > kR1);
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    int src = -1;
+    const unsigned long long mm = m[j] & (~0ull << wv::lane());
+    if (mm) src = j * 64 + __ffsll((long long)mm) - 1;
+#pragma unroll
+    for (int j2 = j + 1; j2 < CH; ++j2)
+      if (src < 0 && m[j2]) src = j2 * 64 + __ffsll((long long)m[j2]) - 1;
+    const R r1 = wv::at_level(raw1, src < 0 ? 0 : src), r2 = wv::at_level(raw2, src < 0 ? 0 : src);
+    out1[j] = src < 0 ? 0.0 : double(r1);
+    out2[j] = src < 0 ? 0.0 : double(r2);
+  }
+}
+
+// a level's part of semi_rain_refresh: the checks on the 1-d state with the
+// tendencies so far, and the raw fall speeds
+template <class R>
+__device__ __forceinline__ void semi_rain_level(const StepArgs<R>& a, R rho, R rhof, R qr, R nr, double& qrten,
+                                                double& nrten, double& rr, double& rn, R& v1, R& v2) {
+  const Const<S_t<R>>& C = *a.cst;
+  Lvl<R> L;
+  L.rho = rho;
+  L.qrten = R(qrten);
+  L.nrten = R(nrten);
+  const R q0 = L.qrten, n0 = L.nrten;
+  rain_check(C, L, qr, nr, R(a.dt), R(a.odt));
+  if (L.qrten != q0) qrten = double(L.qrten);
+  if (L.nrten != n0) nrten = double(L.nrten);
+  rr = double(L.rr);
+  rn = double(L.nr);
+  if (L.rr > R(kR1)) rain_fallspeed(C, rhof, R(1.0) / L.ilamr, v1, v2);
+}
+// ... and of semi_graupel_refresh
+template <class R>
+__device__ __forceinline__ void semi_graupel_level(const StepArgs<R>& a, R rho, R rhof, R visco, R qg, R ng, R qb,
+                                                   double& qgten, double& ngten, double& qbten, double& rg, double& rn,
+                                                   double& rb, R& v1, R& v2) {
+  const Const<S_t<R>>& C = *a.cst;
+  const bool has_ngqb = a.f[F_NG] && a.f[F_QB];
+  Lvl<R> L;
+  L.rho = rho;
+  L.qgten = R(qgten);
+  L.ngten = R(ngten);
+  L.qbten = R(qbten);
+  const R g0 = L.qgten, n0 = L.ngten, b0 = L.qbten;
+  graupel_check(C, L, qg, ng, qb, has_ngqb, R(a.dt), R(a.odt));
+  if (L.qgten != g0) qgten = double(L.qgten);
+  if (L.ngten != n0) ngten = double(L.ngten);
+  if (L.qbten != b0) qbten = double(L.qbten);
+  rg = double(L.rg);
+  rn = double(L.ng);
+  rb = double(L.rb);
+  if (L.rg > R(kR1)) graupel_fallspeed(C, L, rhof, visco, a.f[F_QB] != nullptr, v1, v2);
+}
+
 // Sedimentation of the column group c0 .. c0 + kSedCols - 1, one wavefront
 // per column (64 * kSedCols threads); scr holds the group's scratch,
 // tile_mem sed_lds_bytes(nz) of LDS.  For a dual working type it runs on the
 // values (V, the scalar type) and writes tendencies with zero tangents: the
 // tangent-free forward of an adjoint.
-template <class R, int CH = kSedChunks, bool kEveryPass = false>
+// kSemi: semi-Lagrangian rain and graupel, with semi_lds_bytes(nz) more LDS
+// behind the tile.
+template <class R, int CH = kSedChunks, bool kEveryPass = false, bool kSemi = false>
 __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>& scr, int c0, void* tile_mem) {
   __shared__ unsigned blk_any;
   const int w = int(threadIdx.x >> 6);
@@ -352,7 +677,29 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
   const unsigned bany = blk_any;
 
   double pr[5] = {0, 0, 0, 0, 0};
-  int kst[10] = {1, 1, 1, 1, 1, 1, 1, 1, 1, 1};
+  int kst[kSubRows] = {1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 0, 0};
+  SemiCol<CH> sg;
+  unsigned hash[2] = {0u, 0u};
+  V rhof[CH], visco[CH];
+  if constexpr (kSemi) {
+    double* rows = reinterpret_cast<double*>(static_cast<char*>(tile_mem) + sed_lds_bytes<E>(a.nz));
+    sg.row = rows + w * (kSemiRows * semi_row(a.nz));
+    sg.len = semi_row(a.nz);
+    sg.nz = g.nzc;
+    sg.dt = dt;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      const int k = j * 64 + wv::lane();
+      sg.dz[j] = double(dz[j]);
+      sg.orho[j] = g.orho[j];
+      rhof[j] = visco[j] = V(0);
+      if ((any & (PF_QR | PF_QG)) && k < g.nzc) {
+        rhof[j] = value(sr[SR_RHOF * plane + scr.at(c, k)]);
+        visco[j] = value(sr[SR_VISCO * plane + scr.at(c, k)]);
+      }
+    }
+    if (any & (PF_QR | PF_QG)) sg.heights();
+  }
 
   // ---- rain (:603-630) ----
   if (bany & PF_QR) {
@@ -369,7 +716,28 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
     if (any & PF_QR) {
       int steps, ktop;
       wave_fill(rr, raw1, raw2, true, true, dz, g.nzc, dt, vr, v2, steps, ktop);
-      for (int n = 0; n < steps; ++n) {
+      if constexpr (kSemi) {  // (:599-615): far fewer substeps, fall speeds refreshed after each
+        steps = max(int(R(steps) / R(10.0)) + 1, 1);
+        V q[CH], qn[CH];
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+          const int k = j * 64 + wv::lane();
+          const bool in = k < g.nzc;
+          q[j] = in ? a.fa[F_QR][TEMPO_IDX_STATE(a, c, k)] : V(0);
+          qn[j] = in ? a.fa[F_NR][TEMPO_IDX_STATE(a, c, k)] : V(0);
+        }
+        for (int n = 0; n < steps; ++n) {
+          wave_semi_sediment(sg, rr, tr, vr, steps, kR1, &pr[0], hash[0]);
+          wave_semi_sediment(sg, xn, tn, v2, steps, kR2, nullptr, hash[0]);
+#pragma unroll
+          for (int j = 0; j < CH; ++j) {
+            raw1[j] = raw2[j] = V(0);
+            if (j * 64 + wv::lane() < g.nzc)
+              semi_rain_level(a, rho[j], rhof[j], q[j], qn[j], tr[j], tn[j], rr[j], xn[j], raw1[j], raw2[j]);
+          }
+          wave_refill(rr, g.nzc, raw1, raw2, vr, v2);
+        }
+      } else for (int n = 0; n < steps; ++n) {
         pr[0] += wave_sediment(g, rr, vr, tr, kR1, steps, ktop, dt, true);
         wave_sediment(g, xn, v2, tn, kR2, steps, ktop, dt, false);
       }
@@ -406,7 +774,32 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
       int steps, ktop;
       wave_fill(xg, raw1, raw2, true, false, dz, g.nzc, dt, v1, v2, steps, ktop);
       const double rb_lim = kM3ToL * kR1 / 800.0;
-      for (int n = 0; n < steps; ++n) {
+      if constexpr (kSemi) {  // (:641-667)
+        steps = max(int(R(steps) / R(10.0)) + 1, 1);
+        const bool has_ngqb = a.f[F_NG] && a.f[F_QB];
+        V q[CH], qn[CH], qb[CH];
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+          const int k = j * 64 + wv::lane();
+          const bool in = k < g.nzc;
+          q[j] = in ? a.fa[F_QG][TEMPO_IDX_STATE(a, c, k)] : V(0);
+          qn[j] = in && has_ngqb ? a.fa[F_NG][TEMPO_IDX_STATE(a, c, k)] : V(0);
+          qb[j] = in && has_ngqb ? a.fa[F_QB][TEMPO_IDX_STATE(a, c, k)] : V(0);
+        }
+        for (int n = 0; n < steps; ++n) {
+          wave_semi_sediment(sg, xg, tg, v1, steps, kR1, &pr[1], hash[1]);
+          wave_semi_sediment(sg, xn, tn, v2, steps, kR2, nullptr, hash[1]);
+          wave_semi_sediment(sg, xb, tb, v1, steps, rb_lim, nullptr, hash[1]);
+#pragma unroll
+          for (int j = 0; j < CH; ++j) {
+            raw1[j] = raw2[j] = V(0);
+            if (j * 64 + wv::lane() < g.nzc)
+              semi_graupel_level(a, rho[j], rhof[j], visco[j], q[j], qn[j], qb[j], tg[j], tn[j], tb[j], xg[j], xn[j],
+                                 xb[j], raw1[j], raw2[j]);
+          }
+          wave_refill(xg, g.nzc, raw1, raw2, v1, v2);
+        }
+      } else for (int n = 0; n < steps; ++n) {
         pr[1] += wave_sediment(g, xg, v1, tg, kR1, steps, ktop, dt, true);
         wave_sediment(g, xn, v2, tn, kR2, steps, ktop, dt, false);
         wave_sediment(g, xb, v1, tb, rb_lim, steps, ktop, dt, false);
@@ -529,8 +922,10 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
 
   if (!col_ok || wv::lane() != 0) return;
   for (int q = 0; q < 5; ++q) a.precip[size_t(q) * a.ncol + c] = pr[q];
+  kst[10] = int(hash[0]);
+  kst[11] = int(hash[1]);
   if (a.ksub)
-    for (int q = 0; q < kSubRows; ++q) a.ksub[size_t(q) * a.ncol + c] = q < 10 ? kst[q] : 0;
+    for (int q = 0; q < kSubRows; ++q) a.ksub[size_t(q) * a.ncol + c] = kst[q];
   // column diagnostics (src/module_mp_tempo_main.F90:784-794, driver :452-457)
   const size_t d2 = size_t(c % a.ni) + size_t(c / a.ni) * a.d2ldj;
   const R rain = R(pr[0]), graupel = R(pr[1]), snow = R(pr[2]), ice = R(pr[3]), cloud = R(pr[4]);
@@ -561,6 +956,22 @@ template <class R, int CH, bool kEveryPass = false>
 __global__ void __launch_bounds__(64 * kSedCols) __attribute__((amdgpu_waves_per_eu(sed_waves(CH)))) k_phase_b_wave(StepArgs<R> a) {
   extern __shared__ double tile_mem[];  // sed_lds_bytes<SedStage<R>>(nz)
   phase_b_group<R, CH, kEveryPass>(a, batch_scr(a), int(blockIdx.x) * kSedCols, tile_mem);
+}
+
+// ... with semi-Lagrangian rain and graupel
+template <class R, int CH>
+__global__ void __launch_bounds__(64 * kSedCols) k_phase_b_semi_wave(StepArgs<R> a) {
+  extern __shared__ double tile_mem[];  // sed_lds_bytes<SedStage<R>>(nz) + semi_lds_bytes(nz)
+  phase_b_group<R, CH, false, true>(a, batch_scr(a), int(blockIdx.x) * kSedCols, tile_mem);
+}
+template <class R>
+void launch_phase_b_semi_wave(const StepArgs<R>& a, hipStream_t s) {
+  const dim3 g(unsigned((a.ncol + kSedCols - 1) / kSedCols)), b(64 * kSedCols);
+  const size_t lds = sed_lds_bytes<SedStage<R>>(a.nz) + semi_lds_bytes(a.nz);
+  if (a.nz <= 64)
+    hipLaunchKernelGGL((k_phase_b_semi_wave<R, 1>), g, b, lds, s, a);
+  else
+    hipLaunchKernelGGL((k_phase_b_semi_wave<R, 2>), g, b, lds, s, a);
 }
 
 // nz <= kSedMaxLevels (dual working types: kSedLevels)
@@ -602,6 +1013,8 @@ hipError_t launch_step_impl(const StepArgs<T>& a, const StepArgs<RA>& ga, const 
                        dim3(64 * kSedCols), sed_lds_bytes<SedStage<T>>(a.nz), s, a);
   else if (lc.sed_wave && a.nz <= kSedMaxLevels && !a.fl.semi_sedi)
     launch_phase_b_wave(a, s);
+  else if (lc.sed_wave && a.nz <= kSemiLevels && a.fl.semi_sedi && !a.sig)
+    launch_phase_b_semi_wave(a, s);
   else
     hipLaunchKernelGGL(k_phase_b<T>, dim3(unsigned((a.ncol + 127) / 128)), dim3(128), 0, s, a, vtbuf);
   if (a.fl.refl_from_melting && a.fl.refl10cm && a.d3[D3_REFL]) {

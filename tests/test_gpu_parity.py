@@ -1231,3 +1231,39 @@ def test_gpu_sedimentation_level_counts(hip, dtype, nz):
     for k, v in got[1].items():
         assert np.array_equal(v, got[0][k], equal_nan=True), (k, nz)
     assert got[1]["substeps"].max() > 1 or nz < 64
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "fp64"])
+@pytest.mark.parametrize("hail", [True, False])
+@pytest.mark.parametrize("nz", [2, 3, 5, 59, 63, 64, 65, 127, 128, 129])
+def test_gpu_semi_lagrangian_level_counts(hip, dtype, hail, nz):
+    """semi-Lagrangian sedimentation with a wavefront per column against one
+    lane per column, bit for bit, decision hashes included: 45 columns of
+    uneven depth, layers stretched from 25 m, long steps (several substeps)"""
+    import torch
+    from tempo_amd import generator as gen
+    ctx = context(hip, dict(aerosolaware=True, hailaware=hail, semi_sedi=True))
+    prec = hip.FP32 if dtype == "fp32" else hip.FP64
+    st, m = gen.generate("multistep", ncol=45, col0=9876)
+    if not hail:
+        st.pop("ng")
+        st.pop("qb")
+    x_old, x_new = np.arange(90, dtype=np.float64), np.linspace(0.0, 60.0, nz)
+    st = {k: np.ascontiguousarray(np.stack([np.interp(x_new, x_old, v[:, c]) for c in range(45)], axis=1))
+          for k, v in st.items()}
+    st["dz"] = np.ascontiguousarray(np.broadcast_to(np.minimum(200.0, 25.0 * 1.06 ** np.arange(nz))[:, None], (nz, 45)))
+    nlev = np.maximum(2, nz - np.arange(45) % max(1, nz // 2)).astype(np.int32)
+    got = {}
+    try:
+        for wave in (1, 0):
+            ctx.tune(prec, hip.TUNE_SED_WAVE, wave)
+            dev = {k: torch.tensor(v, dtype=torch.float32 if dtype == "fp32" else torch.float64, device="cuda")
+                   for k, v in st.items()}
+            for k in range(2):
+                d = ctx.run(dev, 120.0, 2 + k, nlev=torch.tensor(nlev, device="cuda"))
+            got[wave] = {**{k: v.cpu().numpy() for k, v in dev.items()}, **{k: v.cpu().numpy() for k, v in d.items()},
+                         "substeps": ctx.substeps(45, decisions=True)}
+    finally:
+        ctx.tune(prec, hip.TUNE_SED_WAVE, 1)
+    for k, v in got[1].items():
+        assert np.array_equal(v, got[0][k], equal_nan=True), (k, nz)
