@@ -22,6 +22,9 @@
 //   pow: exp of y*log(x) with the product carried in double-double; whole
 //   exponents known to the compiler by double-double products.
 //
+// Contraction is off in every function, so that the error-free
+// transformations hold in the FP32 unit too.
+//
 // Everything here is straight-line code without a call: the step evaluates
 // about a hundred of these per point, all inlined.  With the device libm's
 // log for the first approximation and its exp, log and pow as the fallback
@@ -47,17 +50,20 @@ struct dd {
 };
 
 __device__ __host__ __forceinline__ dd two_sum(double a, double b) {
+#pragma clang fp contract(off)
   const double s = a + b;
   const double bb = s - a;
   return {s, (a - (s - bb)) + (b - bb)};
 }
 
 __device__ __host__ __forceinline__ dd fast_two_sum(double a, double b) {  // |a| >= |b|
+#pragma clang fp contract(off)
   const double s = a + b;
   return {s, b - (s - a)};
 }
 
 __device__ __host__ __forceinline__ dd two_prod(double a, double b) {
+#pragma clang fp contract(off)
   const double p = a * b;
   return {p, fma(a, b, -p)};
 }
@@ -67,6 +73,7 @@ __device__ __host__ __forceinline__ dd two_prod(double a, double b) {
 // below 2^-85)
 template <bool kSmall = false>
 __device__ __host__ __forceinline__ dd exp_dd(double zh, double zl, int& k) {
+#pragma clang fp contract(off)
   const double n = rint(zh * kInvLn2x64);
   const int ni = int(n);
   const double r1 = fma(-n, kLn2o64C1, zh);  // exact: n*c1 exact, Sterbenz
@@ -101,6 +108,7 @@ __device__ __host__ __forceinline__ dd exp_dd(double zh, double zl, int& k) {
 // 2^-23), u = m e^-y - 1 in double-double, log m = y + log1p(u) with four
 // terms of the series (u^5/5 < 2^-107 is dropped).
 __device__ __host__ __forceinline__ dd log_dd(double x) {
+#pragma clang fp contract(off)
   int e;
   double m = frexp(x, &e);
   if (m < 0.70710678118654752440) {
@@ -128,6 +136,7 @@ __device__ __host__ __forceinline__ dd log_dd(double x) {
 // Results outside the normal range are formed by the final scaling (an
 // argument past the clamps overflows to infinity or vanishes).
 __device__ __host__ __forceinline__ double exp_cr(double x) {
+#pragma clang fp contract(off)
   const double z = x > 710.0 ? 710.0 : (x < -746.0 ? -746.0 : x);
   int k;
   const dd r = exp_dd(z, 0.0, k);
@@ -135,20 +144,24 @@ __device__ __host__ __forceinline__ double exp_cr(double x) {
 }
 
 __device__ __host__ __forceinline__ bool positive_finite(double x) {
+#pragma clang fp contract(off)
   return x > 0.0 && x <= 1.7976931348623157e308;
 }
 
 // log of 0, negative, infinite and NaN arguments, and of 1
 __device__ __host__ __forceinline__ double log_special(double x) {
+#pragma clang fp contract(off)
   return x == 1.0 ? 0.0 : x == 0.0 ? -__builtin_huge_val() : x > 0.0 ? x : __builtin_nan("");
 }
 
 __device__ __host__ __forceinline__ double log_cr(double x) {
+#pragma clang fp contract(off)
   if (!positive_finite(x) || x == 1.0) return log_special(x);
   return log_dd(x).hi;
 }
 
 __device__ __host__ __forceinline__ double log10_cr(double x) {
+#pragma clang fp contract(off)
   if (!positive_finite(x) || x == 1.0) return log_special(x);
   const dd l = log_dd(x);
   const dd p = two_prod(l.hi, kInvLn10Hi);
@@ -159,6 +172,7 @@ __device__ __host__ __forceinline__ double log10_cr(double x) {
 // pow where x is not a positive finite number other than 1, or y is zero,
 // infinite or NaN: r = |x|**y as computed below, of use for negative x
 __device__ __host__ __forceinline__ double pow_special(double x, double y, double r) {
+#pragma clang fp contract(off)
   const double inf = __builtin_huge_val(), ax = fabs(x);
   if (x == 1.0 || y == 0.0) return 1.0;
   if (x != x || y != y) return x + y;
@@ -180,6 +194,7 @@ __device__ __host__ __forceinline__ double pow_special(double x, double y, doubl
 // exact, the plain product: it overflows or vanishes as the power does.
 template <int n>
 __device__ __host__ __forceinline__ dd pow_whole_dd(double x) {
+#pragma clang fp contract(off)
   static_assert(n >= 1 && n <= 8, "small whole exponents");
   if constexpr (n == 1) return {x, 0.0};
   else if constexpr (n % 2 == 0) {
@@ -194,6 +209,7 @@ __device__ __host__ __forceinline__ dd pow_whole_dd(double x) {
 }
 template <int n>
 __device__ __host__ __forceinline__ double pow_whole(double x) {
+#pragma clang fp contract(off)
   if constexpr (n < 0) {
     const dd d = pow_whole_dd<-n>(x);
     const double q = 1.0 / d.hi;
@@ -208,6 +224,7 @@ __device__ __host__ __forceinline__ double pow_whole(double x) {
 // x^(n + 1/2), and its inverse: the square root with its residual, times x^n
 template <int n, bool kInverse = false>
 __device__ __host__ __forceinline__ double pow_half(double x) {
+#pragma clang fp contract(off)
   const double s = sqrt(x);
   const double sl = fma(-s, s, x) * double(0.5f / float(s));
   const dd w = pow_whole_dd<n>(x);
@@ -224,6 +241,7 @@ __device__ __host__ __forceinline__ double pow_half(double x) {
 // last residual in double-double (relative error near 2^-95), times
 // x^-1.85e-17 = 1 - 1.85e-17 log x.  Of use for positive finite x.
 __device__ __host__ __forceinline__ dd pow_third_dd(double x, int& q) {
+#pragma clang fp contract(off)
   int e;
   double m = frexp(x, &e);
   q = int(float(e + 1200) * (1.0f / 3.0f)) - 400;  // near e/3: m 2^(e - 3q) lies in [1/4, 8)
@@ -248,6 +266,7 @@ __device__ __host__ __forceinline__ dd pow_third_dd(double x, int& q) {
 }
 
 __device__ __host__ __forceinline__ double pow_cr(double x, double y) {
+#pragma clang fp contract(off)
   // exponents known to the compiler
   if (__builtin_constant_p(y) && y == 1.0 / 3.0) {
     int q;

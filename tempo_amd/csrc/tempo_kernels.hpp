@@ -1028,13 +1028,16 @@ __global__ void __launch_bounds__(128) k_phase_b(StepArgs<R> a, W_t<R>* vtbuf) {
 // find_melting_level (src/module_mp_tempo_diags.F90:124-141) on the state
 // the final update will check: rain present at a level above freezing with
 // snow or graupel present at the level above; presence as the final
-// checks decide it (mass after the step's tendencies above r1).  One lane
-// per column, before the final update.
+// checks decide it (mass after the step's tendencies above r1).  Before the
+// final update, in blocks of 64 columns x 4 waves that test every fourth
+// level from the top (the answer is the highest such level).
 template <class R>
 __global__ void __launch_bounds__(256) k_melt_level(StepArgs<R> a) {
-  const int c = int(blockIdx.x * blockDim.x + threadIdx.x);
-  if (c >= a.ncol || (a.cf[c] & CF_EXIT)) return;
-  const int nzc = a.nlev ? min(max(a.nlev[c], 1), a.nz) : a.nz;
+  __shared__ int found[4][64];
+  const int lane = int(threadIdx.x & 63u), w = int(threadIdx.x >> 6);
+  const int c = int(blockIdx.x) * 64 + lane;
+  const bool in = c < a.ncol && !(a.cf[c] & CF_EXIT);
+  const int nzc = !in ? 0 : a.nlev ? min(max(a.nlev[c], 1), a.nz) : a.nz;
   const R dt = R(a.dt);
   const size_t plane = a.plane;
   auto present = [&](int f, int ten, int k) {
@@ -1042,15 +1045,17 @@ __global__ void __launch_bounds__(256) k_melt_level(StepArgs<R> a) {
     return a.fa[f][o] + R(a.sd[size_t(ten) * plane + s]) * dt > R(kR1);
   };
   int k_melt = 1;
-  for (int k = nzc - 2; k >= 0; --k) {
+  for (int k = nzc - 2 - w; k >= 0; k -= 4) {
     const R temp = a.sr[SR_TEMP * plane + TEMPO_IDX_SCR(a, c, k)];
     if (temp > R(kT0) && present(F_QR, SD_QRTEN, k) &&
         (present(F_QS, SD_QSTEN, k + 1) || present(F_QG, SD_QGTEN, k + 1))) {
-      k_melt = max(k + 2, k_melt);
+      k_melt = k + 2;
       break;
     }
   }
-  a.kmelt[c] = k_melt;
+  found[w][lane] = k_melt;
+  __syncthreads();
+  if (w == 0 && in) a.kmelt[c] = max(max(found[0][lane], found[1][lane]), max(found[2][lane], found[3][lane]));
 }
 
 // a level below the column's melting level, where reflectivity_10cm takes
@@ -1065,52 +1070,79 @@ __device__ __forceinline__ bool melt_level(const StepArgs<R>& a, int c, int k) {
 // operands), dry rain and the binned wet-particle reflectivity of snow and
 // graupel.  Its own launch, before the final update (which leaves these
 // levels' reflectivity to it), so that the final update keeps its register
-// budget.
+// budget.  Each thread of a block of 64 columns x 4 levels prepares its
+// point; the points that melt are listed in LDS, the block's wavefronts take
+// them in turn with a bin per lane, and each thread finishes its own.
 template <class R>
 __global__ void __launch_bounds__(256) k_melt_refl(StepArgs<R> a) {
-  const int c = int(blockIdx.x) * 64 + int(threadIdx.x & 63u);
-  const int k = int(blockIdx.y) * int(blockDim.x >> 6) + int(threadIdx.x >> 6);
-  if (c >= a.ncol || k >= a.nz) return;
-  if ((a.nlev && k >= a.nlev[c]) || (a.cf[c] & CF_EXIT) || !melt_level(a, c, k)) return;
+  __shared__ radar::Wet pts[256];
+  __shared__ double ze[2][256];
+  __shared__ unsigned short list[256];
+  __shared__ int count;
+  const int tid = int(threadIdx.x);
+  const int c = int(blockIdx.x) * 64 + (tid & 63), k = int(blockIdx.y) * int(blockDim.x >> 6) + (tid >> 6);
+  const bool on = c < a.ncol && k < a.nz && !(a.nlev && k >= a.nlev[c]) && !(a.cf[c] & CF_EXIT) && melt_level(a, c, k);
+  if (tid == 0) count = 0;
+  if (!__syncthreads_or(on)) return;
   const Const<S_t<R>>& C = *a.cst;
-  const size_t o = TEMPO_IDX_STATE(a, c, k), s = TEMPO_IDX_SCR(a, c, k), plane = a.plane;
-  const R dt = R(a.dt), odt = R(a.odt);
-  const bool has_ngqb = a.f[F_NG] && a.f[F_QB];
-  Lvl<R> L;
-  L.temp = a.sr[SR_TEMP * plane + s];
-  L.qv = a.sr[SR_QV * plane + s];
-  L.pres = a.f[F_P][o];
-  L.rho = rho_of(C, L.pres, L.temp, L.qv);
-  L.qrten = R(a.sd[SD_QRTEN * plane + s]);
-  L.nrten = R(a.sd[SD_NRTEN * plane + s]);
-  L.qsten = R(a.sd[SD_QSTEN * plane + s]);
-  L.qgten = R(a.sd[SD_QGTEN * plane + s]);
-  L.ngten = R(a.sd[SD_NGTEN * plane + s]);
-  L.qbten = R(a.sd[SD_QBTEN * plane + s]);
-  R qr1d = a.fa[F_QR][o], nr1d = a.fa[F_NR][o], qs1d = a.fa[F_QS][o], qg1d = a.fa[F_QG][o];
-  R ng1d = has_ngqb ? a.fa[F_NG][o] : R(0), qb1d = has_ngqb ? a.fa[F_QB][o] : R(0);
-  rain_check(C, L, qr1d, nr1d, dt, odt);
-  snow_check(L, qs1d, dt, odt);
-  L.smob = L.smoc = R(0);
-  if (L.l_qs) snow_moments(C, L.rs, mn(R(-0.1), L.temp - R(kT0)), 0, L);
-  graupel_check(C, L, qg1d, ng1d, qb1d, has_ngqb, dt, odt);
-  if (!(L.l_qs || L.l_qg)) return;
-  constexpr bool kCR = sizeof(S_t<R>) == 8;
   R ze_r = R(1.e-22), ze_s = R(1.e-22), ze_g = R(1.e-22);
-  if (L.l_qr) {
-    const R lamr = R(1.0) / L.ilamr;
-    const R n0_r = L.nr * C.org2 * mpow(lamr, R(kCre[1]));
-    ze_r = n0_r * C.crg[3] * mpow(L.ilamr, R(kCre[3]));
+  bool wet = false, wet_s = false, wet_g = false;
+  if (on) {
+    const size_t o = TEMPO_IDX_STATE(a, c, k), s = TEMPO_IDX_SCR(a, c, k), plane = a.plane;
+    const R dt = R(a.dt), odt = R(a.odt);
+    const bool has_ngqb = a.f[F_NG] && a.f[F_QB];
+    Lvl<R> L;
+    L.temp = a.sr[SR_TEMP * plane + s];
+    L.qv = a.sr[SR_QV * plane + s];
+    L.pres = a.f[F_P][o];
+    L.rho = rho_of(C, L.pres, L.temp, L.qv);
+    L.qrten = R(a.sd[SD_QRTEN * plane + s]);
+    L.nrten = R(a.sd[SD_NRTEN * plane + s]);
+    L.qsten = R(a.sd[SD_QSTEN * plane + s]);
+    L.qgten = R(a.sd[SD_QGTEN * plane + s]);
+    L.ngten = R(a.sd[SD_NGTEN * plane + s]);
+    L.qbten = R(a.sd[SD_QBTEN * plane + s]);
+    R qr1d = a.fa[F_QR][o], nr1d = a.fa[F_NR][o], qs1d = a.fa[F_QS][o], qg1d = a.fa[F_QG][o];
+    R ng1d = has_ngqb ? a.fa[F_NG][o] : R(0), qb1d = has_ngqb ? a.fa[F_QB][o] : R(0);
+    rain_check(C, L, qr1d, nr1d, dt, odt);
+    snow_check(L, qs1d, dt, odt);
+    L.smob = L.smoc = R(0);
+    if (L.l_qs) snow_moments(C, L.rs, mn(R(-0.1), L.temp - R(kT0)), 0, L);
+    graupel_check(C, L, qg1d, ng1d, qb1d, has_ngqb, dt, odt);
+    wet_s = L.l_qs;
+    wet_g = L.l_qg;
+    wet = wet_s || wet_g;
+    if (wet) {
+      if (L.l_qr) {
+        const R lamr = R(1.0) / L.ilamr;
+        const R n0_r = L.nr * C.org2 * mpow(lamr, R(kCre[1]));
+        ze_r = n0_r * C.crg[3] * mpow(L.ilamr, R(kCre[3]));
+      }
+      pts[tid] = radar::Wet{double(value(L.rs)), double(value(L.smob)), double(value(L.smoc)), double(value(L.rr)),
+                            double(value(L.rg)), double(value(L.ng)), double(value(L.ilamg)),
+                            double(C.am_g[L.idx_bg - 1]), L.idx_bg};
+      list[atomicAdd(&count, 1)] = static_cast<unsigned short>(tid | (wet_s ? 0x4000 : 0) | (wet_g ? 0x8000 : 0));
+    }
   }
-  if (L.l_qs)
-    ze_s = R(S_t<R>(radar::melting_snow<kCR>(*a.radar, double(value(L.rs)), double(value(L.smob)),
-                                             double(value(L.smoc)), double(value(L.rr)))));
-  if (L.l_qg) {
-    const int idx = L.idx_bg;
-    ze_g = R(S_t<R>(radar::melting_graupel<kCR>(*a.radar, double(C.am_g[idx - 1]), double(C.ogg2),
-                                                kCge1, double(value(L.rg)), double(value(L.ng)),
-                                                double(value(L.ilamg)), idx, double(value(L.rr)))));
+  __syncthreads();
+  constexpr bool kCR = sizeof(S_t<R>) == 8;
+  const int n = count;
+  for (int i = tid >> 6; i < n; i += int(blockDim.x >> 6)) {
+    const int e = __builtin_amdgcn_readfirstlane(int(list[i])), t = e & 0xff;
+    const radar::Wet p = pts[t];
+    if (e & 0x4000) {
+      const double z = radar::melting_snow<kCR>(*a.radar, p);
+      if ((tid & 63) == 0) ze[0][t] = z;
+    }
+    if (e & 0x8000) {
+      const double z = radar::melting_graupel<kCR>(*a.radar, double(C.ogg2), kCge1, p);
+      if ((tid & 63) == 0) ze[1][t] = z;
+    }
   }
+  __syncthreads();
+  if (!wet) return;
+  if (wet_s) ze_s = R(S_t<R>(ze[0][tid]));
+  if (wet_g) ze_g = R(S_t<R>(ze[1][tid]));
   const size_t d3 = size_t(c % a.ni) + size_t(k) * a.dldk + size_t(c / a.ni) * a.dldj;
   a.d3[D3_REFL][d3] = mx(R(-35.0), R(10.0) * mlog10((ze_r + ze_s + ze_g) * R(1.e18)));
 }

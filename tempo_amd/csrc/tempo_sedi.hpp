@@ -312,7 +312,7 @@ __device__ __forceinline__ double wave_sediment(const SedCol<CH>& g, double (&xr
 // Arrays that are read at other levels live in LDS rows of the column (kSemiRows
 // of nz + 2 doubles): a column's work needs about 30 loads from them per
 // level, which in global memory, one lane per column, took 2.43 ms for
-// 10,007 columns of 59 levels (157 wavefronts on 256 CUs); here 0.15 ms.
+// 10,007 columns of 59 levels (157 wavefronts on 256 CUs); here 0.25 ms.
 constexpr int kSemiLevels = 128;  // the tile's and these rows' LDS: 119 KB in FP64 at 128 levels
 enum SemiRow { SW_ZI, SW_ZA, SW_DZA, SW_QA, SW_QMI, SW_QPI, kSemiRows };
 __host__ __device__ constexpr int semi_row(int nz) { return nz + 2; }
@@ -1018,7 +1018,7 @@ hipError_t launch_step_impl(const StepArgs<T>& a, const StepArgs<RA>& ga, const 
   else
     hipLaunchKernelGGL(k_phase_b<T>, dim3(unsigned((a.ncol + 127) / 128)), dim3(128), 0, s, a, vtbuf);
   if (a.fl.refl_from_melting && a.fl.refl10cm && a.d3[D3_REFL]) {
-    hipLaunchKernelGGL(k_melt_level<T>, dim3(unsigned((a.ncol + 255) / 256)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_melt_level<T>, dim3(unsigned((a.ncol + 63) / 64)), dim3(256), 0, s, a);
     hipLaunchKernelGGL(k_melt_refl<T>, level_grid(a, 256), dim3(256), 0, s, a);
   }
   if (ev) (void)hipEventRecord(ev[3], s);

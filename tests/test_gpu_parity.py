@@ -1267,3 +1267,26 @@ def test_gpu_semi_lagrangian_level_counts(hip, dtype, hail, nz):
         ctx.tune(prec, hip.TUNE_SED_WAVE, 1)
     for k, v in got[1].items():
         assert np.array_equal(v, got[0][k], equal_nan=True), (k, nz)
+
+
+@pytest.mark.parametrize("ncol", [1, 63, 65, 200])
+def test_gpu_melting_points_of_a_block(hip, gpu_tables, ncol):
+    """melting-layer reflectivity where a block's 64 x 4 points melt all, in
+    part or not at all (every level from the ground up to the freezing level
+    wet in the even columns, every third column dry, the last block cut
+    short): FP64 path vs the oracle"""
+    from oracle import oracle as orc
+    from tempo_amd import generator as gen
+    flags = dict(aerosolaware=True, hailaware=True, refl_from_melting=True)
+    st, m = gen.generate("multistep", ncol=ncol, col0=31_000)
+    wet = np.zeros_like(st["p"], bool)
+    wet[:30, ::2] = True
+    wet[:, ::3] = False
+    for k, v in (("qr", 2e-4), ("qs", 1e-4), ("qg", 3e-4), ("nr", 400.0), ("ng", 150.0), ("qb", 6e-4)):
+        st[k] = np.where(wet, v, np.where(np.arange(ncol)[None, :] % 3 == 0, 0.0, st[k]))
+    ctx = context(hip, flags)
+    _, d = gpu_run(ctx, st, m["dt"], m["itimestep"])
+    orc.init(gpu_tables, **flags)
+    want = {k: v.copy() for k, v in st.items()}
+    _, d3 = orc.run(want, m["dt"], m["itimestep"])
+    assert rel_inf(d["refl10cm"], d3["refl10cm"]) <= 1e-12, rel_inf(d["refl10cm"], d3["refl10cm"])
