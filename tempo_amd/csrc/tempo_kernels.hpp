@@ -54,33 +54,44 @@ __device__ __forceinline__ R column_nc(const StepArgs<R>& a, int c) {
 }
 
 // ------------------------------------------------------------ pre-pass ----
-// Blocks of 64 columns x 4 waves: wave w tests levels w, w + 4, ... of its
-// lane's column, so that every load is one coalesced row of 64 columns and
-// the chip holds four times as many waves as columns/64; the waves' answers
-// are combined through LDS.  The tests are ORs over levels, so their order
-// does not matter; the first-step sums and the height prefix keep the
-// reference's sequential order in wave 0.
-constexpr int kPrepassCols = 64;
+// Blocks of 64 columns x n waves: wave w tests levels w, w + n, ... of its
+// lane's column, so that every load is one coalesced row of 64 columns; the
+// waves' answers are combined through LDS.  The tests are ORs over levels, so
+// their order does not matter.  The kernel waits for memory: a column's test
+// is a chain of up to nz/n dependent rounds of loads, ended by the first
+// level that answers it.  n = 16 where 64-column blocks leave CUs idle, and
+// where they fill the chip n = 4, which reads fewer levels past the first
+// answer (100,000 x 90: 27 us against 47; 1,024 x 60, height prefix
+// included: 7 us against 22).  The first-step sums and the height
+// prefix keep the reference's sequential order, in wave 0; the layer depths
+// reach it, and the heights leave it, through LDS with all waves loading and
+// storing.
+constexpr int kPrepassCols = 64, kPrepassWaves = 16;
 template <class R>
-__global__ void __launch_bounds__(256) k_prepass(StepArgs<R> a) {
-  __shared__ unsigned char flag[4][kPrepassCols];
-  const int lane = int(threadIdx.x & 63u), w = int(threadIdx.x >> 6);
+__global__ void __launch_bounds__(64 * kPrepassWaves) k_prepass(StepArgs<R> a) {
+  __shared__ unsigned flag[kPrepassCols];
+  constexpr int kRows = sizeof(R) > 8 ? 32 : 64;
+  __shared__ alignas(16) unsigned char mem[kRows * kPrepassCols * sizeof(R)];
+  R(*row)[kPrepassCols] = reinterpret_cast<R(*)[kPrepassCols]>(mem);
+  const int lane = int(threadIdx.x & 63u), w = int(threadIdx.x >> 6), nw = int(blockDim.x >> 6);
   const int c = int(blockIdx.x) * kPrepassCols + lane;
   const bool in = c < a.ncol;
   const int nzc = !in ? 0 : a.nlev ? min(max(a.nlev[c], 1), a.nz) : a.nz;
+  if (w == 0) flag[lane] = 0u;
+  __syncthreads();
   // early exit (:416-418): any hydrometeor above r1 after the initial checks
   // (tendencies are still zero, so l_q == q1d > r1), or ice supersaturation
   bool q = false;
-  for (int k = w; k < nzc && !q; k += 4) {
+  for (int k = w; k < nzc && !q; k += nw) {
     const size_t o = TEMPO_IDX_STATE(a, c, k);
-    q = a.f[F_QC][o] > R(kR1) || a.f[F_QR][o] > R(kR1) || a.f[F_QI][o] > R(kR1) || a.f[F_QS][o] > R(kR1) ||
-        a.f[F_QG][o] > R(kR1);
+    const R qc = a.f[F_QC][o], qr = a.f[F_QR][o], qi = a.f[F_QI][o], qs = a.f[F_QS][o], qg = a.f[F_QG][o];
+    q = (qc > R(kR1)) | (qr > R(kR1)) | (qi > R(kR1)) | (qs > R(kR1)) | (qg > R(kR1));
   }
-  flag[w][lane] = q;
+  if (q) flag[lane] = 1u;
   __syncthreads();
-  const bool any_q = flag[0][lane] | flag[1][lane] | flag[2][lane] | flag[3][lane];
+  const bool any_q = flag[lane] != 0u;
   bool sup = false;
-  for (int k = w; !any_q && k < nzc && !sup; k += 4) {
+  for (int k = w; !any_q && k < nzc && !sup; k += nw) {
     const size_t o = TEMPO_IDX_STATE(a, c, k);
     const R temp = load_t(a, o), pres = a.f[F_P][o], qv = mx(R(kMinQv), a.f[F_QV][o]);
     const R qvs = rslf(pres, temp);
@@ -90,11 +101,28 @@ __global__ void __launch_bounds__(256) k_prepass(StepArgs<R> a) {
     sup = ssati > R(0.0);
   }
   __syncthreads();  // every wave has read the first answers
-  flag[w][lane] = sup;
+  if (sup) flag[lane] = 1u;
   __syncthreads();
+  // height prefix of the default aerosol profile (src/module_mp_tempo_aerosols.F90:24-28)
+  if (!a.f[F_NWFA] || !a.f[F_NIFA]) {
+    R h = R(0);
+    for (int k0 = 0; k0 < a.nz; k0 += kRows) {
+      const int n = min(kRows, nzc - k0);
+      for (int i = w; i < n; i += nw) row[i][lane] = a.f[F_DZ][TEMPO_IDX_STATE(a, c, k0 + i)];
+      __syncthreads();
+      if (w == 0)
+        for (int i = 0; i < n; ++i) {
+          if (k0 + i > 0) h = h + row[i][lane];
+          row[i][lane] = h;
+        }
+      __syncthreads();
+      for (int i = w; i < n; i += nw) a.sr[size_t(SR_HGT) * a.plane + TEMPO_IDX_SCR(a, c, k0 + i)] = row[i][lane];
+      __syncthreads();
+    }
+  }
   if (w != 0 || !in) return;
   unsigned cf = 0;
-  if (!any_q && !(flag[0][lane] | flag[1][lane] | flag[2][lane] | flag[3][lane])) cf |= CF_EXIT;
+  if (!flag[lane]) cf |= CF_EXIT;
   // first-step graupel initialisation test (:387-393)
   if (a.first_step && a.f[F_NG] && a.f[F_QB]) {
     R sqg = R(0), sng = R(0), sqb = R(0);
@@ -106,19 +134,12 @@ __global__ void __launch_bounds__(256) k_prepass(StepArgs<R> a) {
     }
     if (sqg > R(kR1) && sng < R(kEps) && sqb < R(kEps)) cf |= CF_GINIT;
   }
-  // height prefix of the default aerosol profile (src/module_mp_tempo_aerosols.F90:24-28)
-  if (!a.f[F_NWFA] || !a.f[F_NIFA]) {
-    R h = R(0);
-    for (int k = 0; k < nzc; ++k) {
-      if (k > 0) h = h + a.f[F_DZ][TEMPO_IDX_STATE(a, c, k)];
-      a.sr[size_t(SR_HGT) * a.plane + TEMPO_IDX_SCR(a, c, k)] = h;
-    }
-  }
   a.cf[c] = cf;
 }
 template <class R>
-dim3 prepass_grid(const StepArgs<R>& a) {
-  return dim3(unsigned((a.ncol + kPrepassCols - 1) / kPrepassCols));
+void launch_prepass(const StepArgs<R>& a, hipStream_t s) {
+  const int blocks = (a.ncol + kPrepassCols - 1) / kPrepassCols;
+  hipLaunchKernelGGL(k_prepass<R>, dim3(unsigned(blocks)), dim3(64 * (blocks >= 1024 ? 4 : kPrepassWaves)), 0, s, a);
 }
 
 // ------------------------------------------------ point grouping ----
@@ -1515,7 +1536,7 @@ hipError_t launch_dual_unpack(const Dual<T>* in, const DualGeom& g, T* v, T* t, 
 // the four launches of one tangent-linear step (sedimentation one lane per column)
 template <class D>
 hipError_t launch_step_tlm_impl(const StepArgs<D>& a, Dual<double>* vtbuf, hipStream_t s) {
-  hipLaunchKernelGGL(k_prepass<D>, prepass_grid(a), dim3(256), 0, s, a);
+  launch_prepass(a, s);
   hipLaunchKernelGGL(k_phase_a<D>, level_grid(a, 256), dim3(256), 0, s, a);
   hipLaunchKernelGGL(k_phase_b<D>, dim3(unsigned((a.ncol + 127) / 128)), dim3(128), 0, s, a, vtbuf);
   hipLaunchKernelGGL(k_phase_c<D>, level_grid(a, 256), dim3(256), 0, s, a);

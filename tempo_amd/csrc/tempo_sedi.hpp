@@ -1000,7 +1000,7 @@ template <class T, class RA>
 hipError_t launch_step_impl(const StepArgs<T>& a, const StepArgs<RA>& ga, const LaunchCfg& lc, double* vtbuf,
                             hipStream_t s, hipEvent_t* ev) {
   if (ev) (void)hipEventRecord(ev[0], s);
-  hipLaunchKernelGGL(k_prepass<T>, prepass_grid(a), dim3(256), 0, s, a);
+  launch_prepass(a, s);
   if (ev) (void)hipEventRecord(ev[1], s);
   if (lc.waves_a && std::is_same<RA, T>::value)
     hipLaunchKernelGGL((k_phase_a<RA, WavesPerEu<RA>::a_alt>), level_grid(a, lc.block_a), dim3(unsigned(lc.block_a)),

@@ -1290,3 +1290,26 @@ def test_gpu_melting_points_of_a_block(hip, gpu_tables, ncol):
     want = {k: v.copy() for k, v in st.items()}
     _, d3 = orc.run(want, m["dt"], m["itimestep"])
     assert rel_inf(d["refl10cm"], d3["refl10cm"]) <= 1e-12, rel_inf(d["refl10cm"], d3["refl10cm"])
+
+
+@pytest.mark.parametrize("workload", ["plain", "ragged"])
+def test_gpu_large_batch_equals_its_columns(hip, workload):
+    """the pre-pass takes 16 waves per 64 columns in small batches and 4 in
+    large ones: the last 131 columns of a batch of 65,601, and the same
+    columns alone, give the same bits (no aerosol fields: the heights of the
+    default profile are the pre-pass's; some columns without hydrometeors)"""
+    from tempo_amd import generator as gen
+    n, tail = 65_601, 131
+    ctx = context(hip, dict(aerosolaware=False, hailaware=workload == "ragged"))
+    st, m = gen.generate_torch(workload, ncol=n, dtype=torch.float32)
+    for q in ("qc", "qr", "qi", "qs", "qg"):
+        st[q][:, ::7] = 0.0
+    st["qv"][:, ::14] *= 0.5
+    small = {k: v[:, n - tail:].contiguous() for k, v in st.items()}
+    nlev = m.get("nlev")
+    d = ctx.run(st, m["dt"], 1, nlev=nlev)
+    e = ctx.run(small, m["dt"], 1, nlev=None if nlev is None else nlev[n - tail:].contiguous())
+    for k, v in small.items():
+        assert torch.equal(st[k][:, n - tail:], v), k
+    for k, v in e.items():
+        assert torch.equal(d[k][..., n - tail:], v), k
