@@ -133,6 +133,8 @@ template <class R>
 __global__ void __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(FusedWaves<R>::n)))
 k_step_fused(StepArgs<R> a) {
   extern __shared__ double tile_mem[];  // sed_lds_bytes<SedStage<R>>(nz)
+  pow10_fill<S_t<R>>();
+  __syncthreads();
   __shared__ int item_s;
   __shared__ int nzc_s[kSedCols];
   const int tid = int(threadIdx.x), w = tid >> 6;

@@ -380,8 +380,10 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>
   R vtboost = R(1.0);
   if (micro) {
     warm_rain(C, a.tab, L, t, odt);
-    rain_snow_graupel(C, a.tab, L, t, odt);
-    ice_nucleation(C, a.tab, L, t, has_nwfa, has_nifa, w, dt, odt);
+    int ir = 1, ir1 = 1;
+    if (needs_rain_index(L)) rain_index(C, L.rr, L.ilamr, ir, ir1);
+    rain_snow_graupel(C, a.tab, L, t, odt, ir, ir1);
+    ice_nucleation(C, a.tab, L, t, has_nwfa, has_nifa, w, dt, odt, ir, ir1);
     const R t1s = t1_subl(C, L);
     ice_processes(C, a.tab, L, t, t1s, w, odt);
     vtboost = riming(C, a.tab, L, t, odt);
@@ -533,11 +535,12 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>
 template <class R, int kWaves = WavesPerEu<R>::a>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) k_phase_a(StepArgs<R> a) {
   __shared__ float ccn_s[kCcnSlice];
+  pow10_fill<S_t<R>>();
   if (a.ccn_lds) {
     for (int i = int(threadIdx.x); i < kCcnSlice; i += int(blockDim.x)) ccn_s[i] = a.tab.ccn[i];
-    __syncthreads();
     a.tab.ccn = ccn_s;
   }
+  __syncthreads();
   const int2 pt = block_point<R, false>(a);
   const int c = pt.x, k = pt.y;
   if (c >= a.ncol || k >= a.nz) return;

@@ -843,16 +843,40 @@ __device__ void graupel_check(const Const<T>& C, Lvl<Sig<T>>& L, Sig<T>& qg1d, S
 }
 
 // ---- table indices (src/module_mp_tempo_main.F90:2493-2635, 2839-2858) ----
+// 10**n for n = -kPow10..kPow10-1 as powi forms it, in LDS: the decade search
+// below divides by it two or three times per index, and a point with rain,
+// snow, graupel, ice and cloud looks up some ten indices.  Forming each power
+// by repeated squaring took about half of a cloudy wavefront's instructions.
+constexpr int kPow10 = 32;
+template <class S>
+__device__ __forceinline__ S* pow10_table() {
+  __shared__ S table[2 * kPow10];
+  return table;
+}
+// by the block's first threads; the caller has the block wait before its use
+template <class S>
+__device__ __forceinline__ void pow10_fill() {
+  for (int i = int(threadIdx.x); i < 2 * kPow10; i += int(blockDim.x)) pow10_table<S>()[i] = powi(S(10.0), i - kPow10);
+}
+
+// first n of nx-1, nx, nx+1 (nx = nint(log10 x)) with 1 <= x/10**n < 10, else
+// nx+1; nx is held to the table's range, far outside which the index has
+// long reached 1 or nmax
 template <class R>
 __device__ __forceinline__ int decade_index(R x, int base, int nmax) {
-  const int nx = nint_exact(mlog10(x));
-  int n = nx + 1;
-  for (int nn = nx - 1; nn <= nx + 1; ++nn) {
-    n = nn;
-    const R q = x / powi(R(10.0), nn);
-    if (q >= R(1.0) && q < R(10.0)) break;
+  const S_t<R>* p10 = pow10_table<S_t<R>>() + kPow10;
+  const int nx = max(2 - kPow10, min(nint_exact(mlog10(x)), kPow10 - 2));
+  int n = nx - 1;
+  R q = x / R(p10[n]);
+  if (!(q >= R(1.0) && q < R(10.0))) {
+    n = nx;
+    q = x / R(p10[n]);
+    if (!(q >= R(1.0) && q < R(10.0))) {
+      n = nx + 1;
+      q = x / R(p10[n]);
+    }
   }
-  const int idx = int(x / powi(R(10.0), n)) + 10 * (n - base) - (n - base);
+  const int idx = int(q) + 10 * (n - base) - (n - base);
   return max(1, min(idx, nmax));
 }
 
@@ -865,7 +889,7 @@ __device__ __forceinline__ int temperature_index(R tempk) {
 }
 
 template <class R>
-__device__ void rain_index(const Const<S_t<R>>& C, R rr, R ilamr, int& ir, int& ir1) {
+__device__ __forceinline__ void rain_index(const Const<S_t<R>>& C, R rr, R ilamr, int& ir, int& ir1) {
   ir = decade_index(rr, C.nir2, kNtbR);
   const R lamr = R(1.) / ilamr;
   const R lam_exp = lamr * mpow(C.crg[2] * C.org2 * C.org1, R(kBmR));
@@ -929,13 +953,21 @@ __device__ __forceinline__ void warm_rain(const Const<S_t<R>>& C, const Tables<S
   }
 }
 
+// whether rain_snow_graupel or ice_nucleation looks up a table by the rain
+// content (ir, ir1 of rain_index, formed once for all of them)
+template <class R>
+__device__ __forceinline__ bool needs_rain_index(const Lvl<R>& L) {
+  using S = S_t<R>;
+  if (!L.l_qr || !(value(L.rr) >= S(1.e-6))) return false;
+  return value(L.temp) < S(kT0) || (L.l_qs && value(L.rs) >= S(1.e-6)) || (L.l_qg && value(L.rg) >= S(1.e-6));
+}
+
 // rain_snow_rain_graupel (:2638-2727)
 template <class R>
-__device__ __forceinline__ void rain_snow_graupel(const Const<S_t<R>>& C, const Tables<S_t<R>>& T, const Lvl<R>& L, Tend<R>& t, R odt) {
+__device__ __forceinline__ void rain_snow_graupel(const Const<S_t<R>>& C, const Tables<S_t<R>>& T, const Lvl<R>& L, Tend<R>& t, R odt,
+                                  int ir, int ir1) {
   if (L.l_qr && L.l_qs && L.rr >= R(1.e-6) && L.rs >= R(1.e-6)) {
     const int it = temperature_index(L.temp);
-    int ir, ir1;
-    rain_index(C, L.rr, L.ilamr, ir, ir1);
     const int is = decade_index(L.rs, C.nis2, kNtbS);
     const size_t e = size_t(is - 1) + kNtbS * (size_t(it - 1) + kNtbT * (size_t(ir1 - 1) + kNtbR1 * size_t(ir - 1)));
     const S_t<R>* q = T.qs + e * 12;
@@ -959,9 +991,8 @@ __device__ __forceinline__ void rain_snow_graupel(const Const<S_t<R>>& C, const 
     }
   }
   if (L.l_qr && L.l_qg && L.rr >= R(1.e-6) && L.rg >= R(1.e-6)) {
-    int ir, ir1, ig, ig1;
+    int ig, ig1;
     const int idx = L.idx_bg;
-    rain_index(C, L.rr, L.ilamr, ir, ir1);
     graupel_index(C, L.rg, L.ilamg, idx, ig, ig1);
     const size_t e = size_t(ig1 - 1) +
                      kNtbG1 * (size_t(ig - 1) + kNtbG * (size_t(idx - 1) + kNrhg * (size_t(ir1 - 1) + kNtbR1 * size_t(ir - 1))));
@@ -1010,7 +1041,7 @@ __device__ R koop(const Const<S_t<R>>& C, R temp, R satw, R naero, R dt) {
 // ice_nucleation (:2730-2820)
 template <class R>
 __device__ __forceinline__ void ice_nucleation(const Const<S_t<R>>& C, const Tables<S_t<R>>& T, const Lvl<R>& L, Tend<R>& t, bool has_nwfa,
-                               bool has_nifa, R w, R dt, R odt) {
+                               bool has_nifa, R w, R dt, R odt, int ir, int ir1) {
   if (!(L.temp < R(kT0))) return;
   const R tempc = L.temp - R(kT0);
   const int idx_tc = max(1, min(nint_exact(-tempc), kNtbT1));
@@ -1018,8 +1049,6 @@ __device__ __forceinline__ void ice_nucleation(const Const<S_t<R>>& C, const Tab
   R xni = has_nifa ? demott(C, tempc, L.rho, L.nifa) : R(1.0) * R(1000.0);
   const int idx_in = (xni > R(1.0)) ? decade_index(xni, C.niin2, kNtbIn) : 1;
   if (L.rr > R(1.e-6)) {
-    int ir, ir1;
-    rain_index(C, L.rr, L.ilamr, ir, ir1);
     const size_t e = size_t(ir - 1) + kNtbR * (size_t(ir1 - 1) + kNtbR1 * (size_t(idx_tc - 1) + kNtbT1 * size_t(idx_in - 1)));
     const S_t<R>* q = T.fzr + e * 4;  // tpi_qrfz tni_qrfz tpg_qrfz tnr_qrfz
     t.prg_rfz = q[2] * odt;
