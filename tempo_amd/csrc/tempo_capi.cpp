@@ -133,10 +133,10 @@ hipError_t upload(DevBuf& b, const std::vector<T>& v) {
 // Const<double> -> Const<float>: the R-typed members form one contiguous
 // prefix followed by the int members.
 void narrow(const Const<double>& d, Const<float>& f) {
-  constexpr size_t nr = offsetof(Const<double>, nic2) / sizeof(double);
-  static_assert(offsetof(Const<float>, nic2) == nr * sizeof(float), "Const layout");
+  static_assert(sizeof(LaneConst<double>) == 2 * sizeof(LaneConst<float>), "LaneConst layout");
   const double* src = reinterpret_cast<const double*>(&d);
   float* dst = reinterpret_cast<float*>(&f);
+  const size_t nr = size_t(reinterpret_cast<const double*>(&d.nic2) - src);
   for (size_t i = 0; i < nr; ++i) dst[i] = float(src[i]);
   std::memcpy(&f.nic2, &d.nic2, sizeof(int) * 10);
 }

@@ -78,17 +78,25 @@ constexpr size_t kNFzC1 = size_t(kNtbC) * kNbins * kNtbT1 * kNtbIn;           //
 constexpr size_t kNCcn = size_t(kNtbArc) * kNtbArw * kNtbArt * kNtbArr * kNtbArk;
 constexpr int kNQsArr = 12, kNQgArr = 5, kNFzRArr = 4, kNFzCArr = 2;
 
+// Derived constants that a point picks by its graupel density index or its
+// cloud's shape index: read per lane, so kernels of many such reads keep a
+// copy in LDS (lane_const).
+template <class R>
+struct LaneConst {
+  R av_g[kNrhg], bv_g[kNrhg], am_g[kNrhg];
+  R cce[5][16], ccg[5][16], ocg1[16], ocg2[16];  // [a-1][n], n = 1..15 (index 0 unused)
+  R cge[12][kNrhg], cgg[12][kNrhg];
+};
+
 // Derived constants (gamma-function values, prefactors, bins) in precision R.
 template <class R>
-struct Const {
-  R av_g[kNrhg], bv_g[kNrhg], am_g[kNrhg];
+struct Const : LaneConst<R> {
   R am_i, am_r, ar_volume, lfus, olfus, roverrv, orv, rho_not, rho_not0, sc3;
   R d0i, obmi, obmr, obmg, oams;
-  R cce[5][16], ccg[5][16], ocg1[16], ocg2[16];  // [a-1][n], n = 1..15 (index 0 unused)
   R cie[7], cig[7], oig1, oig2;
   R cre[13], crg[13], ore1, org1, org2, org3;
   R cse[17], csg[17];
-  R cge[12][kNrhg], cgg[12][kNrhg], oge1, ogg1, ogg2, ogg3;
+  R oge1, ogg1, ogg2, ogg3;
   R t1_qr_qc, t1_qr_qi, t2_qr_qi, t1_qs_qc, t1_qs_qi, t1_qr_ev, t2_qr_ev;
   R t1_qs_sd, t2_qs_sd, t1_qs_me, t2_qs_me, t1_qg_sd, t1_qg_me;
   // snow moment regression, with the per-moment polynomial in the second

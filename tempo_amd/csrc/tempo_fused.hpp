@@ -134,6 +134,7 @@ __global__ void __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per
 k_step_fused(StepArgs<R> a) {
   extern __shared__ double tile_mem[];  // sed_lds_bytes<SedStage<R>>(nz)
   pow10_fill<S_t<R>>();
+  lane_const_fill(a.cst);
   __syncthreads();
   __shared__ int item_s;
   __shared__ int nzc_s[kSedCols];

@@ -274,12 +274,12 @@ struct SigScope<Sig<T>> {
 // rain_fallspeed (:1771-1774) and graupel_fallspeed (:1815-1832) of one level:
 // mass- and number-weighted speeds
 template <class R>
-__device__ __forceinline__ void rain_fallspeed(const Const<S_t<R>>& C, R rhof, R lamr, R& v1, R& v2) {
-  v1 = rhof * R(kAvR) * C.crg[5] * C.org3 * mpow(lamr, R(kCre[2])) * mpow(lamr + R(kFvR), -R(kCre[5]));
-  v2 = rhof * R(kAvR) * C.crg[6] / C.crg[11] * mpow(lamr, R(kCre[11])) * mpow(lamr + R(kFvR), -R(kCre[6]));
+__device__ __forceinline__ void rain_fallspeed(const ConstView<S_t<R>>& C, R rhof, R lamr, R& v1, R& v2) {
+  v1 = rhof * R(kAvR) * C.u.crg[5] * C.u.org3 * mpow(lamr, R(kCre[2])) * mpow(lamr + R(kFvR), -R(kCre[5]));
+  v2 = rhof * R(kAvR) * C.u.crg[6] / C.u.crg[11] * mpow(lamr, R(kCre[11])) * mpow(lamr + R(kFvR), -R(kCre[6]));
 }
 template <class R>
-__device__ __forceinline__ void graupel_fallspeed(const Const<S_t<R>>& C, const Lvl<R>& L, R rhof, R visco, bool has_qb,
+__device__ __forceinline__ void graupel_fallspeed(const ConstView<S_t<R>>& C, const Lvl<R>& L, R rhof, R visco, bool has_qb,
                                                   R& v1, R& v2) {
   R afall, bfall;
   if (has_qb) {
@@ -292,15 +292,15 @@ __device__ __forceinline__ void graupel_fallspeed(const Const<S_t<R>>& C, const 
     bfall = R(kBvGOld);
   }
   const int idx = L.idx_bg;
-  v1 = rhof * afall * C.cgg[5][idx - 1] * C.ogg3 * mpow(L.ilamg, bfall);
-  v2 = rhof * afall * C.cgg[6][idx - 1] / C.cgg[11][idx - 1] * mpow(L.ilamg, bfall);
+  v1 = rhof * afall * C.l.cgg[5][idx - 1] * C.u.ogg3 * mpow(L.ilamg, bfall);
+  v2 = rhof * afall * C.l.cgg[6][idx - 1] / C.l.cgg[11][idx - 1] * mpow(L.ilamg, bfall);
 }
 
 // the level-local physics of point (c, k), from the initial checks to the
 // fall speeds (src/module_mp_tempo_main.F90:320-588); scratch in scr
 template <class R>
 __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>& scr, int c, int k) {
-  const Const<S_t<R>>& C = *a.cst;
+  const ConstView<S_t<R>> C = lds_const_view(a.cst);
   const size_t o = TEMPO_IDX_STATE(a, c, k);
   const size_t s = scr.at(c, k);
   const size_t plane = scr.plane;
@@ -352,7 +352,7 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>
     const R rb = rg * R(kM3ToL) / rho_g<R>(kIdxBg1);
     const int idx = max(1, min(nint_exact(R(10.0) * rg / rb) + 1, kNrhg));
     const R lamg = (R(3.0) + R(kMuG) + R(0.672)) / R(5.e-3);
-    const R ng = C.cgg[1][0] * C.ogg3 * rg * mpow(lamg, R(kBmG)) / C.am_g[idx - 1];
+    const R ng = C.u.cgg[1][0] * C.u.ogg3 * rg * mpow(lamg, R(kBmG)) / C.l.am_g[idx - 1];
     ng1d = ng / L.rho;
     qb1d = rb / L.rho;
   }
@@ -460,13 +460,13 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>
     const R xds = L.smoc / L.smob;
     const R mrat = R(1.0) / xds;
     R ils1 = R(1.0) / (mrat * R(kLam0) + R(kFvS)), ils2 = R(1.0) / (mrat * R(kLam1) + R(kFvS));
-    const R t1v = R(kKap0) * C.csg[3] * mpow(ils1, C.cse[3]);
+    const R t1v = R(kKap0) * C.u.csg[3] * mpow(ils1, C.u.cse[3]);
     const R mm = mpow(mrat, R(kMuS));
-    const R t2v = R(kKap1) * mm * C.csg[9] * mpow(ils2, C.cse[9]);
+    const R t2v = R(kKap1) * mm * C.u.csg[9] * mpow(ils2, C.u.cse[9]);
     ils1 = R(1.0) / (mrat * R(kLam0));
     ils2 = R(1.0) / (mrat * R(kLam1));
-    const R t3v = R(kKap0) * C.csg[0] * mpow(ils1, C.cse[0]);
-    const R t4v = R(kKap1) * mm * C.csg[6] * mpow(ils2, C.cse[6]);
+    const R t3v = R(kKap0) * C.u.csg[0] * mpow(ils1, C.u.cse[0]);
+    const R t4v = R(kKap1) * mm * C.u.csg[6] * mpow(ils2, C.u.cse[6]);
     vts = L.rhof * R(kAvS) * (t1v + t2v) / (t3v + t4v);
     if (t.prr_sml > R(0.0))
       pf |= PF_SNOWMIX;
@@ -474,13 +474,13 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>
       vts = vts * vtboost;
   }
   if (L.ri > R(kR1)) {  // ice_fallspeed (:1928-1930)
-    vtri = L.rhof * R(kAvI) * C.cig[2] * C.oig2 * mpow(L.ilami, R(kBvI));
-    vtni = L.rhof * R(kAvI) * C.cig[5] / C.cig[6] * mpow(L.ilami, R(kBvI));
+    vtri = L.rhof * R(kAvI) * C.u.cig[2] * C.u.oig2 * mpow(L.ilami, R(kBvI));
+    vtni = L.rhof * R(kAvI) * C.u.cig[5] / C.u.cig[6] * mpow(L.ilami, R(kBvI));
   }
   if (L.rc > R(kR1) && w < R(0.1)) {  // cloud_fallspeed (:1971-1974)
     const int nu = get_nuc(L.nc);
-    vtrc = L.rhof * R(kAvC) * C.ccg[4][nu] * C.ocg2[nu] * mpow(L.ilamc, R(kBvC));
-    vtnc = L.rhof * R(kAvC) * C.ccg[3][nu] * C.ocg1[nu] * mpow(L.ilamc, R(kBvC));
+    vtrc = L.rhof * R(kAvC) * C.l.ccg[4][nu] * C.l.ocg2[nu] * mpow(L.ilamc, R(kBvC));
+    vtnc = L.rhof * R(kAvC) * C.l.ccg[3][nu] * C.l.ocg1[nu] * mpow(L.ilamc, R(kBvC));
   }
 
   R* sr = scr.sr;
@@ -536,6 +536,7 @@ template <class R, int kWaves = WavesPerEu<R>::a>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) k_phase_a(StepArgs<R> a) {
   __shared__ float ccn_s[kCcnSlice];
   pow10_fill<S_t<R>>();
+  lane_const_fill(a.cst);
   if (a.ccn_lds) {
     for (int i = int(threadIdx.x); i < kCcnSlice; i += int(blockDim.x)) ccn_s[i] = a.tab.ccn[i];
     a.tab.ccn = ccn_s;
@@ -806,7 +807,7 @@ template <class R>
 __device__ void semi_rain_refresh(const StepArgs<R>& a, int c, int nzc, W_t<R>* sd, W_t<R>* vt1, W_t<R>* vt2,
                                   SemiRec& rec) {
   using W = W_t<R>;
-  const Const<S_t<R>>& C = *a.cst;
+  const ConstView<S_t<R>> C = const_view(a.cst);
   const size_t plane = a.plane;
   const R* sr = a.sr;
   const R dt = R(a.dt), odt = R(a.odt);
@@ -839,7 +840,7 @@ template <class R>
 __device__ void semi_graupel_refresh(const StepArgs<R>& a, int c, int nzc, W_t<R>* sd, W_t<R>* vt1, W_t<R>* vt2,
                                      SemiRec& rec) {
   using W = W_t<R>;
-  const Const<S_t<R>>& C = *a.cst;
+  const ConstView<S_t<R>> C = const_view(a.cst);
   const size_t plane = a.plane;
   const R* sr = a.sr;
   const R dt = R(a.dt), odt = R(a.odt);
@@ -1108,7 +1109,7 @@ __global__ void __launch_bounds__(256) k_melt_refl(StepArgs<R> a) {
   const bool on = c < a.ncol && k < a.nz && !(a.nlev && k >= a.nlev[c]) && !(a.cf[c] & CF_EXIT) && melt_level(a, c, k);
   if (tid == 0) count = 0;
   if (!__syncthreads_or(on)) return;
-  const Const<S_t<R>>& C = *a.cst;
+  const ConstView<S_t<R>> C = const_view(a.cst);
   R ze_r = R(1.e-22), ze_s = R(1.e-22), ze_g = R(1.e-22);
   bool wet = false, wet_s = false, wet_g = false;
   if (on) {
@@ -1139,12 +1140,12 @@ __global__ void __launch_bounds__(256) k_melt_refl(StepArgs<R> a) {
     if (wet) {
       if (L.l_qr) {
         const R lamr = R(1.0) / L.ilamr;
-        const R n0_r = L.nr * C.org2 * mpow(lamr, R(kCre[1]));
-        ze_r = n0_r * C.crg[3] * mpow(L.ilamr, R(kCre[3]));
+        const R n0_r = L.nr * C.u.org2 * mpow(lamr, R(kCre[1]));
+        ze_r = n0_r * C.u.crg[3] * mpow(L.ilamr, R(kCre[3]));
       }
       pts[tid] = radar::Wet{double(value(L.rs)), double(value(L.smob)), double(value(L.smoc)), double(value(L.rr)),
                             double(value(L.rg)), double(value(L.ng)), double(value(L.ilamg)),
-                            double(C.am_g[L.idx_bg - 1]), L.idx_bg};
+                            double(C.l.am_g[L.idx_bg - 1]), L.idx_bg};
       list[atomicAdd(&count, 1)] = static_cast<unsigned short>(tid | (wet_s ? 0x4000 : 0) | (wet_g ? 0x8000 : 0));
     }
   }
@@ -1159,7 +1160,7 @@ __global__ void __launch_bounds__(256) k_melt_refl(StepArgs<R> a) {
       if ((tid & 63) == 0) ze[0][t] = z;
     }
     if (e & 0x8000) {
-      const double z = radar::melting_graupel<kCR>(*a.radar, double(C.ogg2), kCge1, p);
+      const double z = radar::melting_graupel<kCR>(*a.radar, double(C.u.ogg2), kCge1, p);
       if ((tid & 63) == 0) ze[1][t] = z;
     }
   }
@@ -1187,7 +1188,7 @@ __device__ __forceinline__ void atomic_max_pos(Dual<T>* p, Dual<T> v) {
 // freeze_cloud_melt_ice (src/module_mp_tempo_main.F90:2124-2165), on the
 // tendencies of the final update
 template <class R>
-__device__ __forceinline__ void freeze_cloud_melt_ice(const Const<S_t<R>>& C, Lvl<R>& L, R qc1d, R qi1d, R ni1d,
+__device__ __forceinline__ void freeze_cloud_melt_ice(const ConstView<S_t<R>>& C, Lvl<R>& L, R qc1d, R qi1d, R ni1d,
                                                       R nc1d, bool has_nc, R ncv, R lvap, R ocp, R dt, R odt) {
   // uncontracted, as the final checks: a fully frozen or melted mass then
   // cancels to zero as in the reference
@@ -1198,7 +1199,7 @@ __device__ __forceinline__ void freeze_cloud_melt_ice(const Const<S_t<R>>& C, Lv
     L.ncten = L.ncten + ni1d * odt;
     L.qiten = L.qiten - xri * odt;
     L.niten = -ni1d * odt;
-    L.tten = L.tten - C.lfus * ocp * xri * odt;
+    L.tten = L.tten - C.u.lfus * ocp * xri * odt;
   }
   const R xrc = mx(R(0.0), qc1d + L.qcten * dt);
   if ((L.temp < R(kHgFrz)) && (xrc > R(0.0))) {
@@ -1214,7 +1215,7 @@ __device__ __forceinline__ void freeze_cloud_melt_ice(const Const<S_t<R>>& C, Lv
 // a signature run executes it on the plain type (its contraction pragma
 // applies to the plain type only) and records its two decisions
 template <class T>
-__device__ __forceinline__ void freeze_cloud_melt_ice(const Const<T>& C, Lvl<Sig<T>>& L, Sig<T> qc1d, Sig<T> qi1d,
+__device__ __forceinline__ void freeze_cloud_melt_ice(const ConstView<T>& C, Lvl<Sig<T>>& L, Sig<T> qc1d, Sig<T> qi1d,
                                                       Sig<T> ni1d, Sig<T> nc1d, bool has_nc, Sig<T> ncv, Sig<T> lvap,
                                                       Sig<T> ocp, Sig<T> dt, Sig<T> odt) {
   Lvl<T> M = sig_unwrap(L);
@@ -1233,7 +1234,7 @@ __device__ __forceinline__ void atomic_max_pos(Sig<T>* p, Sig<T> v) {
 // (src/module_mp_tempo_main.F90:729-863); scratch in scr
 template <class R>
 __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, const Scr<R>& scr, int c, int k) {
-  const Const<S_t<R>>& C = *a.cst;
+  const ConstView<S_t<R>> C = const_view(a.cst);
   const size_t o = TEMPO_IDX_STATE(a, c, k);
   const size_t s = scr.at(c, k);
   const size_t plane = scr.plane;
@@ -1328,21 +1329,21 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, const Scr<R>
     R hail = R(0.0);
     if (L.rg / L.rho >= R(1.e-6) && rho_g<R>(L.idx_bg) >= R(350.0)) {
       const R lamg = R(1.0) / L.ilamg;
-      const R n0_g = L.ng * C.ogg2 * mpow(lamg, R(kCge1));
+      const R n0_g = L.ng * C.u.ogg2 * mpow(lamg, R(kCge1));
       R sum_nh = R(0), sum_t = R(0);
       const R thr = R(0.0005);
       int n;
       for (n = kNhbins; n >= 1; --n) {
-        const R f_d = n0_g * mpow(C.hbins[n - 1], R(kMuG)) * mexp(-lamg * C.hbins[n - 1]) * C.dhbins[n - 1];
+        const R f_d = n0_g * mpow(C.u.hbins[n - 1], R(kMuG)) * mexp(-lamg * C.u.hbins[n - 1]) * C.u.dhbins[n - 1];
         sum_nh = sum_nh + f_d;
         if (sum_nh > thr) break;
         sum_t = sum_nh;
       }
       R hmax;
       if (n >= kNhbins)
-        hmax = C.hbins[kNhbins - 1];
-      else if (C.hbins[n] > R(1.e-3))
-        hmax = C.hbins[n - 1] - (sum_nh - thr) / (sum_nh - sum_t) * (C.hbins[n - 1] - C.hbins[n]);
+        hmax = C.u.hbins[kNhbins - 1];
+      else if (C.u.hbins[n] > R(1.e-3))
+        hmax = C.u.hbins[n - 1] - (sum_nh - thr) / (sum_nh - sum_t) * (C.u.hbins[n - 1] - C.u.hbins[n]);
       else
         hmax = R(1.e-4);
       hail = R(1000.0) * hmax;
@@ -1357,15 +1358,15 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, const Scr<R>
       R ze_r = R(1.e-22), ze_s = R(1.e-22), ze_g = R(1.e-22);
       if (L.l_qr) {
         const R lamr = R(1.0) / L.ilamr;
-        const R n0_r = L.nr * C.org2 * mpow(lamr, R(kCre[1]));
-        ze_r = n0_r * C.crg[3] * mpow(L.ilamr, R(kCre[3]));
+        const R n0_r = L.nr * C.u.org2 * mpow(lamr, R(kCre[1]));
+        ze_r = n0_r * C.u.crg[3] * mpow(L.ilamr, R(kCre[3]));
       }
       const R k6 = R(0.176 / 0.93) * (R(6.0) / R(kPi)) * (R(6.0) / R(kPi));
       if (L.l_qs) ze_s = k6 * (R(kAmS) / R(900.0)) * (R(kAmS) / R(900.0)) * L.smoz;
       if (L.l_qg) {
         const int idx = L.idx_bg;
-        const R n0_g = L.ng * C.ogg2 * mpow(R(1.0) / L.ilamg, R(kCge1));
-        ze_g = k6 * (C.am_g[idx - 1] / R(900.0)) * (C.am_g[idx - 1] / R(900.0)) * n0_g * C.cgg[3][0] *
+        const R n0_g = L.ng * C.u.ogg2 * mpow(R(1.0) / L.ilamg, R(kCge1));
+        ze_g = k6 * (C.l.am_g[idx - 1] / R(900.0)) * (C.l.am_g[idx - 1] / R(900.0)) * n0_g * C.u.cgg[3][0] *
                mpow(L.ilamg, R(kCge3));
       }
       dbz = mx(R(-35.0), R(10.0) * mlog10((ze_r + ze_s + ze_g) * R(1.e18)));
@@ -1421,7 +1422,7 @@ template <class R>
 __global__ void __launch_bounds__(256) k_check_update(CheckArgs<R> g, int which) {
   const int i = int(blockIdx.x * blockDim.x + threadIdx.x);
   if (i >= g.n) return;
-  const Const<S_t<R>>& C = *g.cst;
+  const ConstView<S_t<R>> C = const_view(g.cst);
   Lvl<R> L;
   L.rho = g.rho[i];
   R q = g.q[i];

@@ -582,7 +582,7 @@ __device__ __forceinline__ void wave_refill(const double (&mass)[CH], int nzc, c
 template <class R>
 __device__ __forceinline__ void semi_rain_level(const StepArgs<R>& a, R rho, R rhof, R qr, R nr, double& qrten,
                                                 double& nrten, double& rr, double& rn, R& v1, R& v2) {
-  const Const<S_t<R>>& C = *a.cst;
+  const ConstView<S_t<R>> C = const_view(a.cst);
   Lvl<R> L;
   L.rho = rho;
   L.qrten = R(qrten);
@@ -600,7 +600,7 @@ template <class R>
 __device__ __forceinline__ void semi_graupel_level(const StepArgs<R>& a, R rho, R rhof, R visco, R qg, R ng, R qb,
                                                    double& qgten, double& ngten, double& qbten, double& rg, double& rn,
                                                    double& rb, R& v1, R& v2) {
-  const Const<S_t<R>>& C = *a.cst;
+  const ConstView<S_t<R>> C = const_view(a.cst);
   const bool has_ngqb = a.f[F_NG] && a.f[F_QB];
   Lvl<R> L;
   L.rho = rho;
