@@ -309,14 +309,9 @@ int tempo_hip_substeps(tempo_hip_ctx *ctx, int *host_out, size_t n);
  *                               form of the staging; nz <= 128, else as 1)
  *   TEMPO_HIP_TUNE_BLOCK_A   threads per block of the level-local physics
  *   TEMPO_HIP_TUNE_BLOCK_C   ... and of the final update: 64, 128 or 256
- *   TEMPO_HIP_TUNE_FUSED     1: the whole step as one persistent launch that
- *                               pulls column groups from a work queue and
- *                               keeps their scratch in the caches (for
- *                               flux-form sedimentation on at most 128 levels
- *                               without the melting-layer reflectivity) --
- *                               currently switched off: 1 returns
- *                               TEMPO_HIP_E_UNSUPPORTED;
- *                               0: four launches over the batch (default)
+ *   TEMPO_HIP_TUNE_FUSED     0: four launches over the batch (default);
+ *                               1 (the whole step as one persistent launch)
+ *                               returns TEMPO_HIP_E_UNSUPPORTED
  *   TEMPO_HIP_TUNE_ORDER     point grouping of the level-local kernels, a
  *                               bit mask: bit 0 (level-local physics), bit 1
  *                               (final update) set = each block hands its

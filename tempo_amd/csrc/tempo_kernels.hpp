@@ -218,12 +218,12 @@ dim3 level_grid(const StepArgs<R>& a, int threads) {
 
 // ----------------------------------------------------------- phase A ----
 template <class R>
-__device__ __forceinline__ R default_aerosol(const Scr<R>& scr, int c, int k, R n0, R n1) {
+__device__ __forceinline__ R default_aerosol(const StepArgs<R>& a, int c, int k, R n0, R n1) {
   // init_water/ice_friendly_aerosols (src/module_mp_tempo_aerosols.F90:14-73):
   // hgt(1) = 0, so h_01 = 0.8; level 1 uses hgt(2)
-  const R* hgt = scr.sr + size_t(SR_HGT) * scr.plane;
-  const R h1 = hgt[scr.at(c, 0)];
-  const R hk = hgt[scr.at(c, (k == 0 ? 1 : k))];
+  const R* hgt = a.sr + size_t(SR_HGT) * a.plane;
+  const R h1 = hgt[TEMPO_IDX_SCR(a, c, 0)];
+  const R hk = hgt[TEMPO_IDX_SCR(a, c, (k == 0 ? 1 : k))];
   const R ni3 = R(-1.0) * mlog(n1 / n0) / R(0.8);
   return n1 + n0 * mexp(-((hk - h1) / R(1000.0)) * ni3);
 }
@@ -297,13 +297,13 @@ __device__ __forceinline__ void graupel_fallspeed(const ConstView<S_t<R>>& C, co
 }
 
 // the level-local physics of point (c, k), from the initial checks to the
-// fall speeds (src/module_mp_tempo_main.F90:320-588); scratch in scr
+// fall speeds (src/module_mp_tempo_main.F90:320-588)
 template <class R>
-__device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>& scr, int c, int k) {
+__device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k) {
   const ConstView<S_t<R>> C = lds_const_view(a.cst);
   const size_t o = TEMPO_IDX_STATE(a, c, k);
-  const size_t s = scr.at(c, k);
-  const size_t plane = scr.plane;
+  const size_t s = TEMPO_IDX_SCR(a, c, k);
+  const size_t plane = a.plane;
   const R dt = R(a.dt), odt = R(a.odt);
   const unsigned cf = a.cf[c];
   const bool has_nc = a.f[F_NC], has_nwfa = a.f[F_NWFA], has_nifa = a.f[F_NIFA];
@@ -324,8 +324,8 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>
   L.pres = a.f[F_P][o];
   L.rho = rho_of(C, L.pres, L.temp, L.qv);
   // aerosols: a present field overrides the default profile (:328-345)
-  L.nwfa = has_nwfa ? nwfa1d * L.rho : default_aerosol(scr, c, k, R(kNaccn0), R(kNaccn1));
-  L.nifa = has_nifa ? nifa1d * L.rho : default_aerosol(scr, c, k, R(kNain0), R(kNain1));
+  L.nwfa = has_nwfa ? nwfa1d * L.rho : default_aerosol(a, c, k, R(kNaccn0), R(kNaccn1));
+  L.nifa = has_nifa ? nifa1d * L.rho : default_aerosol(a, c, k, R(kNain0), R(kNain1));
   L.nwfa = mx(R(kNwfaDefault) * L.rho, mn(R(kAeroMax) * L.rho, L.nwfa));
   L.nifa = mx(R(kNifaDefault) * L.rho, mn(R(kAeroMax) * L.rho, L.nifa));
 
@@ -341,7 +341,7 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>
   if (a.fl.ml_for_nc && !has_nc) {
     const R xrx = qc1d <= R(S_t<R>(1.e-12)) ? R(0.0) : qc1d;
     ncv = ml_cloud_number(xrx, qr1d, qi1d, qs1d, L.pres, L.temp, w) * L.rho;
-    scr.sr[SR_NCSAVE * plane + s] = ncv;
+    a.sr[SR_NCSAVE * plane + s] = ncv;
   } else {
     ncv = column_nc(a, c);
   }
@@ -483,7 +483,7 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>
     vtnc = L.rhof * R(kAvC) * C.l.ccg[3][nu] * C.l.ocg1[nu] * mpow(L.ilamc, R(kBvC));
   }
 
-  R* sr = scr.sr;
+  R* sr = a.sr;
   sr[SR_TEMP * plane + s] = L.temp;
   sr[SR_QV * plane + s] = L.qv;
   sr[SR_RHO * plane + s] = L.rho;
@@ -505,7 +505,7 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>
     sr[SR_VISCO * plane + s] = L.visco;
   }
   using D = Sd_t<R>;
-  D* sd = scr.sd;
+  D* sd = a.sd;
   sd[SD_RR * plane + s] = D(L.rr);
   sd[SD_NR * plane + s] = D(L.nr);
   sd[SD_RG * plane + s] = D(L.rg);
@@ -526,7 +526,7 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, const Scr<R>
   sd[SD_NITEN * plane + s] = D(L.niten);
   sd[SD_QCTEN * plane + s] = D(L.qcten);
   sd[SD_NCTEN * plane + s] = D(L.ncten);
-  scr.pf[s] = pf;
+  a.pf[s] = pf;
 }
 
 // kWaves: waves per SIMD the kernel is compiled for.  With a.ccn_lds the
@@ -548,7 +548,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves
   if (a.nlev && k >= a.nlev[c]) return;
   if (IsDual<R>::value && a.pt_on && !a.pt_on[size_t(c) + size_t(k) * a.ncol]) return;  // an adjoint's local pass
   SigScope<R> scope(a, c, k, 0);
-  phase_a_point(a, batch_scr(a), c, k);
+  phase_a_point(a, c, k);
 }
 
 // ----------------------------------------------------------- phase B ----
@@ -1231,13 +1231,13 @@ __device__ __forceinline__ void atomic_max_pos(Sig<T>* p, Sig<T> v) {
 }
 
 // freeze/melt, final update, final checks and diagnostics of point (c, k)
-// (src/module_mp_tempo_main.F90:729-863); scratch in scr
+// (src/module_mp_tempo_main.F90:729-863)
 template <class R>
-__device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, const Scr<R>& scr, int c, int k) {
+__device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k) {
   const ConstView<S_t<R>> C = const_view(a.cst);
   const size_t o = TEMPO_IDX_STATE(a, c, k);
-  const size_t s = scr.at(c, k);
-  const size_t plane = scr.plane;
+  const size_t s = TEMPO_IDX_SCR(a, c, k);
+  const size_t plane = a.plane;
   const size_t d3 = size_t(c % a.ni) + size_t(k) * a.dldk + size_t(c / a.ni) * a.dldj;
   const R dt = R(a.dt), odt = R(a.odt);
   const bool live = !(a.cf[c] & CF_EXIT);
@@ -1250,8 +1250,8 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, const Scr<R>
     return;
   }
   Lvl<R> L;
-  const R* sr = scr.sr;
-  const Sd_t<R>* sd = scr.sd;
+  const R* sr = a.sr;
+  const Sd_t<R>* sd = a.sd;
   L.temp = sr[SR_TEMP * plane + s];
   L.qv = sr[SR_QV * plane + s];
   L.rho = sr[SR_RHO * plane + s];
@@ -1411,7 +1411,7 @@ __global__ void __launch_bounds__(256) TEMPO_ATTR_C k_phase_c(StepArgs<R> a) {
   if (a.nlev && k >= a.nlev[c]) return;
   if (a.lvl_on && !a.lvl_on[k]) return;
   SigScope<R> scope(a, c, k, 1);
-  phase_c_point(a, batch_scr(a), c, k);
+  phase_c_point(a, c, k);
 }
 
 // ------------------------------------ public check-and-update routines ----

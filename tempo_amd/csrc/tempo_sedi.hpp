@@ -34,7 +34,7 @@ constexpr int kSedCols = kScrW;           // columns (wavefronts) per block: one
 constexpr int kSedSlots = 8;              // LDS planes staged at once
 constexpr int kSedMaxChunks = 4;          // register chunks of 64 levels of the largest form
 constexpr int kSedMaxLevels = 64 * kSedMaxChunks;
-constexpr int kSedChunks = 2;             // chunks of the adjoint's and the fused step's column kernels
+constexpr int kSedChunks = 2;             // chunks of the adjoint's column kernels
 constexpr int kSedLevels = 64 * kSedChunks;
 
 // Staged values are kept as the scratch holds them: 4 bytes in the FP32
@@ -619,24 +619,24 @@ __device__ __forceinline__ void semi_graupel_level(const StepArgs<R>& a, R rho, 
 }
 
 // Sedimentation of the column group c0 .. c0 + kSedCols - 1, one wavefront
-// per column (64 * kSedCols threads); scr holds the group's scratch,
-// tile_mem sed_lds_bytes(nz) of LDS.  For a dual working type it runs on the
+// per column (64 * kSedCols threads); tile_mem: sed_lds_bytes(nz)
+// of LDS.  For a dual working type it runs on the
 // values (V, the scalar type) and writes tendencies with zero tangents: the
 // tangent-free forward of an adjoint.
 // kSemi: semi-Lagrangian rain and graupel, with semi_lds_bytes(nz) more LDS
 // behind the tile.
 template <class R, int CH = kSedChunks, bool kEveryPass = false, bool kSemi = false>
-__device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>& scr, int c0, void* tile_mem) {
+__device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void* tile_mem) {
   __shared__ unsigned blk_any;
   const int w = int(threadIdx.x >> 6);
   const int c = c0 + w;
   const bool col_ok = c < a.ncol;
-  const size_t plane = scr.plane;
+  const size_t plane = a.plane;
   using E = SedStage<R>;
-  const SedTile<E, CH, kEveryPass> T{static_cast<E*>(tile_mem), c0, a.ncol, a.nz, scr.nzs, sed_row<E>(a.nz), scr.at(c0, 0)};
+  const SedTile<E, CH, kEveryPass> T{static_cast<E*>(tile_mem), c0, a.ncol, a.nz, a.nzs, sed_row<E>(a.nz), TEMPO_IDX_SCR(a, c0, 0)};
   const double dt = a.dt;
-  Sd_t<R>* sd = scr.sd;
-  const R* sr = scr.sr;
+  Sd_t<R>* sd = a.sd;
+  const R* sr = a.sr;
   using V = typename Num<R>::S;
 
   SedCol<CH> g;
@@ -654,7 +654,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
 
   // column flags (which species hold mass) and the level geometry
   if (threadIdx.x == 0) blk_any = 0;
-  T.load_head(a, scr.pf, sr + SR_RHO * plane, sd + SD_RR * plane);
+  T.load_head(a, a.pf, sr + SR_RHO * plane, sd + SD_RR * plane);
   __syncthreads();
   unsigned pfl[CH];
   V dz[CH], rho[CH];
@@ -694,8 +694,8 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
       sg.orho[j] = g.orho[j];
       rhof[j] = visco[j] = V(0);
       if ((any & (PF_QR | PF_QG)) && k < g.nzc) {
-        rhof[j] = value(sr[SR_RHOF * plane + scr.at(c, k)]);
-        visco[j] = value(sr[SR_VISCO * plane + scr.at(c, k)]);
+        rhof[j] = value(sr[SR_RHOF * plane + TEMPO_IDX_SCR(a, c, k)]);
+        visco[j] = value(sr[SR_VISCO * plane + TEMPO_IDX_SCR(a, c, k)]);
       }
     }
     if (any & (PF_QR | PF_QG)) sg.heights();
@@ -937,7 +937,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, const Scr<R>
     a.d2[D2_FROZEN][d2] = live ? (ice + snow + graupel) / (ice + snow + graupel + rain + R(kR1)) : R(0);
   if (a.d2[D2_FRZRAIN]) {
     R frz = R(0);
-    if (live && (sr[SR_TEMP * plane + scr.at(c, 0)] - R(kT0)) < R(-0.5)) frz = rain + cloud;
+    if (live && (sr[SR_TEMP * plane + TEMPO_IDX_SCR(a, c, 0)] - R(kT0)) < R(-0.5)) frz = rain + cloud;
     a.d2[D2_FRZRAIN][d2] = frz;
   }
   if (a.d2[D2_HAIL_SFC]) a.d2[D2_HAIL_SFC][d2] = R(0);
@@ -955,14 +955,14 @@ constexpr int sed_waves(int chunks) { return chunks <= 1 ? 8 : chunks == 2 ? 6 :
 template <class R, int CH, bool kEveryPass = false>
 __global__ void __launch_bounds__(64 * kSedCols) __attribute__((amdgpu_waves_per_eu(sed_waves(CH)))) k_phase_b_wave(StepArgs<R> a) {
   extern __shared__ double tile_mem[];  // sed_lds_bytes<SedStage<R>>(nz)
-  phase_b_group<R, CH, kEveryPass>(a, batch_scr(a), int(blockIdx.x) * kSedCols, tile_mem);
+  phase_b_group<R, CH, kEveryPass>(a, int(blockIdx.x) * kSedCols, tile_mem);
 }
 
 // ... with semi-Lagrangian rain and graupel
 template <class R, int CH>
 __global__ void __launch_bounds__(64 * kSedCols) k_phase_b_semi_wave(StepArgs<R> a) {
   extern __shared__ double tile_mem[];  // sed_lds_bytes<SedStage<R>>(nz) + semi_lds_bytes(nz)
-  phase_b_group<R, CH, false, true>(a, batch_scr(a), int(blockIdx.x) * kSedCols, tile_mem);
+  phase_b_group<R, CH, false, true>(a, int(blockIdx.x) * kSedCols, tile_mem);
 }
 template <class R>
 void launch_phase_b_semi_wave(const StepArgs<R>& a, hipStream_t s) {

@@ -303,8 +303,6 @@ struct StepArgs {
   // x + (-x/dt)*dt of a fully removed mass from cancelling
   double odt;
   int first_step;
-  // work queue of the fused step (a counter of column groups handed out)
-  int* queue;
   // adjoint passes of the final update: levels whose output cotangents are
   // all zero (lvl_on[k] == 0) are skipped, their contributions being zero;
   // nullptr = every level
@@ -350,7 +348,6 @@ struct DualGeom {
 
 // launch shape of one step (host-side choice, see tempo_hip_tune)
 struct LaunchCfg {
-  int fused = 0;      // 1: the whole step in one persistent launch where it applies (k_step_fused)
   int sed_wave = 1;   // sedimentation: 1 = one wavefront per column (nz <= 128), 0 = one lane per column,
                       // 2 = the wavefront kernel issuing every staging pass (check form)
   int order = 0;      // point grouping within blocks: bit 0 phase A, bit 1 final update
@@ -373,31 +370,8 @@ struct LaunchCfg {
 constexpr int kScrW = 8;
 constexpr int kScrLevels = 16;
 __host__ __device__ constexpr int scratch_levels(int nz) { return (nz + kScrLevels - 1) / kScrLevels * kScrLevels; }
-// elements of one plane of a fused-step block's scratch slot: one column tile
-__host__ __device__ constexpr size_t fused_slot_plane(int nz) { return size_t(kScrW) * size_t(scratch_levels(nz)); }
 #define TEMPO_IDX_SCR(a, c, k) \
   ((size_t((c) / kScrW) * size_t((a).nzs) + size_t(k)) * kScrW + size_t((c) % kScrW))
-
-// Where the per-point scratch of a kernel lives: the batch's column-tiled
-// planes (c0 = 0; element of (c, k) at TEMPO_IDX_SCR), or the tile of one
-// column group starting at column c0 (the fused step's block-private slot),
-// indexed the same way relative to c0.
-template <class R>
-struct Scr {
-  R* sr;
-  Sd_t<R>* sd;
-  unsigned* pf;
-  size_t plane;  // elements per plane
-  int c0, nzs;
-  __device__ __forceinline__ size_t at(int c, int k) const {
-    const int cc = c - c0;
-    return (size_t(cc / kScrW) * size_t(nzs) + size_t(k)) * kScrW + size_t(cc % kScrW);
-  }
-};
-template <class R>
-__device__ __forceinline__ Scr<R> batch_scr(const StepArgs<R>& a) {
-  return Scr<R>{a.sr, a.sd, a.pf, a.plane, 0, a.nzs};
-}
 
 // ------------------------------------------------ level-local physics ----
 // Per-level working state: the scalars of one (column, level) point.  The
