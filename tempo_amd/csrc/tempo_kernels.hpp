@@ -173,9 +173,12 @@ __device__ bool point_active_c(const StepArgs<R>& a, int c, int k) {
   if ((a.nlev && k >= a.nlev[c]) || (a.cf[c] & CF_EXIT)) return false;
   const size_t o = TEMPO_IDX_STATE(a, c, k), s = TEMPO_IDX_SCR(a, c, k);
   const R dt = R(a.dt);
-  auto present = [&](int f, int ten) { return a.fa[f][o] + R(a.sd[size_t(ten) * a.plane + s]) * dt > R(kR1); };
-  return present(F_QC, SD_QCTEN) || present(F_QR, SD_QRTEN) || present(F_QI, SD_QITEN) ||
-         present(F_QS, SD_QSTEN) || present(F_QG, SD_QGTEN);
+  const unsigned pf = a.pf[s];
+  auto present = [&](int f, int ten, unsigned bit) {
+    return a.fa[f][o] + (pf & bit ? R(a.sd[size_t(ten) * a.plane + s]) : R(0)) * dt > R(kR1);
+  };
+  return present(F_QC, SD_QCTEN, PF_TC) || present(F_QR, SD_QRTEN, PF_TR) || present(F_QI, SD_QITEN, PF_TI) ||
+         present(F_QS, SD_QSTEN, PF_TS) || present(F_QG, SD_QGTEN, PF_TG);
 }
 
 // The level-local kernels run blocks of 64 columns x blockDim.x/64 levels,
@@ -296,6 +299,53 @@ __device__ __forceinline__ void graupel_fallspeed(const ConstView<S_t<R>>& C, co
   v2 = rhof * afall * C.l.cgg[6][idx - 1] / C.l.cgg[11][idx - 1] * mpow(L.ilamg, bfall);
 }
 
+// ---- clear air ----
+// A point without hydrometeors, below liquid saturation by a part in a
+// thousand and below ice saturation's nucleation thresholds by a margin: the
+// level-local physics does nothing there but evaporate the floor of the
+// cloud mass and number (r1 and Nt_c_min) that cloud_condensation sees
+// (:1980-2056), which moves vapour, temperature and aerosol by their last
+// digits.  A wavefront of clear points takes these few operations instead of
+// the 1,200 instructions that lead to the same result; they are the general
+// path's own, in its order, with its fused multiply-adds (mad).
+__device__ __forceinline__ float mad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double mad(double a, double b, double c) {
+#pragma clang fp contract(off)
+  return a * b + c;
+}
+template <class T>
+__device__ __forceinline__ Sig<T> mad(Sig<T> a, Sig<T> b, Sig<T> c) { return mad(a.v, b.v, c.v); }
+template <class T>
+__device__ __forceinline__ Dual<T> mad(Dual<T> a, Dual<T> b, Dual<T> c) { return a * b + c; }
+
+template <class R>
+__device__ __forceinline__ bool clear_air(R pres, R temp, R qv) {
+  return qv < R(0.999) * rslf(pres, temp) && (temp >= R(kT0) || qv < R(1.2) * rsif(pres, temp));
+}
+template <class R>
+struct ClearAir {
+  R temp, qv, rho;              // after the step's tendencies
+  R tten, qvten, nwfaten;       // the ice-friendly aerosol's and the hydrometeors' are zero
+};
+template <class R>
+__device__ __forceinline__ ClearAir<R> clear_air_tendencies(const ConstView<S_t<R>>& C, R pres, R t1d, R qv1d, R dt,
+                                                            R odt) {
+#pragma clang fp contract(off)
+  ClearAir<R> q;
+  const R qv0 = mx(R(kMinQv), qv1d);
+  const R orho = R(1.0) / rho_of(C, pres, t1d, qv0);
+  const R prw = -R(kR1) * orho * odt, pnc = -R(kNtCMin) * orho * odt;
+  const R lvap = mad(R(2106.0 - 4218.0), t1d - R(kT0), R(kLvap0));
+  const R ocp = R(1.0) / (R(kCp) * mad(R(0.887), qv0, R(1.0)));
+  q.tten = lvap * ocp * prw;
+  q.qvten = R(0) - prw;
+  q.nwfaten = R(0) - pnc;
+  q.qv = mx(R(kMinQv), mad(q.qvten, dt, qv1d));
+  q.temp = mad(q.tten, dt, t1d);
+  q.rho = rho_of(C, pres, q.temp, q.qv);
+  return q;
+}
+
 // the level-local physics of point (c, k), from the initial checks to the
 // fall speeds (src/module_mp_tempo_main.F90:320-588)
 template <class R>
@@ -315,6 +365,29 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
   R ni1d = a.f[F_NI][o], nr1d = a.f[F_NR][o];
   R nc1d = has_nc ? a.f[F_NC][o] : R(0), ng1d = has_ngqb ? a.f[F_NG][o] : R(0), qb1d = has_ngqb ? a.f[F_QB][o] : R(0);
   const R nwfa1d = has_nwfa ? a.f[F_NWFA][o] : R(0), nifa1d = has_nifa ? a.f[F_NIFA][o] : R(0);
+
+  if constexpr (!IsDual<R>::value) {
+    if (a.sparse & SPARSE_CLEAR) {
+      const R pres = a.f[F_P][o];
+      const bool dry = !(qc1d > R(kR1) || qr1d > R(kR1) || qi1d > R(kR1) || qs1d > R(kR1) || qg1d > R(kR1));
+      if (__all(dry && ((cf & CF_EXIT) || clear_air(pres, t1d, mx(R(kMinQv), qv1d))))) {
+        // the initial checks remove what is below r1, and its number
+        const int fz[] = {F_QC, F_QR, F_NR, F_QI, F_NI, F_QS, F_QG};
+        for (int f : fz) put_post_check(a, f, o, R(0));
+        if (has_nc) put_post_check(a, F_NC, o, R(0));
+        if (has_ngqb) {
+          put_post_check(a, F_NG, o, R(0));
+          put_post_check(a, F_QB, o, R(0));
+        }
+        if (cf & CF_EXIT) return;
+        const ClearAir<R> q = clear_air_tendencies<R>(C, pres, t1d, qv1d, dt, odt);
+        a.sr[SR_RHO * plane + s] = q.rho;
+        if (k == 0) a.sr[SR_TEMP * plane + s] = q.temp;
+        a.pf[s] = PF_CLEAR;
+        return;
+      }
+    }
+  }
 
   L.tten = L.qvten = L.qcten = L.qiten = L.qrten = L.qsten = L.qgten = L.qbten = R(0);
   L.niten = L.nrten = L.ncten = L.ngten = L.nwfaten = L.nifaten = R(0);
@@ -491,41 +564,72 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
   sr[SR_QVTEN * plane + s] = L.qvten;
   sr[SR_NWFATEN * plane + s] = L.nwfaten;
   sr[SR_NIFATEN * plane + s] = L.nifaten;
-  sr[SR_VTRR * plane + s] = vtrr;
-  sr[SR_VTNR * plane + s] = vtnr;
-  sr[SR_VTRG * plane + s] = vtrg;
-  sr[SR_VTNG * plane + s] = vtng;
-  sr[SR_VTS * plane + s] = vts;
-  sr[SR_VTRI * plane + s] = vtri;
-  sr[SR_VTNI * plane + s] = vtni;
-  sr[SR_VTRC * plane + s] = vtrc;
-  sr[SR_VTNC * plane + s] = vtnc;
   if (a.fl.semi_sedi) {  // the fall-speed refresh between semi-Lagrangian substeps reads these
     sr[SR_RHOF * plane + s] = L.rhof;
     sr[SR_VISCO * plane + s] = L.visco;
   }
+  // the species' planes, where one of the sector's columns (8 lanes) needs them
+  const bool all = IsDual<R>::value || !(a.sparse & SPARSE_PLANES);
+  auto sector = [&](bool x) {
+    return all || ((__ballot(x) >> (threadIdx.x & 56u)) & 0xffull) != 0ull;
+  };
+  auto moves = [](const R& x) { return value(x) != S_t<R>(0); };
+  const bool tr = all || moves(L.qrten) || moves(L.nrten);
+  const bool tg = all || moves(L.qgten) || moves(L.ngten) || moves(L.qbten);
+  const bool ts = all || moves(L.qsten);
+  const bool ti = all || moves(L.qiten) || moves(L.niten);
+  // (without prognostic cloud number its tendency counts only with a cloud)
+  const bool tc = all || L.l_qc || moves(L.qcten) || (has_nc && moves(L.ncten));
+  pf |= (tr ? PF_TR : 0u) | (tg ? PF_TG : 0u) | (ts ? PF_TS : 0u) | (ti ? PF_TI : 0u) | (tc ? PF_TC : 0u);
   using D = Sd_t<R>;
   D* sd = a.sd;
-  sd[SD_RR * plane + s] = D(L.rr);
-  sd[SD_NR * plane + s] = D(L.nr);
-  sd[SD_RG * plane + s] = D(L.rg);
-  sd[SD_NG * plane + s] = D(L.ng);
-  sd[SD_RB * plane + s] = D(L.rb);
-  sd[SD_RS * plane + s] = D(L.rs);
-  sd[SD_RI * plane + s] = D(L.ri);
-  sd[SD_NI * plane + s] = D(L.ni);
-  sd[SD_RC * plane + s] = D(L.rc);
-  sd[SD_NC * plane + s] = D(L.nc);
-  sd[SD_QRTEN * plane + s] = D(L.qrten);
-  sd[SD_NRTEN * plane + s] = D(L.nrten);
-  sd[SD_QGTEN * plane + s] = D(L.qgten);
-  sd[SD_NGTEN * plane + s] = D(L.ngten);
-  sd[SD_QBTEN * plane + s] = D(L.qbten);
-  sd[SD_QSTEN * plane + s] = D(L.qsten);
-  sd[SD_QITEN * plane + s] = D(L.qiten);
-  sd[SD_NITEN * plane + s] = D(L.niten);
-  sd[SD_QCTEN * plane + s] = D(L.qcten);
-  sd[SD_NCTEN * plane + s] = D(L.ncten);
+  if (sector(L.l_qr)) {
+    sd[SD_RR * plane + s] = D(L.rr);
+    sd[SD_NR * plane + s] = D(L.nr);
+    sr[SR_VTRR * plane + s] = vtrr;
+    sr[SR_VTNR * plane + s] = vtnr;
+  }
+  if (sector(L.l_qg)) {
+    sd[SD_RG * plane + s] = D(L.rg);
+    sd[SD_NG * plane + s] = D(L.ng);
+    sd[SD_RB * plane + s] = D(L.rb);
+    sr[SR_VTRG * plane + s] = vtrg;
+    sr[SR_VTNG * plane + s] = vtng;
+  }
+  if (sector(L.l_qs)) {
+    sd[SD_RS * plane + s] = D(L.rs);
+    sr[SR_VTS * plane + s] = vts;
+  }
+  if (sector(L.l_qi)) {
+    sd[SD_RI * plane + s] = D(L.ri);
+    sd[SD_NI * plane + s] = D(L.ni);
+    sr[SR_VTRI * plane + s] = vtri;
+    sr[SR_VTNI * plane + s] = vtni;
+  }
+  if (sector(L.l_qc)) {
+    sd[SD_RC * plane + s] = D(L.rc);
+    sd[SD_NC * plane + s] = D(L.nc);
+    sr[SR_VTRC * plane + s] = vtrc;
+    sr[SR_VTNC * plane + s] = vtnc;
+  }
+  if (sector(tr)) {
+    sd[SD_QRTEN * plane + s] = D(L.qrten);
+    sd[SD_NRTEN * plane + s] = D(L.nrten);
+  }
+  if (sector(tg)) {
+    sd[SD_QGTEN * plane + s] = D(L.qgten);
+    sd[SD_NGTEN * plane + s] = D(L.ngten);
+    sd[SD_QBTEN * plane + s] = D(L.qbten);
+  }
+  if (sector(ts)) sd[SD_QSTEN * plane + s] = D(L.qsten);
+  if (sector(ti)) {
+    sd[SD_QITEN * plane + s] = D(L.qiten);
+    sd[SD_NITEN * plane + s] = D(L.niten);
+  }
+  if (sector(tc)) {
+    sd[SD_QCTEN * plane + s] = D(L.qcten);
+    sd[SD_NCTEN * plane + s] = D(L.ncten);
+  }
   a.pf[s] = pf;
 }
 
@@ -1065,15 +1169,15 @@ __global__ void __launch_bounds__(256) k_melt_level(StepArgs<R> a) {
   const int nzc = !in ? 0 : a.nlev ? min(max(a.nlev[c], 1), a.nz) : a.nz;
   const R dt = R(a.dt);
   const size_t plane = a.plane;
-  auto present = [&](int f, int ten, int k) {
+  auto present = [&](int f, int ten, unsigned bit, int k) {
     const size_t o = TEMPO_IDX_STATE(a, c, k), s = TEMPO_IDX_SCR(a, c, k);
-    return a.fa[f][o] + R(a.sd[size_t(ten) * plane + s]) * dt > R(kR1);
+    return a.fa[f][o] + (a.pf[s] & bit ? R(a.sd[size_t(ten) * plane + s]) : R(0)) * dt > R(kR1);
   };
   int k_melt = 1;
   for (int k = nzc - 2 - w; k >= 0; k -= 4) {
     const R temp = a.sr[SR_TEMP * plane + TEMPO_IDX_SCR(a, c, k)];
-    if (temp > R(kT0) && present(F_QR, SD_QRTEN, k) &&
-        (present(F_QS, SD_QSTEN, k + 1) || present(F_QG, SD_QGTEN, k + 1))) {
+    if (temp > R(kT0) && present(F_QR, SD_QRTEN, PF_TR, k) &&
+        (present(F_QS, SD_QSTEN, PF_TS, k + 1) || present(F_QG, SD_QGTEN, PF_TG, k + 1))) {
       k_melt = k + 2;
       break;
     }
@@ -1121,12 +1225,13 @@ __global__ void __launch_bounds__(256) k_melt_refl(StepArgs<R> a) {
     L.qv = a.sr[SR_QV * plane + s];
     L.pres = a.f[F_P][o];
     L.rho = rho_of(C, L.pres, L.temp, L.qv);
-    L.qrten = R(a.sd[SD_QRTEN * plane + s]);
-    L.nrten = R(a.sd[SD_NRTEN * plane + s]);
-    L.qsten = R(a.sd[SD_QSTEN * plane + s]);
-    L.qgten = R(a.sd[SD_QGTEN * plane + s]);
-    L.ngten = R(a.sd[SD_NGTEN * plane + s]);
-    L.qbten = R(a.sd[SD_QBTEN * plane + s]);
+    const unsigned pf = a.pf[s];
+    L.qrten = pf & PF_TR ? R(a.sd[SD_QRTEN * plane + s]) : R(0);
+    L.nrten = pf & PF_TR ? R(a.sd[SD_NRTEN * plane + s]) : R(0);
+    L.qsten = pf & PF_TS ? R(a.sd[SD_QSTEN * plane + s]) : R(0);
+    L.qgten = pf & PF_TG ? R(a.sd[SD_QGTEN * plane + s]) : R(0);
+    L.ngten = pf & PF_TG ? R(a.sd[SD_NGTEN * plane + s]) : R(0);
+    L.qbten = pf & PF_TG ? R(a.sd[SD_QBTEN * plane + s]) : R(0);
     R qr1d = a.fa[F_QR][o], nr1d = a.fa[F_NR][o], qs1d = a.fa[F_QS][o], qg1d = a.fa[F_QG][o];
     R ng1d = has_ngqb ? a.fa[F_NG][o] : R(0), qb1d = has_ngqb ? a.fa[F_QB][o] : R(0);
     rain_check(C, L, qr1d, nr1d, dt, odt);
@@ -1249,35 +1354,87 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
       if (a.d3[q]) a.d3[q][d3] = R(0);
     return;
   }
-  Lvl<R> L;
   const R* sr = a.sr;
   const Sd_t<R>* sd = a.sd;
-  L.temp = sr[SR_TEMP * plane + s];
-  L.qv = sr[SR_QV * plane + s];
-  L.rho = sr[SR_RHO * plane + s];
-  L.tten = sr[SR_TTEN * plane + s];
-  L.qvten = sr[SR_QVTEN * plane + s];
-  L.nwfaten = sr[SR_NWFATEN * plane + s];
-  L.nifaten = sr[SR_NIFATEN * plane + s];
+  const unsigned pf = a.pf[s];
+  if constexpr (!IsDual<R>::value) {
+    // a wavefront of points without hydrometeors and without tendencies of
+    // them (PF_ANYQ, PF_ANYT): temperature, vapour and aerosols take their
+    // tendencies where these change them, the diagnostics are constants
+    if (!a.qc_bl && !(a.fl.nc_mixing_ratio && a.d3[D3_NC_MIX]) && __all(!(pf & (PF_ANYQ | PF_ANYT)))) {
+      const R t1d = load_t(a, o), qv1d = a.f[F_QV][o];
+      R tten, qvten, nwfaten, nifaten = R(0);
+      if (pf & PF_CLEAR) {
+        const ClearAir<R> q = clear_air_tendencies<R>(C, a.f[F_P][o], t1d, qv1d, dt, odt);
+        tten = q.tten;
+        qvten = q.qvten;
+        nwfaten = q.nwfaten;
+      } else {
+        tten = sr[SR_TTEN * plane + s];
+        qvten = sr[SR_QVTEN * plane + s];
+        nwfaten = sr[SR_NWFATEN * plane + s];
+        nifaten = sr[SR_NIFATEN * plane + s];
+      }
+      auto put = [&](int f, R v) {
+        if (!same_bits(a.f[f][o], v)) a.fo[f][o] = v;
+      };
+      const R t_new = t1d + tten * dt;
+      if (a.f[F_T])
+        put(F_T, t_new);
+      else
+        put(F_TH, t_new / a.f[F_PII][o]);
+      put(F_QV, mx(R(kMinQv), (qv1d + qvten * dt)));
+      if (has_nwfa) put(F_NWFA, mx(R(kNwfaDefault), mn(R(kAeroMax), (a.f[F_NWFA][o] + nwfaten * dt))));
+      if (has_nifa) put(F_NIFA, mx(R(kNifaDefault), mn(R(kAeroMax), (a.f[F_NIFA][o] + nifaten * dt))));
+      if (a.d3[D3_NC_MIX]) a.d3[D3_NC_MIX][d3] = R(0);
+      if (a.d3[D3_MVD_R]) a.d3[D3_MVD_R][d3] = a.fl.mvd_r ? R(kD0R) : R(0);
+      if (a.d3[D3_MVD_G]) a.d3[D3_MVD_G][d3] = a.fl.mvd_g ? R(kD0G) : R(0);
+      if (a.d3[D3_REFL]) a.d3[D3_REFL][d3] = R(-35.0);
+      for (int q = D3_RE_C; q <= D3_RE_S; ++q)
+        if (a.d3[q]) a.d3[q][d3] = R(0);
+      return;
+    }
+  }
+  Lvl<R> L;
+  if (!IsDual<R>::value && (pf & PF_CLEAR)) {
+    const ClearAir<R> q = clear_air_tendencies<R>(C, a.f[F_P][o], load_t(a, o), a.f[F_QV][o], dt, odt);
+    L.temp = q.temp;
+    L.qv = q.qv;
+    L.rho = q.rho;
+    L.tten = q.tten;
+    L.qvten = q.qvten;
+    L.nwfaten = q.nwfaten;
+    L.nifaten = R(0);
+  } else {
+    L.temp = sr[SR_TEMP * plane + s];
+    L.qv = sr[SR_QV * plane + s];
+    L.rho = sr[SR_RHO * plane + s];
+    L.tten = sr[SR_TTEN * plane + s];
+    L.qvten = sr[SR_QVTEN * plane + s];
+    L.nwfaten = sr[SR_NWFATEN * plane + s];
+    L.nifaten = sr[SR_NIFATEN * plane + s];
+  }
   // the post-sedimentation tendencies; an adjoint's local pass takes their
   // values from a.post and their (local) tangents from the scratch
-  auto ten = [&](int m) {
+  auto ten = [&](int m, unsigned bit) {
     const Sd_t<R>& x = sd[size_t(SD_QRTEN + m) * plane + s];
     if constexpr (IsDual<R>::value) {
       if (a.post) return R(Sd_t<R>(a.post[size_t(m) * plane + s], x.d));
+      return R(x);
+    } else {
+      return pf & bit ? R(x) : R(0);
     }
-    return R(x);
   };
-  L.qrten = ten(0);
-  L.nrten = ten(1);
-  L.qgten = ten(2);
-  L.ngten = ten(3);
-  L.qbten = ten(4);
-  L.qsten = ten(5);
-  L.qiten = ten(6);
-  L.niten = ten(7);
-  L.qcten = ten(8);
-  L.ncten = ten(9);
+  L.qrten = ten(0, PF_TR);
+  L.nrten = ten(1, PF_TR);
+  L.qgten = ten(2, PF_TG);
+  L.ngten = ten(3, PF_TG);
+  L.qbten = ten(4, PF_TG);
+  L.qsten = ten(5, PF_TS);
+  L.qiten = ten(6, PF_TI);
+  L.niten = ten(7, PF_TI);
+  L.qcten = ten(8, PF_TC);
+  L.ncten = ten(9, PF_TC);
   L.pres = a.f[F_P][o];
   const R lvap = R(kLvap0) + R(2106.0 - 4218.0) * (L.temp - R(kT0));
   const R ocp = R(1.0) / (R(kCp) * (R(1.0) + R(0.887) * L.qv));

@@ -111,62 +111,72 @@ struct SedTile {
   size_t sbase; // scratch offset of the group's first element
 
   __device__ E* slot(int s) const { return lds + s * (kSedCols * row); }
-  // Several scratch planes of one stage (the block's column group of each is
-  // one contiguous run).  Every global load of the stage is issued into
-  // registers before the first LDS write, so the stage waits for one memory
-  // latency instead of one per plane and pass (a load-convert-write loop per
-  // plane waits for each load before its write).  The block has
-  // 64 * kSedCols threads and nz <= 64 * CH, so CH passes cover
+  // One species' planes (the block's column group of each is one contiguous
+  // run): masses and numbers pm and raw speeds ph where the point holds the
+  // species (pbit of its flags), tendencies pt where they are stored (tbit),
+  // elsewhere dm, 0 and td(x), x the element's place in its LDS plane.  Every
+  // global load is issued into registers before the first LDS write, so the
+  // stage waits for one memory latency instead of one per plane and pass (a
+  // load-convert-write loop per plane waits for each load before its write).
+  // The block has 64 * kSedCols threads and nz <= 64 * CH, so CH passes cover
   // the column group; a pass runs only when the group reaches it (a
   // block-uniform test), and its elements past the group's end load the last
-  // one (the index is clamped, not branched on per lane, so that the loads
-  // issue back to back) and are not written.
-  template <class TA, int NA, class TB, int NB>
-  __device__ void load_many(const int (&sa)[NA], const TA* const (&pa)[NA], const int (&sb)[NB],
-                            const TB* const (&pb)[NB]) const {
-    TA va[CH][NA];
-    TB vb[CH][NB];
+  // one (the index is clamped) and are not written.  kAll: every point is
+  // stored (dual planes).
+  template <bool kAll, class M, class H, int NM, int NH, int NT, class TD>
+  __device__ void load_species(const unsigned (&pfe)[CH], unsigned pbit, unsigned tbit, const int (&sm)[NM],
+                               const M* const (&pm)[NM], const E (&dm)[NM], const int (&sh)[NH],
+                               const H* const (&ph)[NH], const int (&st)[NT], const M* const (&pt)[NT], TD td) const {
+    M vm[CH][NM], vt[CH][NT];
+    H vh[CH][NH];
     const int n = kSedCols * nz;
     const size_t base = sbase;
 #pragma unroll
     for (int it = 0; it < CH; ++it) {
       if (!kEveryPass && it * 64 * kSedCols >= n) break;
       const int e = min(int(threadIdx.x) + it * 64 * kSedCols, n - 1);
+      if (kAll || (pfe[it] & pbit)) {
 #pragma unroll
-      for (int p = 0; p < NA; ++p) va[it][p] = pa[p][base + e];
+        for (int p = 0; p < NM; ++p) vm[it][p] = pm[p][base + e];
 #pragma unroll
-      for (int p = 0; p < NB; ++p) vb[it][p] = pb[p][base + e];
+        for (int p = 0; p < NH; ++p) vh[it][p] = ph[p][base + e];
+      }
+      if (kAll || (pfe[it] & tbit)) {
+#pragma unroll
+        for (int p = 0; p < NT; ++p) vt[it][p] = pt[p][base + e];
+      }
     }
 #pragma unroll
     for (int it = 0; it < CH; ++it) {
       const int e = int(threadIdx.x) + it * 64 * kSedCols;
       if (e < n) {
-        const int cc = e % kSedCols, k = e / kSedCols;
+        const int cc = e % kSedCols, k = e / kSedCols, x = cc * row + k;
+        const bool p_ = kAll || (pfe[it] & pbit), t_ = kAll || (pfe[it] & tbit);
 #pragma unroll
-        for (int p = 0; p < NA; ++p) slot(sa[p])[cc * row + k] = E(sval(va[it][p]));
+        for (int p = 0; p < NM; ++p) slot(sm[p])[x] = p_ ? E(sval(vm[it][p])) : dm[p];
 #pragma unroll
-        for (int p = 0; p < NB; ++p) slot(sb[p])[cc * row + k] = E(sval(vb[it][p]));
+        for (int p = 0; p < NH; ++p) slot(sh[p])[x] = p_ ? E(sval(vh[it][p])) : E(0);
+#pragma unroll
+        for (int p = 0; p < NT; ++p) slot(st[p])[x] = t_ ? E(sval(vt[it][p])) : td(p, x);
       }
     }
   }
-  // the first stage in the same way: per-point flags (slot 0), layer depths
-  // from the state (slot 1), density (slot 2) and rain mass (slot 3)
-  template <class R, class H, class M>
-  __device__ void load_head(const StepArgs<R>& a, const unsigned* pf, const H* rho, const M* rr) const {
-    unsigned vf[CH];
+  // the first stage in the same way: per-point flags (slot 0, and pfe for this
+  // thread's elements), layer depths from the state (slot 1), density (slot 2)
+  template <class R, class H>
+  __device__ void load_head(const StepArgs<R>& a, const unsigned* pf, const H* rho, unsigned (&pfe)[CH]) const {
     R vz[CH];
     H vh[CH];
-    M vr[CH];
     const int n = kSedCols * nz;
     const size_t base = sbase;
 #pragma unroll
     for (int it = 0; it < CH; ++it) {
-      if (!kEveryPass && it * 64 * kSedCols >= n) break;
+      pfe[it] = 0u;
+      if (!kEveryPass && it * 64 * kSedCols >= n) continue;
       const int e = min(int(threadIdx.x) + it * 64 * kSedCols, n - 1);
       const int cc = e % kSedCols, k = e / kSedCols, c = min(c0 + cc, ncol - 1);
-      vf[it] = pf[base + e];
+      pfe[it] = pf[base + e];
       vh[it] = rho[base + e];
-      vr[it] = rr[base + e];
       vz[it] = a.f[F_DZ][TEMPO_IDX_STATE(a, c, k)];
     }
 #pragma unroll
@@ -174,20 +184,38 @@ struct SedTile {
       const int e = int(threadIdx.x) + it * 64 * kSedCols;
       if (e < n) {
         const int cc = e % kSedCols, k = e / kSedCols, x = cc * row + k;
-        slot(0)[x] = E(vf[it]);
+        slot(0)[x] = E(pfe[it]);
         slot(1)[x] = c0 + cc < ncol ? E(sval(vz[it])) : E(0);
         slot(2)[x] = E(sval(vh[it]));
-        slot(3)[x] = E(sval(vr[it]));
       }
     }
   }
-  template <class T>
-  __device__ void store(int s, T* plane) const {
-    const E* d = slot(s);
-    T* dst = plane + sbase;
-    for (int e = threadIdx.x; e < kSedCols * nz; e += blockDim.x) {
+  // a species' tendencies back to their planes: the sectors (8 consecutive
+  // threads: the columns of one level) where one is non-zero or was stored;
+  // the flags of the elements that are non-zero gain tbit.  cond: which of
+  // the tendencies make an element count (a bit per plane).
+  template <bool kAll, class T, int NT>
+  __device__ void store_species(unsigned (&pfe)[CH], unsigned tbit, const int (&st)[NT], T* const (&pt)[NT],
+                                unsigned cond) const {
+#pragma unroll
+    for (int it = 0; it < CH; ++it) {
+      if (it * 64 * kSedCols >= kSedCols * nz) break;
+      const int e = int(threadIdx.x) + it * 64 * kSedCols;
       const int cc = e % kSedCols, k = e / kSedCols;
-      if (c0 + cc < ncol) dst[e] = T(d[cc * row + k]);
+      const bool in = e < kSedCols * nz && c0 + cc < ncol;
+      E v[NT];
+      bool counts = false;
+#pragma unroll
+      for (int p = 0; p < NT; ++p) {
+        v[p] = in ? slot(st[p])[cc * row + k] : E(0);
+        counts = counts || (((cond >> p) & 1u) && v[p] != E(0));
+      }
+      if (in && counts) pfe[it] |= tbit;
+      const bool sector = kAll || ((__ballot(in && (pfe[it] & tbit)) >> (threadIdx.x & 56u)) & 0xffull) != 0ull;
+      if (in && sector) {
+#pragma unroll
+        for (int p = 0; p < NT; ++p) pt[p][sbase + e] = T(v[p]);
+      }
     }
   }
   // this wavefront's column <-> registers
@@ -653,8 +681,15 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   const bool live = col_ok && !(cf & CF_EXIT);
 
   // column flags (which species hold mass) and the level geometry
+  constexpr bool kAll = IsDual<R>::value;
+  unsigned pfe[CH];  // flags of the elements this thread loads and stores
   if (threadIdx.x == 0) blk_any = 0;
-  T.load_head(a, a.pf, sr + SR_RHO * plane, sd + SD_RR * plane);
+  T.load_head(a, a.pf, sr + SR_RHO * plane, pfe);
+  unsigned pf0[CH];
+#pragma unroll
+  for (int j = 0; j < CH; ++j) pf0[j] = pfe[j];
+  const auto none = [](int, int) { return E(0); };
+  const E r1 = E(S_t<R>(kR1)), r2 = E(S_t<R>(kR2));
   __syncthreads();
   unsigned pfl[CH];
   V dz[CH], rho[CH];
@@ -662,7 +697,6 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   T.get(0, w, pfl);
   T.get(1, w, dz);
   T.get(2, w, rho);
-  T.get(3, w, rr);
   unsigned any = 0;
 #pragma unroll
   for (int j = 0; j < CH; ++j) {
@@ -670,6 +704,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     g.odz[j] = 1.0 / double(dz[j]);
     g.orho[j] = 1.0 / double(rho[j]);
     vr[j] = 0.0;
+    rr[j] = r1;
   }
   any = live ? wv::uor(any) : 0u;
   if (wv::lane() == 0 && any) atomicOr(&blk_any, any);
@@ -705,9 +740,11 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   if (bany & PF_QR) {
     double xn[CH], tr[CH], tn[CH], v2[CH];
     V raw1[CH], raw2[CH];
-    T.load_many({0, 1, 2}, {sd + SD_NR * plane, sd + SD_QRTEN * plane, sd + SD_NRTEN * plane}, {4, 5},
-                {sr + SR_VTRR * plane, sr + SR_VTNR * plane});
+    T.template load_species<kAll>(pfe, PF_QR, PF_TR, {3, 0}, {sd + SD_RR * plane, sd + SD_NR * plane}, {r1, r2}, {4, 5},
+                                  {sr + SR_VTRR * plane, sr + SR_VTNR * plane}, {1, 2},
+                                  {sd + SD_QRTEN * plane, sd + SD_NRTEN * plane}, none);
     __syncthreads();
+    T.get(3, w, rr);
     T.get(0, w, xn);
     T.get(1, w, tr);
     T.get(2, w, tn);
@@ -747,8 +784,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     T.put(1, w, tr);
     T.put(2, w, tn);
     __syncthreads();
-    T.store(1, sd + SD_QRTEN * plane);
-    T.store(2, sd + SD_NRTEN * plane);
+    T.template store_species<kAll>(pfe, PF_TR, {1, 2}, {sd + SD_QRTEN * plane, sd + SD_NRTEN * plane}, 3u);
     __syncthreads();
   }
 
@@ -757,10 +793,10 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     double xg[CH], xn[CH], xb[CH], tg[CH], tn[CH], tb[CH];
     double v1[CH], v2[CH];
     V raw1[CH], raw2[CH];
-    T.load_many({0, 1, 2, 4, 5, 6},
-                {sd + SD_RG * plane, sd + SD_NG * plane, sd + SD_RB * plane, sd + SD_QGTEN * plane,
-                 sd + SD_NGTEN * plane, sd + SD_QBTEN * plane},
-                {7, 3}, {sr + SR_VTRG * plane, sr + SR_VTNG * plane});
+    const E rb0 = E(S_t<R>(kM3ToL) * S_t<R>(kR1) / rho_g<S_t<R>>(kIdxBg1));
+    T.template load_species<kAll>(pfe, PF_QG, PF_TG, {0, 1, 2}, {sd + SD_RG * plane, sd + SD_NG * plane, sd + SD_RB * plane},
+                                  {r1, r2, rb0}, {7, 3}, {sr + SR_VTRG * plane, sr + SR_VTNG * plane}, {4, 5, 6},
+                                  {sd + SD_QGTEN * plane, sd + SD_NGTEN * plane, sd + SD_QBTEN * plane}, none);
     __syncthreads();
     T.get(0, w, xg);
     T.get(1, w, xn);
@@ -811,9 +847,8 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     T.put(5, w, tn);
     T.put(6, w, tb);
     __syncthreads();
-    T.store(4, sd + SD_QGTEN * plane);
-    T.store(5, sd + SD_NGTEN * plane);
-    T.store(6, sd + SD_QBTEN * plane);
+    T.template store_species<kAll>(pfe, PF_TG, {4, 5, 6},
+                                   {sd + SD_QGTEN * plane, sd + SD_NGTEN * plane, sd + SD_QBTEN * plane}, 7u);
     __syncthreads();
   }
 
@@ -822,7 +857,8 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   if (bany & PF_QS) {
     double xs[CH], ts[CH], v1[CH];
     V raw[CH];
-    T.load_many({0, 1}, {sd + SD_RS * plane, sd + SD_QSTEN * plane}, {2}, {sr + SR_VTS * plane});
+    T.template load_species<kAll>(pfe, PF_QS, PF_TS, {0}, {sd + SD_RS * plane}, {r1}, {2}, {sr + SR_VTS * plane}, {1},
+                                  {sd + SD_QSTEN * plane}, none);
     __syncthreads();
     T.get(0, w, xs);
     T.get(1, w, ts);
@@ -848,7 +884,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     }
     T.put(1, w, ts);
     __syncthreads();
-    T.store(1, sd + SD_QSTEN * plane);
+    T.template store_species<kAll>(pfe, PF_TS, {1}, {sd + SD_QSTEN * plane}, 1u);
     __syncthreads();
   }
 
@@ -856,8 +892,9 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   if (bany & PF_QI) {
     double xi[CH], xn[CH], ti[CH], tn[CH], v1[CH], v2[CH];
     V raw1[CH], raw2[CH];
-    T.load_many({0, 1, 2, 4}, {sd + SD_RI * plane, sd + SD_NI * plane, sd + SD_QITEN * plane, sd + SD_NITEN * plane},
-                {5, 6}, {sr + SR_VTRI * plane, sr + SR_VTNI * plane});
+    T.template load_species<kAll>(pfe, PF_QI, PF_TI, {0, 1}, {sd + SD_RI * plane, sd + SD_NI * plane}, {r1, r2}, {5, 6},
+                                  {sr + SR_VTRI * plane, sr + SR_VTNI * plane}, {2, 4},
+                                  {sd + SD_QITEN * plane, sd + SD_NITEN * plane}, none);
     __syncthreads();
     T.get(0, w, xi);
     T.get(1, w, xn);
@@ -876,8 +913,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     T.put(2, w, ti);
     T.put(4, w, tn);
     __syncthreads();
-    T.store(2, sd + SD_QITEN * plane);
-    T.store(4, sd + SD_NITEN * plane);
+    T.template store_species<kAll>(pfe, PF_TI, {2, 4}, {sd + SD_QITEN * plane, sd + SD_NITEN * plane}, 3u);
     __syncthreads();
   }
 
@@ -885,8 +921,20 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   if (bany & PF_QC) {
     double xc[CH], xn[CH], tc[CH], tn[CH], v1[CH], v2[CH];
     V raw1[CH], raw2[CH];
-    T.load_many({0, 1, 2, 4}, {sd + SD_RC * plane, sd + SD_NC * plane, sd + SD_QCTEN * plane, sd + SD_NCTEN * plane},
-                {5, 6}, {sr + SR_VTRC * plane, sr + SR_VTNC * plane});
+    // slot 3 keeps the density while slot 2 takes the tendency: a one-moment
+    // cloud's number tendency is, where not stored, that of clear air
+    const bool has_nc = a.f[F_NC] != nullptr;
+    for (int j = 0; j < CH; ++j) {
+      const int k = j * 64 + wv::lane();
+      if (k < a.nz) T.slot(3)[w * T.row + k] = E(rho[j]);
+    }
+    __syncthreads();
+    T.template load_species<kAll>(
+        pfe, PF_QC, PF_TC, {0, 1}, {sd + SD_RC * plane, sd + SD_NC * plane}, {r1, E(S_t<R>(kNtCMin))}, {5, 6},
+        {sr + SR_VTRC * plane, sr + SR_VTNC * plane}, {2, 4}, {sd + SD_QCTEN * plane, sd + SD_NCTEN * plane},
+        [&](int p, int x) {
+          return p == 0 || has_nc ? E(0) : E(-S_t<R>(kNtCMin) * (S_t<R>(1) / S_t<R>(T.slot(3)[x])) * S_t<R>(a.odt));
+        });
     __syncthreads();
     T.get(0, w, xc);
     T.get(1, w, xn);
@@ -916,8 +964,15 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     T.put(2, w, tc);
     T.put(4, w, tn);
     __syncthreads();
-    T.store(2, sd + SD_QCTEN * plane);
-    T.store(4, sd + SD_NCTEN * plane);
+    T.template store_species<kAll>(pfe, PF_TC, {2, 4}, {sd + SD_QCTEN * plane, sd + SD_NCTEN * plane},
+                                   a.f[F_NC] ? 3u : 1u);
+  }
+  if (!kAll) {  // the flags the final update reads
+#pragma unroll
+    for (int it = 0; it < CH; ++it) {
+      const int e = int(threadIdx.x) + it * 64 * kSedCols;
+      if (e < kSedCols * a.nz && c0 + e % kSedCols < a.ncol && pfe[it] != pf0[it]) a.pf[T.sbase + e] = pfe[it];
+    }
   }
 
   if (!col_ok || wv::lane() != 0) return;
@@ -997,8 +1052,20 @@ void launch_phase_b_wave(const StepArgs<R>& a, hipStream_t s) {
 // that records branch signatures (StepArgs<T> and StepArgs<Sig<T>> have the
 // same layout).
 template <class T, class RA>
-hipError_t launch_step_impl(const StepArgs<T>& a, const StepArgs<RA>& ga, const LaunchCfg& lc, double* vtbuf,
+hipError_t launch_step_impl(const StepArgs<T>& args, const StepArgs<RA>& gargs, const LaunchCfg& lc, double* vtbuf,
                             hipStream_t s, hipEvent_t* ev) {
+  StepArgs<T> a = args;
+  StepArgs<RA> ga = gargs;
+  // the lane-per-column kernel reads every point's planes.  The clear-air path
+  // leaves out planes that the semi-Lagrangian refresh, the melting level and
+  // the network's one-moment cloud number need, is the general path's result
+  // only where condensation runs, and is off in signature runs, whose records
+  // are of the decisions themselves.
+  const bool semi_wave = lc.sed_wave && a.nz <= kSemiLevels && a.fl.semi_sedi && !a.sig;
+  const bool wave = semi_wave || (lc.sed_wave && a.nz <= kSedMaxLevels && !a.fl.semi_sedi);
+  const bool clear = wave && !a.sig && !a.fl.semi_sedi && !(a.fl.refl_from_melting && a.fl.refl10cm) &&
+                     !(a.fl.ml_for_nc && !a.f[F_NC]) && !a.fl.turn_off_micro && a.fl.cloud_condensation;
+  a.sparse = ga.sparse = (wave ? SPARSE_PLANES : 0) | (clear ? SPARSE_CLEAR : 0);
   if (ev) (void)hipEventRecord(ev[0], s);
   launch_prepass(a, s);
   if (ev) (void)hipEventRecord(ev[1], s);
@@ -1011,10 +1078,10 @@ hipError_t launch_step_impl(const StepArgs<T>& a, const StepArgs<RA>& ga, const 
   if (lc.sed_wave == 2 && a.nz <= kSedLevels && !a.fl.semi_sedi)
     hipLaunchKernelGGL((k_phase_b_wave<T, kSedChunks, true>), dim3(unsigned((a.ncol + kSedCols - 1) / kSedCols)),
                        dim3(64 * kSedCols), sed_lds_bytes<SedStage<T>>(a.nz), s, a);
-  else if (lc.sed_wave && a.nz <= kSedMaxLevels && !a.fl.semi_sedi)
-    launch_phase_b_wave(a, s);
-  else if (lc.sed_wave && a.nz <= kSemiLevels && a.fl.semi_sedi && !a.sig)
+  else if (semi_wave)
     launch_phase_b_semi_wave(a, s);
+  else if (wave)
+    launch_phase_b_wave(a, s);
   else
     hipLaunchKernelGGL(k_phase_b<T>, dim3(unsigned((a.ncol + 127) / 128)), dim3(128), 0, s, a, vtbuf);
   if (a.fl.refl_from_melting && a.fl.refl10cm && a.d3[D3_REFL]) {

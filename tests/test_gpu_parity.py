@@ -1313,3 +1313,49 @@ def test_gpu_large_batch_equals_its_columns(hip, workload):
         assert torch.equal(st[k][:, n - tail:], v), k
     for k, v in e.items():
         assert torch.equal(d[k][..., n - tail:], v), k
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "fp64"])
+@pytest.mark.parametrize("form", ["aerosol", "plain", "hail", "theta", "no_condensation", "micro_off"])
+def test_gpu_clear_air_and_sparse_planes(hip, dtype, form):
+    """the step whose scratch holds what the point flags say, with its
+    clear-air path, against the one that stores every point (one lane per
+    column), bit for bit: cloud-free columns and levels, masses and numbers
+    below the presence threshold, vapour through both saturations (the
+    thresholds of nucleation included), columns that leave early, two steps"""
+    from tempo_amd import generator as gen
+    flags = dict(aerosolaware=form != "plain", hailaware=form == "hail")
+    ctx = context(hip, flags)
+    ctx.set_run_cfg(cloud_condensation_flag=int(form != "no_condensation"), turn_off_micro_flag=int(form == "micro_off"))
+    prec = hip.FP32 if dtype == "fp32" else hip.FP64
+    st, m = gen.generate("multistep", ncol=203, col0=5_000)
+    for k in ("ng", "qb") if form != "hail" else ():
+        st.pop(k)
+    for k in ("nc", "nwfa", "nifa") if form in ("plain", "hail") else ():
+        st.pop(k)
+    rng = np.random.default_rng(3)
+    col = np.arange(203)
+    clear = (col % 4 == 0) | ((col >= 64) & (col < 128))   # one whole wavefront, and every fourth column
+    for q in ("qc", "qr", "qi", "qs", "qg"):
+        st[q][:, clear] = 0.0
+    tiny = rng.random(st["qr"].shape) < 0.05
+    st["qr"][:, clear] = np.where(tiny, 5e-13, 0.0)[:, clear]
+    sat = gen.rslf(st["p"], st["t"])
+    st["qv"][:, clear] = (sat * rng.choice([1e-7, 0.3, 0.9, 0.998, 0.9995, 1.0, 1.2], size=sat.shape))[:, clear]
+    st["qv"][:, 64:96] = 0.2 * sat[:, 64:96]               # nothing supersaturated: these columns leave early
+    if form == "theta":
+        pii = (st["p"] / 1e5) ** 0.2857
+        st["pii"], st["th"] = pii, st.pop("t") / pii
+    got = {}
+    try:
+        for wave in (1, 0):
+            ctx.tune(prec, hip.TUNE_SED_WAVE, wave)
+            dev = to_dev(st, torch.float32 if dtype == "fp32" else torch.float64)
+            for i in range(2):
+                d = ctx.run(dev, m["dt"], 2 + i)
+            got[wave] = {k: v.cpu().numpy() for k, v in {**dev, **d}.items()}
+    finally:
+        ctx.tune(prec, hip.TUNE_SED_WAVE, 1)
+        ctx.set_run_cfg(cloud_condensation_flag=1, turn_off_micro_flag=0)
+    for k, v in got[1].items():
+        assert np.array_equal(v, got[0][k], equal_nan=True), k
