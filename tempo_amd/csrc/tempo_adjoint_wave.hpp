@@ -19,10 +19,7 @@ namespace wv {
 // value of x at level k-1 for every lane's level k in chunk j (0 below level 0)
 template <class T>
 __device__ __forceinline__ T below(const T (&x)[kSedChunks], int j) {
-  const T dn = __shfl_up(x[j], 1, 64);
-  T prv = T(0);
-  if (j > 0) prv = __shfl(x[j > 0 ? j - 1 : 0], 63, 64);
-  return lane() == 0 ? prv : dn;
+  return dpp<0x138>(j > 0 ? read_lane(x[j > 0 ? j - 1 : 0], 63) : T(0), x[j]);
 }
 }  // namespace wv
 
@@ -142,7 +139,7 @@ __device__ __forceinline__ void wave_sed_adjoint(const WaveCol& q, const double 
         post[j] = v > limit ? v : limit;
       }
     }
-    const double x0post = __shfl(post[0], 0, 64);
+    const double x0post = wv::read_lane(post[0], 0);
 #pragma unroll
     for (int j = 0; j < kSedChunks; ++j) {
       const double fbl = wv::below(fb, j);

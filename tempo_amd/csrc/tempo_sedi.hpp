@@ -30,6 +30,7 @@
 
 namespace tempo {
 
+constexpr unsigned kFlagsChanged = 1u << 31;  // of a thread's copy of a point's flags: to be written back
 constexpr int kSedCols = kScrW;           // columns (wavefronts) per block: one scratch column group
 constexpr int kSedSlots = 8;              // LDS planes staged at once
 constexpr int kSedMaxChunks = 4;          // register chunks of 64 levels of the largest form
@@ -58,15 +59,56 @@ __host__ __device__ constexpr size_t sed_lds_bytes(int nz) {
 
 namespace wv {
 __device__ __forceinline__ int lane() { return int(threadIdx.x & 63u); }
+// Data-parallel-primitive moves between lanes: one VALU instruction per 32
+// bits, against an LDS permute (and its wait) for a general shuffle.  The
+// sedimentation's substeps are chains of such moves (131,072 uneven columns
+// of up to 22 substeps: 1.02 -> 0.86 ms).
+template <int ctrl, int rows = 0xf, class T>
+__device__ __forceinline__ T dpp(T old, T x) {
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8, "32- or 64-bit values");
+  if constexpr (sizeof(T) == 4) {
+    const int r = __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old), __builtin_bit_cast(int, x), ctrl, rows, 0xf, false);
+    return __builtin_bit_cast(T, r);
+  } else {
+    const long long o = __builtin_bit_cast(long long, old), v = __builtin_bit_cast(long long, x);
+    const unsigned lo = unsigned(__builtin_amdgcn_update_dpp(int(o), int(v), ctrl, rows, 0xf, false));
+    const unsigned hi = unsigned(__builtin_amdgcn_update_dpp(int(o >> 32), int(v >> 32), ctrl, rows, 0xf, false));
+    return __builtin_bit_cast(T, (static_cast<unsigned long long>(hi) << 32) | lo);
+  }
+}
+// x of lane l (the same l in every lane)
+template <class T>
+__device__ __forceinline__ T read_lane(T x, int l) {
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l));
+  } else {
+    const long long v = __builtin_bit_cast(long long, x);
+    const unsigned lo = unsigned(__builtin_amdgcn_readlane(int(v), l));
+    const unsigned hi = unsigned(__builtin_amdgcn_readlane(int(v >> 32), l));
+    return __builtin_bit_cast(T, (static_cast<unsigned long long>(hi) << 32) | lo);
+  }
+}
+// maximum (of non-negative values) and bitwise or over the wavefront: row
+// shifts by 1, 2, 4, 8, then the rows' last lanes broadcast upwards
 __device__ __forceinline__ int imax(int v) {
-  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-  return v;
+  v = max(v, dpp<0x111>(0, v));
+  v = max(v, dpp<0x112>(0, v));
+  v = max(v, dpp<0x114>(0, v));
+  v = max(v, dpp<0x118>(0, v));
+  v = max(v, dpp<0x142, 0xa>(0, v));
+  v = max(v, dpp<0x143, 0xc>(0, v));
+  return __builtin_amdgcn_readlane(v, 63);
 }
 __device__ __forceinline__ unsigned uor(unsigned v) {
-  for (int o = 32; o > 0; o >>= 1) v |= unsigned(__shfl_xor(int(v), o, 64));
-  return v;
+  v |= dpp<0x111>(0u, v);
+  v |= dpp<0x112>(0u, v);
+  v |= dpp<0x114>(0u, v);
+  v |= dpp<0x118>(0u, v);
+  v |= dpp<0x142, 0xa>(0u, v);
+  v |= dpp<0x143, 0xc>(0u, v);
+  return unsigned(__builtin_amdgcn_readlane(int(v), 63));
 }
-// value of x at level k (k uniform or per lane), chunks held in x[]
+// value of x at level k (per lane), chunks held in x[]
 template <class T, int CH>
 __device__ __forceinline__ T at_level(const T (&x)[CH], int k) {
   T v = T(0);
@@ -77,13 +119,21 @@ __device__ __forceinline__ T at_level(const T (&x)[CH], int k) {
   }
   return v;
 }
+// ... at a level that is the same in every lane
+template <class T, int CH>
+__device__ __forceinline__ T at_uniform(const T (&x)[CH], int k) {
+  T v = read_lane(x[0], k & 63);
+#pragma unroll
+  for (int j = 1; j < CH; ++j)
+    if ((k >> 6) == j) v = read_lane(x[j], k & 63);
+  return v;
+}
 // value of x at level k+1 for every lane's level k in chunk j (0 above the top chunk)
 template <class T, int CH>
 __device__ __forceinline__ T above(const T (&x)[CH], int j) {
-  const T up = __shfl_down(x[j], 1, 64);
-  T nxt = T(0);
-  if (j + 1 < CH) nxt = __shfl(x[j + 1 < CH ? j + 1 : j], 0, 64);
-  return lane() == 63 ? nxt : up;
+  T top = T(0);
+  if (j + 1 < CH) top = read_lane(x[j + 1 < CH ? j + 1 : j], 0);
+  return dpp<0x130>(top, x[j]);  // whole-wavefront shift: lane l takes lane l + 1
 }
 }  // namespace wv
 
@@ -111,10 +161,18 @@ struct SedTile {
   size_t sbase; // scratch offset of the group's first element
 
   __device__ E* slot(int s) const { return lds + s * (kSedCols * row); }
+  // element e of this group in a scratch plane: a base that the block shares
+  // (scalar registers) and a 32-bit byte offset, so that a load needs no
+  // 64-bit address arithmetic per plane
+  template <class T>
+  __device__ __forceinline__ T& elem(T* plane, int e) const {
+    using B = typename std::conditional<std::is_const<T>::value, const char, char>::type;
+    return *reinterpret_cast<T*>(reinterpret_cast<B*>(plane + sbase) + unsigned(e) * unsigned(sizeof(T)));
+  }
   // One species' planes (the block's column group of each is one contiguous
   // run): masses and numbers pm and raw speeds ph where the point holds the
   // species (pbit of its flags), tendencies pt where they are stored (tbit),
-  // elsewhere dm, 0 and td(x), x the element's place in its LDS plane.  Every
+  // elsewhere dm, 0 and td(plane, element).  Every
   // global load is issued into registers before the first LDS write, so the
   // stage waits for one memory latency instead of one per plane and pass (a
   // load-convert-write loop per plane waits for each load before its write).
@@ -130,20 +188,19 @@ struct SedTile {
     M vm[CH][NM], vt[CH][NT];
     H vh[CH][NH];
     const int n = kSedCols * nz;
-    const size_t base = sbase;
 #pragma unroll
     for (int it = 0; it < CH; ++it) {
       if (!kEveryPass && it * 64 * kSedCols >= n) break;
       const int e = min(int(threadIdx.x) + it * 64 * kSedCols, n - 1);
       if (kAll || (pfe[it] & pbit)) {
 #pragma unroll
-        for (int p = 0; p < NM; ++p) vm[it][p] = pm[p][base + e];
+        for (int p = 0; p < NM; ++p) vm[it][p] = elem(pm[p], e);
 #pragma unroll
-        for (int p = 0; p < NH; ++p) vh[it][p] = ph[p][base + e];
+        for (int p = 0; p < NH; ++p) vh[it][p] = elem(ph[p], e);
       }
       if (kAll || (pfe[it] & tbit)) {
 #pragma unroll
-        for (int p = 0; p < NT; ++p) vt[it][p] = pt[p][base + e];
+        for (int p = 0; p < NT; ++p) vt[it][p] = elem(pt[p], e);
       }
     }
 #pragma unroll
@@ -157,7 +214,7 @@ struct SedTile {
 #pragma unroll
         for (int p = 0; p < NH; ++p) slot(sh[p])[x] = p_ ? E(sval(vh[it][p])) : E(0);
 #pragma unroll
-        for (int p = 0; p < NT; ++p) slot(st[p])[x] = t_ ? E(sval(vt[it][p])) : td(p, x);
+        for (int p = 0; p < NT; ++p) slot(st[p])[x] = t_ ? E(sval(vt[it][p])) : td(p, e);
       }
     }
   }
@@ -168,15 +225,14 @@ struct SedTile {
     R vz[CH];
     H vh[CH];
     const int n = kSedCols * nz;
-    const size_t base = sbase;
 #pragma unroll
     for (int it = 0; it < CH; ++it) {
       pfe[it] = 0u;
       if (!kEveryPass && it * 64 * kSedCols >= n) continue;
       const int e = min(int(threadIdx.x) + it * 64 * kSedCols, n - 1);
       const int cc = e % kSedCols, k = e / kSedCols, c = min(c0 + cc, ncol - 1);
-      pfe[it] = pf[base + e];
-      vh[it] = rho[base + e];
+      pfe[it] = elem(pf, e) & ~kFlagsChanged;
+      vh[it] = elem(rho, e);
       vz[it] = a.f[F_DZ][TEMPO_IDX_STATE(a, c, k)];
     }
 #pragma unroll
@@ -210,11 +266,11 @@ struct SedTile {
         v[p] = in ? slot(st[p])[cc * row + k] : E(0);
         counts = counts || (((cond >> p) & 1u) && v[p] != E(0));
       }
-      if (in && counts) pfe[it] |= tbit;
+      if (in && counts && !(pfe[it] & tbit)) pfe[it] |= tbit | kFlagsChanged;
       const bool sector = kAll || ((__ballot(in && (pfe[it] & tbit)) >> (threadIdx.x & 56u)) & 0xffull) != 0ull;
       if (in && sector) {
 #pragma unroll
-        for (int p = 0; p < NT; ++p) pt[p][sbase + e] = T(v[p]);
+        for (int p = 0; p < NT; ++p) elem(pt[p], e) = T(v[p]);
       }
     }
   }
@@ -306,7 +362,7 @@ __device__ __forceinline__ double wave_sediment(const SedCol<CH>& g, double (&xr
   double sed[CH];
 #pragma unroll
   for (int j = 0; j < CH; ++j) sed[j] = vt[j] * xr[j];
-  const double s0 = __shfl(sed[0], 0, 64);
+  const double s0 = wv::read_lane(sed[0], 0);
 #pragma unroll
   for (int j = 0; j < CH; ++j) {
     const double up = wv::above(sed, j);
@@ -319,7 +375,7 @@ __device__ __forceinline__ double wave_sediment(const SedCol<CH>& g, double (&xr
     }
   }
   if (!precip) return 0.0;
-  const double x0 = __shfl(xr[0], 0, 64);
+  const double x0 = wv::read_lane(xr[0], 0);
   return x0 > kLowLimitPrecip ? s0 * dt * ost : 0.0;
 }
 
@@ -385,12 +441,9 @@ template <int CH>
 __device__ __forceinline__ double wave_up(const double (&x)[CH], int j) { return wv::above(x, j); }
 template <int CH>
 __device__ __forceinline__ double wave_down(const double (&x)[CH], int j, int d) {
-  double v = __shfl_up(x[j], d, 64);
-  if (wv::lane() < d) v = 0.0;
-  if (j > 0) {
-    const double p = __shfl(x[j > 0 ? j - 1 : 0], 64 - d + wv::lane(), 64);
-    if (wv::lane() < d) v = p;
-  }
+  // one level at a time: whole-wavefront shift, lane l takes lane l - 1
+  double v = wv::dpp<0x138>(j > 0 ? wv::read_lane(x[j > 0 ? j - 1 : 0], 63) : 0.0, x[j]);
+  if (d == 2) v = wv::dpp<0x138>(j > 0 ? wv::read_lane(x[j > 0 ? j - 1 : 0], 62) : 0.0, v);
   return v;
 }
 
@@ -685,9 +738,6 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   unsigned pfe[CH];  // flags of the elements this thread loads and stores
   if (threadIdx.x == 0) blk_any = 0;
   T.load_head(a, a.pf, sr + SR_RHO * plane, pfe);
-  unsigned pf0[CH];
-#pragma unroll
-  for (int j = 0; j < CH; ++j) pf0[j] = pfe[j];
   const auto none = [](int, int) { return E(0); };
   const E r1 = E(S_t<R>(kR1)), r2 = E(S_t<R>(kR2));
   __syncthreads();
@@ -711,10 +761,23 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   __syncthreads();
   const unsigned bany = blk_any;
 
-  double pr[5] = {0, 0, 0, 0, 0};
-  int kst[kSubRows] = {1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 0, 0};
+  // each species' precipitation and substep record wait in LDS for the
+  // column's diagnostics
+  __shared__ double pr_s[kSedCols][5];
+  __shared__ int kst_s[kSedCols][kSubRows];
+  double* pr = pr_s[w];
+  int* kst = kst_s[w];
+  if (wv::lane() < 5) pr[wv::lane()] = 0.0;
+  if (wv::lane() < kSubRows) kst[wv::lane()] = wv::lane() < 10 ? 1 : 0;
+  auto record = [&](int q, double precip, int steps, int ktop) {
+    if (wv::lane() == 0) {
+      pr[q] = precip;
+      kst[2 * q] = steps;
+      kst[2 * q + 1] = ktop;
+    }
+  };
   SemiCol<CH> sg;
-  unsigned hash[2] = {0u, 0u};
+  unsigned hash = 0u;
   V rhof[CH], visco[CH];
   if constexpr (kSemi) {
     double* rows = reinterpret_cast<double*>(static_cast<char*>(tile_mem) + sed_lds_bytes<E>(a.nz));
@@ -752,6 +815,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     T.get(5, w, raw2);
     if (any & PF_QR) {
       int steps, ktop;
+      double pq = 0.0;
       wave_fill(rr, raw1, raw2, true, true, dz, g.nzc, dt, vr, v2, steps, ktop);
       if constexpr (kSemi) {  // (:599-615): far fewer substeps, fall speeds refreshed after each
         steps = max(int(R(steps) / R(10.0)) + 1, 1);
@@ -764,8 +828,8 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
           qn[j] = in ? a.fa[F_NR][TEMPO_IDX_STATE(a, c, k)] : V(0);
         }
         for (int n = 0; n < steps; ++n) {
-          wave_semi_sediment(sg, rr, tr, vr, steps, kR1, &pr[0], hash[0]);
-          wave_semi_sediment(sg, xn, tn, v2, steps, kR2, nullptr, hash[0]);
+          wave_semi_sediment(sg, rr, tr, vr, steps, kR1, &pq, hash);
+          wave_semi_sediment(sg, xn, tn, v2, steps, kR2, nullptr, hash);
 #pragma unroll
           for (int j = 0; j < CH; ++j) {
             raw1[j] = raw2[j] = V(0);
@@ -775,11 +839,11 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
           wave_refill(rr, g.nzc, raw1, raw2, vr, v2);
         }
       } else for (int n = 0; n < steps; ++n) {
-        pr[0] += wave_sediment(g, rr, vr, tr, kR1, steps, ktop, dt, true);
+        pq += wave_sediment(g, rr, vr, tr, kR1, steps, ktop, dt, true);
         wave_sediment(g, xn, v2, tn, kR2, steps, ktop, dt, false);
       }
-      kst[0] = steps;
-      kst[1] = ktop;
+      record(0, pq, steps, ktop);
+      if (kSemi && wv::lane() == 0) kst[10] = int(hash);
     }
     T.put(1, w, tr);
     T.put(2, w, tn);
@@ -808,6 +872,8 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     T.get(3, w, raw2);
     if (any & PF_QG) {
       int steps, ktop;
+      double pq = 0.0;
+      hash = 0u;
       wave_fill(xg, raw1, raw2, true, false, dz, g.nzc, dt, v1, v2, steps, ktop);
       const double rb_lim = kM3ToL * kR1 / 800.0;
       if constexpr (kSemi) {  // (:641-667)
@@ -823,9 +889,9 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
           qb[j] = in && has_ngqb ? a.fa[F_QB][TEMPO_IDX_STATE(a, c, k)] : V(0);
         }
         for (int n = 0; n < steps; ++n) {
-          wave_semi_sediment(sg, xg, tg, v1, steps, kR1, &pr[1], hash[1]);
-          wave_semi_sediment(sg, xn, tn, v2, steps, kR2, nullptr, hash[1]);
-          wave_semi_sediment(sg, xb, tb, v1, steps, rb_lim, nullptr, hash[1]);
+          wave_semi_sediment(sg, xg, tg, v1, steps, kR1, &pq, hash);
+          wave_semi_sediment(sg, xn, tn, v2, steps, kR2, nullptr, hash);
+          wave_semi_sediment(sg, xb, tb, v1, steps, rb_lim, nullptr, hash);
 #pragma unroll
           for (int j = 0; j < CH; ++j) {
             raw1[j] = raw2[j] = V(0);
@@ -836,12 +902,12 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
           wave_refill(xg, g.nzc, raw1, raw2, v1, v2);
         }
       } else for (int n = 0; n < steps; ++n) {
-        pr[1] += wave_sediment(g, xg, v1, tg, kR1, steps, ktop, dt, true);
+        pq += wave_sediment(g, xg, v1, tg, kR1, steps, ktop, dt, true);
         wave_sediment(g, xn, v2, tn, kR2, steps, ktop, dt, false);
         wave_sediment(g, xb, v1, tb, rb_lim, steps, ktop, dt, false);
       }
-      kst[2] = steps;
-      kst[3] = ktop;
+      record(1, pq, steps, ktop);
+      if (kSemi && wv::lane() == 0) kst[11] = int(hash);
     }
     T.put(4, w, tg);
     T.put(5, w, tn);
@@ -878,9 +944,9 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
       double unused[CH];
       int steps, ktop;
       wave_fill(xs, vraw, vraw, false, false, dz, g.nzc, dt, v1, unused, steps, ktop);
-      for (int n = 0; n < steps; ++n) pr[2] += wave_sediment(g, xs, v1, ts, kR1, steps, ktop, dt, true);
-      kst[4] = steps;
-      kst[5] = ktop;
+      double pq = 0.0;
+      for (int n = 0; n < steps; ++n) pq += wave_sediment(g, xs, v1, ts, kR1, steps, ktop, dt, true);
+      record(2, pq, steps, ktop);
     }
     T.put(1, w, ts);
     __syncthreads();
@@ -905,10 +971,9 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     if (any & PF_QI) {
       int steps, ktop;
       wave_fill(xi, raw1, raw2, true, false, dz, g.nzc, dt, v1, v2, steps, ktop);
-      pr[3] += wave_sediment(g, xi, v1, ti, kR1, steps, ktop, dt, true);
+      const double pq = wave_sediment(g, xi, v1, ti, kR1, steps, ktop, dt, true);
       wave_sediment(g, xn, v2, tn, kR2, steps, ktop, dt, false);
-      kst[6] = steps;
-      kst[7] = ktop;
+      record(3, pq, steps, ktop);
     }
     T.put(2, w, ti);
     T.put(4, w, tn);
@@ -921,19 +986,15 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   if (bany & PF_QC) {
     double xc[CH], xn[CH], tc[CH], tn[CH], v1[CH], v2[CH];
     V raw1[CH], raw2[CH];
-    // slot 3 keeps the density while slot 2 takes the tendency: a one-moment
-    // cloud's number tendency is, where not stored, that of clear air
+    // a one-moment cloud's number tendency is, where not stored, clear air's
     const bool has_nc = a.f[F_NC] != nullptr;
-    for (int j = 0; j < CH; ++j) {
-      const int k = j * 64 + wv::lane();
-      if (k < a.nz) T.slot(3)[w * T.row + k] = E(rho[j]);
-    }
-    __syncthreads();
+    const R* rho_p = sr + SR_RHO * plane;
     T.template load_species<kAll>(
         pfe, PF_QC, PF_TC, {0, 1}, {sd + SD_RC * plane, sd + SD_NC * plane}, {r1, E(S_t<R>(kNtCMin))}, {5, 6},
         {sr + SR_VTRC * plane, sr + SR_VTNC * plane}, {2, 4}, {sd + SD_QCTEN * plane, sd + SD_NCTEN * plane},
-        [&](int p, int x) {
-          return p == 0 || has_nc ? E(0) : E(-S_t<R>(kNtCMin) * (S_t<R>(1) / S_t<R>(T.slot(3)[x])) * S_t<R>(a.odt));
+        [&](int p, int e) {
+          if (p == 0 || has_nc) return E(0);
+          return E(-S_t<R>(kNtCMin) * (S_t<R>(1) / S_t<R>(sval(T.elem(rho_p, e)))) * S_t<R>(a.odt));
         });
     __syncthreads();
     T.get(0, w, xc);
@@ -946,8 +1007,8 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
       int kt = 1;
       V hgt = V(0.0);
       for (int k = 0; k < g.nzc - 1; ++k) {  // uniform loop: every lane follows level k
-        if (wv::at_level(xc, k) > kR2) kt = k + 1;
-        hgt = hgt + wv::at_level(dz, k);
+        if (wv::at_uniform(xc, k) > kR2) kt = k + 1;
+        hgt = hgt + wv::at_uniform(dz, k);
         if (hgt > V(500.0)) break;
       }
 #pragma unroll
@@ -956,10 +1017,9 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
         v1[j] = (k < kt) ? double(raw1[j]) : 0.0;
         v2[j] = (k < kt) ? double(raw2[j]) : 0.0;
       }
-      pr[4] += wave_sediment(g, xc, v1, tc, kR1, 1, kt, dt, true);
+      const double pq = wave_sediment(g, xc, v1, tc, kR1, 1, kt, dt, true);
       wave_sediment(g, xn, v2, tn, kR2, 1, kt, dt, false);
-      kst[8] = 1;
-      kst[9] = kt;
+      record(4, pq, 1, kt);
     }
     T.put(2, w, tc);
     T.put(4, w, tn);
@@ -971,14 +1031,13 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
 #pragma unroll
     for (int it = 0; it < CH; ++it) {
       const int e = int(threadIdx.x) + it * 64 * kSedCols;
-      if (e < kSedCols * a.nz && c0 + e % kSedCols < a.ncol && pfe[it] != pf0[it]) a.pf[T.sbase + e] = pfe[it];
+      if (e < kSedCols * a.nz && c0 + e % kSedCols < a.ncol && (pfe[it] & kFlagsChanged))
+        T.elem(a.pf, e) = pfe[it] & ~kFlagsChanged;
     }
   }
 
   if (!col_ok || wv::lane() != 0) return;
   for (int q = 0; q < 5; ++q) a.precip[size_t(q) * a.ncol + c] = pr[q];
-  kst[10] = int(hash[0]);
-  kst[11] = int(hash[1]);
   if (a.ksub)
     for (int q = 0; q < kSubRows; ++q) a.ksub[size_t(q) * a.ncol + c] = kst[q];
   // column diagnostics (src/module_mp_tempo_main.F90:784-794, driver :452-457)
@@ -1000,13 +1059,15 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
 }
 
 // waves per SIMD by chunks: one chunk fits 8 without spills, two are held to
-// 6 (56 B of spills; measured faster than 4 without), three and four take
-// what their registers allow.  Against one lane per column the wavefront
-// form takes, for the whole step, 0.41 instead of 2.93 ms at 8,191 x 160
-// (FP32; one lane per column is 128 wavefronts on 256 CUs).  Two chunks with
-// 4-byte instead of 8-byte staging: 131,072 uneven columns of 30-128 levels
-// 4.70 -> 4.42 ms a step.
-constexpr int sed_waves(int chunks) { return chunks <= 1 ? 8 : chunks == 2 ? 6 : chunks == 3 ? 4 : 3; }
+// 6, three and four take what their registers allow.  A spill is a
+// scratch-memory access in every stage and dominates soon: two chunks held to
+// 8 waves (128 B of spills) take 1.20 ms at 100,000 x 90 against 0.50 at 6
+// (52 B) and 0.42 with precipitation sums and substep records kept in LDS
+// and 32-bit plane offsets (12 B); at 5 waves 0.49 before that.
+// Against one lane per column the wavefront form takes, for the whole step,
+// 0.33 instead of 2.93 ms at 8,191 x 160 (FP32; one lane per column is 128
+// wavefronts on 256 CUs).
+constexpr int sed_waves(int chunks) { return chunks <= 1 ? 7 : chunks == 2 ? 6 : chunks == 3 ? 4 : 3; }
 template <class R, int CH, bool kEveryPass = false>
 __global__ void __launch_bounds__(64 * kSedCols) __attribute__((amdgpu_waves_per_eu(sed_waves(CH)))) k_phase_b_wave(StepArgs<R> a) {
   extern __shared__ double tile_mem[];  // sed_lds_bytes<SedStage<R>>(nz)
