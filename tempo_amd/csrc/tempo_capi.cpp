@@ -26,8 +26,8 @@ hipError_t launch_step(const StepArgs<float>& a, const LaunchCfg& lc, double* vt
 hipError_t launch_step(const StepArgs<double>& a, const LaunchCfg& lc, double* vtbuf, hipStream_t s, hipEvent_t* ev);
 hipError_t launch_step_sig(const StepArgs<float>& a, const LaunchCfg& lc, double* vtbuf, hipStream_t s);
 hipError_t launch_step_sig(const StepArgs<double>& a, const LaunchCfg& lc, double* vtbuf, hipStream_t s);
-hipError_t launch_step_tlm(const StepArgs<Dual<float>>& a, Dual<double>* vtbuf, hipStream_t s);
-hipError_t launch_step_tlm(const StepArgs<Dual<double>>& a, Dual<double>* vtbuf, hipStream_t s);
+hipError_t launch_step_tlm(const StepArgs<Dual<float>>& a, const LaunchCfg& lc, Dual<double>* vtbuf, hipStream_t s);
+hipError_t launch_step_tlm(const StepArgs<Dual<double>>& a, const LaunchCfg& lc, Dual<double>* vtbuf, hipStream_t s);
 template <class T>
 hipError_t launch_dual_pack(const T* v, const T* t, const DualGeom& g, Dual<T>* out, hipStream_t s);
 template <class R>
@@ -743,7 +743,7 @@ int run_tlm(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_fields*
   a.d2ldj = ncol;
   int rc = bind_common(x, a, dt, itimestep);
   if (rc) return rc;
-  HIP_TRY(launch_step_tlm(a, x->vtbuf.as<Dual<double>>(), s));
+  HIP_TRY(launch_step_tlm(a, x->launch[sizeof(T) == 8 ? 1 : 0], x->vtbuf.as<Dual<double>>(), s));
   for (int i = 0; i < F_NFIELDS; ++i)
     if (fp[i]) HIP_TRY(launch_dual_unpack(a.f[i], g3, static_cast<T*>(fp[i]), static_cast<T*>(tp[i]), s));
   DualGeom g2{dm->ni, dm->nj, 1, 0, dm->d2ldj};

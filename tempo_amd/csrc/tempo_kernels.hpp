@@ -1694,14 +1694,4 @@ hipError_t launch_dual_unpack(const Dual<T>* in, const DualGeom& g, T* v, T* t, 
   return hipGetLastError();
 }
 
-// the four launches of one tangent-linear step (sedimentation one lane per column)
-template <class D>
-hipError_t launch_step_tlm_impl(const StepArgs<D>& a, Dual<double>* vtbuf, hipStream_t s) {
-  launch_prepass(a, s);
-  hipLaunchKernelGGL(k_phase_a<D>, level_grid(a, 256), dim3(256), 0, s, a);
-  hipLaunchKernelGGL(k_phase_b<D>, dim3(unsigned((a.ncol + 127) / 128)), dim3(128), 0, s, a, vtbuf);
-  hipLaunchKernelGGL(k_phase_c<D>, level_grid(a, 256), dim3(256), 0, s, a);
-  return hipGetLastError();
-}
-
 }  // namespace tempo

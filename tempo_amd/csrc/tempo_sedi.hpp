@@ -45,6 +45,16 @@ constexpr int kSedLevels = 64 * kSedChunks;
 // where eight FP64 planes take 82 KB, it decides between one block and four.
 template <class R>
 using SedStage = typename std::conditional<std::is_same<Sd_t<R>, float>::value, float, double>::type;
+// The kernel's types: X of masses, tendencies and speeds while they sediment,
+// V of level geometry and raw speeds, E of the staged planes.  A dual working
+// type runs on the values alone (the tangent-free forward of an adjoint), or,
+// with kTan, on duals throughout (the tangent-linear step).
+template <class R, bool kTan>
+struct SedTypes {
+  using X = typename std::conditional<kTan, W_t<R>, double>::type;
+  using V = typename std::conditional<kTan, R, S_t<R>>::type;
+  using E = typename std::conditional<kTan, W_t<R>, SedStage<R>>::type;
+};
 // LDS row of one column, in stage elements: at least nz, and an odd multiple
 // of 8 (4-byte elements) or 4 (8-byte), so that the 8 columns x 8 (4) levels
 // that a wavefront (half one) writes at a time fall in 64 different banks
@@ -87,6 +97,14 @@ __device__ __forceinline__ T read_lane(T x, int l) {
     const unsigned hi = unsigned(__builtin_amdgcn_readlane(int(v >> 32), l));
     return __builtin_bit_cast(T, (static_cast<unsigned long long>(hi) << 32) | lo);
   }
+}
+template <int ctrl, int rows = 0xf, class T>
+__device__ __forceinline__ Dual<T> dpp(Dual<T> old, Dual<T> x) {
+  return {dpp<ctrl, rows>(old.v, x.v), dpp<ctrl, rows>(old.d, x.d)};
+}
+template <class T>
+__device__ __forceinline__ Dual<T> read_lane(Dual<T> x, int l) {
+  return {read_lane(x.v, l), read_lane(x.d, l)};
 }
 // maximum (of non-negative values) and bitwise or over the wavefront: row
 // shifts by 1, 2, 4, 8, then the rows' last lanes broadcast upwards
@@ -144,6 +162,13 @@ __device__ __forceinline__ double sval(float x) { return double(x); }
 template <class T>
 __device__ __forceinline__ double sval(const Dual<T>& x) {
   return double(x.v);
+}
+
+// a stored number as a staged one
+template <class E, class T>
+__device__ __forceinline__ E staged(const T& x) {
+  if constexpr (IsDual<E>::value) return E(x);
+  else return E(sval(x));
 }
 
 // Block-wide staging of (level, column) planes through LDS slots.  Loads
@@ -210,11 +235,11 @@ struct SedTile {
         const int cc = e % kSedCols, k = e / kSedCols, x = cc * row + k;
         const bool p_ = kAll || (pfe[it] & pbit), t_ = kAll || (pfe[it] & tbit);
 #pragma unroll
-        for (int p = 0; p < NM; ++p) slot(sm[p])[x] = p_ ? E(sval(vm[it][p])) : dm[p];
+        for (int p = 0; p < NM; ++p) slot(sm[p])[x] = p_ ? staged<E>(vm[it][p]) : dm[p];
 #pragma unroll
-        for (int p = 0; p < NH; ++p) slot(sh[p])[x] = p_ ? E(sval(vh[it][p])) : E(0);
+        for (int p = 0; p < NH; ++p) slot(sh[p])[x] = p_ ? staged<E>(vh[it][p]) : E(0);
 #pragma unroll
-        for (int p = 0; p < NT; ++p) slot(st[p])[x] = t_ ? E(sval(vt[it][p])) : td(p, e);
+        for (int p = 0; p < NT; ++p) slot(st[p])[x] = t_ ? staged<E>(vt[it][p]) : td(p, e);
       }
     }
   }
@@ -240,9 +265,9 @@ struct SedTile {
       const int e = int(threadIdx.x) + it * 64 * kSedCols;
       if (e < n) {
         const int cc = e % kSedCols, k = e / kSedCols, x = cc * row + k;
-        slot(0)[x] = E(pfe[it]);
-        slot(1)[x] = c0 + cc < ncol ? E(sval(vz[it])) : E(0);
-        slot(2)[x] = E(sval(vh[it]));
+        slot(0)[x] = E(double(pfe[it]));
+        slot(1)[x] = c0 + cc < ncol ? staged<E>(vz[it]) : E(0);
+        slot(2)[x] = staged<E>(vh[it]);
       }
     }
   }
@@ -296,20 +321,20 @@ struct SedTile {
 };
 
 // Per-column level geometry held by every lane.
-template <int CH>
+template <int CH, class X = double>
 struct SedCol {
   int nzc;                          // active levels
-  double odz[CH], orho[CH];
+  X odz[CH], orho[CH];
 };
 
 // top-down fill (:1768-1789): out(k) = raw(k') at the lowest k' >= k whose
 // mass exceeds r1 (0 when none); CFL substeps and ktop from the filled
 // speeds in the working precision.
-template <class R, int CH>
-__device__ __forceinline__ void wave_fill(const double (&mass)[CH], const R (&raw1)[CH],
+template <class R, int CH, class X>
+__device__ __forceinline__ void wave_fill(const X (&mass)[CH], const R (&raw1)[CH],
                                           const R (&raw2)[CH], bool two, bool use_max,
-                                          const R (&dz)[CH], int nzc, double dt, double (&out1)[CH],
-                                          double (&out2)[CH], int& substeps, int& ktop) {
+                                          const R (&dz)[CH], int nzc, double dt, X (&out1)[CH],
+                                          X (&out2)[CH], int& substeps, int& ktop) {
 #pragma clang fp contract(off)  // as the lane-per-column kernel: every operation rounded on its own
   unsigned long long m[CH];
 #pragma unroll
@@ -332,8 +357,8 @@ __device__ __forceinline__ void wave_fill(const double (&mass)[CH], const R (&ra
     }
     const R r1 = wv::at_level(raw1, src < 0 ? 0 : src);
     const R r2 = two ? wv::at_level(raw2, src < 0 ? 0 : src) : R(0);
-    const double v1 = src < 0 ? 0.0 : double(r1);
-    const double v2 = src < 0 ? 0.0 : double(r2);
+    const X v1 = src < 0 ? X(0.0) : X(r1);
+    const X v2 = src < 0 ? X(0.0) : X(r2);
     out1[j] = v1;
     out2[j] = v2;
     if (k < nzc) {
@@ -353,30 +378,29 @@ __device__ __forceinline__ void wave_fill(const double (&mass)[CH], const R (&ra
 
 // one flux-form substep of one field (:1516-1559); returns the surface
 // precipitation increment (0 when the caller does not accumulate it)
-template <int CH>
-__device__ __forceinline__ double wave_sediment(const SedCol<CH>& g, double (&xr)[CH],
-                                                const double (&vt)[CH], double (&xten)[CH],
-                                                double limit, int steps, int ktop, double dt, bool precip) {
+template <int CH, class X>
+__device__ __forceinline__ X wave_sediment(const SedCol<CH, X>& g, X (&xr)[CH], const X (&vt)[CH], X (&xten)[CH],
+                                           double limit, int steps, int ktop, double dt, bool precip) {
 #pragma clang fp contract(off)  // as the lane-per-column kernel: every operation rounded on its own
   const double ost = 1.0 / double(steps);
-  double sed[CH];
+  X sed[CH];
 #pragma unroll
   for (int j = 0; j < CH; ++j) sed[j] = vt[j] * xr[j];
-  const double s0 = wv::read_lane(sed[0], 0);
+  const X s0 = wv::read_lane(sed[0], 0);
 #pragma unroll
   for (int j = 0; j < CH; ++j) {
-    const double up = wv::above(sed, j);
+    const X up = wv::above(sed, j);
     const int k = j * 64 + wv::lane();
     if (k < g.nzc && (k == g.nzc - 1 || k <= ktop - 1)) {
-      const double flux = (k == g.nzc - 1) ? -sed[j] : (up - sed[j]);
+      const X flux = (k == g.nzc - 1) ? -sed[j] : (up - sed[j]);
       xten[j] = xten[j] + flux * g.odz[j] * ost * g.orho[j];
-      const double v = xr[j] + flux * g.odz[j] * dt * ost;
-      xr[j] = v > limit ? v : limit;
+      const X v = xr[j] + flux * g.odz[j] * dt * ost;
+      xr[j] = v > limit ? v : X(limit);
     }
   }
-  if (!precip) return 0.0;
-  const double x0 = wv::read_lane(xr[0], 0);
-  return x0 > kLowLimitPrecip ? s0 * dt * ost : 0.0;
+  if (!precip) return X(0.0);
+  const X x0 = wv::read_lane(xr[0], 0);
+  return x0 > kLowLimitPrecip ? s0 * dt * ost : X(0.0);
 }
 
 // ---- semi-Lagrangian sedimentation on the wavefront --------------------
@@ -706,21 +730,22 @@ __device__ __forceinline__ void semi_graupel_level(const StepArgs<R>& a, R rho, 
 // tangent-free forward of an adjoint.
 // kSemi: semi-Lagrangian rain and graupel, with semi_lds_bytes(nz) more LDS
 // behind the tile.
-template <class R, int CH = kSedChunks, bool kEveryPass = false, bool kSemi = false>
+template <class R, int CH = kSedChunks, bool kEveryPass = false, bool kSemi = false, bool kTan = false>
 __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void* tile_mem) {
   __shared__ unsigned blk_any;
   const int w = int(threadIdx.x >> 6);
   const int c = c0 + w;
   const bool col_ok = c < a.ncol;
   const size_t plane = a.plane;
-  using E = SedStage<R>;
+  using E = typename SedTypes<R, kTan>::E;
+  using X = typename SedTypes<R, kTan>::X;
   const SedTile<E, CH, kEveryPass> T{static_cast<E*>(tile_mem), c0, a.ncol, a.nz, a.nzs, sed_row<E>(a.nz), TEMPO_IDX_SCR(a, c0, 0)};
   const double dt = a.dt;
   Sd_t<R>* sd = a.sd;
   const R* sr = a.sr;
-  using V = typename Num<R>::S;
+  using V = typename SedTypes<R, kTan>::V;
 
-  SedCol<CH> g;
+  SedCol<CH, X> g;
   g.nzc = col_ok ? (a.nlev ? min(max(a.nlev[c], 1), a.nz) : a.nz) : 0;
   if (a.sig && col_ok) {  // signature run: this kernel's decisions are per column (tempo_hip_substeps)
     const size_t n3 = size_t(a.ncol) * size_t(a.nz);
@@ -743,7 +768,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   __syncthreads();
   unsigned pfl[CH];
   V dz[CH], rho[CH];
-  double rr[CH], vr[CH];
+  X rr[CH], vr[CH];
   T.get(0, w, pfl);
   T.get(1, w, dz);
   T.get(2, w, rho);
@@ -751,10 +776,10 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
 #pragma unroll
   for (int j = 0; j < CH; ++j) {
     if (j * 64 + wv::lane() < g.nzc) any |= pfl[j];
-    g.odz[j] = 1.0 / double(dz[j]);
-    g.orho[j] = 1.0 / double(rho[j]);
-    vr[j] = 0.0;
-    rr[j] = r1;
+    g.odz[j] = X(1.0) / X(dz[j]);
+    g.orho[j] = X(1.0) / X(rho[j]);
+    vr[j] = X(0.0);
+    rr[j] = X(r1);
   }
   any = live ? wv::uor(any) : 0u;
   if (wv::lane() == 0 && any) atomicOr(&blk_any, any);
@@ -763,13 +788,13 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
 
   // each species' precipitation and substep record wait in LDS for the
   // column's diagnostics
-  __shared__ double pr_s[kSedCols][5];
+  __shared__ double pr_s[kSedCols][5 * (sizeof(X) / sizeof(double))];
   __shared__ int kst_s[kSedCols][kSubRows];
-  double* pr = pr_s[w];
+  X* pr = reinterpret_cast<X*>(pr_s[w]);
   int* kst = kst_s[w];
-  if (wv::lane() < 5) pr[wv::lane()] = 0.0;
+  if (wv::lane() < 5) pr[wv::lane()] = X(0.0);
   if (wv::lane() < kSubRows) kst[wv::lane()] = wv::lane() < 10 ? 1 : 0;
-  auto record = [&](int q, double precip, int steps, int ktop) {
+  auto record = [&](int q, X precip, int steps, int ktop) {
     if (wv::lane() == 0) {
       pr[q] = precip;
       kst[2 * q] = steps;
@@ -801,7 +826,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
 
   // ---- rain (:603-630) ----
   if (bany & PF_QR) {
-    double xn[CH], tr[CH], tn[CH], v2[CH];
+    X xn[CH], tr[CH], tn[CH], v2[CH];
     V raw1[CH], raw2[CH];
     T.template load_species<kAll>(pfe, PF_QR, PF_TR, {3, 0}, {sd + SD_RR * plane, sd + SD_NR * plane}, {r1, r2}, {4, 5},
                                   {sr + SR_VTRR * plane, sr + SR_VTNR * plane}, {1, 2},
@@ -815,7 +840,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     T.get(5, w, raw2);
     if (any & PF_QR) {
       int steps, ktop;
-      double pq = 0.0;
+      X pq = X(0.0);
       wave_fill(rr, raw1, raw2, true, true, dz, g.nzc, dt, vr, v2, steps, ktop);
       if constexpr (kSemi) {  // (:599-615): far fewer substeps, fall speeds refreshed after each
         steps = max(int(R(steps) / R(10.0)) + 1, 1);
@@ -854,8 +879,8 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
 
   // ---- graupel (:632-660) ----
   if (bany & PF_QG) {
-    double xg[CH], xn[CH], xb[CH], tg[CH], tn[CH], tb[CH];
-    double v1[CH], v2[CH];
+    X xg[CH], xn[CH], xb[CH], tg[CH], tn[CH], tb[CH];
+    X v1[CH], v2[CH];
     V raw1[CH], raw2[CH];
     const E rb0 = E(S_t<R>(kM3ToL) * S_t<R>(kR1) / rho_g<S_t<R>>(kIdxBg1));
     T.template load_species<kAll>(pfe, PF_QG, PF_TG, {0, 1, 2}, {sd + SD_RG * plane, sd + SD_NG * plane, sd + SD_RB * plane},
@@ -872,7 +897,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     T.get(3, w, raw2);
     if (any & PF_QG) {
       int steps, ktop;
-      double pq = 0.0;
+      X pq = X(0.0);
       hash = 0u;
       wave_fill(xg, raw1, raw2, true, false, dz, g.nzc, dt, v1, v2, steps, ktop);
       const double rb_lim = kM3ToL * kR1 / 800.0;
@@ -921,7 +946,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   // ---- snow (:662-697): mixes in the filled rain speed where snow melts,
   // with the rain mass after rain sedimentation ----
   if (bany & PF_QS) {
-    double xs[CH], ts[CH], v1[CH];
+    X xs[CH], ts[CH], v1[CH];
     V raw[CH];
     T.template load_species<kAll>(pfe, PF_QS, PF_TS, {0}, {sd + SD_RS * plane}, {r1}, {2}, {sr + SR_VTS * plane}, {1},
                                   {sd + SD_QSTEN * plane}, none);
@@ -941,10 +966,10 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
         }
         vraw[j] = v;
       }
-      double unused[CH];
+      X unused[CH];
       int steps, ktop;
       wave_fill(xs, vraw, vraw, false, false, dz, g.nzc, dt, v1, unused, steps, ktop);
-      double pq = 0.0;
+      X pq = X(0.0);
       for (int n = 0; n < steps; ++n) pq += wave_sediment(g, xs, v1, ts, kR1, steps, ktop, dt, true);
       record(2, pq, steps, ktop);
     }
@@ -956,7 +981,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
 
   // ---- ice (:699-715): one call with steps = substeps ----
   if (bany & PF_QI) {
-    double xi[CH], xn[CH], ti[CH], tn[CH], v1[CH], v2[CH];
+    X xi[CH], xn[CH], ti[CH], tn[CH], v1[CH], v2[CH];
     V raw1[CH], raw2[CH];
     T.template load_species<kAll>(pfe, PF_QI, PF_TI, {0, 1}, {sd + SD_RI * plane, sd + SD_NI * plane}, {r1, r2}, {5, 6},
                                   {sr + SR_VTRI * plane, sr + SR_VTNI * plane}, {2, 4},
@@ -971,7 +996,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     if (any & PF_QI) {
       int steps, ktop;
       wave_fill(xi, raw1, raw2, true, false, dz, g.nzc, dt, v1, v2, steps, ktop);
-      const double pq = wave_sediment(g, xi, v1, ti, kR1, steps, ktop, dt, true);
+      const X pq = wave_sediment(g, xi, v1, ti, kR1, steps, ktop, dt, true);
       wave_sediment(g, xn, v2, tn, kR2, steps, ktop, dt, false);
       record(3, pq, steps, ktop);
     }
@@ -984,7 +1009,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
 
   // ---- cloud (:717-727, cloud_fallspeed :1945-1977): below 500 m only ----
   if (bany & PF_QC) {
-    double xc[CH], xn[CH], tc[CH], tn[CH], v1[CH], v2[CH];
+    X xc[CH], xn[CH], tc[CH], tn[CH], v1[CH], v2[CH];
     V raw1[CH], raw2[CH];
     // a one-moment cloud's number tendency is, where not stored, clear air's
     const bool has_nc = a.f[F_NC] != nullptr;
@@ -1014,10 +1039,10 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
 #pragma unroll
       for (int j = 0; j < CH; ++j) {
         const int k = j * 64 + wv::lane();
-        v1[j] = (k < kt) ? double(raw1[j]) : 0.0;
-        v2[j] = (k < kt) ? double(raw2[j]) : 0.0;
+        v1[j] = (k < kt) ? X(raw1[j]) : X(0.0);
+        v2[j] = (k < kt) ? X(raw2[j]) : X(0.0);
       }
-      const double pq = wave_sediment(g, xc, v1, tc, kR1, 1, kt, dt, true);
+      const X pq = wave_sediment(g, xc, v1, tc, kR1, 1, kt, dt, true);
       wave_sediment(g, xn, v2, tn, kR2, 1, kt, dt, false);
       record(4, pq, 1, kt);
     }
@@ -1088,6 +1113,34 @@ void launch_phase_b_semi_wave(const StepArgs<R>& a, hipStream_t s) {
     hipLaunchKernelGGL((k_phase_b_semi_wave<R, 1>), g, b, lds, s, a);
   else
     hipLaunchKernelGGL((k_phase_b_semi_wave<R, 2>), g, b, lds, s, a);
+}
+
+// ... of the tangent-linear step: duals throughout
+template <class R, int CH>
+__global__ void __launch_bounds__(64 * kSedCols) k_phase_b_tan_wave(StepArgs<R> a) {
+  extern __shared__ double tile_mem[];  // sed_lds_bytes<W_t<R>>(nz)
+  phase_b_group<R, CH, false, false, true>(a, int(blockIdx.x) * kSedCols, tile_mem);
+}
+// the four launches of one tangent-linear step; sedimentation one wavefront
+// per column in flux form up to kSedLevels levels, else one lane per column.
+// 8,192 columns are 128 wavefronts at one lane per column: 840 of the step's
+// 1364 us at 64 levels (FP32), against 63 of 553 us here.
+template <class D>
+hipError_t launch_step_tlm_impl(const StepArgs<D>& a, const LaunchCfg& lc, Dual<double>* vtbuf, hipStream_t s) {
+  launch_prepass(a, s);
+  hipLaunchKernelGGL(k_phase_a<D>, level_grid(a, 256), dim3(256), 0, s, a);
+  if (lc.sed_wave && a.nz <= kSedLevels && !a.fl.semi_sedi) {
+    const dim3 g(unsigned((a.ncol + kSedCols - 1) / kSedCols)), b(64 * kSedCols);
+    const size_t lds = sed_lds_bytes<Dual<double>>(a.nz);
+    if (a.nz <= 64)
+      hipLaunchKernelGGL((k_phase_b_tan_wave<D, 1>), g, b, lds, s, a);
+    else
+      hipLaunchKernelGGL((k_phase_b_tan_wave<D, 2>), g, b, lds, s, a);
+  } else {
+    hipLaunchKernelGGL(k_phase_b<D>, dim3(unsigned((a.ncol + 127) / 128)), dim3(128), 0, s, a, vtbuf);
+  }
+  hipLaunchKernelGGL(k_phase_c<D>, level_grid(a, 256), dim3(256), 0, s, a);
+  return hipGetLastError();
 }
 
 // nz <= kSedMaxLevels (dual working types: kSedLevels)

@@ -18,8 +18,8 @@ hipError_t launch_step_sig(const StepArgs<float>& a, const LaunchCfg& lc, double
 }
 
 // tangent-linear step in this precision (same contraction flags as the step)
-hipError_t launch_step_tlm(const StepArgs<Dual<float>>& a, Dual<double>* vtbuf, hipStream_t s) {
-  return launch_step_tlm_impl(a, vtbuf, s);
+hipError_t launch_step_tlm(const StepArgs<Dual<float>>& a, const LaunchCfg& lc, Dual<double>* vtbuf, hipStream_t s) {
+  return launch_step_tlm_impl(a, lc, vtbuf, s);
 }
 template hipError_t launch_check_update<float>(const CheckArgs<float>&, int, hipStream_t);
 template hipError_t launch_surface_emissions<float>(float*, const float*, int, int, long long, long long, long long, int,

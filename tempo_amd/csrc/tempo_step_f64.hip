@@ -18,8 +18,8 @@ hipError_t launch_step_sig(const StepArgs<double>& a, const LaunchCfg& lc, doubl
 }
 
 // tangent-linear step in this precision (same contraction flags as the step)
-hipError_t launch_step_tlm(const StepArgs<Dual<double>>& a, Dual<double>* vtbuf, hipStream_t s) {
-  return launch_step_tlm_impl(a, vtbuf, s);
+hipError_t launch_step_tlm(const StepArgs<Dual<double>>& a, const LaunchCfg& lc, Dual<double>* vtbuf, hipStream_t s) {
+  return launch_step_tlm_impl(a, lc, vtbuf, s);
 }
 template hipError_t launch_check_update<double>(const CheckArgs<double>&, int, hipStream_t);
 template hipError_t launch_surface_emissions<double>(double*, const double*, int, int, long long, long long, long long, int,

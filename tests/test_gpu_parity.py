@@ -1359,3 +1359,49 @@ def test_gpu_clear_air_and_sparse_planes(hip, dtype, form):
         ctx.set_run_cfg(cloud_condensation_flag=1, turn_off_micro_flag=0)
     for k, v in got[1].items():
         assert np.array_equal(v, got[0][k], equal_nan=True), k
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "fp64"])
+@pytest.mark.parametrize("hail", [True, False])
+@pytest.mark.parametrize("nz", [2, 63, 64, 65, 127, 128, 129])
+def test_gpu_tangent_sedimentation_level_counts(hip, dtype, hail, nz):
+    """the tangent-linear step with a wavefront per column against one lane
+    per column at the chunk edges, 45 columns (the last group cut short): FP64
+    values and tangents bit for bit; FP32 to 128 levels' worth of roundings of
+    the largest element (the two kernels may fuse different multiply-adds)"""
+    import torch
+    from tempo_amd import generator as gen
+    ctx = context(hip, dict(aerosolaware=True, hailaware=hail))
+    prec = hip.FP32 if dtype == "fp32" else hip.FP64
+    td = torch.float32 if dtype == "fp32" else torch.float64
+    st, m = gen.generate("multistep", ncol=45, col0=2468)
+    if not hail:
+        st.pop("ng")
+        st.pop("qb")
+    x_old, x_new = np.arange(90, dtype=np.float64), np.linspace(0.0, 60.0, nz)
+    st = {k: np.ascontiguousarray(np.stack([np.interp(x_new, x_old, v[:, c]) for c in range(45)], axis=1))
+          for k, v in st.items()}
+    st["dz"] = st["dz"] * min(1.0, 90.0 / nz) * 0.5
+    nlev = np.maximum(2, nz - np.arange(45) % max(1, nz // 2)).astype(np.int32)
+    rng = np.random.default_rng(nz)
+    tan = {k: v * rng.uniform(-1e-3, 1e-3, v.shape) for k, v in st.items()}
+    got = {}
+    try:
+        for wave in (1, 0):
+            ctx.tune(prec, hip.TUNE_SED_WAVE, wave)
+            dev = {k: torch.tensor(v, dtype=td, device="cuda") for k, v in st.items()}
+            dtan = {k: torch.tensor(v, dtype=td, device="cuda") for k, v in tan.items()}
+            d, t, dtan = ctx.tlm(dev, dtan, m["dt"], 2, nlev=torch.tensor(nlev, device="cuda"))
+            got[wave] = {**{k: v.cpu().numpy() for k, v in dev.items()},
+                         **{"tan_" + k: v.cpu().numpy() for k, v in dtan.items()},
+                         **{k: v.cpu().numpy() for k, v in d.items()},
+                         **{"tan_" + k: v.cpu().numpy() for k, v in t.items()}}
+    finally:
+        ctx.tune(prec, hip.TUNE_SED_WAVE, 1)
+    below = np.arange(nz)[:, None] < nlev[None, :]  # diagnostics are not defined above a column's depth
+    for k, v in got[1].items():
+        v, w = (v[below], got[0][k][below]) if v.ndim == 2 else (v, got[0][k])
+        if dtype == "fp64":
+            assert np.array_equal(v, w, equal_nan=True), (k, nz)
+        else:
+            assert np.abs(v - w).max() <= 128 * 2.0**-23 * np.abs(w).max(), (k, nz)
