@@ -516,65 +516,69 @@ __global__ void __launch_bounds__(64) k_adj_sedimentation(StepArgs<D> a, AdjArgs
 
 namespace tempo {
 
-// caller array (layout g, precision T, may be NULL = zeros) <-> compact FP64 plane
-template <class T>
-__global__ void __launch_bounds__(256) k_to_compact(const T* __restrict__ src, DualGeom g, double* __restrict__ dst) {
-  const size_t ncol = size_t(g.ni) * g.nj;
-  const size_t e = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= ncol * size_t(g.nk)) return;
-  const size_t c = e % ncol, k = e / ncol;
-  dst[e] = src ? double(src[(c % g.ni) + k * g.ldk + (c / g.ni) * g.ldj]) : 0.0;
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) k_from_compact(const double* __restrict__ src, DualGeom g, T* __restrict__ dst) {
-  const size_t ncol = size_t(g.ni) * g.nj;
-  const size_t e = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= ncol * size_t(g.nk)) return;
-  const size_t c = e % ncol, k = e / ncol;
-  dst[(c % g.ni) + k * g.ldk + (c / g.ni) * g.ldj] = T(src[e]);
-}
-
-
-// several arrays of one layout in one launch (blockIdx.y: the array)
+// ---- caller arrays <-> compact planes (element (c, k) at c + k*ncol) ----
+// Several arrays of one layout in one launch: 256 columns per block, the
+// level in blockIdx.y, the array in blockIdx.z, so that an element's place
+// needs no division but the column's by ni, and that only where nj > 1.
 constexpr int kBatchMax = 24;
 template <class S, class D>
 struct PlaneBatch {
   const S* src[kBatchMax];
   D* dst[kBatchMax];
 };
+// values and tangents beside their dual planes
+template <class T>
+struct DualBatch {
+  T* v[kBatchMax];
+  T* t[kBatchMax];
+  Dual<T>* d[kBatchMax];
+};
+struct PlanePoint {
+  size_t e, o;  // compact and caller offsets
+  bool in;
+};
+__device__ __forceinline__ PlanePoint plane_point(const DualGeom& g) {
+  const unsigned ncol = unsigned(g.ni) * unsigned(g.nj), c = blockIdx.x * 256u + threadIdx.x, k = blockIdx.y;
+  size_t o = size_t(c) + size_t(k) * size_t(g.ldk);
+  if (g.nj > 1) o = size_t(c % unsigned(g.ni)) + size_t(k) * size_t(g.ldk) + size_t(c / unsigned(g.ni)) * size_t(g.ldj);
+  return {size_t(c) + size_t(k) * ncol, o, c < ncol};
+}
+// src may be NULL: zeros
 template <class T>
 __global__ void __launch_bounds__(256) k_to_compact_n(PlaneBatch<T, double> b, DualGeom g) {
-  const size_t ncol = size_t(g.ni) * g.nj;
-  const size_t e = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= ncol * size_t(g.nk)) return;
-  const T* src = b.src[blockIdx.y];
-  const size_t c = e % ncol, k = e / ncol;
-  b.dst[blockIdx.y][e] = src ? double(src[(c % g.ni) + k * g.ldk + (c / g.ni) * g.ldj]) : 0.0;
+  const PlanePoint p = plane_point(g);
+  if (!p.in) return;
+  const T* src = b.src[blockIdx.z];
+  b.dst[blockIdx.z][p.e] = src ? double(src[p.o]) : 0.0;
 }
 template <class T>
 __global__ void __launch_bounds__(256) k_from_compact_n(PlaneBatch<double, T> b, DualGeom g) {
-  const size_t ncol = size_t(g.ni) * g.nj;
-  const size_t e = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= ncol * size_t(g.nk)) return;
-  const size_t c = e % ncol, k = e / ncol;
-  b.dst[blockIdx.y][(c % g.ni) + k * g.ldk + (c / g.ni) * g.ldj] = T(b.src[blockIdx.y][e]);
+  const PlanePoint p = plane_point(g);
+  if (p.in) b.dst[blockIdx.z][p.o] = T(b.src[blockIdx.z][p.e]);
 }
-// values into compact duals with zero tangents
+// values (tangents may be NULL: zeros) into duals
 template <class T>
-__global__ void __launch_bounds__(256) k_dual_pack_n(PlaneBatch<T, Dual<T>> b, DualGeom g) {
-  const size_t ncol = size_t(g.ni) * g.nj;
-  const size_t e = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= ncol * size_t(g.nk)) return;
-  const size_t c = e % ncol, k = e / ncol;
-  b.dst[blockIdx.y][e] = Dual<T>(b.src[blockIdx.y][(c % g.ni) + k * g.ldk + (c / g.ni) * g.ldj], T(0));
+__global__ void __launch_bounds__(256) k_dual_pack_n(DualBatch<T> b, DualGeom g) {
+  const PlanePoint p = plane_point(g);
+  if (!p.in) return;
+  const T* t = b.t[blockIdx.z];
+  b.d[blockIdx.z][p.e] = Dual<T>(b.v[blockIdx.z][p.o], t ? t[p.o] : T(0));
+}
+// duals into values and tangents (either may be NULL)
+template <class T>
+__global__ void __launch_bounds__(256) k_dual_unpack_n(DualBatch<T> b, DualGeom g) {
+  const PlanePoint p = plane_point(g);
+  if (!p.in) return;
+  const Dual<T> x = b.d[blockIdx.z][p.e];
+  if (b.v[blockIdx.z]) b.v[blockIdx.z][p.o] = x.v;
+  if (b.t[blockIdx.z]) b.t[blockIdx.z][p.o] = x.d;
 }
 template <class K, class B>
 hipError_t launch_batch(K kernel, const B& b, int n, const DualGeom& g, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   if (n > kBatchMax) return hipErrorInvalidValue;
-  const size_t m = size_t(g.ni) * g.nj * g.nk;
-  hipLaunchKernelGGL(kernel, dim3(unsigned((m + 255) / 256), unsigned(n)), dim3(256), 0, s, b, g);
+  const unsigned blocks = (unsigned(g.ni) * unsigned(g.nj) + 255u) / 256u;
+  hipLaunchKernelGGL(kernel, dim3(blocks, unsigned(g.nk), unsigned(n)), dim3(256), 0, s, b, g);
   return hipGetLastError();
 }
 template <class T>
@@ -586,22 +590,12 @@ hipError_t launch_from_compact_n(const PlaneBatch<double, T>& b, int n, const Du
   return launch_batch(k_from_compact_n<T>, b, n, g, s);
 }
 template <class T>
-hipError_t launch_dual_pack_n(const PlaneBatch<T, Dual<T>>& b, int n, const DualGeom& g, hipStream_t s) {
+hipError_t launch_dual_pack_n(const DualBatch<T>& b, int n, const DualGeom& g, hipStream_t s) {
   return launch_batch(k_dual_pack_n<T>, b, n, g, s);
 }
-
 template <class T>
-hipError_t launch_to_compact(const T* src, const DualGeom& g, double* dst, hipStream_t s) {
-  const size_t n = size_t(g.ni) * g.nj * g.nk;
-  hipLaunchKernelGGL(k_to_compact<T>, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, src, g, dst);
-  return hipGetLastError();
-}
-
-template <class T>
-hipError_t launch_from_compact(const double* src, const DualGeom& g, T* dst, hipStream_t s) {
-  const size_t n = size_t(g.ni) * g.nj * g.nk;
-  hipLaunchKernelGGL(k_from_compact<T>, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, src, g, dst);
-  return hipGetLastError();
+hipError_t launch_dual_unpack_n(const DualBatch<T>& b, int n, const DualGeom& g, hipStream_t s) {
+  return launch_batch(k_dual_unpack_n<T>, b, n, g, s);
 }
 
 }  // namespace tempo

@@ -28,29 +28,23 @@ hipError_t launch_step_sig(const StepArgs<float>& a, const LaunchCfg& lc, double
 hipError_t launch_step_sig(const StepArgs<double>& a, const LaunchCfg& lc, double* vtbuf, hipStream_t s);
 hipError_t launch_step_tlm(const StepArgs<Dual<float>>& a, const LaunchCfg& lc, Dual<double>* vtbuf, hipStream_t s);
 hipError_t launch_step_tlm(const StepArgs<Dual<double>>& a, const LaunchCfg& lc, Dual<double>* vtbuf, hipStream_t s);
-template <class T>
-hipError_t launch_dual_pack(const T* v, const T* t, const DualGeom& g, Dual<T>* out, hipStream_t s);
 template <class R>
 hipError_t launch_check_update(const CheckArgs<R>& g, int which, hipStream_t s);
 template <class R>
 hipError_t launch_surface_emissions(R* nwfa, const R* nwfa2d, int ni, int nj, long long ldk, long long ldj,
                                     long long d2ldj, int k, double dt, hipStream_t s);
-template <class T>
-hipError_t launch_dual_unpack(const Dual<T>* in, const DualGeom& g, T* v, T* t, hipStream_t s);
 hipError_t launch_adjoint(const StepArgs<Dual<float>>& a, const AdjArgs& g, Dual<double>* vtbuf, size_t sr_bytes,
                           size_t sd_bytes, AdjSnap snap, const bool* have_x, hipStream_t s);
 hipError_t launch_adjoint(const StepArgs<Dual<double>>& a, const AdjArgs& g, Dual<double>* vtbuf, size_t sr_bytes,
                           size_t sd_bytes, AdjSnap snap, const bool* have_x, hipStream_t s);
 template <class T>
-hipError_t launch_to_compact(const T* src, const DualGeom& g, double* dst, hipStream_t s);
-template <class T>
-hipError_t launch_from_compact(const double* src, const DualGeom& g, T* dst, hipStream_t s);
-template <class T>
 hipError_t launch_to_compact_n(const PlaneBatch<T, double>& b, int n, const DualGeom& g, hipStream_t s);
 template <class T>
 hipError_t launch_from_compact_n(const PlaneBatch<double, T>& b, int n, const DualGeom& g, hipStream_t s);
 template <class T>
-hipError_t launch_dual_pack_n(const PlaneBatch<T, Dual<T>>& b, int n, const DualGeom& g, hipStream_t s);
+hipError_t launch_dual_pack_n(const DualBatch<T>& b, int n, const DualGeom& g, hipStream_t s);
+template <class T>
+hipError_t launch_dual_unpack_n(const DualBatch<T>& b, int n, const DualGeom& g, hipStream_t s);
 hipError_t launch_table_qg(const double*, const double*, const double*, const double*, double*, hipStream_t);
 hipError_t launch_table_qs(const double*, const double*, const double*, const double*, double*, hipStream_t);
 hipError_t launch_table_fz(const double*, const double*, const double*, const double*, double, const double*,
@@ -710,18 +704,27 @@ int run_tlm(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_fields*
   field_ptrs(ft, tp);
   D* st = x->tl_state.as<D>();
   DualGeom g3{dm->ni, dm->nj, nz, dm->ldk, dm->ldj};
+  // one launch per layout, in and out
+  DualBatch<T> pk{};
+  int npk = 0;
   for (int i = 0; i < F_NFIELDS; ++i) {
     if (!fp[i]) continue;
     a.f[i] = st + size_t(i) * n3;
-    HIP_TRY(launch_dual_pack(static_cast<const T*>(fp[i]), static_cast<const T*>(tp[i]), g3, a.f[i], s));
+    pk.v[npk] = static_cast<T*>(fp[i]);
+    pk.t[npk] = static_cast<T*>(tp[i]);
+    pk.d[npk++] = a.f[i];
   }
+  const int nstate = npk;
   if (bl) {  // boundary-layer cloud: constants of the step (zero tangent)
     D* qbl = st + F_NFIELDS * n3;
-    HIP_TRY(launch_dual_pack(static_cast<const T*>(f->qc_bl), static_cast<const T*>(nullptr), g3, qbl, s));
-    HIP_TRY(launch_dual_pack(static_cast<const T*>(f->qcfrac_bl), static_cast<const T*>(nullptr), g3, qbl + n3, s));
+    pk.v[npk] = static_cast<T*>(const_cast<void*>(f->qc_bl));
+    pk.d[npk++] = qbl;
+    pk.v[npk] = static_cast<T*>(const_cast<void*>(f->qcfrac_bl));
+    pk.d[npk++] = qbl + n3;
     a.qc_bl = qbl;
     a.qcfrac_bl = qbl + n3;
   }
+  HIP_TRY(launch_dual_pack_n(pk, npk, g3, s));
   void *d2[D2_N] = {}, *d3[D3_N] = {}, *t2[D2_N] = {}, *t3[D3_N] = {};
   if (d) diag_ptrs(d, d2, d3);
   if (dt_) diag_ptrs(dt_, t2, t3);
@@ -744,14 +747,25 @@ int run_tlm(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_fields*
   int rc = bind_common(x, a, dt, itimestep);
   if (rc) return rc;
   HIP_TRY(launch_step_tlm(a, x->launch[sizeof(T) == 8 ? 1 : 0], x->vtbuf.as<Dual<double>>(), s));
-  for (int i = 0; i < F_NFIELDS; ++i)
-    if (fp[i]) HIP_TRY(launch_dual_unpack(a.f[i], g3, static_cast<T*>(fp[i]), static_cast<T*>(tp[i]), s));
+  HIP_TRY(launch_dual_unpack_n(pk, nstate, g3, s));  // the state's entries come first
   DualGeom g2{dm->ni, dm->nj, 1, 0, dm->d2ldj};
   DualGeom gd3{dm->ni, dm->nj, nz, dm->dldk, dm->dldj};
-  for (int i = 0; i < D2_N; ++i)
-    if (a.d2[i]) HIP_TRY(launch_dual_unpack(a.d2[i], g2, static_cast<T*>(d2[i]), static_cast<T*>(t2[i]), s));
-  for (int i = 0; i < D3_N; ++i)
-    if (a.d3[i]) HIP_TRY(launch_dual_unpack(a.d3[i], gd3, static_cast<T*>(d3[i]), static_cast<T*>(t3[i]), s));
+  DualBatch<T> u2{}, u3{};
+  int n2 = 0, nd3 = 0;
+  for (int i = 0; i < D2_N; ++i) {
+    if (!a.d2[i]) continue;
+    u2.v[n2] = static_cast<T*>(d2[i]);
+    u2.t[n2] = static_cast<T*>(t2[i]);
+    u2.d[n2++] = a.d2[i];
+  }
+  for (int i = 0; i < D3_N; ++i) {
+    if (!a.d3[i]) continue;
+    u3.v[nd3] = static_cast<T*>(d3[i]);
+    u3.t[nd3] = static_cast<T*>(t3[i]);
+    u3.d[nd3++] = a.d3[i];
+  }
+  HIP_TRY(launch_dual_unpack_n(u2, n2, g2, s));
+  HIP_TRY(launch_dual_unpack_n(u3, nd3, gd3, s));
   return TEMPO_HIP_OK;
 }
 
@@ -800,12 +814,12 @@ int run_adjoint(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_fie
   const DualGeom g3{dm->ni, dm->nj, nz, dm->ldk, dm->ldj};
   // the inputs, the output cotangents and the precipitation cotangents, one
   // launch per layout
-  PlaneBatch<T, Dual<T>> pk{};
+  DualBatch<T> pk{};
   int npk = 0;
   for (int i = 0; i < F_NFIELDS; ++i) {
     if (!fp[i]) continue;
-    pk.src[npk] = static_cast<const T*>(fp[i]);
-    pk.dst[npk++] = in + size_t(i) * n3;
+    pk.v[npk] = static_cast<T*>(fp[i]);
+    pk.d[npk++] = in + size_t(i) * n3;
     a.f[i] = st + size_t(i) * n3;
   }
   HIP_TRY(launch_dual_pack_n(pk, npk, g3, s));
@@ -821,7 +835,10 @@ int run_adjoint(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_fie
   if (db) diag_ptrs(db, d2, d3);
   const DualGeom gd3{dm->ni, dm->nj, nz, dm->dldk, dm->dldj};
   const DualGeom g2{dm->ni, dm->nj, 1, 0, dm->d2ldj};
-  HIP_TRY(launch_to_compact(static_cast<const T*>(d3[D3_REFL]), gd3, ybar + size_t(AY_REFL) * n3, s));
+  PlaneBatch<T, double> rb{};
+  rb.src[0] = static_cast<const T*>(d3[D3_REFL]);
+  rb.dst[0] = ybar + size_t(AY_REFL) * n3;
+  HIP_TRY(launch_to_compact_n(rb, 1, gd3, s));
   const int pmap[4] = {D2_RAIN, D2_GRAUPEL, D2_SNOW, D2_ICE};  // S^T order: rain, graupel, snow, ice
   PlaneBatch<T, double> pc{};
   for (int q = 0; q < 4; ++q) {

@@ -1654,44 +1654,4 @@ hipError_t launch_surface_emissions(R* nwfa, const R* nwfa2d, int ni, int nj, lo
   return hipGetLastError();
 }
 
-// ------------------------------------------------ tangent-linear I/O ----
-// caller arrays (value, tangent) <-> one compact dual array, element (c, k)
-// at c + k*ncol
-template <class T>
-__global__ void __launch_bounds__(256) k_dual_pack(const T* __restrict__ v, const T* __restrict__ t, DualGeom g,
-                                                   Dual<T>* __restrict__ out) {
-  const size_t ncol = size_t(g.ni) * g.nj;
-  const size_t e = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= ncol * size_t(g.nk)) return;
-  const size_t c = e % ncol, k = e / ncol;
-  const size_t o = (c % g.ni) + k * g.ldk + (c / g.ni) * g.ldj;
-  out[e] = Dual<T>(v[o], t ? t[o] : T(0));
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) k_dual_unpack(const Dual<T>* __restrict__ in, DualGeom g, T* __restrict__ v,
-                                                     T* __restrict__ t) {
-  const size_t ncol = size_t(g.ni) * g.nj;
-  const size_t e = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= ncol * size_t(g.nk)) return;
-  const size_t c = e % ncol, k = e / ncol;
-  const size_t o = (c % g.ni) + k * g.ldk + (c / g.ni) * g.ldj;
-  if (v) v[o] = in[e].v;
-  if (t) t[o] = in[e].d;
-}
-
-template <class T>
-hipError_t launch_dual_pack(const T* v, const T* t, const DualGeom& g, Dual<T>* out, hipStream_t s) {
-  const size_t n = size_t(g.ni) * g.nj * g.nk;
-  hipLaunchKernelGGL(k_dual_pack<T>, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, v, t, g, out);
-  return hipGetLastError();
-}
-
-template <class T>
-hipError_t launch_dual_unpack(const Dual<T>* in, const DualGeom& g, T* v, T* t, hipStream_t s) {
-  const size_t n = size_t(g.ni) * g.nj * g.nk;
-  hipLaunchKernelGGL(k_dual_unpack<T>, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, in, g, v, t);
-  return hipGetLastError();
-}
-
 }  // namespace tempo

@@ -24,17 +24,14 @@ hipError_t launch_step_tlm(const StepArgs<Dual<float>>& a, const LaunchCfg& lc, 
 template hipError_t launch_check_update<float>(const CheckArgs<float>&, int, hipStream_t);
 template hipError_t launch_surface_emissions<float>(float*, const float*, int, int, long long, long long, long long, int,
                                                      double, hipStream_t);
-template hipError_t launch_dual_pack<float>(const float*, const float*, const DualGeom&, Dual<float>*, hipStream_t);
-template hipError_t launch_dual_unpack<float>(const Dual<float>*, const DualGeom&, float*, float*, hipStream_t);
 
 hipError_t launch_adjoint(const StepArgs<Dual<float>>& a, const AdjArgs& g, Dual<double>* vtbuf, size_t sr_bytes,
                           size_t sd_bytes, AdjSnap snap, const bool* have_x, hipStream_t s) {
   return adjoint_passes(a, g, vtbuf, sr_bytes, sd_bytes, snap, have_x, s);
 }
-template hipError_t launch_to_compact<float>(const float*, const DualGeom&, double*, hipStream_t);
-template hipError_t launch_from_compact<float>(const double*, const DualGeom&, float*, hipStream_t);
 template hipError_t launch_to_compact_n<float>(const PlaneBatch<float, double>&, int, const DualGeom&, hipStream_t);
 template hipError_t launch_from_compact_n<float>(const PlaneBatch<double, float>&, int, const DualGeom&, hipStream_t);
-template hipError_t launch_dual_pack_n<float>(const PlaneBatch<float, Dual<float>>&, int, const DualGeom&, hipStream_t);
+template hipError_t launch_dual_pack_n<float>(const DualBatch<float>&, int, const DualGeom&, hipStream_t);
+template hipError_t launch_dual_unpack_n<float>(const DualBatch<float>&, int, const DualGeom&, hipStream_t);
 
 }  // namespace tempo

@@ -24,17 +24,14 @@ hipError_t launch_step_tlm(const StepArgs<Dual<double>>& a, const LaunchCfg& lc,
 template hipError_t launch_check_update<double>(const CheckArgs<double>&, int, hipStream_t);
 template hipError_t launch_surface_emissions<double>(double*, const double*, int, int, long long, long long, long long, int,
                                                      double, hipStream_t);
-template hipError_t launch_dual_pack<double>(const double*, const double*, const DualGeom&, Dual<double>*, hipStream_t);
-template hipError_t launch_dual_unpack<double>(const Dual<double>*, const DualGeom&, double*, double*, hipStream_t);
 
 hipError_t launch_adjoint(const StepArgs<Dual<double>>& a, const AdjArgs& g, Dual<double>* vtbuf, size_t sr_bytes,
                           size_t sd_bytes, AdjSnap snap, const bool* have_x, hipStream_t s) {
   return adjoint_passes(a, g, vtbuf, sr_bytes, sd_bytes, snap, have_x, s);
 }
-template hipError_t launch_to_compact<double>(const double*, const DualGeom&, double*, hipStream_t);
-template hipError_t launch_from_compact<double>(const double*, const DualGeom&, double*, hipStream_t);
 template hipError_t launch_to_compact_n<double>(const PlaneBatch<double, double>&, int, const DualGeom&, hipStream_t);
 template hipError_t launch_from_compact_n<double>(const PlaneBatch<double, double>&, int, const DualGeom&, hipStream_t);
-template hipError_t launch_dual_pack_n<double>(const PlaneBatch<double, Dual<double>>&, int, const DualGeom&, hipStream_t);
+template hipError_t launch_dual_pack_n<double>(const DualBatch<double>&, int, const DualGeom&, hipStream_t);
+template hipError_t launch_dual_unpack_n<double>(const DualBatch<double>&, int, const DualGeom&, hipStream_t);
 
 }  // namespace tempo
