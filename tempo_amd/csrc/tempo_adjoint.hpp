@@ -53,8 +53,10 @@ struct AdjArgs {
   int* pt_loc;          // compact plane: 1 where a local pass's phase A runs (see k_adj_point_flags)
   const double* pbar;   // 4 x ncol: rain, graupel, snow, ice precipitation
   double* xbar;         // AX_N planes (compact)
-  double* ubar;         // 10 planes (compact): tendency cotangents, SD_QRTEN order
-  double* zbar;         // AZ_N planes (compact)
+  // the planes that S^T reads and writes are tiled like the step scratch: its
+  // wavefronts take a column each, and a column group's levels are contiguous
+  double* ubar;         // 10 planes (tiled): tendency cotangents, SD_QRTEN order
+  double* zbar;         // AZ_N planes (tiled)
   double* work;         // AW_N scratch planes (tiled like the step scratch)
 };
 
@@ -92,7 +94,7 @@ template <class D>
 __global__ void __launch_bounds__(256) k_adj_capture(StepArgs<D> a, AdjArgs g, double* __restrict__ xb) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
   if (c >= a.ncol) return;
-  const size_t s = TEMPO_IDX_SCR(a, c, k), e = size_t(c) + size_t(k) * a.ncol, n3 = size_t(a.ncol) * a.nz;
+  const size_t s = TEMPO_IDX_SCR(a, c, k), e = size_t(c) + size_t(k) * a.ncol;
   if (!g.pt_loc[e]) {  // skipped by phase A: zero tangents against zero zbar, no final update
     xb[e] = 0.0;
     return;
@@ -104,15 +106,15 @@ __global__ void __launch_bounds__(256) k_adj_capture(StepArgs<D> a, AdjArgs g, d
   double acc = 0.0;
 #pragma unroll
   for (int q = 0; q < 10; ++q) {
-    const double z = g.zbar[size_t(AZ_RR + q) * n3 + e];
+    const double z = g.zbar[size_t(AZ_RR + q) * a.plane + s];
     if (z != 0.0) acc += double(a.sd[size_t(sdf[q]) * a.plane + s].d) * z;
   }
 #pragma unroll
   for (int q = 0; q < 9; ++q) {
-    const double z = g.zbar[size_t(AZ_VTRR + q) * n3 + e];
+    const double z = g.zbar[size_t(AZ_VTRR + q) * a.plane + s];
     if (z != 0.0) acc += double(a.sr[size_t(srf[q]) * a.plane + s].d) * z;
   }
-  const double zr = g.zbar[size_t(AZ_RHO) * n3 + e];
+  const double zr = g.zbar[size_t(AZ_RHO) * a.plane + s];
   if (zr != 0.0) acc += double(a.sr[size_t(SR_RHO) * a.plane + s].d) * zr;
   xb[e] = acc;
 }
@@ -163,9 +165,9 @@ template <class D>
 __global__ void __launch_bounds__(256) k_adj_point_flags(StepArgs<D> a, AdjArgs g) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
   if (c >= a.ncol) return;
-  const size_t e = size_t(c) + size_t(k) * a.ncol, n3 = size_t(a.ncol) * a.nz;
+  const size_t e = size_t(c) + size_t(k) * a.ncol, s = TEMPO_IDX_SCR(a, c, k);
   bool on = g.lvl_on[k] != 0;
-  for (int q = 0; q < AZ_N && !on; ++q) on = g.zbar[size_t(q) * n3 + e] != 0.0;
+  for (int q = 0; q < AZ_N && !on; ++q) on = g.zbar[size_t(q) * a.plane + s] != 0.0;
   g.pt_loc[e] = on ? 1 : 0;
 }
 
@@ -177,22 +179,24 @@ struct AdjSeed {
   int kind, set, clear;
 };
 
-// out[e] (+)= sum over outputs of ybar * tangent (0 at a level without
+// out (+)= sum over outputs of ybar * tangent (0 at a level without
 // output cotangents, whose final update a.lvl_on skipped); then the next
 // pass's seed at this point.  A point the step leaves as it is (an
 // early-exit column, a level at or above the column's nlev) has no final
 // update writing its new state: its output tangents are its input tangents,
 // and its reflectivity is no function of the inputs (a constant in an
-// early-exit column, left as it is above nlev).
+// early-exit column, left as it is above nlev).  out is compact, or tiled
+// (the tendency cotangents, which S^T reads).
 template <class D>
 __global__ void __launch_bounds__(256) k_adj_contract(StepArgs<D> a, AdjArgs g, double* out, int accumulate,
-                                                      AdjSeed nx) {
+                                                      int tiled, AdjSeed nx) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
   if (c >= a.ncol) return;
   const size_t o = TEMPO_IDX_STATE(a, c, k), e = size_t(c) + size_t(k) * a.ncol, n3 = size_t(a.ncol) * a.nz;
+  const size_t w = tiled ? TEMPO_IDX_SCR(a, c, k) : e;
   const bool kept = (a.cf[c] & CF_EXIT) || (a.nlev && k >= a.nlev[c]);
   if (a.lvl_on && !a.lvl_on[k]) {
-    if (!accumulate) out[e] = 0.0;
+    if (!accumulate) out[w] = 0.0;
   } else {
     double acc = 0.0;  // tangents read only where their cotangent is non-zero
     for (int q = 0; q < AY_REFL; ++q) {
@@ -205,7 +209,7 @@ __global__ void __launch_bounds__(256) k_adj_contract(StepArgs<D> a, AdjArgs g, 
       const double y = g.ybar[size_t(AY_REFL) * n3 + e];
       if (y != 0.0) acc += y * double(a.d3[D3_REFL][o].d);
     }
-    out[e] = accumulate ? out[e] + acc : acc;
+    out[w] = accumulate ? out[w] + acc : acc;
   }
   if (nx.kind == 1) {
     if (nx.clear >= 0 && a.f[nx.clear]) a.f[nx.clear][o].d = 0;
@@ -244,7 +248,6 @@ __device__ void sed_adjoint(const StepArgs<D>& a, const SedAdjCol& q, const AdjA
   const double ost = 1.0 / double(steps), dt = q.dt;
   const int top = q.nzc - 1;
   auto updated = [&](int k) { return k == top || k <= ktop - 1; };
-  const size_t n3 = size_t(a.ncol) * a.nz;
   for (int n = nsub - 1; n >= 0; --n) {
     // masses at the start of substep n, recomputed from the initial ones
     for (int k = 0; k < q.nzc; ++k) xr[TEMPO_IDX_SCR(a, q.c, k)] = xr0(k);
@@ -271,7 +274,7 @@ __device__ void sed_adjoint(const StepArgs<D>& a, const SedAdjCol& q, const AdjA
         const double flux = (k == top) ? -sed : (above - sed);
         const double v = xr[s] + flux * odz(k) * dt * ost;
         const double vb = v > limit ? xb[s] : 0.0;
-        const double tb = tenbar ? tenbar[size_t(q.c) + size_t(k) * a.ncol] : 0.0;
+        const double tb = tenbar ? tenbar[s] : 0.0;
         fbar = vb * odz(k) * dt * ost + tb * odz(k) * ost * orho(k);
         if (tb != 0.0) rhobar[s] += -orho(k) * orho(k) * tb * flux * odz(k) * ost;
         xb[s] = vb;  // cotangent of the pre-substep mass through v (identity part)
@@ -292,7 +295,6 @@ __device__ void sed_adjoint(const StepArgs<D>& a, const SedAdjCol& q, const AdjA
       vbar[s] += sb * xr[s];
     }
   }
-  (void)n3;
 }
 
 template <class D>
@@ -303,8 +305,8 @@ __global__ void __launch_bounds__(64) k_adj_sedimentation(StepArgs<D> a, AdjArgs
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= a.ncol) return;
   const int nzc = a.nlev ? min(max(a.nlev[c], 1), a.nz) : a.nz;
-  const size_t plane = a.plane, n3 = size_t(a.ncol) * a.nz;
-  auto zb = [&](int z, int k) -> double& { return g.zbar[size_t(z) * n3 + size_t(c) + size_t(k) * a.ncol]; };
+  const size_t plane = a.plane;
+  auto zb = [&](int z, int k) -> double& { return g.zbar[size_t(z) * plane + TEMPO_IDX_SCR(a, c, k)]; };
   for (int z = 0; z < AZ_N; ++z)
     for (int k = 0; k < a.nz; ++k) zb(z, k) = 0.0;
   if (a.cf[c] & CF_EXIT) return;
@@ -318,7 +320,7 @@ __global__ void __launch_bounds__(64) k_adj_sedimentation(StepArgs<D> a, AdjArgs
   auto odz = [&](int k) { return 1.0 / double(a.f[F_DZ][TEMPO_IDX_STATE(a, c, k)].v); };
   auto orho = [&](int k) { return 1.0 / double(a.sr[size_t(SR_RHO) * plane + S(k)].v); };
   const double* ub = g.ubar;
-  auto ubp = [&](int m) { return ub + size_t(m) * n3; };
+  auto ubp = [&](int m) { return ub + size_t(m) * plane; };
   double* w = g.work;
   double* vb1 = w + AW_VB1 * plane;
   double* vb2 = w + AW_VB2 * plane;

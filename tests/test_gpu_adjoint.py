@@ -697,3 +697,34 @@ def test_cloud_number_network_derivatives(hip, ref_tables, which):
           int((any_ok & ~central_ok).sum()), "unmatched", int((~any_ok).sum()), "of", ncol)
     assert any_ok.all(), np.where(~any_ok)[0]
     assert central_ok.mean() >= 0.9
+
+
+@pytest.mark.parametrize("sparse", [False, True])
+@pytest.mark.parametrize("nz", [63, 64, 65, 127, 128])
+def test_adjoint_dot_product_level_counts(ctx, sample, nz, sparse):
+    """the dot-product test at the edges of the column kernels' 64-level
+    chunks, on 67 columns of uneven depth; sparse: output cotangents at three
+    levels only"""
+    st0, m = sample
+    st = refine({k: v[:, :67] for k, v in st0.items()}, nz)
+    ncol = 67
+    nlev = np.maximum(2, nz - np.arange(ncol) % 9).astype(np.int32)
+    rng = np.random.default_rng(nz)
+    v = direction(st, 37)
+    active = np.arange(nz)[:, None] < nlev[None, :]
+    rows = np.isin(np.arange(nz), LEVELS)[:, None] if sparse else np.ones((nz, 1), bool)
+    ybar = {k: torch.tensor(rng.standard_normal(st[k].shape) / (np.abs(st[k]).max() + 1e-30) * rows, device="cuda")
+            for k in ("t", "qv", "qc", "qr", "qi", "qs", "qg", "ni", "nr", "nc", "nwfa", "nifa") if k in st}
+    dbar = {"refl10cm": torch.tensor(rng.standard_normal((nz, ncol)) * 0.01 * active * rows, device="cuda")}
+    for k in ("rain_precip", "ice_liquid_equiv_precip", "snow_liquid_equiv_precip", "graupel_liquid_equiv_precip"):
+        dbar[k] = torch.tensor(rng.standard_normal(ncol) * 1e3, device="cuda")
+    nl = torch.tensor(nlev, device="cuda")
+    _, dtl, tb = ctx.tlm(dev(st), {k: torch.tensor(x, device="cuda") for k, x in v.items()}, m["dt"], m["itimestep"],
+                         nlev=nl)
+    # the tangent of a diagnostic above a column's levels is not defined
+    dtl["refl10cm"] = torch.where(torch.tensor(active, device="cuda"), dtl["refl10cm"], 0.0)
+    lhs = sum(float((ybar[k] * tb[k]).sum()) for k in ybar) + sum(float((dbar[k] * dtl[k]).sum()) for k in dbar)
+    xbar = ctx.adjoint(dev(st), ybar, dbar, m["dt"], m["itimestep"], nlev=nl)
+    rhs = sum(float((xbar[k] * torch.tensor(v[k], device="cuda")).sum()) for k in v)
+    print(nz, "levels, dot test", lhs, rhs)
+    assert abs(lhs - rhs) <= 1e-10 * abs(lhs)
