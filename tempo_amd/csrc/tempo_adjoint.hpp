@@ -47,6 +47,13 @@ __host__ __device__ constexpr int adj_y_field(int i) {
        : i == AY_NWFA ? F_NWFA : i == AY_NIFA ? F_NIFA : i == AY_NG ? F_NG : F_QB;
 }
 
+// output cotangent of a field (a constant f: folded)
+__host__ __device__ constexpr int adj_y_of(int f) {
+  int q = 0;
+  while (q < AY_REFL && adj_y_field(q) != f) ++q;
+  return q;
+}
+
 struct AdjArgs {
   const double* ybar;   // AY_N planes (compact c + k*ncol), absent outputs all zero
   int* lvl_on;          // nz: 1 where some output cotangent of the level is non-zero
@@ -119,17 +126,6 @@ __global__ void __launch_bounds__(256) k_adj_capture(StepArgs<D> a, AdjArgs g, d
   xb[e] = acc;
 }
 
-// seed the tangent of one post-sedimentation tendency plane (u pass),
-// clearing the previous pass's seed (m_prev < 0: none)
-template <class D>
-__global__ void __launch_bounds__(256) k_adj_seed_ten(StepArgs<D> a, int m, int m_prev) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
-  if (c >= a.ncol) return;
-  const size_t s = TEMPO_IDX_SCR(a, c, k);
-  if (m_prev >= 0) a.sd[size_t(SD_QRTEN + m_prev) * a.plane + s].d = 0;
-  a.sd[size_t(SD_QRTEN + m) * a.plane + s].d = 1;
-}
-
 // out[0, n) = 0 (a kernel rather than a memset, so that the sequence may be
 // captured in a graph)
 template <class T>
@@ -171,12 +167,55 @@ __global__ void __launch_bounds__(256) k_adj_point_flags(StepArgs<D> a, AdjArgs 
   g.pt_loc[e] = on ? 1 : 0;
 }
 
-// the seed of the next pass, moved by the contraction that ends a pass
-// (the seeding runs on the same grid): kind 1 an input field's tangent
-// (a.f), kind 2 a post-sedimentation tendency plane's (scratch); the
-// field or plane `clear` loses its seed, `set` gets one (< 0: none)
+// passes seeded on the post-sedimentation tendencies: ubar_m = sum over
+// outputs of ybar * d(output)/d(tendency m), one direction per blockIdx.z,
+// all in one launch.  The final update contracts its outputs where it has
+// them, so no pass stores a new state, and the seed goes into the tendency as
+// it is read.  A single direction over the three levels of 64 where an
+// assimilation's loss has cotangents is too little for the chip: 24 us for
+// the update and 17 for a separate contraction, eight times over; 45 us
+// for all eight at 16,384 x 64 (FP32).
+struct AdjDirs {
+  int n, id[AX_N];
+};
+template <class D>
+struct UpassOutputs {
+  static constexpr bool kAdjoint = true;
+  const double* ybar;  // at the point
+  size_t n3;
+  int seed;
+  double acc;
+  __device__ __forceinline__ double ten_tangent(int m) const { return m == seed ? 1.0 : 0.0; }
+  // a tangent counts only where its cotangent is non-zero
+  __device__ __forceinline__ void add_y(int q, const D& v) {
+    const double y = ybar[size_t(q) * n3];
+    if (y != 0.0) acc += y * double(v.d);
+  }
+  __device__ __forceinline__ void add(int f, const D& v) { add_y(adj_y_of(f), v); }
+  __device__ __forceinline__ bool wants_refl() const { return ybar[size_t(AY_REFL) * n3] != 0.0; }
+  __device__ __forceinline__ void add_refl(const D& v) { add_y(AY_REFL, v); }
+};
+template <class D>
+__global__ void __launch_bounds__(256) k_adj_upass(StepArgs<D> a, AdjArgs g, AdjDirs dirs) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y, m = dirs.id[blockIdx.z];
+  if (c >= a.ncol) return;
+  const size_t e = size_t(c) + size_t(k) * a.ncol, n3 = size_t(a.ncol) * a.nz;
+  double* out = g.ubar + size_t(m) * a.plane + TEMPO_IDX_SCR(a, c, k);
+  // no cotangents, or a point that the step leaves as it is
+  if (!g.lvl_on[k] || (a.cf[c] & CF_EXIT) || (a.nlev && k >= a.nlev[c])) {
+    *out = 0.0;
+    return;
+  }
+  UpassOutputs<D> u{g.ybar + e, n3, m, 0.0};
+  phase_c_point(a, c, k, u);
+  *out = u.acc;
+}
+
+// the seed of the next pass, moved by the contraction that ends a pass (the
+// seeding runs on the same grid): the input field `clear` loses its tangent
+// seed, `set` gets one (< 0: none)
 struct AdjSeed {
-  int kind, set, clear;
+  int set, clear;
 };
 
 // out (+)= sum over outputs of ybar * tangent (0 at a level without
@@ -185,18 +224,16 @@ struct AdjSeed {
 // early-exit column, a level at or above the column's nlev) has no final
 // update writing its new state: its output tangents are its input tangents,
 // and its reflectivity is no function of the inputs (a constant in an
-// early-exit column, left as it is above nlev).  out is compact, or tiled
-// (the tendency cotangents, which S^T reads).
+// early-exit column, left as it is above nlev).
 template <class D>
 __global__ void __launch_bounds__(256) k_adj_contract(StepArgs<D> a, AdjArgs g, double* out, int accumulate,
-                                                      int tiled, AdjSeed nx) {
+                                                      AdjSeed nx) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
   if (c >= a.ncol) return;
   const size_t o = TEMPO_IDX_STATE(a, c, k), e = size_t(c) + size_t(k) * a.ncol, n3 = size_t(a.ncol) * a.nz;
-  const size_t w = tiled ? TEMPO_IDX_SCR(a, c, k) : e;
   const bool kept = (a.cf[c] & CF_EXIT) || (a.nlev && k >= a.nlev[c]);
   if (a.lvl_on && !a.lvl_on[k]) {
-    if (!accumulate) out[w] = 0.0;
+    if (!accumulate) out[e] = 0.0;
   } else {
     double acc = 0.0;  // tangents read only where their cotangent is non-zero
     for (int q = 0; q < AY_REFL; ++q) {
@@ -209,16 +246,10 @@ __global__ void __launch_bounds__(256) k_adj_contract(StepArgs<D> a, AdjArgs g, 
       const double y = g.ybar[size_t(AY_REFL) * n3 + e];
       if (y != 0.0) acc += y * double(a.d3[D3_REFL][o].d);
     }
-    out[w] = accumulate ? out[w] + acc : acc;
+    out[e] = accumulate ? out[e] + acc : acc;
   }
-  if (nx.kind == 1) {
-    if (nx.clear >= 0 && a.f[nx.clear]) a.f[nx.clear][o].d = 0;
-    if (nx.set >= 0 && a.f[nx.set]) a.f[nx.set][o].d = 1;
-  } else if (nx.kind == 2) {
-    const size_t s = TEMPO_IDX_SCR(a, c, k);
-    if (nx.clear >= 0) a.sd[size_t(SD_QRTEN + nx.clear) * a.plane + s].d = 0;
-    if (nx.set >= 0) a.sd[size_t(SD_QRTEN + nx.set) * a.plane + s].d = 1;
-  }
+  if (nx.clear >= 0 && a.f[nx.clear]) a.f[nx.clear][o].d = 0;
+  if (nx.set >= 0 && a.f[nx.set]) a.f[nx.set][o].d = 1;
 }
 
 

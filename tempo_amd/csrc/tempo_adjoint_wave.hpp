@@ -625,7 +625,6 @@ hipError_t adjoint_passes(const StepArgs<D>& a, const AdjArgs& g, Dual<double>* 
   ac.lvl_on = g.lvl_on;
   hipLaunchKernelGGL(k_adj_level_zero<D>, dim3(unsigned((a.nz + 255) / 256)), dim3(256), 0, s, a, g);
   hipLaunchKernelGGL(k_adj_level_flags<D>, g2, dim3(256), 0, s, a, g);
-  auto phase_c = [&]() { hipLaunchKernelGGL(k_phase_c<D>, level_grid(a, 256), dim3(256), 0, s, ac); };
 
   // tangent-free forward.  Its sedimentation on the values, one wavefront
   // per column (the tangents are zero in this pass), writes only the ten
@@ -646,28 +645,20 @@ hipError_t adjoint_passes(const StepArgs<D>& a, const AdjArgs& g, Dual<double>* 
     hipLaunchKernelGGL(k_phase_b<D>, dim3(unsigned((a.ncol + 127) / 128)), dim3(128), 0, s, a, vtbuf);
   double* post = static_cast<double*>(snap.sd_b);
   hipLaunchKernelGGL(k_adj_keep_post<D>, g2, dim3(256), 0, s, a, post);
-  // passes seeded on the post-sedimentation tendencies (the final update
-  // reads the inputs, a.fa and the scratch, and writes only a.fo).  Without
-  // prognostic graupel number and volume the final update does not read
-  // their tendencies, so those cotangents are zero and need no pass.
-  // Each pass's contraction moves the seed on to the next pass.
+  // passes seeded on the post-sedimentation tendencies.  Without prognostic
+  // graupel number and volume the final update does not read their
+  // tendencies, so those cotangents are zero and need no pass.
   const bool ngqb = a.f[F_NG] && a.f[F_QB];
-  int ms[10], nm = 0;
+  AdjDirs ms{};
   for (int m = 0; m < 10; ++m) {
     if (!ngqb && (SD_QRTEN + m == SD_NGTEN || SD_QRTEN + m == SD_QBTEN)) {
       double* ub = g.ubar + size_t(m) * a.plane;
       hipLaunchKernelGGL(k_adj_zero<double>, dim3(unsigned((a.plane + 255) / 256)), dim3(256), 0, s, ub, a.plane);
       continue;
     }
-    ms[nm++] = m;
+    ms.id[ms.n++] = m;
   }
-  if (nm > 0) hipLaunchKernelGGL(k_adj_seed_ten<D>, g2, dim3(256), 0, s, a, ms[0], -1);
-  for (int j = 0; j < nm; ++j) {
-    phase_c();
-    const AdjSeed nx{2, j + 1 < nm ? ms[j + 1] : -1, j + 1 < nm ? ms[j] : -1};
-    hipLaunchKernelGGL(k_adj_contract<D>, g2, dim3(256), 0, s, ac, g, g.ubar + size_t(ms[j]) * a.plane, 0, 1,
-                       nx);
-  }
+  hipLaunchKernelGGL(k_adj_upass<D>, dim3(gc, unsigned(a.nz), unsigned(ms.n)), dim3(256), 0, s, a, g, ms);
   // S^T on the values after phase A
   if (!wave_b) {
     if ((e = cp(a.sr, snap.sr_a, sr_bytes)) != hipSuccess) return e;
@@ -699,8 +690,8 @@ hipError_t adjoint_passes(const StepArgs<D>& a, const AdjArgs& g, Dual<double>* 
     hipLaunchKernelGGL(k_phase_a<D>, level_grid(a, 256), dim3(256), 0, s, al);
     hipLaunchKernelGGL(k_adj_capture<D>, g2, dim3(256), 0, s, a, g, xb);
     hipLaunchKernelGGL(k_phase_c<D>, level_grid(a, 256), dim3(256), 0, s, acl);
-    const AdjSeed nx{1, j + 1 < nxs ? adj_x_field(xs[j + 1]) : -1, j + 1 < nxs ? adj_x_field(xs[j]) : -1};
-    hipLaunchKernelGGL(k_adj_contract<D>, g2, dim3(256), 0, s, ac, g, xb, 1, 0, nx);
+    const AdjSeed nx{j + 1 < nxs ? adj_x_field(xs[j + 1]) : -1, j + 1 < nxs ? adj_x_field(xs[j]) : -1};
+    hipLaunchKernelGGL(k_adj_contract<D>, g2, dim3(256), 0, s, ac, g, xb, 1, nx);
   }
   return hipGetLastError();
 }

@@ -1335,10 +1335,38 @@ __device__ __forceinline__ void atomic_max_pos(Sig<T>* p, Sig<T> v) {
   atomic_max_pos(&p->v, v.v);
 }
 
-// freeze/melt, final update, final checks and diagnostics of point (c, k)
-// (src/module_mp_tempo_main.F90:729-863)
+// reflectivity_10cm (src/module_mp_tempo_diags.F90:59-121) of the checked
+// rain, snow and graupel, none of them melting
 template <class R>
-__device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k) {
+__device__ __forceinline__ R dry_reflectivity(const ConstView<S_t<R>>& C, const Lvl<R>& L) {
+  R ze_r = R(1.e-22), ze_s = R(1.e-22), ze_g = R(1.e-22);
+  if (L.l_qr) {
+    const R lamr = R(1.0) / L.ilamr;
+    const R n0_r = L.nr * C.u.org2 * mpow(lamr, R(kCre[1]));
+    ze_r = n0_r * C.u.crg[3] * mpow(L.ilamr, R(kCre[3]));
+  }
+  const R k6 = R(0.176 / 0.93) * (R(6.0) / R(kPi)) * (R(6.0) / R(kPi));
+  if (L.l_qs) ze_s = k6 * (R(kAmS) / R(900.0)) * (R(kAmS) / R(900.0)) * L.smoz;
+  if (L.l_qg) {
+    const int idx = L.idx_bg;
+    const R n0_g = L.ng * C.u.ogg2 * mpow(R(1.0) / L.ilamg, R(kCge1));
+    ze_g = k6 * (C.l.am_g[idx - 1] / R(900.0)) * (C.l.am_g[idx - 1] / R(900.0)) * n0_g * C.u.cgg[3][0] *
+           mpow(L.ilamg, R(kCge3));
+  }
+  return mx(R(-35.0), R(10.0) * mlog10((ze_r + ze_s + ze_g) * R(1.e18)));
+}
+
+// the step's own final update: new state and diagnostics stored
+struct StoreOutputs {
+  static constexpr bool kAdjoint = false;
+};
+
+// freeze/melt, final update, final checks and diagnostics of point (c, k)
+// (src/module_mp_tempo_main.F90:729-863).  An adjoint pass (Out::kAdjoint)
+// stores nothing: out takes the new state and the reflectivity as they are,
+// and supplies the tangents of the post-sedimentation tendencies.
+template <class R, class Out>
+__device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k, Out& out) {
   const ConstView<S_t<R>> C = const_view(a.cst);
   const size_t o = TEMPO_IDX_STATE(a, c, k);
   const size_t s = TEMPO_IDX_SCR(a, c, k);
@@ -1419,6 +1447,7 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
   auto ten = [&](int m, unsigned bit) {
     const Sd_t<R>& x = sd[size_t(SD_QRTEN + m) * plane + s];
     if constexpr (IsDual<R>::value) {
+      if constexpr (Out::kAdjoint) return R(Sd_t<R>(x.v, out.ten_tangent(m)));
       if (a.post) return R(Sd_t<R>(a.post[size_t(m) * plane + s], x.d));
       return R(x);
     } else {
@@ -1449,8 +1478,12 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
   const R t_new = load_t(a, o) + L.tten * dt;
   const R qv_new = mx(R(kMinQv), (a.f[F_QV][o] + L.qvten * dt));
   L.rho = rho_of(C, L.pres, L.temp, L.qv);
-  if (has_nwfa) a.fo[F_NWFA][o] = mx(R(kNwfaDefault), mn(R(kAeroMax), (a.f[F_NWFA][o] + L.nwfaten * dt)));
-  if (has_nifa) a.fo[F_NIFA][o] = mx(R(kNifaDefault), mn(R(kAeroMax), (a.f[F_NIFA][o] + L.nifaten * dt)));
+  auto nwfa_new = [&]() { return mx(R(kNwfaDefault), mn(R(kAeroMax), (a.f[F_NWFA][o] + L.nwfaten * dt))); };
+  auto nifa_new = [&]() { return mx(R(kNifaDefault), mn(R(kAeroMax), (a.f[F_NIFA][o] + L.nifaten * dt))); };
+  if constexpr (!Out::kAdjoint) {
+    if (has_nwfa) a.fo[F_NWFA][o] = nwfa_new();
+    if (has_nifa) a.fo[F_NIFA][o] = nifa_new();
+  }
   // final checks (:750-781)
   cloud_check(C, L, qc1d, nc1d, has_nc, ncv, dt, odt);
   rain_check(C, L, qr1d, nr1d, dt, odt);
@@ -1460,6 +1493,26 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
   if (L.l_qs) snow_moments(C, L.rs, mn(R(-0.1), L.temp - R(kT0)), 4 | 32, L);
   graupel_check(C, L, qg1d, ng1d, qb1d, has_ngqb, dt, odt);
 
+  if constexpr (Out::kAdjoint) {  // (temperature form only)
+    out.add(F_T, t_new);
+    out.add(F_QV, qv_new);
+    out.add(F_QC, qc1d);
+    out.add(F_QR, qr1d);
+    out.add(F_QI, qi1d);
+    out.add(F_QS, qs1d);
+    out.add(F_QG, qg1d);
+    out.add(F_NI, ni1d);
+    out.add(F_NR, nr1d);
+    if (has_nc) out.add(F_NC, nc1d);
+    if (has_nwfa) out.add(F_NWFA, nwfa_new());
+    if (has_nifa) out.add(F_NIFA, nifa_new());
+    if (has_ngqb) {
+      out.add(F_NG, ng1d);
+      out.add(F_QB, qb1d);
+    }
+    if (a.fl.refl10cm && out.wants_refl()) out.add_refl(dry_reflectivity(C, L));
+    return;
+  }
   if (a.f[F_T])
     a.fo[F_T][o] = t_new;
   else
@@ -1511,23 +1564,7 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
   }
   if (a.d3[D3_REFL]) {  // reflectivity_10cm (:59-121)
     R dbz = R(-35.0);
-    if (a.fl.refl10cm) {
-      R ze_r = R(1.e-22), ze_s = R(1.e-22), ze_g = R(1.e-22);
-      if (L.l_qr) {
-        const R lamr = R(1.0) / L.ilamr;
-        const R n0_r = L.nr * C.u.org2 * mpow(lamr, R(kCre[1]));
-        ze_r = n0_r * C.u.crg[3] * mpow(L.ilamr, R(kCre[3]));
-      }
-      const R k6 = R(0.176 / 0.93) * (R(6.0) / R(kPi)) * (R(6.0) / R(kPi));
-      if (L.l_qs) ze_s = k6 * (R(kAmS) / R(900.0)) * (R(kAmS) / R(900.0)) * L.smoz;
-      if (L.l_qg) {
-        const int idx = L.idx_bg;
-        const R n0_g = L.ng * C.u.ogg2 * mpow(R(1.0) / L.ilamg, R(kCge1));
-        ze_g = k6 * (C.l.am_g[idx - 1] / R(900.0)) * (C.l.am_g[idx - 1] / R(900.0)) * n0_g * C.u.cgg[3][0] *
-               mpow(L.ilamg, R(kCge3));
-      }
-      dbz = mx(R(-35.0), R(10.0) * mlog10((ze_r + ze_s + ze_g) * R(1.e18)));
-    }
+    if (a.fl.refl10cm) dbz = dry_reflectivity(C, L);
     // levels with melting snow or graupel are k_melt_refl's
     if (!(melt_level(a, c, k) && (L.l_qs || L.l_qg))) a.d3[D3_REFL][d3] = dbz;
   }
@@ -1568,7 +1605,8 @@ __global__ void __launch_bounds__(256) TEMPO_ATTR_C k_phase_c(StepArgs<R> a) {
   if (a.nlev && k >= a.nlev[c]) return;
   if (a.lvl_on && !a.lvl_on[k]) return;
   SigScope<R> scope(a, c, k, 1);
-  phase_c_point(a, c, k);
+  StoreOutputs out;
+  phase_c_point(a, c, k, out);
 }
 
 // ------------------------------------ public check-and-update routines ----
