@@ -278,8 +278,8 @@ struct SigScope<Sig<T>> {
 // mass- and number-weighted speeds
 template <class R>
 __device__ __forceinline__ void rain_fallspeed(const ConstView<S_t<R>>& C, R rhof, R lamr, R& v1, R& v2) {
-  v1 = rhof * R(kAvR) * C.u.crg[5] * C.u.org3 * mpow(lamr, R(kCre[2])) * mpow(lamr + R(kFvR), -R(kCre[5]));
-  v2 = rhof * R(kAvR) * C.u.crg[6] / C.u.crg[11] * mpow(lamr, R(kCre[11])) * mpow(lamr + R(kFvR), -R(kCre[6]));
+  v1 = rhof * R(kAvR) * C.u.crg[5] * C.u.org3 * mpow(lamr, expo<R>(C.u.cre[2], kCre[2])) * mpow(lamr + R(kFvR), -expo<R>(C.u.cre[5], kCre[5]));
+  v2 = rhof * R(kAvR) * C.u.crg[6] / C.u.crg[11] * mpow(lamr, expo<R>(C.u.cre[11], kCre[11])) * mpow(lamr + R(kFvR), -expo<R>(C.u.cre[6], kCre[6]));
 }
 template <class R>
 __device__ __forceinline__ void graupel_fallspeed(const ConstView<S_t<R>>& C, const Lvl<R>& L, R rhof, R visco, bool has_qb,
@@ -1245,8 +1245,8 @@ __global__ void __launch_bounds__(256) k_melt_refl(StepArgs<R> a) {
     if (wet) {
       if (L.l_qr) {
         const R lamr = R(1.0) / L.ilamr;
-        const R n0_r = L.nr * C.u.org2 * mpow(lamr, R(kCre[1]));
-        ze_r = n0_r * C.u.crg[3] * mpow(L.ilamr, R(kCre[3]));
+        const R n0_r = L.nr * C.u.org2 * mpow(lamr, expo<R>(C.u.cre[1], kCre[1]));
+        ze_r = n0_r * C.u.crg[3] * mpow(L.ilamr, expo<R>(C.u.cre[3], kCre[3]));
       }
       pts[tid] = radar::Wet{double(value(L.rs)), double(value(L.smob)), double(value(L.smoc)), double(value(L.rr)),
                             double(value(L.rg)), double(value(L.ng)), double(value(L.ilamg)),
@@ -1342,16 +1342,16 @@ __device__ __forceinline__ R dry_reflectivity(const ConstView<S_t<R>>& C, const 
   R ze_r = R(1.e-22), ze_s = R(1.e-22), ze_g = R(1.e-22);
   if (L.l_qr) {
     const R lamr = R(1.0) / L.ilamr;
-    const R n0_r = L.nr * C.u.org2 * mpow(lamr, R(kCre[1]));
-    ze_r = n0_r * C.u.crg[3] * mpow(L.ilamr, R(kCre[3]));
+    const R n0_r = L.nr * C.u.org2 * mpow(lamr, expo<R>(C.u.cre[1], kCre[1]));
+    ze_r = n0_r * C.u.crg[3] * mpow(L.ilamr, expo<R>(C.u.cre[3], kCre[3]));
   }
   const R k6 = R(0.176 / 0.93) * (R(6.0) / R(kPi)) * (R(6.0) / R(kPi));
   if (L.l_qs) ze_s = k6 * (R(kAmS) / R(900.0)) * (R(kAmS) / R(900.0)) * L.smoz;
   if (L.l_qg) {
     const int idx = L.idx_bg;
-    const R n0_g = L.ng * C.u.ogg2 * mpow(R(1.0) / L.ilamg, R(kCge1));
+    const R n0_g = L.ng * C.u.ogg2 * mpow(R(1.0) / L.ilamg, expo<R>(C.l.cge[1][0], kCge1));
     ze_g = k6 * (C.l.am_g[idx - 1] / R(900.0)) * (C.l.am_g[idx - 1] / R(900.0)) * n0_g * C.u.cgg[3][0] *
-           mpow(L.ilamg, R(kCge3));
+           mpow(L.ilamg, expo<R>(C.l.cge[3][0], kCge3));
   }
   return mx(R(-35.0), R(10.0) * mlog10((ze_r + ze_s + ze_g) * R(1.e18)));
 }
@@ -1539,7 +1539,7 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
     R hail = R(0.0);
     if (L.rg / L.rho >= R(1.e-6) && rho_g<R>(L.idx_bg) >= R(350.0)) {
       const R lamg = R(1.0) / L.ilamg;
-      const R n0_g = L.ng * C.u.ogg2 * mpow(lamg, R(kCge1));
+      const R n0_g = L.ng * C.u.ogg2 * mpow(lamg, expo<R>(C.l.cge[1][0], kCge1));
       R sum_nh = R(0), sum_t = R(0);
       const R thr = R(0.0005);
       int n;
