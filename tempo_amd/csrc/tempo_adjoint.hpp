@@ -57,7 +57,9 @@ __host__ __device__ constexpr int adj_y_of(int f) {
 struct AdjArgs {
   const double* ybar;   // AY_N planes (compact c + k*ncol), absent outputs all zero
   int* lvl_on;          // nz: 1 where some output cotangent of the level is non-zero
-  int* pt_loc;          // compact plane: 1 where a local pass's phase A runs (see k_adj_point_flags)
+  const double* post;   // 10 planes (tiled): post-sedimentation tendency values, SD_QRTEN order
+  unsigned* list;       // points the local passes run at (see k_adj_point_list), c + k*ncol each
+  unsigned* count;      // how many
   const double* pbar;   // 4 x ncol: rain, graupel, snow, ice precipitation
   double* xbar;         // AX_N planes (compact)
   // the planes that S^T reads and writes are tiled like the step scratch: its
@@ -67,18 +69,7 @@ struct AdjArgs {
   double* work;         // AW_N scratch planes (tiled like the step scratch)
 };
 
-// ---- tangent seeding and collection (one lane per (column, level)) ------
-// seed the tangent of one input field, clearing the previous pass's seed
-// (prev < 0: none)
-template <class D>
-__global__ void __launch_bounds__(256) k_adj_seed_input(StepArgs<D> a, int field, int prev) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
-  if (c >= a.ncol) return;
-  const size_t o = TEMPO_IDX_STATE(a, c, k);
-  if (prev >= 0 && a.f[prev]) a.f[prev][o].d = 0;
-  if (a.f[field]) a.f[field][o].d = 1;
-}
-
+// ---- flags, lists and direct passes (one lane per (column, level)) ------
 // the values of the ten post-sedimentation tendency planes after the
 // tangent-free forward's sedimentation, plane m at post[m * plane + s]
 template <class D>
@@ -88,42 +79,6 @@ __global__ void __launch_bounds__(256) k_adj_keep_post(StepArgs<D> a, double* __
   const size_t s = TEMPO_IDX_SCR(a, c, k);
 #pragma unroll
   for (int m = 0; m < 10; ++m) post[size_t(m) * a.plane + s] = a.sd[size_t(SD_QRTEN + m) * a.plane + s].v;
-}
-
-// after phase A of a local pass: the S^T part of xbar_i, (dz/dx_i) . zbar,
-// from the tangents of the sedimentation inputs (masses, numbers, raw fall
-// speeds, density) and the cotangents zbar that S^T has already produced.
-// The final update then reads the forward's post-sedimentation tendency
-// values (k_adj_keep_post, a.post) with the local tangents phase A left in
-// the scratch (S frozen out); it reads neither the sedimenting masses nor
-// the fall speeds, so their tangents need not be cleared.
-template <class D>
-__global__ void __launch_bounds__(256) k_adj_capture(StepArgs<D> a, AdjArgs g, double* __restrict__ xb) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
-  if (c >= a.ncol) return;
-  const size_t s = TEMPO_IDX_SCR(a, c, k), e = size_t(c) + size_t(k) * a.ncol;
-  if (!g.pt_loc[e]) {  // skipped by phase A: zero tangents against zero zbar, no final update
-    xb[e] = 0.0;
-    return;
-  }
-  const int sdf[10] = {SD_RR, SD_NR, SD_RG, SD_NG, SD_RB, SD_RS, SD_RI, SD_NI, SD_RC, SD_NC};
-  const int srf[9] = {SR_VTRR, SR_VTNR, SR_VTRG, SR_VTNG, SR_VTS, SR_VTRI, SR_VTNI, SR_VTRC, SR_VTNC};
-  // a tangent is read only where its cotangent is non-zero (a finite
-  // tangent times zero adds nothing)
-  double acc = 0.0;
-#pragma unroll
-  for (int q = 0; q < 10; ++q) {
-    const double z = g.zbar[size_t(AZ_RR + q) * a.plane + s];
-    if (z != 0.0) acc += double(a.sd[size_t(sdf[q]) * a.plane + s].d) * z;
-  }
-#pragma unroll
-  for (int q = 0; q < 9; ++q) {
-    const double z = g.zbar[size_t(AZ_VTRR + q) * a.plane + s];
-    if (z != 0.0) acc += double(a.sr[size_t(srf[q]) * a.plane + s].d) * z;
-  }
-  const double zr = g.zbar[size_t(AZ_RHO) * a.plane + s];
-  if (zr != 0.0) acc += double(a.sr[size_t(SR_RHO) * a.plane + s].d) * zr;
-  xb[e] = acc;
 }
 
 // out[0, n) = 0 (a kernel rather than a memset, so that the sequence may be
@@ -141,6 +96,7 @@ template <class D>
 __global__ void __launch_bounds__(256) k_adj_level_zero(StepArgs<D> a, AdjArgs g) {
   const int k = int(blockIdx.x * blockDim.x + threadIdx.x);
   if (k < a.nz) g.lvl_on[k] = 0;
+  if (k == 0) *g.count = 0;
 }
 template <class D>
 __global__ void __launch_bounds__(256) k_adj_level_flags(StepArgs<D> a, AdjArgs g) {
@@ -152,19 +108,40 @@ __global__ void __launch_bounds__(256) k_adj_level_flags(StepArgs<D> a, AdjArgs 
   }
   if (__ballot(nz) != 0ull && (threadIdx.x & 63u) == 0) atomicOr(&g.lvl_on[k], 1);
 }
-// after S^T: the points where the local passes' phase A runs (g.pt_loc).
-// At a point whose zbar are all zero, on a level whose final update is
-// skipped, the capture adds tangent * 0 and nothing else reads phase A's
-// results, so every local pass skips it; its tangents stay those of the
-// tangent-free forward (zero).
+// directions of a launch: ids of the passes, one per blockIdx.z
+struct AdjDirs {
+  int n, id[AX_N];
+};
+
+// after S^T: lists the points where the local passes run (g.list).  At a
+// point whose zbar are all zero, on a level without output cotangents, every
+// tangent meets a zero cotangent: its input cotangents are zero.
 template <class D>
-__global__ void __launch_bounds__(256) k_adj_point_flags(StepArgs<D> a, AdjArgs g) {
+__global__ void __launch_bounds__(256) k_adj_point_list(StepArgs<D> a, AdjArgs g, AdjDirs dirs) {
+  __shared__ unsigned n_w[4], first;
   const int c = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
-  if (c >= a.ncol) return;
-  const size_t e = size_t(c) + size_t(k) * a.ncol, s = TEMPO_IDX_SCR(a, c, k);
-  bool on = g.lvl_on[k] != 0;
-  for (int q = 0; q < AZ_N && !on; ++q) on = g.zbar[size_t(q) * a.plane + s] != 0.0;
-  g.pt_loc[e] = on ? 1 : 0;
+  const unsigned w = threadIdx.x >> 6, l = threadIdx.x & 63u;
+  const size_t e = size_t(c) + size_t(k) * a.ncol, n3 = size_t(a.ncol) * a.nz;
+  bool on = false;
+  if (c < a.ncol) {
+    const size_t s = TEMPO_IDX_SCR(a, c, k);
+    on = g.lvl_on[k] != 0;
+    for (int q = 0; q < AZ_N && !on; ++q) on = g.zbar[size_t(q) * a.plane + s] != 0.0;
+    if (!on)
+      for (int z = 0; z < dirs.n; ++z) g.xbar[size_t(dirs.id[z]) * n3 + e] = 0.0;
+  }
+  const unsigned long long m = __ballot(on);
+  if (l == 0) n_w[w] = unsigned(__popcll(m));
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned n = n_w[0] + n_w[1] + n_w[2] + n_w[3];
+    first = n ? atomicAdd(g.count, n) : 0u;
+  }
+  __syncthreads();
+  if (!on) return;
+  unsigned i = first + unsigned(__popcll(m & ((1ull << l) - 1ull)));
+  for (unsigned j = 0; j < w; ++j) i += n_w[j];
+  g.list[i] = unsigned(e);
 }
 
 // passes seeded on the post-sedimentation tendencies: ubar_m = sum over
@@ -175,17 +152,15 @@ __global__ void __launch_bounds__(256) k_adj_point_flags(StepArgs<D> a, AdjArgs 
 // assimilation's loss has cotangents is too little for the chip: 24 us for
 // the update and 17 for a separate contraction, eight times over; 45 us
 // for all eight at 16,384 x 64 (FP32).
-struct AdjDirs {
-  int n, id[AX_N];
-};
+
+// sum over outputs of ybar * tangent, in the order the final update hands
+// them over
 template <class D>
-struct UpassOutputs {
+struct Contraction {
   static constexpr bool kAdjoint = true;
   const double* ybar;  // at the point
   size_t n3;
-  int seed;
   double acc;
-  __device__ __forceinline__ double ten_tangent(int m) const { return m == seed ? 1.0 : 0.0; }
   // a tangent counts only where its cotangent is non-zero
   __device__ __forceinline__ void add_y(int q, const D& v) {
     const double y = ybar[size_t(q) * n3];
@@ -195,63 +170,153 @@ struct UpassOutputs {
   __device__ __forceinline__ bool wants_refl() const { return ybar[size_t(AY_REFL) * n3] != 0.0; }
   __device__ __forceinline__ void add_refl(const D& v) { add_y(AY_REFL, v); }
 };
+// the forward's point with one tendency seeded (the forward's tangents are zero)
+template <class D>
+struct UpassPoint : StepPoint<D>, Contraction<D> {
+  static constexpr bool kAdjoint = true;
+  int seed;
+  __device__ __forceinline__ UpassPoint(const StepArgs<D>& a, const AdjArgs& g, int c, int k, int m)
+      : StepPoint<D>(a, c, k),
+        Contraction<D>{g.ybar + size_t(c) + size_t(k) * a.ncol, size_t(a.ncol) * a.nz, 0.0},
+        seed(m) {}
+  __device__ __forceinline__ D t() const { return this->f(F_T); }
+  __device__ __forceinline__ Sd_t<D> ten(int m, const Sd_t<D>& x) const { return Sd_t<D>(x.v, m == seed ? 1.0 : 0.0); }
+};
 template <class D>
 __global__ void __launch_bounds__(256) k_adj_upass(StepArgs<D> a, AdjArgs g, AdjDirs dirs) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y, m = dirs.id[blockIdx.z];
   if (c >= a.ncol) return;
-  const size_t e = size_t(c) + size_t(k) * a.ncol, n3 = size_t(a.ncol) * a.nz;
   double* out = g.ubar + size_t(m) * a.plane + TEMPO_IDX_SCR(a, c, k);
   // no cotangents, or a point that the step leaves as it is
   if (!g.lvl_on[k] || (a.cf[c] & CF_EXIT) || (a.nlev && k >= a.nlev[c])) {
     *out = 0.0;
     return;
   }
-  UpassOutputs<D> u{g.ybar + e, n3, m, 0.0};
-  phase_c_point(a, c, k, u);
-  *out = u.acc;
+  UpassPoint<D> p(a, g, c, k, m);
+  phase_c_point(a, c, k, p);
+  *out = p.acc;
 }
 
-// the seed of the next pass, moved by the contraction that ends a pass (the
-// seeding runs on the same grid): the input field `clear` loses its tangent
-// seed, `set` gets one (< 0: none)
-struct AdjSeed {
-  int set, clear;
-};
-
-// out (+)= sum over outputs of ybar * tangent (0 at a level without
-// output cotangents, whose final update a.lvl_on skipped); then the next
-// pass's seed at this point.  A point the step leaves as it is (an
-// early-exit column, a level at or above the column's nlev) has no final
-// update writing its new state: its output tangents are its input tangents,
-// and its reflectivity is no function of the inputs (a constant in an
-// early-exit column, left as it is above nlev).
+// ---- local passes: xbar_i = (dz/dx_i) . zbar + the local part through A and
+// C, one direction i per seeded input field.  They run at the listed points
+// only, `points` of them times the launch's directions at a time, and keep
+// what phase A hands to the final update by position in the launch, not by
+// point, so that all directions fit into the scratch of one.  A direction
+// alone leaves the chip waiting (an assimilation's loss flags an eighth of
+// the points: 2,000 wavefronts, one per slot, 104 us of one wavefront's
+// latency for each of nine, and 58 us in three kernels after it); together
+// 348 us at 16,384 x 64 (FP32) against 1458.
 template <class D>
-__global__ void __launch_bounds__(256) k_adj_contract(StepArgs<D> a, AdjArgs g, double* out, int accumulate,
-                                                      AdjSeed nx) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
-  if (c >= a.ncol) return;
-  const size_t o = TEMPO_IDX_STATE(a, c, k), e = size_t(c) + size_t(k) * a.ncol, n3 = size_t(a.ncol) * a.nz;
-  const bool kept = (a.cf[c] & CF_EXIT) || (a.nlev && k >= a.nlev[c]);
-  if (a.lvl_on && !a.lvl_on[k]) {
-    if (!accumulate) out[e] = 0.0;
-  } else {
-    double acc = 0.0;  // tangents read only where their cotangent is non-zero
-    for (int q = 0; q < AY_REFL; ++q) {
-      const D* f = kept ? a.f[adj_y_field(q)] : a.fo[adj_y_field(q)];
-      if (!f) continue;
-      const double y = g.ybar[size_t(q) * n3 + e];
-      if (y != 0.0) acc += y * double(f[o].d);
-    }
-    if (a.d3[D3_REFL] && !kept) {
-      const double y = g.ybar[size_t(AY_REFL) * n3 + e];
-      if (y != 0.0) acc += y * double(a.d3[D3_REFL][o].d);
-    }
-    out[e] = accumulate ? out[e] + acc : acc;
+struct AdjLocal {
+  D* sr;
+  Sd_t<D>* sd;
+  unsigned* pf;
+  D* fa;                 // F_NFIELDS planes: state after the initial checks
+  size_t plane, fplane;  // strides of the scratch and fa planes
+  size_t room;           // point-directions they hold
+};
+// position in a launch, point and direction of a thread
+struct LocalSlot {
+  size_t v;  // blockIdx.z * points + the place among the launch's points
+  int c, k;
+  bool in;
+};
+__device__ __forceinline__ LocalSlot local_slot(const AdjArgs& g, int ncol, unsigned first, unsigned points) {
+  const unsigned w = blockIdx.x * blockDim.x + threadIdx.x;
+  LocalSlot q{size_t(blockIdx.z) * points + w, 0, 0, w < points && first + w < *g.count};
+  if (q.in) {
+    const unsigned e = g.list[first + w];
+    q.k = int(e / unsigned(ncol));
+    q.c = int(e % unsigned(ncol));
   }
-  if (nx.clear >= 0 && a.f[nx.clear]) a.f[nx.clear][o].d = 0;
-  if (nx.set >= 0 && a.f[nx.set]) a.f[nx.set][o].d = 1;
+  return q;
 }
-
+template <class D>
+struct LocalPoint : Contraction<D> {
+  static constexpr bool kAdjoint = true;
+  const StepArgs<D>& a;
+  const AdjLocal<D>& q;
+  const double* post;
+  size_t o, s, fwd;  // inputs, position, the forward's scratch
+  int seed;          // seeded input field
+  __device__ __forceinline__ LocalPoint(const StepArgs<D>& args, const AdjArgs& g, const AdjLocal<D>& scr, int c, int k,
+                                        size_t v, int field)
+      : Contraction<D>{g.ybar + size_t(c) + size_t(k) * args.ncol, size_t(args.ncol) * args.nz, 0.0},
+        a(args),
+        q(scr),
+        post(g.post),
+        o(TEMPO_IDX_STATE(args, c, k)),
+        s(v),
+        fwd(TEMPO_IDX_SCR(args, c, k)),
+        seed(field) {}
+  __device__ __forceinline__ D f(int i) const { return D(a.f[i][o].v, i == seed ? S_t<D>(1) : S_t<D>(0)); }
+  __device__ __forceinline__ D t() const { return f(F_T); }
+  __device__ __forceinline__ void put(int i, const D& x) const { q.fa[size_t(i) * q.fplane + s] = x; }
+  __device__ __forceinline__ D fa(int i) const { return q.fa[size_t(i) * q.fplane + s]; }
+  __device__ __forceinline__ D* sr() const { return q.sr; }
+  __device__ __forceinline__ Sd_t<D>* sd() const { return q.sd; }
+  __device__ __forceinline__ unsigned* pf() const { return q.pf; }
+  __device__ __forceinline__ size_t plane() const { return q.plane; }
+  // the forward's value after sedimentation with phase A's local tangent (S
+  // frozen out)
+  __device__ __forceinline__ Sd_t<D> ten(int m, const Sd_t<D>& x) const {
+    return Sd_t<D>(post[size_t(m) * a.plane + fwd], x.d);
+  }
+};
+template <class D>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WavesPerEu<D>::a)))
+k_adj_local_a(StepArgs<D> a, AdjArgs g, AdjLocal<D> scr, AdjDirs dirs, unsigned first, unsigned points) {
+  __shared__ float ccn_s[kCcnSlice];
+  if (first + blockIdx.x * blockDim.x >= *g.count) return;  // the whole block
+  phase_a_lds(a, ccn_s);
+  const LocalSlot q = local_slot(g, a.ncol, first, points);
+  if (!q.in || (a.nlev && q.k >= a.nlev[q.c])) return;
+  phase_a_point(a, q.c, q.k, LocalPoint<D>(a, g, scr, q.c, q.k, q.v, adj_x_field(dirs.id[blockIdx.z])));
+}
+// the S^T part from phase A's tangents of the sedimentation inputs (masses,
+// numbers, raw fall speeds, density) and zbar, then the final update and the
+// contraction of its outputs.  A point the step leaves as it is (an
+// early-exit column, a level at or above the column's nlev) has zero zbar,
+// its output tangents are its input tangents, and its reflectivity is no
+// function of the inputs.
+template <class D>
+__global__ void __launch_bounds__(256) k_adj_local_c(StepArgs<D> a, AdjArgs g, AdjLocal<D> scr, AdjDirs dirs,
+                                                     unsigned first, unsigned points) {
+  const LocalSlot q = local_slot(g, a.ncol, first, points);
+  if (!q.in) return;
+  const int i = dirs.id[blockIdx.z], field = adj_x_field(i);
+  const size_t n3 = size_t(a.ncol) * a.nz;
+  double* out = g.xbar + size_t(i) * n3 + size_t(q.c) + size_t(q.k) * a.ncol;
+  LocalPoint<D> p(a, g, scr, q.c, q.k, q.v, field);
+  if ((a.cf[q.c] & CF_EXIT) || (a.nlev && q.k >= a.nlev[q.c])) {
+    if (g.lvl_on[q.k]) p.add(field, D(S_t<D>(0), S_t<D>(1)));
+    *out = p.acc;
+    return;
+  }
+  const int sdf[10] = {SD_RR, SD_NR, SD_RG, SD_NG, SD_RB, SD_RS, SD_RI, SD_NI, SD_RC, SD_NC};
+  const int srf[9] = {SR_VTRR, SR_VTNR, SR_VTRG, SR_VTNG, SR_VTS, SR_VTRI, SR_VTNI, SR_VTRC, SR_VTNC};
+  // a tangent is read only where its cotangent is non-zero (a finite
+  // tangent times zero adds nothing)
+  const double* zb = g.zbar + p.fwd;
+  double acc = 0.0;
+#pragma unroll
+  for (int j = 0; j < 10; ++j) {
+    const double z = zb[size_t(AZ_RR + j) * a.plane];
+    if (z != 0.0) acc += double(scr.sd[size_t(sdf[j]) * scr.plane + q.v].d) * z;
+  }
+#pragma unroll
+  for (int j = 0; j < 9; ++j) {
+    const double z = zb[size_t(AZ_VTRR + j) * a.plane];
+    if (z != 0.0) acc += double(scr.sr[size_t(srf[j]) * scr.plane + q.v].d) * z;
+  }
+  const double zr = zb[size_t(AZ_RHO) * a.plane];
+  if (zr != 0.0) acc += double(scr.sr[size_t(SR_RHO) * scr.plane + q.v].d) * zr;
+  if (g.lvl_on[q.k]) {
+    phase_c_point(a, q.c, q.k, p);
+    acc += p.acc;
+  }
+  *out = acc;
+}
 
 // ---- S^T: sedimentation adjoint, one lane per column --------------------
 struct SedAdjCol {

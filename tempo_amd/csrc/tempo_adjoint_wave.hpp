@@ -604,25 +604,21 @@ struct AdjSnap {
 };
 
 // The passes of one adjoint.  The state is out of place: a.f holds the
-// packed inputs (duals, tangents zero except the seeded field), a.fa the
-// state after the initial checks (phase A's output), a.fo the new state
-// (the final update's output), so that no pass has to restore the state.
+// packed inputs (duals, zero tangents: the passes seed what they read), a.fa
+// the state after the initial checks (phase A's output); no pass stores a new
+// state.
 template <class D>
-hipError_t adjoint_passes(const StepArgs<D>& a, const AdjArgs& g, Dual<double>* vtbuf, size_t sr_bytes,
-                          size_t sd_bytes, AdjSnap snap, const bool* have_x, hipStream_t s) {
+hipError_t adjoint_passes(const StepArgs<D>& a, AdjArgs g, Dual<double>* vtbuf, size_t sr_bytes,
+                          size_t sd_bytes, AdjSnap snap, const AdjLocal<D>& scr, const bool* have_x, hipStream_t s) {
   const unsigned gc = unsigned((a.ncol + 255) / 256);
   const dim3 g2(gc, unsigned(a.nz));
-  const size_t n3 = size_t(a.ncol) * a.nz;
   hipError_t e;
   auto cp = [&](void* dst, const void* src, size_t n) { return hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToDevice, s); };
   auto phase_pre_a = [&]() {
     launch_prepass(a, s);
     hipLaunchKernelGGL(k_phase_a<D>, level_grid(a, 256), dim3(256), 0, s, a);
   };
-  // the final update's passes and contractions skip the levels without
-  // output cotangents
-  StepArgs<D> ac = a;
-  ac.lvl_on = g.lvl_on;
+  // the final update's passes skip the levels without output cotangents
   hipLaunchKernelGGL(k_adj_level_zero<D>, dim3(unsigned((a.nz + 255) / 256)), dim3(256), 0, s, a, g);
   hipLaunchKernelGGL(k_adj_level_flags<D>, g2, dim3(256), 0, s, a, g);
 
@@ -644,6 +640,7 @@ hipError_t adjoint_passes(const StepArgs<D>& a, const AdjArgs& g, Dual<double>* 
   else
     hipLaunchKernelGGL(k_phase_b<D>, dim3(unsigned((a.ncol + 127) / 128)), dim3(128), 0, s, a, vtbuf);
   double* post = static_cast<double*>(snap.sd_b);
+  g.post = post;
   hipLaunchKernelGGL(k_adj_keep_post<D>, g2, dim3(256), 0, s, a, post);
   // passes seeded on the post-sedimentation tendencies.  Without prognostic
   // graupel number and volume the final update does not read their
@@ -671,27 +668,27 @@ hipError_t adjoint_passes(const StepArgs<D>& a, const AdjArgs& g, Dual<double>* 
     hipLaunchKernelGGL((k_adj_sed_wave<D, 2>), gw, dim3(64 * kScrW), 0, s, a, g);
   else
     hipLaunchKernelGGL(k_adj_sedimentation<D>, dim3(unsigned((a.ncol + 63) / 64)), dim3(64), 0, s, a, g);
-  // the local passes' phase A runs at the points where they contribute,
-  // their final update on the post-sedimentation tendency values
-  StepArgs<D> al = a, acl = ac;
-  al.pt_on = g.pt_loc;
-  acl.post = post;
-  hipLaunchKernelGGL(k_adj_point_flags<D>, g2, dim3(256), 0, s, a, g);
-  // local passes, one per requested input field: xbar_i = (dz/dx_i) . zbar
-  // + the local part through A and C, phase B replaced by the forward's
-  // post-sedimentation tendency values.  The pre-pass results (column flags,
-  // heights) depend on values only and stay from the first pass.
-  int xs[AX_N], nxs = 0;
+  // the local passes, as many directions in a launch and then as many points
+  // as the scratch holds.  The count of listed points stays on the device:
+  // launches past it end at once.  The pre-pass results (column flags,
+  // heights) depend on values only and stay from the forward.
+  AdjDirs xs{};
   for (int i = 0; i < AX_N; ++i)
-    if (have_x[i]) xs[nxs++] = i;
-  if (nxs > 0) hipLaunchKernelGGL(k_adj_seed_input<D>, g2, dim3(256), 0, s, a, adj_x_field(xs[0]), -1);
-  for (int j = 0; j < nxs; ++j) {
-    double* xb = g.xbar + size_t(xs[j]) * n3;
-    hipLaunchKernelGGL(k_phase_a<D>, level_grid(a, 256), dim3(256), 0, s, al);
-    hipLaunchKernelGGL(k_adj_capture<D>, g2, dim3(256), 0, s, a, g, xb);
-    hipLaunchKernelGGL(k_phase_c<D>, level_grid(a, 256), dim3(256), 0, s, acl);
-    const AdjSeed nx{j + 1 < nxs ? adj_x_field(xs[j + 1]) : -1, j + 1 < nxs ? adj_x_field(xs[j]) : -1};
-    hipLaunchKernelGGL(k_adj_contract<D>, g2, dim3(256), 0, s, ac, g, xb, 1, nx);
+    if (have_x[i]) xs.id[xs.n++] = i;
+  if (xs.n == 0) return hipGetLastError();
+  hipLaunchKernelGGL(k_adj_point_list<D>, g2, dim3(256), 0, s, a, g, xs);
+  const size_t n3 = size_t(a.ncol) * a.nz;
+  const size_t together = std::min(size_t(xs.n), scr.room);
+  size_t points = std::min(scr.room / together, n3);
+  if (points >= 64 && points < n3) points = points / 64 * 64;
+  for (int j = 0; j < xs.n; j += int(together)) {
+    AdjDirs d{};
+    for (int i = j; i < xs.n && i < j + int(together); ++i) d.id[d.n++] = xs.id[i];
+    const dim3 gl(unsigned((points + 255) / 256), 1, unsigned(d.n));
+    for (size_t first = 0; first < n3; first += points) {
+      hipLaunchKernelGGL(k_adj_local_a<D>, gl, dim3(256), 0, s, a, g, scr, d, unsigned(first), unsigned(points));
+      hipLaunchKernelGGL(k_adj_local_c<D>, gl, dim3(256), 0, s, a, g, scr, d, unsigned(first), unsigned(points));
+    }
   }
   return hipGetLastError();
 }

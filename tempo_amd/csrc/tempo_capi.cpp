@@ -34,9 +34,11 @@ template <class R>
 hipError_t launch_surface_emissions(R* nwfa, const R* nwfa2d, int ni, int nj, long long ldk, long long ldj,
                                     long long d2ldj, int k, double dt, hipStream_t s);
 hipError_t launch_adjoint(const StepArgs<Dual<float>>& a, const AdjArgs& g, Dual<double>* vtbuf, size_t sr_bytes,
-                          size_t sd_bytes, AdjSnap snap, const bool* have_x, hipStream_t s);
+                          size_t sd_bytes, AdjSnap snap, const AdjLocal<Dual<float>>& scr, const bool* have_x,
+                          hipStream_t s);
 hipError_t launch_adjoint(const StepArgs<Dual<double>>& a, const AdjArgs& g, Dual<double>* vtbuf, size_t sr_bytes,
-                          size_t sd_bytes, AdjSnap snap, const bool* have_x, hipStream_t s);
+                          size_t sd_bytes, AdjSnap snap, const AdjLocal<Dual<double>>& scr, const bool* have_x,
+                          hipStream_t s);
 template <class T>
 hipError_t launch_to_compact_n(const PlaneBatch<T, double>& b, int n, const DualGeom& g, hipStream_t s);
 template <class T>
@@ -263,7 +265,7 @@ struct tempo_hip_ctx {
   DevBuf sr, sd, pf, cf_, precip, ksub, vtbuf, kmelt, radar;
   DevBuf semiw;  // semi-Lagrangian sedimentation work (allocated only with semi_sedi_flag)
   DevBuf tl_state, tl_diag;  // dual (value, tangent) copies for the tangent-linear step
-  DevBuf adj_in, adj_out, adj_mem;  // adjoint: packed inputs, new state, cotangent/Jacobian planes
+  DevBuf adj_in, adj_local, adj_mem;  // adjoint: packed inputs, local passes' scratch, cotangent/Jacobian planes
   DevBuf adj_snap;                  // adjoint: post-sedimentation tendencies (and scratch after A)
   int last_ncol = 0;
   void* last_ksub = nullptr;  // substep counts of the last run (its scratch)
@@ -786,11 +788,9 @@ int run_adjoint(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_fie
   const int ncol = dm->ni * dm->nj, nz = dm->nz;
   const size_t n3 = size_t(ncol) * nz, sb = F_NFIELDS * n3 * sizeof(D);
   const size_t plane = scratch_plane(size_t(ncol), size_t(nz));
-  const size_t nd = (AY_N + AX_N) * n3 + 4 * size_t(ncol) + (10 + AZ_N + AW_N) * plane + (size_t(nz) + 1) / 2 + (n3 + 1) / 2;
+  const size_t nd = (AY_N + AX_N) * n3 + 4 * size_t(ncol) + (10 + AZ_N + AW_N) * plane + (size_t(nz) + 1) / 2 + (n3 + 2) / 2;
   HIP_TRY(x->tl_state.ensure(sb));
   HIP_TRY(x->adj_in.ensure(sb));
-  HIP_TRY(x->adj_out.ensure(sb));
-  HIP_TRY(x->tl_diag.ensure((D2_N * size_t(ncol) + D3_N * n3) * sizeof(D)));
   HIP_TRY(x->adj_mem.ensure(nd * sizeof(double)));
   double* mem = x->adj_mem.as<double>();
   AdjArgs g;
@@ -803,7 +803,8 @@ int run_adjoint(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_fie
   g.pbar = pbar;
   g.work = pbar + 4 * size_t(ncol);
   g.lvl_on = reinterpret_cast<int*>(g.work + AW_N * plane);
-  g.pt_loc = reinterpret_cast<int*>(g.work + AW_N * plane + (size_t(nz) + 1) / 2);
+  g.list = reinterpret_cast<unsigned*>(g.work + AW_N * plane + (size_t(nz) + 1) / 2);
+  g.count = g.list + n3;
 
   StepArgs<D> a;
   std::memset(&a, 0, sizeof(a));
@@ -846,7 +847,6 @@ int run_adjoint(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_fie
     pc.dst[q] = pbar + size_t(q) * ncol;
   }
   HIP_TRY(launch_to_compact_n(pc, 4, g2, s));
-  a.d3[D3_REFL] = x->tl_diag.as<D>() + D2_N * size_t(ncol);
   a.land = f->land;
   a.nlev = dm->nlev;
   a.ni = ncol;
@@ -871,14 +871,29 @@ int run_adjoint(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_fie
   HIP_TRY(x->adj_snap.ensure(wave_b ? 10 * a.plane * sizeof(double) : srb + 2 * sdb));
   char* sp = static_cast<char*>(x->adj_snap.p);
   const AdjSnap snap = wave_b ? AdjSnap{nullptr, nullptr, sp} : AdjSnap{sp, sp + srb, sp + srb + sdb};
-  // out of place: inputs in adj_in, post-check state in tl_state, new state in adj_out
-  D* out = x->adj_out.as<D>();
+  // out of place: inputs in adj_in, post-check state in tl_state; no pass
+  // stores a new state
+  int ndir = 0;
   for (int i = 0; i < F_NFIELDS; ++i) {
     a.f[i] = fp[i] ? in + size_t(i) * n3 : nullptr;
-    a.fa[i] = fp[i] ? st + size_t(i) * n3 : nullptr;
-    a.fo[i] = fp[i] ? out + size_t(i) * n3 : nullptr;
+    a.fa[i] = a.fo[i] = fp[i] ? st + size_t(i) * n3 : nullptr;
   }
-  HIP_TRY(launch_adjoint(a, g, x->vtbuf.as<Dual<double>>(), srb, sdb, snap, have_x, s));
+  for (bool h : have_x) ndir += h;
+  // the local passes' scratch: of a large batch the forward's, done with by
+  // then; a smaller one's would leave launches that do not fill the chip, so
+  // it gets its own, up to kLocalRoom point-directions
+  constexpr size_t kLocalRoom = size_t(1) << 21;
+  AdjLocal<D> scr{a.sr, a.sd, a.pf, st, a.plane, n3, n3};
+  if (n3 < kLocalRoom && ndir > 1) {
+    const size_t m = std::min(kLocalRoom, (n3 * size_t(ndir) + 63) / 64 * 64);
+    HIP_TRY(x->adj_local.ensure(m * (SD_N * sizeof(Dual<double>) + (SR_N + F_NFIELDS) * sizeof(D) + sizeof(unsigned))));
+    scr.sd = x->adj_local.as<Dual<double>>();
+    scr.sr = reinterpret_cast<D*>(scr.sd + SD_N * m);
+    scr.fa = scr.sr + SR_N * m;
+    scr.pf = reinterpret_cast<unsigned*>(scr.fa + F_NFIELDS * m);
+    scr.plane = scr.fplane = scr.room = m;
+  }
+  HIP_TRY(launch_adjoint(a, g, x->vtbuf.as<Dual<double>>(), srb, sdb, snap, scr, have_x, s));
   PlaneBatch<double, T> xc{};
   int nxc = 0;
   for (int i = 0; i < AX_N; ++i)

@@ -251,6 +251,25 @@ __device__ __forceinline__ void put_post_check(const StepArgs<R>& a, int f, size
   if (a.fa[f] != a.f[f] || !same_bits(a.f[f][o], v)) a.fa[f][o] = v;
 }
 
+// where a level-local kernel finds point (c, k) and puts its results: the
+// step's own arrays (an adjoint pass has others)
+template <class R>
+struct StepPoint {
+  static constexpr bool kAdjoint = false;
+  const StepArgs<R>& a;
+  size_t o, s;  // of the state and the scratch
+  __device__ __forceinline__ StepPoint(const StepArgs<R>& args, int c, int k)
+      : a(args), o(TEMPO_IDX_STATE(args, c, k)), s(TEMPO_IDX_SCR(args, c, k)) {}
+  __device__ __forceinline__ R f(int i) const { return a.f[i][o]; }
+  __device__ __forceinline__ R fa(int i) const { return a.fa[i][o]; }
+  __device__ __forceinline__ R t() const { return load_t(a, o); }
+  __device__ __forceinline__ void put(int i, const R& v) const { put_post_check(a, i, o, v); }
+  __device__ __forceinline__ R* sr() const { return a.sr; }
+  __device__ __forceinline__ Sd_t<R>* sd() const { return a.sd; }
+  __device__ __forceinline__ unsigned* pf() const { return a.pf; }
+  __device__ __forceinline__ size_t plane() const { return a.plane; }
+};
+
 // branch signature of a level-local kernel's point: opened on entry, stored
 // at every exit (the plain types record nothing)
 template <class R>
@@ -348,42 +367,40 @@ __device__ __forceinline__ ClearAir<R> clear_air_tendencies(const ConstView<S_t<
 
 // the level-local physics of point (c, k), from the initial checks to the
 // fall speeds (src/module_mp_tempo_main.F90:320-588)
-template <class R>
-__device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k) {
+template <class R, class Point>
+__device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k, const Point& pt) {
   const ConstView<S_t<R>> C = lds_const_view(a.cst);
-  const size_t o = TEMPO_IDX_STATE(a, c, k);
-  const size_t s = TEMPO_IDX_SCR(a, c, k);
-  const size_t plane = a.plane;
+  const size_t s = pt.s, plane = pt.plane();
   const R dt = R(a.dt), odt = R(a.odt);
   const unsigned cf = a.cf[c];
   const bool has_nc = a.f[F_NC], has_nwfa = a.f[F_NWFA], has_nifa = a.f[F_NIFA];
   const bool has_ngqb = a.f[F_NG] && a.f[F_QB];
 
   Lvl<R> L;
-  const R t1d = load_t(a, o), qv1d = a.f[F_QV][o], w = a.f[F_W][o];
-  R qc1d = a.f[F_QC][o], qr1d = a.f[F_QR][o], qi1d = a.f[F_QI][o], qs1d = a.f[F_QS][o], qg1d = a.f[F_QG][o];
-  R ni1d = a.f[F_NI][o], nr1d = a.f[F_NR][o];
-  R nc1d = has_nc ? a.f[F_NC][o] : R(0), ng1d = has_ngqb ? a.f[F_NG][o] : R(0), qb1d = has_ngqb ? a.f[F_QB][o] : R(0);
-  const R nwfa1d = has_nwfa ? a.f[F_NWFA][o] : R(0), nifa1d = has_nifa ? a.f[F_NIFA][o] : R(0);
+  const R t1d = pt.t(), qv1d = pt.f(F_QV), w = pt.f(F_W);
+  R qc1d = pt.f(F_QC), qr1d = pt.f(F_QR), qi1d = pt.f(F_QI), qs1d = pt.f(F_QS), qg1d = pt.f(F_QG);
+  R ni1d = pt.f(F_NI), nr1d = pt.f(F_NR);
+  R nc1d = has_nc ? pt.f(F_NC) : R(0), ng1d = has_ngqb ? pt.f(F_NG) : R(0), qb1d = has_ngqb ? pt.f(F_QB) : R(0);
+  const R nwfa1d = has_nwfa ? pt.f(F_NWFA) : R(0), nifa1d = has_nifa ? pt.f(F_NIFA) : R(0);
 
   if constexpr (!IsDual<R>::value) {
     if (a.sparse & SPARSE_CLEAR) {
-      const R pres = a.f[F_P][o];
+      const R pres = pt.f(F_P);
       const bool dry = !(qc1d > R(kR1) || qr1d > R(kR1) || qi1d > R(kR1) || qs1d > R(kR1) || qg1d > R(kR1));
       if (__all(dry && ((cf & CF_EXIT) || clear_air(pres, t1d, mx(R(kMinQv), qv1d))))) {
         // the initial checks remove what is below r1, and its number
         const int fz[] = {F_QC, F_QR, F_NR, F_QI, F_NI, F_QS, F_QG};
-        for (int f : fz) put_post_check(a, f, o, R(0));
-        if (has_nc) put_post_check(a, F_NC, o, R(0));
+        for (int f : fz) pt.put(f, R(0));
+        if (has_nc) pt.put(F_NC, R(0));
         if (has_ngqb) {
-          put_post_check(a, F_NG, o, R(0));
-          put_post_check(a, F_QB, o, R(0));
+          pt.put(F_NG, R(0));
+          pt.put(F_QB, R(0));
         }
         if (cf & CF_EXIT) return;
         const ClearAir<R> q = clear_air_tendencies<R>(C, pres, t1d, qv1d, dt, odt);
-        a.sr[SR_RHO * plane + s] = q.rho;
-        if (k == 0) a.sr[SR_TEMP * plane + s] = q.temp;
-        a.pf[s] = PF_CLEAR;
+        pt.sr()[SR_RHO * plane + s] = q.rho;
+        if (k == 0) pt.sr()[SR_TEMP * plane + s] = q.temp;
+        pt.pf()[s] = PF_CLEAR;
         return;
       }
     }
@@ -394,7 +411,7 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
   L.smob = L.smoc = L.smo0 = L.smo1 = L.smo2 = L.smoe = L.smof = L.smoz = R(0);
   L.temp = t1d;
   L.qv = mx(R(kMinQv), qv1d);
-  L.pres = a.f[F_P][o];
+  L.pres = pt.f(F_P);
   L.rho = rho_of(C, L.pres, L.temp, L.qv);
   // aerosols: a present field overrides the default profile (:328-345)
   L.nwfa = has_nwfa ? nwfa1d * L.rho : default_aerosol(a, c, k, R(kNaccn0), R(kNaccn1));
@@ -414,7 +431,7 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
   if (a.fl.ml_for_nc && !has_nc) {
     const R xrx = qc1d <= R(S_t<R>(1.e-12)) ? R(0.0) : qc1d;
     ncv = ml_cloud_number(xrx, qr1d, qi1d, qs1d, L.pres, L.temp, w) * L.rho;
-    a.sr[SR_NCSAVE * plane + s] = ncv;
+    pt.sr()[SR_NCSAVE * plane + s] = ncv;
   } else {
     ncv = column_nc(a, c);
   }
@@ -432,17 +449,17 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
   graupel_check(C, L, qg1d, ng1d, qb1d, has_ngqb, dt, odt);
   // the post-check state is the 1-d state for the rest of the step; a step
   // in place writes back only the values the checks changed
-  put_post_check(a, F_QC, o, qc1d);
-  put_post_check(a, F_QR, o, qr1d);
-  put_post_check(a, F_NR, o, nr1d);
-  put_post_check(a, F_QI, o, qi1d);
-  put_post_check(a, F_NI, o, ni1d);
-  put_post_check(a, F_QS, o, qs1d);
-  put_post_check(a, F_QG, o, qg1d);
-  if (has_nc) put_post_check(a, F_NC, o, nc1d);
+  pt.put(F_QC, qc1d);
+  pt.put(F_QR, qr1d);
+  pt.put(F_NR, nr1d);
+  pt.put(F_QI, qi1d);
+  pt.put(F_NI, ni1d);
+  pt.put(F_QS, qs1d);
+  pt.put(F_QG, qg1d);
+  if (has_nc) pt.put(F_NC, nc1d);
   if (has_ngqb) {
-    put_post_check(a, F_NG, o, ng1d);
-    put_post_check(a, F_QB, o, qb1d);
+    pt.put(F_NG, ng1d);
+    pt.put(F_QB, qb1d);
   }
   if (cf & CF_EXIT) return;
   L.qcten = L.qiten = L.qrten = L.qsten = L.qgten = L.ngten = L.qbten = L.niten = L.nrten = L.ncten = R(0);
@@ -556,7 +573,7 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
     vtnc = L.rhof * R(kAvC) * C.l.ccg[3][nu] * C.l.ocg1[nu] * mpow(L.ilamc, R(kBvC));
   }
 
-  R* sr = a.sr;
+  R* sr = pt.sr();
   sr[SR_TEMP * plane + s] = L.temp;
   sr[SR_QV * plane + s] = L.qv;
   sr[SR_RHO * plane + s] = L.rho;
@@ -582,7 +599,7 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
   const bool tc = all || L.l_qc || moves(L.qcten) || (has_nc && moves(L.ncten));
   pf |= (tr ? PF_TR : 0u) | (tg ? PF_TG : 0u) | (ts ? PF_TS : 0u) | (ti ? PF_TI : 0u) | (tc ? PF_TC : 0u);
   using D = Sd_t<R>;
-  D* sd = a.sd;
+  D* sd = pt.sd();
   if (sector(L.l_qr)) {
     sd[SD_RR * plane + s] = D(L.rr);
     sd[SD_NR * plane + s] = D(L.nr);
@@ -630,7 +647,19 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
     sd[SD_QCTEN * plane + s] = D(L.qcten);
     sd[SD_NCTEN * plane + s] = D(L.ncten);
   }
-  a.pf[s] = pf;
+  pt.pf()[s] = pf;
+}
+
+// what phase A reads from LDS, by the whole block
+template <class R>
+__device__ __forceinline__ void phase_a_lds(StepArgs<R>& a, float* ccn_s) {
+  pow10_fill<S_t<R>>();
+  lane_const_fill(a.cst);
+  if (a.ccn_lds) {
+    for (int i = int(threadIdx.x); i < kCcnSlice; i += int(blockDim.x)) ccn_s[i] = a.tab.ccn[i];
+    a.tab.ccn = ccn_s;
+  }
+  __syncthreads();
 }
 
 // kWaves: waves per SIMD the kernel is compiled for.  With a.ccn_lds the
@@ -639,20 +668,13 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
 template <class R, int kWaves = WavesPerEu<R>::a>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) k_phase_a(StepArgs<R> a) {
   __shared__ float ccn_s[kCcnSlice];
-  pow10_fill<S_t<R>>();
-  lane_const_fill(a.cst);
-  if (a.ccn_lds) {
-    for (int i = int(threadIdx.x); i < kCcnSlice; i += int(blockDim.x)) ccn_s[i] = a.tab.ccn[i];
-    a.tab.ccn = ccn_s;
-  }
-  __syncthreads();
+  phase_a_lds(a, ccn_s);
   const int2 pt = block_point<R, false>(a);
   const int c = pt.x, k = pt.y;
   if (c >= a.ncol || k >= a.nz) return;
   if (a.nlev && k >= a.nlev[c]) return;
-  if (IsDual<R>::value && a.pt_on && !a.pt_on[size_t(c) + size_t(k) * a.ncol]) return;  // an adjoint's local pass
   SigScope<R> scope(a, c, k, 0);
-  phase_a_point(a, c, k);
+  phase_a_point(a, c, k, StepPoint<R>(a, c, k));
 }
 
 // ----------------------------------------------------------- phase B ----
@@ -1356,21 +1378,14 @@ __device__ __forceinline__ R dry_reflectivity(const ConstView<S_t<R>>& C, const 
   return mx(R(-35.0), R(10.0) * mlog10((ze_r + ze_s + ze_g) * R(1.e18)));
 }
 
-// the step's own final update: new state and diagnostics stored
-struct StoreOutputs {
-  static constexpr bool kAdjoint = false;
-};
-
 // freeze/melt, final update, final checks and diagnostics of point (c, k)
-// (src/module_mp_tempo_main.F90:729-863).  An adjoint pass (Out::kAdjoint)
-// stores nothing: out takes the new state and the reflectivity as they are,
-// and supplies the tangents of the post-sedimentation tendencies.
-template <class R, class Out>
-__device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k, Out& out) {
+// (src/module_mp_tempo_main.F90:729-863).  An adjoint pass (Point::kAdjoint)
+// stores nothing: pt takes the new state and the reflectivity as they are,
+// and supplies the post-sedimentation tendencies.
+template <class R, class Point>
+__device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k, Point& pt) {
   const ConstView<S_t<R>> C = const_view(a.cst);
-  const size_t o = TEMPO_IDX_STATE(a, c, k);
-  const size_t s = TEMPO_IDX_SCR(a, c, k);
-  const size_t plane = a.plane;
+  const size_t o = pt.o, s = pt.s, plane = pt.plane();
   const size_t d3 = size_t(c % a.ni) + size_t(k) * a.dldk + size_t(c / a.ni) * a.dldj;
   const R dt = R(a.dt), odt = R(a.odt);
   const bool live = !(a.cf[c] & CF_EXIT);
@@ -1382,18 +1397,18 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
       if (a.d3[q]) a.d3[q][d3] = R(0);
     return;
   }
-  const R* sr = a.sr;
-  const Sd_t<R>* sd = a.sd;
-  const unsigned pf = a.pf[s];
+  const R* sr = pt.sr();
+  const Sd_t<R>* sd = pt.sd();
+  const unsigned pf = pt.pf()[s];
   if constexpr (!IsDual<R>::value) {
     // a wavefront of points without hydrometeors and without tendencies of
     // them (PF_ANYQ, PF_ANYT): temperature, vapour and aerosols take their
     // tendencies where these change them, the diagnostics are constants
     if (!a.qc_bl && !(a.fl.nc_mixing_ratio && a.d3[D3_NC_MIX]) && __all(!(pf & (PF_ANYQ | PF_ANYT)))) {
-      const R t1d = load_t(a, o), qv1d = a.f[F_QV][o];
+      const R t1d = pt.t(), qv1d = pt.f(F_QV);
       R tten, qvten, nwfaten, nifaten = R(0);
       if (pf & PF_CLEAR) {
-        const ClearAir<R> q = clear_air_tendencies<R>(C, a.f[F_P][o], t1d, qv1d, dt, odt);
+        const ClearAir<R> q = clear_air_tendencies<R>(C, pt.f(F_P), t1d, qv1d, dt, odt);
         tten = q.tten;
         qvten = q.qvten;
         nwfaten = q.nwfaten;
@@ -1404,16 +1419,16 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
         nifaten = sr[SR_NIFATEN * plane + s];
       }
       auto put = [&](int f, R v) {
-        if (!same_bits(a.f[f][o], v)) a.fo[f][o] = v;
+        if (!same_bits(pt.f(f), v)) a.fo[f][o] = v;
       };
       const R t_new = t1d + tten * dt;
       if (a.f[F_T])
         put(F_T, t_new);
       else
-        put(F_TH, t_new / a.f[F_PII][o]);
+        put(F_TH, t_new / pt.f(F_PII));
       put(F_QV, mx(R(kMinQv), (qv1d + qvten * dt)));
-      if (has_nwfa) put(F_NWFA, mx(R(kNwfaDefault), mn(R(kAeroMax), (a.f[F_NWFA][o] + nwfaten * dt))));
-      if (has_nifa) put(F_NIFA, mx(R(kNifaDefault), mn(R(kAeroMax), (a.f[F_NIFA][o] + nifaten * dt))));
+      if (has_nwfa) put(F_NWFA, mx(R(kNwfaDefault), mn(R(kAeroMax), (pt.f(F_NWFA) + nwfaten * dt))));
+      if (has_nifa) put(F_NIFA, mx(R(kNifaDefault), mn(R(kAeroMax), (pt.f(F_NIFA) + nifaten * dt))));
       if (a.d3[D3_NC_MIX]) a.d3[D3_NC_MIX][d3] = R(0);
       if (a.d3[D3_MVD_R]) a.d3[D3_MVD_R][d3] = a.fl.mvd_r ? R(kD0R) : R(0);
       if (a.d3[D3_MVD_G]) a.d3[D3_MVD_G][d3] = a.fl.mvd_g ? R(kD0G) : R(0);
@@ -1425,7 +1440,7 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
   }
   Lvl<R> L;
   if (!IsDual<R>::value && (pf & PF_CLEAR)) {
-    const ClearAir<R> q = clear_air_tendencies<R>(C, a.f[F_P][o], load_t(a, o), a.f[F_QV][o], dt, odt);
+    const ClearAir<R> q = clear_air_tendencies<R>(C, pt.f(F_P), pt.t(), pt.f(F_QV), dt, odt);
     L.temp = q.temp;
     L.qv = q.qv;
     L.rho = q.rho;
@@ -1442,13 +1457,11 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
     L.nwfaten = sr[SR_NWFATEN * plane + s];
     L.nifaten = sr[SR_NIFATEN * plane + s];
   }
-  // the post-sedimentation tendencies; an adjoint's local pass takes their
-  // values from a.post and their (local) tangents from the scratch
+  // the post-sedimentation tendencies
   auto ten = [&](int m, unsigned bit) {
     const Sd_t<R>& x = sd[size_t(SD_QRTEN + m) * plane + s];
     if constexpr (IsDual<R>::value) {
-      if constexpr (Out::kAdjoint) return R(Sd_t<R>(x.v, out.ten_tangent(m)));
-      if (a.post) return R(Sd_t<R>(a.post[size_t(m) * plane + s], x.d));
+      if constexpr (Point::kAdjoint) return R(pt.ten(m, x));
       return R(x);
     } else {
       return pf & bit ? R(x) : R(0);
@@ -1464,23 +1477,23 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
   L.niten = ten(7, PF_TI);
   L.qcten = ten(8, PF_TC);
   L.ncten = ten(9, PF_TC);
-  L.pres = a.f[F_P][o];
+  L.pres = pt.f(F_P);
   const R lvap = R(kLvap0) + R(2106.0 - 4218.0) * (L.temp - R(kT0));
   const R ocp = R(1.0) / (R(kCp) * (R(1.0) + R(0.887) * L.qv));
-  R qc1d = a.fa[F_QC][o], qr1d = a.fa[F_QR][o], qi1d = a.fa[F_QI][o], qs1d = a.fa[F_QS][o], qg1d = a.fa[F_QG][o];
-  R ni1d = a.fa[F_NI][o], nr1d = a.fa[F_NR][o];
-  R nc1d = has_nc ? a.fa[F_NC][o] : R(0), ng1d = has_ngqb ? a.fa[F_NG][o] : R(0);
-  R qb1d = has_ngqb ? a.fa[F_QB][o] : R(0);
+  R qc1d = pt.fa(F_QC), qr1d = pt.fa(F_QR), qi1d = pt.fa(F_QI), qs1d = pt.fa(F_QS), qg1d = pt.fa(F_QG);
+  R ni1d = pt.fa(F_NI), nr1d = pt.fa(F_NR);
+  R nc1d = has_nc ? pt.fa(F_NC) : R(0), ng1d = has_ngqb ? pt.fa(F_NG) : R(0);
+  R qb1d = has_ngqb ? pt.fa(F_QB) : R(0);
   const R ncv = (a.fl.ml_for_nc && !has_nc) ? sr[SR_NCSAVE * plane + s] : column_nc(a, c);
 
   if (!a.fl.turn_off_micro) freeze_cloud_melt_ice(C, L, qc1d, qi1d, ni1d, nc1d, has_nc, ncv, lvap, ocp, dt, odt);
   // final update (:738-748)
-  const R t_new = load_t(a, o) + L.tten * dt;
-  const R qv_new = mx(R(kMinQv), (a.f[F_QV][o] + L.qvten * dt));
+  const R t_new = pt.t() + L.tten * dt;
+  const R qv_new = mx(R(kMinQv), (pt.f(F_QV) + L.qvten * dt));
   L.rho = rho_of(C, L.pres, L.temp, L.qv);
-  auto nwfa_new = [&]() { return mx(R(kNwfaDefault), mn(R(kAeroMax), (a.f[F_NWFA][o] + L.nwfaten * dt))); };
-  auto nifa_new = [&]() { return mx(R(kNifaDefault), mn(R(kAeroMax), (a.f[F_NIFA][o] + L.nifaten * dt))); };
-  if constexpr (!Out::kAdjoint) {
+  auto nwfa_new = [&]() { return mx(R(kNwfaDefault), mn(R(kAeroMax), (pt.f(F_NWFA) + L.nwfaten * dt))); };
+  auto nifa_new = [&]() { return mx(R(kNifaDefault), mn(R(kAeroMax), (pt.f(F_NIFA) + L.nifaten * dt))); };
+  if constexpr (!Point::kAdjoint) {
     if (has_nwfa) a.fo[F_NWFA][o] = nwfa_new();
     if (has_nifa) a.fo[F_NIFA][o] = nifa_new();
   }
@@ -1493,30 +1506,30 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
   if (L.l_qs) snow_moments(C, L.rs, mn(R(-0.1), L.temp - R(kT0)), 4 | 32, L);
   graupel_check(C, L, qg1d, ng1d, qb1d, has_ngqb, dt, odt);
 
-  if constexpr (Out::kAdjoint) {  // (temperature form only)
-    out.add(F_T, t_new);
-    out.add(F_QV, qv_new);
-    out.add(F_QC, qc1d);
-    out.add(F_QR, qr1d);
-    out.add(F_QI, qi1d);
-    out.add(F_QS, qs1d);
-    out.add(F_QG, qg1d);
-    out.add(F_NI, ni1d);
-    out.add(F_NR, nr1d);
-    if (has_nc) out.add(F_NC, nc1d);
-    if (has_nwfa) out.add(F_NWFA, nwfa_new());
-    if (has_nifa) out.add(F_NIFA, nifa_new());
+  if constexpr (Point::kAdjoint) {  // (temperature form only)
+    pt.add(F_T, t_new);
+    pt.add(F_QV, qv_new);
+    pt.add(F_QC, qc1d);
+    pt.add(F_QR, qr1d);
+    pt.add(F_QI, qi1d);
+    pt.add(F_QS, qs1d);
+    pt.add(F_QG, qg1d);
+    pt.add(F_NI, ni1d);
+    pt.add(F_NR, nr1d);
+    if (has_nc) pt.add(F_NC, nc1d);
+    if (has_nwfa) pt.add(F_NWFA, nwfa_new());
+    if (has_nifa) pt.add(F_NIFA, nifa_new());
     if (has_ngqb) {
-      out.add(F_NG, ng1d);
-      out.add(F_QB, qb1d);
+      pt.add(F_NG, ng1d);
+      pt.add(F_QB, qb1d);
     }
-    if (a.fl.refl10cm && out.wants_refl()) out.add_refl(dry_reflectivity(C, L));
+    if (a.fl.refl10cm && pt.wants_refl()) pt.add_refl(dry_reflectivity(C, L));
     return;
   }
   if (a.f[F_T])
     a.fo[F_T][o] = t_new;
   else
-    a.fo[F_TH][o] = t_new / a.f[F_PII][o];
+    a.fo[F_TH][o] = t_new / pt.f(F_PII);
   a.fo[F_QV][o] = qv_new;
   a.fo[F_QC][o] = qc1d;
   a.fo[F_QR][o] = qr1d;
@@ -1579,7 +1592,7 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
     const R qbl = a.qc_bl[o], fbl = a.qcfrac_bl[o];
     if (xrx <= R(kR1) && qbl > R(S_t<R>(1.e-9)) && fbl > R(0.0)) xrx = xrx + qbl / fbl;
     if (xrx <= R(S_t<R>(1.e-12))) xrx = R(0.0);
-    R xnc = ml_cloud_number(xrx, qr1d, qi1d, qs1d, L.pres, L.temp, a.f[F_W][o]);
+    R xnc = ml_cloud_number(xrx, qr1d, qi1d, qs1d, L.pres, L.temp, pt.f(F_W));
     L.qcten = L.ncten = R(0.0);
     cloud_check(C, L, xrx, xnc, true, ncv, dt, odt);
   }
@@ -1603,10 +1616,9 @@ __global__ void __launch_bounds__(256) TEMPO_ATTR_C k_phase_c(StepArgs<R> a) {
   const int c = pt.x, k = pt.y;
   if (c >= a.ncol || k >= a.nz) return;
   if (a.nlev && k >= a.nlev[c]) return;
-  if (a.lvl_on && !a.lvl_on[k]) return;
   SigScope<R> scope(a, c, k, 1);
-  StoreOutputs out;
-  phase_c_point(a, c, k, out);
+  StepPoint<R> p(a, c, k);
+  phase_c_point(a, c, k, p);
 }
 
 // ------------------------------------ public check-and-update routines ----

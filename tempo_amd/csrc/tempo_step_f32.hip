@@ -26,8 +26,9 @@ template hipError_t launch_surface_emissions<float>(float*, const float*, int, i
                                                      double, hipStream_t);
 
 hipError_t launch_adjoint(const StepArgs<Dual<float>>& a, const AdjArgs& g, Dual<double>* vtbuf, size_t sr_bytes,
-                          size_t sd_bytes, AdjSnap snap, const bool* have_x, hipStream_t s) {
-  return adjoint_passes(a, g, vtbuf, sr_bytes, sd_bytes, snap, have_x, s);
+                          size_t sd_bytes, AdjSnap snap, const AdjLocal<Dual<float>>& scr, const bool* have_x,
+                          hipStream_t s) {
+  return adjoint_passes(a, g, vtbuf, sr_bytes, sd_bytes, snap, scr, have_x, s);
 }
 template hipError_t launch_to_compact_n<float>(const PlaneBatch<float, double>&, int, const DualGeom&, hipStream_t);
 template hipError_t launch_from_compact_n<float>(const PlaneBatch<double, float>&, int, const DualGeom&, hipStream_t);

@@ -26,8 +26,9 @@ template hipError_t launch_surface_emissions<double>(double*, const double*, int
                                                      double, hipStream_t);
 
 hipError_t launch_adjoint(const StepArgs<Dual<double>>& a, const AdjArgs& g, Dual<double>* vtbuf, size_t sr_bytes,
-                          size_t sd_bytes, AdjSnap snap, const bool* have_x, hipStream_t s) {
-  return adjoint_passes(a, g, vtbuf, sr_bytes, sd_bytes, snap, have_x, s);
+                          size_t sd_bytes, AdjSnap snap, const AdjLocal<Dual<double>>& scr, const bool* have_x,
+                          hipStream_t s) {
+  return adjoint_passes(a, g, vtbuf, sr_bytes, sd_bytes, snap, scr, have_x, s);
 }
 template hipError_t launch_to_compact_n<double>(const PlaneBatch<double, double>&, int, const DualGeom&, hipStream_t);
 template hipError_t launch_from_compact_n<double>(const PlaneBatch<double, double>&, int, const DualGeom&, hipStream_t);

@@ -728,3 +728,32 @@ def test_adjoint_dot_product_level_counts(ctx, sample, nz, sparse):
     rhs = sum(float((xbar[k] * torch.tensor(v[k], device="cuda")).sum()) for k in v)
     print(nz, "levels, dot test", lhs, rhs)
     assert abs(lhs - rhs) <= 1e-10 * abs(lhs)
+
+
+@pytest.mark.parametrize("ncol,dtype,sparse", [(1, torch.float64, False), (33, torch.float64, True),
+                                               (33, torch.float32, False), (33_000, torch.float32, False),
+                                               (33_000, torch.float64, True)])
+def test_adjoint_batches_and_directions(ctx, sample, ncol, dtype, sparse):
+    """a column's gradient does not depend on the batch it is in nor on the
+    other requested inputs, bit for bit: batches whose directions share one
+    launch, and a batch (2.1 million points) taken in chunks of the forward's
+    scratch, against 33 columns with one direction at a time"""
+    st0, m = sample
+    nz = st0["p"].shape[0]
+    rng = np.random.default_rng(41)
+    rows = np.isin(np.arange(nz), LEVELS)[:, None] if sparse else np.ones((nz, 1), bool)
+    y0 = {k: rng.standard_normal((nz, 33)) * rows / (np.abs(st0[k]).max() + 1e-30) for k in ("t", "qv", "qr", "ni")}
+    d0 = {"refl10cm": rng.standard_normal((nz, 33)) * 0.01 * rows, "rain_precip": rng.standard_normal(33) * 1e3}
+
+    def columns(v, n):
+        return torch.tensor(np.ascontiguousarray(np.take(v[..., :33], np.arange(n) % 33, axis=-1)), dtype=dtype,
+                            device="cuda")
+
+    def gradient(n, wrt):
+        return ctx.adjoint({k: columns(v, n) for k, v in st0.items()}, {k: columns(v, n) for k, v in y0.items()},
+                           {k: columns(v, n) for k, v in d0.items()}, m["dt"], m["itimestep"], wrt=wrt)
+    names = ("t", "qv", "qc", "qr", "qi", "qs", "qg", "nc", "nr", "ni", "nwfa", "nifa")
+    all_ = gradient(ncol, names)
+    for k in names:
+        one = gradient(33, (k,))[k]
+        assert torch.equal(all_[k], one[:, torch.arange(ncol, device="cuda") % 33]), k
