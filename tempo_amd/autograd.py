@@ -19,6 +19,7 @@ import torch
 
 X_NAMES = ("t", "qv", "qc", "qr", "qi", "qs", "qg", "nc", "nr", "ni", "nwfa", "nifa", "ng", "qb")
 Y_NAMES = ("t", "qv", "qc", "qr", "qi", "qs", "qg", "ni", "nr", "nc", "nwfa", "nifa", "ng", "qb")
+CONSTANTS = ("p", "w", "dz", "pii")  # fields the step only reads
 D_NAMES = ("rain_precip", "ice_liquid_equiv_precip", "snow_liquid_equiv_precip", "graupel_liquid_equiv_precip",
            "refl10cm")
 
@@ -27,7 +28,11 @@ class _TempoStep(torch.autograd.Function):
     @staticmethod
     def forward(fctx, tempo, dt, itimestep, keys, nlev, land, *tensors):
         inputs = dict(zip(keys, tensors))
-        state = {k: v.detach().clone() for k, v in inputs.items()}
+        # outputs without a gradient stay None: the adjoint takes an absent
+        # cotangent as zero without reading it
+        fctx.set_materialize_grads(False)
+        state = {k: v.detach() if k in CONSTANTS and v.is_contiguous() else v.detach().clone()
+                 for k, v in inputs.items()}
         diags = tempo.run(state, dt, itimestep, nlev=nlev, land=land)
         fctx.tempo, fctx.dt, fctx.itimestep, fctx.keys = tempo, dt, itimestep, keys
         fctx.nlev, fctx.land = nlev, land

@@ -52,6 +52,7 @@ FIELD_NAMES = ("t", "th", "pii", "p", "w", "dz", "qv", "qc", "qr", "qi", "qs", "
 # boundary-layer cloud inputs (read only; with the cloud-number network they
 # enter the cloud effective radius)
 BL_NAMES = ("qc_bl", "qcfrac_bl")
+ADJOINT_NAMES = ("t", "qv", "qc", "qr", "qi", "qs", "qg", "nc", "nr", "ni", "nwfa", "nifa", "ng", "qb")  # differentiable
 
 
 class Fields(ctypes.Structure):
@@ -239,12 +240,10 @@ class TempoHip:
                 setattr(d, n, a.data_ptr())
             out = diags
         elif diags:
-            for n in DIAG2_NAMES:
-                out[n] = torch.zeros(ncol, dtype=dtype, device=ref.device)
-                setattr(d, n, out[n].data_ptr())
-            for n in DIAG3_NAMES:
-                out[n] = torch.zeros((nz, ncol), dtype=dtype, device=ref.device)
-                setattr(d, n, out[n].data_ptr())
+            out = self._new_diags(nz, ncol, dtype, ref.device)
+            torch._foreach_zero_(list(out.values()))  # one launch instead of 15
+            for n, a in out.items():
+                setattr(d, n, a.data_ptr())
         dims = Dims(ncol, 1, nz, ncol, nz * ncol, ncol, nz * ncol, ncol, None)
         if nlev is not None:
             nlev = nlev.to(device=ref.device, dtype=torch.int32).contiguous()
@@ -265,6 +264,13 @@ class TempoHip:
         return out
 
     # ---- shared argument marshalling for device tensors ----
+    @staticmethod
+    def _new_diags(nz, ncol, dtype, device):
+        import torch
+        out = {n: torch.empty(ncol, dtype=dtype, device=device) for n in DIAG2_NAMES}
+        out.update({n: torch.empty((nz, ncol), dtype=dtype, device=device) for n in DIAG3_NAMES})
+        return out
+
     def _fields(self, state, nz, ncol, dtype, what="field"):
         f = Fields()
         for name in FIELD_NAMES + BL_NAMES:
@@ -301,9 +307,9 @@ class TempoHip:
                 tangent[k] = torch.zeros_like(v)
         f = self._fields(state, nz, ncol, dtype)
         ft = self._fields(tangent, nz, ncol, dtype, "tangent")
-        out = {n: torch.zeros(ncol, dtype=dtype, device=ref.device) for n in DIAG2_NAMES}
-        out.update({n: torch.zeros((nz, ncol), dtype=dtype, device=ref.device) for n in DIAG3_NAMES})
-        tout = {n: torch.zeros_like(v) for n, v in out.items()}
+        # every element is written (30 fills took 72 of 458 us at 8,192 x 64)
+        out = self._new_diags(nz, ncol, dtype, ref.device)
+        tout = self._new_diags(nz, ncol, dtype, ref.device)
         keep = []
         if land is not None:
             land = land.to(device=ref.device, dtype=torch.int32).contiguous()
@@ -336,7 +342,9 @@ class TempoHip:
         yb = self._fields(ybar, nz, ncol, dtype, "cotangent")
         db = self._diags(dbar, nz, ncol, dtype)
         names = wrt or ("t", "qv", "qc", "qr", "qi", "qs", "qg", "nc", "nr")
-        xbar = {k: torch.zeros((nz, ncol), dtype=dtype, device=ref.device) for k in names if k in state}
+        # every element of a differentiable input's cotangent is written
+        xbar = {k: (torch.empty if k in ADJOINT_NAMES else torch.zeros)((nz, ncol), dtype=dtype, device=ref.device)
+                for k in names if k in state}
         xb = self._fields(xbar, nz, ncol, dtype)
         keep = []
         if land is not None:
