@@ -55,9 +55,10 @@ __host__ __device__ constexpr int adj_y_of(int f) {
 }
 
 struct AdjArgs {
-  const double* ybar;   // AY_N planes (compact c + k*ncol), absent outputs all zero
+  const double* ybar;   // AY_N planes (compact c + k*ncol)
+  unsigned y_on;        // bit q: output q has cotangents (the other planes are not set)
   int* lvl_on;          // nz: 1 where some output cotangent of the level is non-zero
-  const double* post;   // 10 planes (tiled): post-sedimentation tendency values, SD_QRTEN order
+  const double* post;   // 10 planes (tiled): post-sedimentation tendency values, SD_QRTEN order (NULL: in the scratch)
   unsigned* list;       // points the local passes run at (see k_adj_point_list), c + k*ncol each
   unsigned* count;      // how many
   const double* pbar;   // 4 x ncol: rain, graupel, snow, ice precipitation
@@ -104,7 +105,7 @@ __global__ void __launch_bounds__(256) k_adj_level_flags(StepArgs<D> a, AdjArgs 
   bool nz = false;
   if (c < a.ncol) {
     const size_t e = size_t(c) + size_t(k) * a.ncol, n3 = size_t(a.ncol) * a.nz;
-    for (int q = 0; q < AY_N; ++q) nz = nz || g.ybar[size_t(q) * n3 + e] != 0.0;
+    for (int q = 0; q < AY_N; ++q) nz = nz || ((g.y_on >> q & 1u) && g.ybar[size_t(q) * n3 + e] != 0.0);
   }
   if (__ballot(nz) != 0ull && (threadIdx.x & 63u) == 0) atomicOr(&g.lvl_on[k], 1);
 }
@@ -160,14 +161,18 @@ struct Contraction {
   static constexpr bool kAdjoint = true;
   const double* ybar;  // at the point
   size_t n3;
+  unsigned y_on;
   double acc;
   // a tangent counts only where its cotangent is non-zero
   __device__ __forceinline__ void add_y(int q, const D& v) {
+    if (!(y_on >> q & 1u)) return;
     const double y = ybar[size_t(q) * n3];
     if (y != 0.0) acc += y * double(v.d);
   }
   __device__ __forceinline__ void add(int f, const D& v) { add_y(adj_y_of(f), v); }
-  __device__ __forceinline__ bool wants_refl() const { return ybar[size_t(AY_REFL) * n3] != 0.0; }
+  __device__ __forceinline__ bool wants_refl() const {
+    return (y_on >> AY_REFL & 1u) && ybar[size_t(AY_REFL) * n3] != 0.0;
+  }
   __device__ __forceinline__ void add_refl(const D& v) { add_y(AY_REFL, v); }
 };
 // the forward's point with one tendency seeded (the forward's tangents are zero)
@@ -177,7 +182,7 @@ struct UpassPoint : StepPoint<D>, Contraction<D> {
   int seed;
   __device__ __forceinline__ UpassPoint(const StepArgs<D>& a, const AdjArgs& g, int c, int k, int m)
       : StepPoint<D>(a, c, k),
-        Contraction<D>{g.ybar + size_t(c) + size_t(k) * a.ncol, size_t(a.ncol) * a.nz, 0.0},
+        Contraction<D>{g.ybar + size_t(c) + size_t(k) * a.ncol, size_t(a.ncol) * a.nz, g.y_on, 0.0},
         seed(m) {}
   __device__ __forceinline__ D t() const { return this->f(F_T); }
   __device__ __forceinline__ Sd_t<D> ten(int m, const Sd_t<D>& x) const { return Sd_t<D>(x.v, m == seed ? 1.0 : 0.0); }
@@ -241,7 +246,7 @@ struct LocalPoint : Contraction<D> {
   int seed;          // seeded input field
   __device__ __forceinline__ LocalPoint(const StepArgs<D>& args, const AdjArgs& g, const AdjLocal<D>& scr, int c, int k,
                                         size_t v, int field)
-      : Contraction<D>{g.ybar + size_t(c) + size_t(k) * args.ncol, size_t(args.ncol) * args.nz, 0.0},
+      : Contraction<D>{g.ybar + size_t(c) + size_t(k) * args.ncol, size_t(args.ncol) * args.nz, g.y_on, 0.0},
         a(args),
         q(scr),
         post(g.post),
@@ -260,7 +265,8 @@ struct LocalPoint : Contraction<D> {
   // the forward's value after sedimentation with phase A's local tangent (S
   // frozen out)
   __device__ __forceinline__ Sd_t<D> ten(int m, const Sd_t<D>& x) const {
-    return Sd_t<D>(post[size_t(m) * a.plane + fwd], x.d);
+    const size_t i = size_t(m) * a.plane + fwd;
+    return Sd_t<D>(post ? post[i] : a.sd[size_t(SD_QRTEN) * a.plane + i].v, x.d);
   }
 };
 template <class D>

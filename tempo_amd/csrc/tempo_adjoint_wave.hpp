@@ -596,7 +596,7 @@ __global__ void __launch_bounds__(64 * kScrW) k_adj_sed_wave(StepArgs<D> a, AdjA
 // so that the later passes restart from them instead of recomputing.
 // scratch snapshots of the adjoint: working-precision and FP64 planes after
 // phase A (used for nz > 128 only), and the post-sedimentation tendency
-// values
+// values (NULL where nothing overwrites them)
 struct AdjSnap {
   void* sr_a;  // sr_bytes
   void* sd_a;  // sd_bytes
@@ -639,9 +639,11 @@ hipError_t adjoint_passes(const StepArgs<D>& a, AdjArgs g, Dual<double>* vtbuf, 
     launch_phase_b_wave(a, s);
   else
     hipLaunchKernelGGL(k_phase_b<D>, dim3(unsigned((a.ncol + 127) / 128)), dim3(128), 0, s, a, vtbuf);
+  // the post-sedimentation tendency values stay in the scratch for the local
+  // passes, or are copied where these or the restored snapshot overwrite it
   double* post = static_cast<double*>(snap.sd_b);
   g.post = post;
-  hipLaunchKernelGGL(k_adj_keep_post<D>, g2, dim3(256), 0, s, a, post);
+  if (post) hipLaunchKernelGGL(k_adj_keep_post<D>, g2, dim3(256), 0, s, a, post);
   // passes seeded on the post-sedimentation tendencies.  Without prognostic
   // graupel number and volume the final update does not read their
   // tendencies, so those cotangents are zero and need no pass.

@@ -827,19 +827,26 @@ int run_adjoint(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_fie
   void* yp[F_NFIELDS] = {};
   if (yb) field_ptrs(yb, yp);
   PlaneBatch<T, double> yc{};
+  int nyc = 0;
+  g.y_on = 0;
   for (int q = 0; q < AY_REFL; ++q) {
-    yc.src[q] = static_cast<const T*>(a.f[adj_y_field(q)] ? yp[adj_y_field(q)] : nullptr);
-    yc.dst[q] = ybar + size_t(q) * n3;
+    if (!a.f[adj_y_field(q)] || !yp[adj_y_field(q)]) continue;
+    g.y_on |= 1u << q;
+    yc.src[nyc] = static_cast<const T*>(yp[adj_y_field(q)]);
+    yc.dst[nyc++] = ybar + size_t(q) * n3;
   }
-  HIP_TRY(launch_to_compact_n(yc, AY_REFL, g3, s));
+  HIP_TRY(launch_to_compact_n(yc, nyc, g3, s));
   void *d2[D2_N] = {}, *d3[D3_N] = {};
   if (db) diag_ptrs(db, d2, d3);
   const DualGeom gd3{dm->ni, dm->nj, nz, dm->dldk, dm->dldj};
   const DualGeom g2{dm->ni, dm->nj, 1, 0, dm->d2ldj};
-  PlaneBatch<T, double> rb{};
-  rb.src[0] = static_cast<const T*>(d3[D3_REFL]);
-  rb.dst[0] = ybar + size_t(AY_REFL) * n3;
-  HIP_TRY(launch_to_compact_n(rb, 1, gd3, s));
+  if (d3[D3_REFL]) {
+    g.y_on |= 1u << AY_REFL;
+    PlaneBatch<T, double> rb{};
+    rb.src[0] = static_cast<const T*>(d3[D3_REFL]);
+    rb.dst[0] = ybar + size_t(AY_REFL) * n3;
+    HIP_TRY(launch_to_compact_n(rb, 1, gd3, s));
+  }
   const int pmap[4] = {D2_RAIN, D2_GRAUPEL, D2_SNOW, D2_ICE};  // S^T order: rain, graupel, snow, ice
   PlaneBatch<T, double> pc{};
   for (int q = 0; q < 4; ++q) {
@@ -864,27 +871,35 @@ int run_adjoint(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_fie
   if (xb) field_ptrs(xb, xp);
   bool have_x[AX_N];
   for (int i = 0; i < AX_N; ++i) have_x[i] = fp[adj_x_field(i)] && xp[adj_x_field(i)];
-  // snapshots: the post-sedimentation tendency values (10 FP64 planes), and
-  // for the lane-per-column sedimentation (nz > 128) the scratch after A
-  const size_t srb = SR_N * a.plane * sizeof(D), sdb = SD_N * a.plane * sizeof(Dual<double>);
-  const bool wave_b = nz <= kSedLevels;
-  HIP_TRY(x->adj_snap.ensure(wave_b ? 10 * a.plane * sizeof(double) : srb + 2 * sdb));
-  char* sp = static_cast<char*>(x->adj_snap.p);
-  const AdjSnap snap = wave_b ? AdjSnap{nullptr, nullptr, sp} : AdjSnap{sp, sp + srb, sp + srb + sdb};
-  // out of place: inputs in adj_in, post-check state in tl_state; no pass
-  // stores a new state
-  int ndir = 0;
-  for (int i = 0; i < F_NFIELDS; ++i) {
-    a.f[i] = fp[i] ? in + size_t(i) * n3 : nullptr;
-    a.fa[i] = a.fo[i] = fp[i] ? st + size_t(i) * n3 : nullptr;
-  }
-  for (bool h : have_x) ndir += h;
   // the local passes' scratch: of a large batch the forward's, done with by
   // then; a smaller one's would leave launches that do not fill the chip, so
   // it gets its own, up to kLocalRoom point-directions
   constexpr size_t kLocalRoom = size_t(1) << 21;
+  int ndir = 0;
+  for (bool h : have_x) ndir += h;
+  const bool own_scr = n3 < kLocalRoom && ndir > 0;
+  // snapshots: for the lane-per-column sedimentation (nz > 128) the scratch
+  // after A, and the post-sedimentation tendency values (10 FP64 planes)
+  // where they do not stay in the scratch
+  const size_t srb = SR_N * a.plane * sizeof(D), sdb = SD_N * a.plane * sizeof(Dual<double>);
+  const bool wave_b = nz <= kSedLevels;
+  AdjSnap snap{nullptr, nullptr, nullptr};
+  if (!wave_b) {
+    HIP_TRY(x->adj_snap.ensure(srb + 2 * sdb));
+    char* sp = static_cast<char*>(x->adj_snap.p);
+    snap = AdjSnap{sp, sp + srb, sp + srb + sdb};
+  } else if (!own_scr) {
+    HIP_TRY(x->adj_snap.ensure(10 * a.plane * sizeof(double)));
+    snap.sd_b = x->adj_snap.p;
+  }
+  // out of place: inputs in adj_in, post-check state in tl_state; no pass
+  // stores a new state
+  for (int i = 0; i < F_NFIELDS; ++i) {
+    a.f[i] = fp[i] ? in + size_t(i) * n3 : nullptr;
+    a.fa[i] = a.fo[i] = fp[i] ? st + size_t(i) * n3 : nullptr;
+  }
   AdjLocal<D> scr{a.sr, a.sd, a.pf, st, a.plane, n3, n3};
-  if (n3 < kLocalRoom && ndir > 1) {
+  if (own_scr) {
     const size_t m = std::min(kLocalRoom, (n3 * size_t(ndir) + 63) / 64 * 64);
     HIP_TRY(x->adj_local.ensure(m * (SD_N * sizeof(Dual<double>) + (SR_N + F_NFIELDS) * sizeof(D) + sizeof(unsigned))));
     scr.sd = x->adj_local.as<Dual<double>>();
