@@ -318,7 +318,9 @@ int tempo_hip_substeps(tempo_hip_ctx *ctx, int *host_out, size_t n);
  *                               points with microphysics to do to its first
  *                               wavefronts, so that they do not share
  *                               wavefronts with idle points; clear = lane i
- *                               takes column i (default 0)
+ *                               takes column i.  Unless set it is chosen:
+ *                               bit 0 in FP64, both in batches of few columns,
+ *                               else 0 (the results are the same)
  *   TEMPO_HIP_TUNE_WAVES_A   1: the level-local physics compiled for one
  *                               wave per SIMD fewer (more registers, fewer
  *                               spills: 3 instead of 4 in FP32, 2 instead

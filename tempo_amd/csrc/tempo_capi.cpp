@@ -537,6 +537,20 @@ ScratchSizes step_scratch(const tempo_hip_ctx* x, const StepArgs<R>& a, int wave
                       x->cfg.semi_sedi_flag != 0);
 }
 
+// Point grouping of a step that sets none.  The FP64 level physics is bound
+// by its instructions, so wavefronts full of points with work to do pay for
+// finding them at every size (25,000 x 90: 1.85 ms without, 1.56 with; one
+// column x 60: 178, 135 us); its final update, bound by memory, only while
+// a batch leaves the chip idle (128 columns: 139 us, 130 with; 512: the
+// same).  In FP32 both lose by it (100,000 x 90: 2.04 ms, 2.20 with), but
+// where the columns fill half a wavefront at most (one column: 78 us, 60; 32:
+// 67, 64; 64: 65, 65): four levels then share one.  Duals lose or gain under
+// 3 %.
+int point_order(bool r64, int ncol) {
+  if (r64) return ncol <= 256 ? 3 : 1;
+  return ncol <= 32 ? 3 : 0;
+}
+
 // scratch, tables, constants and flags of one launch (a.ncol, a.nz set);
 // sc: the scratch to use (NULL: the context's own, grown as needed)
 template <class R>
@@ -572,7 +586,8 @@ int bind_common(tempo_hip_ctx* x, StepArgs<R>& a, double dt, int itimestep, cons
   x->last_ksub = sc->ksub;
   x->last_vt = sc->vt;
   const bool r64 = sizeof(S) == 8;
-  a.compact = x->launch[r64 ? 1 : 0].order;
+  const int order = x->launch[r64 ? 1 : 0].order;
+  a.compact = order >= 0 ? order : IsDual<R>::value ? 0 : point_order(r64, a.ncol);
   a.ccn_lds = x->launch[r64 ? 1 : 0].ccn_lds;
   a.tab.qg = static_cast<const S*>(r64 ? x->qg64.p : x->qg32.p);
   a.tab.qs = static_cast<const S*>(r64 ? x->qs64.p : x->qs32.p);
@@ -667,6 +682,7 @@ int run_impl(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_diags*
   if (rc) return rc;
   double* vt = static_cast<double*>(x->last_vt);
   if (sig) {
+    if (x->launch[sizeof(R) == 8 ? 1 : 0].order < 0) a.compact = 0;
     a.sig = sig;
     HIP_TRY(launch_step_sig(a, x->launch[sizeof(R) == 8 ? 1 : 0], vt, s));
     return TEMPO_HIP_OK;

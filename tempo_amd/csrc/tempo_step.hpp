@@ -373,7 +373,7 @@ struct DualGeom {
 struct LaunchCfg {
   int sed_wave = 1;   // sedimentation: 1 = one wavefront per column (nz <= 128), 0 = one lane per column,
                       // 2 = the wavefront kernel issuing every staging pass (check form)
-  int order = 0;      // point grouping within blocks: bit 0 phase A, bit 1 final update
+  int order = -1;     // point grouping within blocks: bit 0 phase A, bit 1 final update (-1: point_order)
   int block_a = 256;  // threads per block of the level-local kernels (64, 128 or 256)
   int block_c = 256;
   int waves_a = 0;       // phase A compiled for the default waves per SIMD (0) or one fewer (1)

@@ -1405,3 +1405,29 @@ def test_gpu_tangent_sedimentation_level_counts(hip, dtype, hail, nz):
             assert np.array_equal(v, w, equal_nan=True), (k, nz)
         else:
             assert np.abs(v - w).max() <= 128 * 2.0**-23 * np.abs(w).max(), (k, nz)
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "fp64"])
+@pytest.mark.parametrize("ncol", [1, 2, 31, 32, 33, 64, 255, 256, 257])
+def test_gpu_default_point_grouping(hip, dtype, ncol):
+    """the grouping a step chooses by precision and columns against none, bit
+    for bit, on both sides of the rule's lines (uneven columns)"""
+    import torch
+    from tempo_amd import generator as gen
+    flags = dict(aerosolaware=True, hailaware=True)
+    prec = hip.FP32 if dtype == "fp32" else hip.FP64
+    td = torch.float32 if dtype == "fp32" else torch.float64
+    st, m = gen.generate("multistep", ncol=ncol, col0=555)
+    nz = st["p"].shape[0]
+    nlev = torch.tensor(np.maximum(2, nz - np.arange(ncol) % 40).astype(np.int32), device="cuda")
+    got = []
+    for order in (None, 0):
+        ctx = hip.TempoHip(**{k + "_flag": int(v) for k, v in flags.items()})
+        if order is not None:
+            ctx.tune(prec, hip.TUNE_ORDER, order)
+        dev = {k: torch.tensor(v, dtype=td, device="cuda") for k, v in st.items()}
+        for i in range(2):
+            d = ctx.run(dev, m["dt"], 2 + i, nlev=nlev)
+        got.append({k: v.cpu().numpy() for k, v in {**dev, **d}.items()})
+    for k, v in got[0].items():
+        assert np.array_equal(v, got[1][k], equal_nan=True), k
