@@ -324,7 +324,9 @@ int tempo_hip_substeps(tempo_hip_ctx *ctx, int *host_out, size_t n);
  *   TEMPO_HIP_TUNE_WAVES_A   1: the level-local physics compiled for one
  *                               wave per SIMD fewer (more registers, fewer
  *                               spills: 3 instead of 4 in FP32, 2 instead
- *                               of 3 in FP64), 0: the default
+ *                               of 3 in FP64), 0: not.  Unless set, 1 in
+ *                               FP64 up to 4,096 wavefronts (64 columns of
+ *                               a level each), else 0
  *   TEMPO_HIP_TUNE_CCN_LDS   1: each block of the level-local physics
  *                               copies the CCN activation table's slice
  *                               (441 floats) into LDS and reads it there,

@@ -1183,7 +1183,14 @@ hipError_t launch_step_impl(const StepArgs<T>& args, const StepArgs<RA>& gargs, 
   if (ev) (void)hipEventRecord(ev[0], s);
   launch_prepass(a, s);
   if (ev) (void)hipEventRecord(ev[1], s);
-  if (lc.waves_a && std::is_same<RA, T>::value)
+  // FP64 with the registers of two waves per SIMD has next to no spills and is
+  // faster while the launch is one or two rounds of them at most (2,048 run
+  // at once): 1 column x 60 122 -> 115 us, 2,000 x 90 (2,880 wavefronts) 206 ->
+  // 186, 3,000 x 90 (4,230) 272 -> 265; 5,000 x 60 (4,740) 265 -> 275, 25,000 x
+  // 90 1573 -> 1585.  FP32 gains nothing at any size.
+  const bool fewer = lc.waves_a >= 0 ? lc.waves_a == 1
+                                     : sizeof(T) == 8 && size_t((a.ncol + 63) / 64) * size_t(a.nz) <= 4096;
+  if (fewer && std::is_same<RA, T>::value)
     hipLaunchKernelGGL((k_phase_a<RA, WavesPerEu<RA>::a_alt>), level_grid(a, lc.block_a), dim3(unsigned(lc.block_a)),
                        0, s, ga);
   else

@@ -1431,3 +1431,23 @@ def test_gpu_default_point_grouping(hip, dtype, ncol):
         got.append({k: v.cpu().numpy() for k, v in {**dev, **d}.items()})
     for k, v in got[0].items():
         assert np.array_equal(v, got[1][k], equal_nan=True), k
+
+
+@pytest.mark.parametrize("ncol", [4096, 4097])
+def test_gpu_default_register_budget(hip, ncol):
+    """the FP64 level physics on both sides of the line between its two
+    compiled forms (64 x 64 wavefronts and one column more) against either
+    form, bit for bit"""
+    import torch
+    from tempo_amd import generator as gen
+    st, m = gen.generate("adjoint", ncol=ncol, col0=77)
+    got = []
+    for waves in (None, 0, 1):
+        ctx = hip.TempoHip(aerosolaware_flag=1, hailaware_flag=0)
+        if waves is not None:
+            ctx.tune(hip.FP64, hip.TUNE_WAVES_A, waves)
+        dev = {k: torch.tensor(v, dtype=torch.float64, device="cuda") for k, v in st.items()}
+        d = ctx.run(dev, m["dt"], 2)
+        got.append({**dev, **d})
+    for k, v in got[0].items():
+        assert torch.equal(v, got[1][k]) and torch.equal(v, got[2][k]), k
