@@ -335,9 +335,9 @@ int tempo_hip_substeps(tempo_hip_ctx *ctx, int *host_out, size_t n);
  *                               _run_host_prec): slabs of columns of the
  *                               transfer pipeline, 1..4096 (fewer where the
  *                               tile has fewer j rows, or fewer than 256
- *                               columns per slab when nj = 1); 0 = about
- *                               128 MB of uploads per slab, at most 32
- *                               (default)
+ *                               columns per slab when nj = 1); 0 (default)
+ *                               = the root of the uploads' bytes over 4 MiB,
+ *                               at most 32
  *   TEMPO_HIP_TUNE_HOST_THREADS ... and host threads copying between the
  *                               caller's arrays and pinned memory, 1..64
  *                               (default 8)

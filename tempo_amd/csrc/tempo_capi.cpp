@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <condition_variable>
 #include <cstdio>
 #include <cstring>
@@ -967,8 +968,12 @@ int check_run_args(const tempo_hip_fields* f, const tempo_hip_dims* dm, double d
 // slabs overlap (the link is full duplex), the host copies overlap both,
 // and each column's step is the device path's.
 
-// default upload bytes per slab, and the most slabs
-constexpr size_t kSlabBytes = size_t(128) << 20;
+// Slabs unless set: n slabs cost n times a slab's launches and joins and leave
+// 1/n of the transfers at either end of the pipeline without a partner, so
+// that the best n grows as the root of the bytes.  Uploads of 36 MB (5,000 x 60
+// FP64 fields): 1 slab 2.52 ms, 3 2.12, 6 2.53; 144 MB: 2 6.9, 6 6.0, 12 6.4;
+// 432 MB: 4 15.0, 8 13.7, 12 14.1.
+constexpr double kSlabRoot = double(size_t(4) << 20);
 constexpr int kMaxSlabs = 32;
 
 // elements of one array in one slab: n rows of len elements at element
@@ -1013,7 +1018,7 @@ SlabPlan plan_slabs(const tempo_hip_dims* dm, size_t up_bytes, int tuned) {
   SlabPlan p{dm->nj > 1, 1, 0, 0};
   p.total = p.along_j ? dm->nj : dm->ni;
   const int most = p.along_j ? dm->nj : std::max(1, dm->ni / 256);  // i slabs of at least 256 columns
-  int n = tuned > 0 ? tuned : int(std::min<size_t>(kMaxSlabs, (up_bytes + kSlabBytes - 1) / kSlabBytes));
+  int n = tuned > 0 ? tuned : int(std::min<double>(kMaxSlabs, std::sqrt(double(up_bytes) / kSlabRoot) + 0.5));
   n = std::max(1, std::min(n, most));
   if (n == 1) p.along_j = true;  // one slab: the arrays' whole spans
   if (p.along_j) p.total = dm->nj;

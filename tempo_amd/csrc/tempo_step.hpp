@@ -378,7 +378,7 @@ struct LaunchCfg {
   int block_c = 256;
   int waves_a = -1;      // phase A compiled for the default waves per SIMD (0) or one fewer (1); -1: chosen
   int ccn_lds = 0;       // phase A stages the CCN table's slice in LDS (1)
-  int host_slabs = 0;    // host-array steps: slabs of columns (0: about 128 MB of uploads each)
+  int host_slabs = 0;    // host-array steps: slabs of columns (0: by the upload's bytes)
   int host_threads = 8;  // ... and host threads copying between the caller's arrays and pinned memory
 };
 

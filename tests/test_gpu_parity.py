@@ -1451,3 +1451,20 @@ def test_gpu_default_register_budget(hip, ncol):
         got.append({**dev, **d})
     for k, v in got[0].items():
         assert torch.equal(v, got[1][k]) and torch.equal(v, got[2][k]), k
+
+
+@pytest.mark.parametrize("ncol", [255, 2000, 9000])
+def test_gpu_host_default_slabs(hip, ncol):
+    """the slabs a host-array step chooses from its bytes (one, two and four)
+    against one slab, bit for bit"""
+    from tempo_amd import generator as gen
+    st, m = gen.generate("adjoint", ncol=ncol, col0=42)
+    got = []
+    for slabs in (0, 1):
+        ctx = hip.TempoHip(aerosolaware_flag=1, hailaware_flag=0)
+        ctx.tune(hip.FP64, hip.TUNE_HOST_SLABS, slabs)
+        s = {k: v.copy() for k, v in st.items()}
+        d = ctx.run_host(s, m["dt"], 2)
+        got.append({**s, **d})
+    for k, v in got[0].items():
+        assert np.array_equal(v, got[1][k], equal_nan=True), k
