@@ -8,12 +8,13 @@
 namespace tempo {
 
 // Waves per SIMD the level-local kernels are compiled for, per working type.
-// The FP32 level physics needs 130 VGPRs unconstrained (3 waves per SIMD);
-// held to 128 it runs 4 waves with a few bytes more of private memory and
-// is measured faster.  Tighter budgets spill heavily and are slower.  The
-// FP64 level physics is held to three waves (168 VGPRs, a few hundred
-// bytes of spills per lane), measured faster than two waves without
-// spills.  The dual instantiations keep the compiler's choice (the FP32
+// The FP32 level physics takes 125 VGPRs and 28 bytes of spills held to 4
+// waves per SIMD; tighter budgets spill heavily and are slower.  The FP64
+// level physics is held to three waves (168 VGPRs, 432 bytes of spills per
+// lane) where a launch has wavefronts for them, else to two (256 VGPRs, 80
+// bytes), see launch_step_impl.  The FP32 final update is left at 71-75 VGPRs,
+// 6 waves: held to 7 or 8 it took 489 and 553 us against 466 at 100,000 x 90,
+// and capped at 5, 4 and 3 waves 536, 598 and 690.  The dual instantiations keep the compiler's choice (the FP32
 // dual phase A takes 244 VGPRs, two waves; held to three waves it spilled
 // and made the adjoint 7-13 % slower; its final update at four waves
 // instead of three gained nothing).  One wave fewer (a_alt: 3 in FP32,
