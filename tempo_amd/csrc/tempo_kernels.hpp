@@ -14,11 +14,11 @@ namespace tempo {
 // lane) where a launch has wavefronts for them, else to two (256 VGPRs, 80
 // bytes), see launch_step_impl.  The FP32 final update is left at 71-75 VGPRs,
 // 6 waves: held to 7 or 8 it took 489 and 553 us against 466 at 100,000 x 90,
-// and capped at 5, 4 and 3 waves 536, 598 and 690.  The dual instantiations keep the compiler's choice (the FP32
-// dual phase A takes 244 VGPRs, two waves; held to three waves it spilled
-// and made the adjoint 7-13 % slower; its final update at four waves
-// instead of three gained nothing).  One wave fewer (a_alt: 3 in FP32,
-// 2 in FP64) is a tuning option of phase A (TEMPO_HIP_TUNE_WAVES_A).
+// and capped at 5, 4 and 3 waves 536, 598 and 690.  The dual instantiations
+// keep the compiler's choice (the FP32 dual phase A takes 240 VGPRs, two
+// waves; held to three it spilled and made the adjoint 7-13 % slower; its
+// final update at four waves instead of three gained nothing).  One wave
+// fewer (a_alt: 3 in FP32, 2 in FP64) can also be set (TEMPO_HIP_TUNE_WAVES_A).
 template <class R>
 struct WavesPerEu {
   static constexpr int a = 1, a_alt = 1, c = 1;
