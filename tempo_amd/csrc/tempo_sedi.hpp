@@ -197,19 +197,19 @@ struct SedTile {
   // One species' planes (the block's column group of each is one contiguous
   // run): masses and numbers pm and raw speeds ph where the point holds the
   // species (pbit of its flags), tendencies pt where they are stored (tbit),
-  // elsewhere dm, 0 and td(plane, element).  Every
-  // global load is issued into registers before the first LDS write, so the
-  // stage waits for one memory latency instead of one per plane and pass (a
-  // load-convert-write loop per plane waits for each load before its write).
+  // elsewhere dm and zeros.  Every global load is issued into registers before
+  // the first LDS write, so the stage waits for one memory latency instead of
+  // one per plane and pass (a load-convert-write loop per plane waits for each
+  // load before its write).
   // The block has 64 * kSedCols threads and nz <= 64 * CH, so CH passes cover
   // the column group; a pass runs only when the group reaches it (a
   // block-uniform test), and its elements past the group's end load the last
   // one (the index is clamped) and are not written.  kAll: every point is
   // stored (dual planes).
-  template <bool kAll, class M, class H, int NM, int NH, int NT, class TD>
+  template <bool kAll, class M, class H, int NM, int NH, int NT>
   __device__ void load_species(const unsigned (&pfe)[CH], unsigned pbit, unsigned tbit, const int (&sm)[NM],
                                const M* const (&pm)[NM], const E (&dm)[NM], const int (&sh)[NH],
-                               const H* const (&ph)[NH], const int (&st)[NT], const M* const (&pt)[NT], TD td) const {
+                               const H* const (&ph)[NH], const int (&st)[NT], const M* const (&pt)[NT]) const {
     M vm[CH][NM], vt[CH][NT];
     H vh[CH][NH];
     const int n = kSedCols * nz;
@@ -239,7 +239,7 @@ struct SedTile {
 #pragma unroll
         for (int p = 0; p < NH; ++p) slot(sh[p])[x] = p_ ? staged<E>(vh[it][p]) : E(0);
 #pragma unroll
-        for (int p = 0; p < NT; ++p) slot(st[p])[x] = t_ ? staged<E>(vt[it][p]) : td(p, e);
+        for (int p = 0; p < NT; ++p) slot(st[p])[x] = t_ ? staged<E>(vt[it][p]) : E(0);
       }
     }
   }
@@ -774,7 +774,6 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   unsigned pfe[CH];  // flags of the elements this thread loads and stores
   if (threadIdx.x == 0) blk_any = 0;
   T.load_head(a, a.pf, sr + SR_RHO * plane, pfe);
-  const auto none = [](int, int) { return E(0); };
   const E r1 = E(S_t<R>(kR1)), r2 = E(S_t<R>(kR2));
   __syncthreads();
   unsigned pfl[CH];
@@ -841,7 +840,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     V raw1[CH], raw2[CH];
     T.template load_species<kAll>(pfe, PF_QR, PF_TR, {3, 0}, {sd + SD_RR * plane, sd + SD_NR * plane}, {r1, r2}, {4, 5},
                                   {sr + SR_VTRR * plane, sr + SR_VTNR * plane}, {1, 2},
-                                  {sd + SD_QRTEN * plane, sd + SD_NRTEN * plane}, none);
+                                  {sd + SD_QRTEN * plane, sd + SD_NRTEN * plane});
     __syncthreads();
     T.get(3, w, rr);
     T.get(0, w, xn);
@@ -896,7 +895,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     const E rb0 = E(S_t<R>(kM3ToL) * S_t<R>(kR1) / rho_g<S_t<R>>(kIdxBg1));
     T.template load_species<kAll>(pfe, PF_QG, PF_TG, {0, 1, 2}, {sd + SD_RG * plane, sd + SD_NG * plane, sd + SD_RB * plane},
                                   {r1, r2, rb0}, {7, 3}, {sr + SR_VTRG * plane, sr + SR_VTNG * plane}, {4, 5, 6},
-                                  {sd + SD_QGTEN * plane, sd + SD_NGTEN * plane, sd + SD_QBTEN * plane}, none);
+                                  {sd + SD_QGTEN * plane, sd + SD_NGTEN * plane, sd + SD_QBTEN * plane});
     __syncthreads();
     T.get(0, w, xg);
     T.get(1, w, xn);
@@ -960,7 +959,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     X xs[CH], ts[CH], v1[CH];
     V raw[CH];
     T.template load_species<kAll>(pfe, PF_QS, PF_TS, {0}, {sd + SD_RS * plane}, {r1}, {2}, {sr + SR_VTS * plane}, {1},
-                                  {sd + SD_QSTEN * plane}, none);
+                                  {sd + SD_QSTEN * plane});
     __syncthreads();
     T.get(0, w, xs);
     T.get(1, w, ts);
@@ -996,7 +995,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     V raw1[CH], raw2[CH];
     T.template load_species<kAll>(pfe, PF_QI, PF_TI, {0, 1}, {sd + SD_RI * plane, sd + SD_NI * plane}, {r1, r2}, {5, 6},
                                   {sr + SR_VTRI * plane, sr + SR_VTNI * plane}, {2, 4},
-                                  {sd + SD_QITEN * plane, sd + SD_NITEN * plane}, none);
+                                  {sd + SD_QITEN * plane, sd + SD_NITEN * plane});
     __syncthreads();
     T.get(0, w, xi);
     T.get(1, w, xn);
@@ -1022,16 +1021,10 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   if (bany & PF_QC) {
     X xc[CH], xn[CH], tc[CH], tn[CH], v1[CH], v2[CH];
     V raw1[CH], raw2[CH];
-    // a one-moment cloud's number tendency is, where not stored, clear air's
     const bool has_nc = a.f[F_NC] != nullptr;
-    const R* rho_p = sr + SR_RHO * plane;
-    T.template load_species<kAll>(
-        pfe, PF_QC, PF_TC, {0, 1}, {sd + SD_RC * plane, sd + SD_NC * plane}, {r1, E(S_t<R>(kNtCMin))}, {5, 6},
-        {sr + SR_VTRC * plane, sr + SR_VTNC * plane}, {2, 4}, {sd + SD_QCTEN * plane, sd + SD_NCTEN * plane},
-        [&](int p, int e) {
-          if (p == 0 || has_nc) return E(0);
-          return E(-S_t<R>(kNtCMin) * (S_t<R>(1) / S_t<R>(sval(T.elem(rho_p, e)))) * S_t<R>(a.odt));
-        });
+    T.template load_species<kAll>(pfe, PF_QC, PF_TC, {0, 1}, {sd + SD_RC * plane, sd + SD_NC * plane},
+                                  {r1, E(S_t<R>(kNtCMin))}, {5, 6}, {sr + SR_VTRC * plane, sr + SR_VTNC * plane}, {2, 4},
+                                  {sd + SD_QCTEN * plane, sd + SD_NCTEN * plane});
     __syncthreads();
     T.get(0, w, xc);
     T.get(1, w, xn);
@@ -1053,6 +1046,17 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
         v1[j] = (k < kt) ? X(raw1[j]) : X(0.0);
         v2[j] = (k < kt) ? X(raw2[j]) : X(0.0);
       }
+      // cloud settles into levels without any: theirs is a number tendency too
+      if constexpr (!kAll) {
+        if (!has_nc) {
+#pragma unroll
+          for (int j = 0; j < CH; ++j) {
+            const bool fed = wv::above(v1, j) != X(0.0);
+            const int k = j * 64 + wv::lane();
+            if (fed && k < kt && !(a.pf[TEMPO_IDX_SCR(a, c, k)] & PF_TC)) tn[j] = X(cloudless_ncten(a, c, k));
+          }
+        }
+      }
       const X pq = wave_sediment(g, xc, v1, tc, kR1, 1, kt, (kt + 63) / 64, dt, true);
       wave_sediment(g, xn, v2, tn, kR2, 1, kt, (kt + 63) / 64, dt, false);
       record(4, pq, 1, kt);
@@ -1061,7 +1065,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
     T.put(4, w, tn);
     __syncthreads();
     T.template store_species<kAll>(pfe, PF_TC, {2, 4}, {sd + SD_QCTEN * plane, sd + SD_NCTEN * plane},
-                                   a.f[F_NC] ? 3u : 1u);
+                                   has_nc ? 3u : 1u);
   }
   if (!kAll) {  // the flags the final update reads
 #pragma unroll

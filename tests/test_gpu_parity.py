@@ -1468,3 +1468,45 @@ def test_gpu_host_default_slabs(hip, ncol):
         got.append({**s, **d})
     for k, v in got[0].items():
         assert np.array_equal(v, got[1][k], equal_nan=True), k
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "fp64"])
+@pytest.mark.parametrize("aerosols", [True, False])
+@pytest.mark.parametrize("condensation", [True, False])
+def test_gpu_one_moment_cloud_settles_into_empty_levels(hip, dtype, aerosols, condensation):
+    """cloud of one-moment number that settles into cloud-free levels cold
+    enough to freeze it there, the wavefront sedimentation against one lane per
+    column bit for bit: the number tendency of such a level (none, what
+    condensation left of the cloud's floor, or an activation) enters the number
+    of the ice.  Levels 1 and 7 are dry in every column (clear air), the others
+    between dryness and supersaturation; a cloud number small enough that the
+    ice number is not at its largest."""
+    from tempo_amd import generator as gen
+    ctx = hip.TempoHip(aerosolaware_flag=int(aerosols), hailaware_flag=0, single_moment_nc_opt="1e5")
+    ctx.set_run_cfg(cloud_condensation_flag=int(condensation))
+    prec, td = (hip.FP32, torch.float32) if dtype == "fp32" else (hip.FP64, torch.float64)
+    ncol, nz, dz = 72, 20, 40.0
+    rng = np.random.default_rng(9)
+    k, c = np.arange(nz)[:, None], np.arange(ncol)[None, :]
+    st = {n: np.zeros((nz, ncol)) for n in ("qc", "qr", "qi", "qs", "qg", "ni", "nr", "w")}
+    st["t"] = 228.0 + 0.3 * (k % 5) + 0.05 * (c % 7)
+    st["p"] = 6.0e4 * np.exp(-9.81 * dz * k / (287.0 * 229.0)) + 0.0 * c
+    st["dz"] = np.full((nz, ncol), dz)
+    sat = gen.rslf(st["p"], st["t"])
+    st["qv"] = sat * rng.choice([0.3, 0.9, 0.9995, 1.0, 1.0 + 1e-9, 1.0 + 1e-6, 1.001], size=sat.shape)
+    st["qv"][[1, 7]] = 0.3 * sat[[1, 7]]
+    st["qc"][[2, 5, 8]] = np.exp(rng.uniform(np.log(1e-5), np.log(2e-3), (3, ncol)))
+    st["qc"][:, ::9] = 0.0
+    if aerosols:
+        st["nwfa"], st["nifa"] = np.full((nz, ncol), 3e8), np.full((nz, ncol), 1e5)
+    got = {}
+    for wave in (1, 0):
+        ctx.tune(prec, hip.TUNE_SED_WAVE, wave)
+        dev = to_dev(st, td)
+        d = ctx.run(dev, 300.0, 2)
+        got[wave] = {n: v.cpu().numpy() for n, v in {**dev, **d}.items()}
+    empty = (st["qc"] == 0.0) & (got[0]["qi"] > 1e-9)
+    assert empty[1].sum() > 20 and empty[4].sum() > 20 and empty[7].sum() > 20  # cloud came and froze
+    assert (got[0]["ni"][empty] < 4e6).mean() > 0.5
+    for n, v in got[1].items():
+        assert np.array_equal(v, got[0][n], equal_nan=True), n
