@@ -342,8 +342,10 @@ class TempoHip:
         yb = self._fields(ybar, nz, ncol, dtype, "cotangent")
         db = self._diags(dbar, nz, ncol, dtype)
         names = wrt or ("t", "qv", "qc", "qr", "qi", "qs", "qg", "nc", "nr")
-        # every element of a differentiable input's cotangent is written
-        xbar = {k: (torch.empty if k in ADJOINT_NAMES else torch.zeros)((nz, ncol), dtype=dtype, device=ref.device)
+        # every element of a differentiable input's cotangent is written, if
+        # the state has the field
+        xbar = {k: (torch.empty if k in ADJOINT_NAMES and state[k] is not None else torch.zeros)(
+                    (nz, ncol), dtype=dtype, device=ref.device)
                 for k in names if k in state}
         xb = self._fields(xbar, nz, ncol, dtype)
         keep = []

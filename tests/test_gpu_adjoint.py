@@ -757,3 +757,25 @@ def test_adjoint_batches_and_directions(ctx, sample, ncol, dtype, sparse):
     for k in names:
         one = gradient(33, (k,))[k]
         assert torch.equal(all_[k], one[:, torch.arange(ncol, device="cuda") % 33]), k
+
+
+@pytest.mark.parametrize("wrt", [None, ("t", "qr", "nc", "nwfa", "nifa", "ng", "qb")])
+def test_adjoint_of_fields_given_as_none(hip, wrt):
+    """optional fields that a state holds as None: the cotangents named for
+    them are zeros, whatever the allocator's memory held"""
+    from tempo_amd import generator as gen
+    c = hip.TempoHip(aerosolaware_flag=0, hailaware_flag=0)
+    st, m = gen.generate("adjoint", ncol=96, col0=31)
+    st = {k: torch.tensor(v, dtype=torch.float64, device="cuda") for k, v in st.items()}
+    st.update({k: None for k in ("nc", "nwfa", "nifa", "ng", "qb")})
+    ybar = {"qv": torch.ones_like(st["qv"]), "qr": torch.ones_like(st["qr"])}
+    full = {k: v for k, v in st.items() if v is not None}
+    want = c.adjoint(full, ybar, {}, m["dt"], 2, wrt=tuple(k for k in wrt if k in full) if wrt else None)
+    torch.cuda.synchronize()
+    fill = [torch.full_like(st["t"], float("nan")) for _ in range(32)]
+    del fill  # the allocator hands this memory out again
+    got = c.adjoint(st, ybar, {}, m["dt"], 2, wrt=wrt)
+    names = wrt or X_NAMES
+    assert set(got) == set(names)
+    for k in names:
+        assert torch.equal(got[k], want[k] if k in want else torch.zeros_like(st["t"])), k
