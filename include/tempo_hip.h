@@ -257,7 +257,8 @@ int tempo_hip_snow_check_and_update_host(tempo_hip_ctx *ctx, int n, const double
  * their forward branches (branch-frozen derivatives; with semi_sedi_flag
  * also the semi-Lagrangian remap's source cells, limiters and clamps); in
  * FP64 the values are those of tempo_hip_run bit for bit.  qc_bl and
- * qcfrac_bl of f, when given, are constants of the step.  Returns
+ * qcfrac_bl of f, when given, are constants of the step.  The 3-D diagnostics
+ * and their tangents are zero at levels k >= nlev of a column.  Returns
  * TEMPO_HIP_E_UNSUPPORTED for a context with refl10cm_from_melting_flag. */
 int tempo_hip_tlm(tempo_hip_ctx *ctx, const tempo_hip_fields *f, const tempo_hip_fields *f_tl,
                   const tempo_hip_diags *d, const tempo_hip_diags *d_tl, const tempo_hip_dims *dims, double dt,

@@ -668,21 +668,23 @@ __global__ void __launch_bounds__(256) k_dual_pack_n(DualBatch<T> b, DualGeom g)
   const T* t = b.t[blockIdx.z];
   b.d[blockIdx.z][p.e] = Dual<T>(b.v[blockIdx.z][p.o], t ? t[p.o] : T(0));
 }
-// duals into values and tangents (either may be NULL)
+// duals into values and tangents (either may be NULL); zeros at the levels a
+// column does not have (nlev, may be NULL), where the step sets no diagnostics
 template <class T>
-__global__ void __launch_bounds__(256) k_dual_unpack_n(DualBatch<T> b, DualGeom g) {
+__global__ void __launch_bounds__(256) k_dual_unpack_n(DualBatch<T> b, DualGeom g, const int* __restrict__ nlev) {
   const PlanePoint p = plane_point(g);
   if (!p.in) return;
-  const Dual<T> x = b.d[blockIdx.z][p.e];
+  const bool none = nlev && int(blockIdx.y) >= nlev[blockIdx.x * 256u + threadIdx.x];
+  const Dual<T> x = none ? Dual<T>(T(0), T(0)) : b.d[blockIdx.z][p.e];
   if (b.v[blockIdx.z]) b.v[blockIdx.z][p.o] = x.v;
   if (b.t[blockIdx.z]) b.t[blockIdx.z][p.o] = x.d;
 }
-template <class K, class B>
-hipError_t launch_batch(K kernel, const B& b, int n, const DualGeom& g, hipStream_t s) {
+template <class K, class B, class... More>
+hipError_t launch_batch(K kernel, const B& b, int n, const DualGeom& g, hipStream_t s, More... more) {
   if (n <= 0) return hipSuccess;
   if (n > kBatchMax) return hipErrorInvalidValue;
   const unsigned blocks = (unsigned(g.ni) * unsigned(g.nj) + 255u) / 256u;
-  hipLaunchKernelGGL(kernel, dim3(blocks, unsigned(g.nk), unsigned(n)), dim3(256), 0, s, b, g);
+  hipLaunchKernelGGL(kernel, dim3(blocks, unsigned(g.nk), unsigned(n)), dim3(256), 0, s, b, g, more...);
   return hipGetLastError();
 }
 template <class T>
@@ -698,8 +700,8 @@ hipError_t launch_dual_pack_n(const DualBatch<T>& b, int n, const DualGeom& g, h
   return launch_batch(k_dual_pack_n<T>, b, n, g, s);
 }
 template <class T>
-hipError_t launch_dual_unpack_n(const DualBatch<T>& b, int n, const DualGeom& g, hipStream_t s) {
-  return launch_batch(k_dual_unpack_n<T>, b, n, g, s);
+hipError_t launch_dual_unpack_n(const DualBatch<T>& b, int n, const DualGeom& g, const int* nlev, hipStream_t s) {
+  return launch_batch(k_dual_unpack_n<T>, b, n, g, s, nlev);
 }
 
 }  // namespace tempo

@@ -47,7 +47,7 @@ hipError_t launch_from_compact_n(const PlaneBatch<double, T>& b, int n, const Du
 template <class T>
 hipError_t launch_dual_pack_n(const DualBatch<T>& b, int n, const DualGeom& g, hipStream_t s);
 template <class T>
-hipError_t launch_dual_unpack_n(const DualBatch<T>& b, int n, const DualGeom& g, hipStream_t s);
+hipError_t launch_dual_unpack_n(const DualBatch<T>& b, int n, const DualGeom& g, const int* nlev, hipStream_t s);
 hipError_t launch_table_qg(const double*, const double*, const double*, const double*, double*, hipStream_t);
 hipError_t launch_table_qs(const double*, const double*, const double*, const double*, double*, hipStream_t);
 hipError_t launch_table_fz(const double*, const double*, const double*, const double*, double, const double*,
@@ -766,7 +766,7 @@ int run_tlm(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_fields*
   int rc = bind_common(x, a, dt, itimestep);
   if (rc) return rc;
   HIP_TRY(launch_step_tlm(a, x->launch[sizeof(T) == 8 ? 1 : 0], x->vtbuf.as<Dual<double>>(), s));
-  HIP_TRY(launch_dual_unpack_n(pk, nstate, g3, s));  // the state's entries come first
+  HIP_TRY(launch_dual_unpack_n(pk, nstate, g3, nullptr, s));  // the state's entries come first
   DualGeom g2{dm->ni, dm->nj, 1, 0, dm->d2ldj};
   DualGeom gd3{dm->ni, dm->nj, nz, dm->dldk, dm->dldj};
   DualBatch<T> u2{}, u3{};
@@ -783,8 +783,8 @@ int run_tlm(tempo_hip_ctx* x, const tempo_hip_fields* f, const tempo_hip_fields*
     u3.t[nd3] = static_cast<T*>(t3[i]);
     u3.d[nd3++] = a.d3[i];
   }
-  HIP_TRY(launch_dual_unpack_n(u2, n2, g2, s));
-  HIP_TRY(launch_dual_unpack_n(u3, nd3, gd3, s));
+  HIP_TRY(launch_dual_unpack_n(u2, n2, g2, nullptr, s));
+  HIP_TRY(launch_dual_unpack_n(u3, nd3, gd3, dm->nlev, s));
   return TEMPO_HIP_OK;
 }
 

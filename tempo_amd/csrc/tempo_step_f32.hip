@@ -33,6 +33,6 @@ hipError_t launch_adjoint(const StepArgs<Dual<float>>& a, const AdjArgs& g, Dual
 template hipError_t launch_to_compact_n<float>(const PlaneBatch<float, double>&, int, const DualGeom&, hipStream_t);
 template hipError_t launch_from_compact_n<float>(const PlaneBatch<double, float>&, int, const DualGeom&, hipStream_t);
 template hipError_t launch_dual_pack_n<float>(const DualBatch<float>&, int, const DualGeom&, hipStream_t);
-template hipError_t launch_dual_unpack_n<float>(const DualBatch<float>&, int, const DualGeom&, hipStream_t);
+template hipError_t launch_dual_unpack_n<float>(const DualBatch<float>&, int, const DualGeom&, const int*, hipStream_t);
 
 }  // namespace tempo

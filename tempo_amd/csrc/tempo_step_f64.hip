@@ -33,6 +33,6 @@ hipError_t launch_adjoint(const StepArgs<Dual<double>>& a, const AdjArgs& g, Dua
 template hipError_t launch_to_compact_n<double>(const PlaneBatch<double, double>&, int, const DualGeom&, hipStream_t);
 template hipError_t launch_from_compact_n<double>(const PlaneBatch<double, double>&, int, const DualGeom&, hipStream_t);
 template hipError_t launch_dual_pack_n<double>(const DualBatch<double>&, int, const DualGeom&, hipStream_t);
-template hipError_t launch_dual_unpack_n<double>(const DualBatch<double>&, int, const DualGeom&, hipStream_t);
+template hipError_t launch_dual_unpack_n<double>(const DualBatch<double>&, int, const DualGeom&, const int*, hipStream_t);
 
 }  // namespace tempo

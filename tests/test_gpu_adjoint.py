@@ -779,3 +779,32 @@ def test_adjoint_of_fields_given_as_none(hip, wrt):
     assert set(got) == set(names)
     for k in names:
         assert torch.equal(got[k], want[k] if k in want else torch.zeros_like(st["t"])), k
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("nz", [40, 130])
+def test_tlm_diagnostics_above_a_columns_depth(hip, dtype, nz):
+    """the 3-D diagnostics and their tangents of the tangent-linear step are
+    zero at the levels a column does not have, as the step's own are, not what
+    an earlier call left behind"""
+    from tempo_amd import generator as gen
+    c = hip.TempoHip(**FLAGS)
+    st, m = gen.generate("adjoint", ncol=70, col0=3)
+    x_old, x_new = np.arange(st["p"].shape[0], dtype=np.float64), np.linspace(0.0, st["p"].shape[0] - 1.0, nz)
+    st = {k: np.stack([np.interp(x_new, x_old, v[:, i]) for i in range(70)], axis=1) for k, v in st.items()}
+    nlev = np.maximum(2, nz - np.arange(70) % 30).astype(np.int32)
+    above = torch.tensor(np.arange(nz)[:, None] >= nlev[None, :], device="cuda")
+
+    def tlm(nl):
+        dev = {k: torch.tensor(v, dtype=dtype, device="cuda") for k, v in st.items()}
+        return c.tlm(dev, {k: 0.01 * v for k, v in dev.items()}, m["dt"], 2, nlev=nl)
+    whole = tlm(None)
+    d, t, _ = tlm(torch.tensor(nlev, device="cuda"))
+    assert (whole[0]["refl10cm"][above] != 0).all()
+    for n in hip.DIAG3_NAMES:
+        assert (d[n][above] == 0).all() and (t[n][above] == 0).all(), n
+        assert torch.isfinite(d[n][~above]).all(), n
+    # the deepest columns are the whole ones
+    deep = torch.tensor(nlev == nz, device="cuda")
+    assert torch.equal(d["refl10cm"][:, deep], whole[0]["refl10cm"][:, deep])
+    assert torch.equal(t["refl10cm"][:, deep], whole[1]["refl10cm"][:, deep])
