@@ -319,15 +319,15 @@ int tempo_hip_substeps(tempo_hip_ctx *ctx, int *host_out, size_t n);
  *                               points with microphysics to do to its first
  *                               wavefronts, so that they do not share
  *                               wavefronts with idle points; clear = lane i
- *                               takes column i.  Unless set it is chosen:
- *                               bit 0 in FP64, both in batches of few columns,
- *                               else 0 (the results are the same)
+ *                               takes column i.  -1 (default): chosen for
+ *                               each batch, bit 0 in FP64, both in batches of
+ *                               few columns, else 0 (the results are the same)
  *   TEMPO_HIP_TUNE_WAVES_A   1: the level-local physics compiled for one
  *                               wave per SIMD fewer (more registers, fewer
  *                               spills: 3 instead of 4 in FP32, 2 instead
- *                               of 3 in FP64), 0: not.  Unless set, 1 in
- *                               FP64 up to 4,096 wavefronts (64 columns of
- *                               a level each), else 0
+ *                               of 3 in FP64), 0: not.  -1 (default): chosen
+ *                               for each batch, 1 in FP64 up to 4,096
+ *                               wavefronts (64 columns of a level each), else 0
  *   TEMPO_HIP_TUNE_CCN_LDS   1: each block of the level-local physics
  *                               copies the CCN activation table's slice
  *                               (441 floats) into LDS and reads it there,

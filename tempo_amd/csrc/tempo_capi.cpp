@@ -1664,7 +1664,7 @@ int tempo_hip_tune(tempo_hip_ctx* x, int precision, int key, int value) {
       (key == TEMPO_HIP_TUNE_BLOCK_A ? lc.block_a : lc.block_c) = value;
       return TEMPO_HIP_OK;
     case TEMPO_HIP_TUNE_ORDER:
-      if (value < 0 || value > 3) return fail(TEMPO_HIP_E_ARG, "order must be 0..3");
+      if (value < -1 || value > 3) return fail(TEMPO_HIP_E_ARG, "order must be 0..3, or -1 (chosen)");
       lc.order = value;
       return TEMPO_HIP_OK;
     case TEMPO_HIP_TUNE_FUSED:
@@ -1672,7 +1672,7 @@ int tempo_hip_tune(tempo_hip_ctx* x, int precision, int key, int value) {
       if (value == 1) return fail(TEMPO_HIP_E_UNSUPPORTED, "this library has no single-launch step");
       return TEMPO_HIP_OK;
     case TEMPO_HIP_TUNE_WAVES_A:
-      if (value != 0 && value != 1) return fail(TEMPO_HIP_E_ARG, "waves_a must be 0 or 1");
+      if (value < -1 || value > 1) return fail(TEMPO_HIP_E_ARG, "waves_a must be 0 or 1, or -1 (chosen)");
       lc.waves_a = value;
       return TEMPO_HIP_OK;
     case TEMPO_HIP_TUNE_CCN_LDS:

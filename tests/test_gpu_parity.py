@@ -70,6 +70,17 @@ def context(hip, flags):
     return _ctx_cache[key]
 
 
+@pytest.fixture(autouse=True)
+def launch_choices(hip):
+    """the cached contexts choose their point grouping and register budget in
+    every test, whatever an earlier one set"""
+    yield
+    for ctx in _ctx_cache.values():
+        for prec in (hip.FP32, hip.FP64):
+            ctx.tune(prec, hip.TUNE_ORDER, -1)
+            ctx.tune(prec, hip.TUNE_WAVES_A, -1)
+
+
 @pytest.fixture(scope="module")
 def gpu_tables(hip):
     ctx = context(hip, dict(aerosolaware=True, hailaware=True))
@@ -1510,3 +1521,39 @@ def test_gpu_one_moment_cloud_settles_into_empty_levels(hip, dtype, aerosols, co
     assert (got[0]["ni"][empty] < 4e6).mean() > 0.5
     for n, v in got[1].items():
         assert np.array_equal(v, got[0][n], equal_nan=True), n
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "fp64"])
+def test_gpu_launch_choices_can_be_restored(hip, dtype):
+    """-1 gives the point grouping and the register budget back to the rules,
+    and is a value of these two keys only.  Clear air and sparse planes under
+    every grouping against the lane-per-column sedimentation, bit for bit."""
+    from tempo_amd import generator as gen
+    ctx = hip.TempoHip(aerosolaware_flag=1, hailaware_flag=0)
+    prec, td = (hip.FP32, torch.float32) if dtype == "fp32" else (hip.FP64, torch.float64)
+    st, m = gen.generate("adjoint", ncol=300, col0=7)
+    st["qv"][:, ::3] *= 0.2
+    for q in ("qc", "qr", "qi", "qs", "qg"):
+        st[q][:, ::3] = 0.0
+    out = []
+    for wave, order, waves in ((0, None, None), (1, None, None), (1, 0, 0), (1, -1, -1), (1, 3, 1), (1, 1, 0), (1, 2, 1),
+                               (1, -1, -1)):
+        ctx.tune(prec, hip.TUNE_SED_WAVE, wave)
+        if order is not None:
+            ctx.tune(prec, hip.TUNE_ORDER, order)
+            ctx.tune(prec, hip.TUNE_WAVES_A, waves)
+        dev = to_dev(st, td)
+        for i in range(2):
+            d = ctx.run(dev, m["dt"], 2 + i)
+        out.append({**dev, **d})
+    for o in out[1:]:
+        for k, v in o.items():
+            assert torch.equal(v, out[0][k]), k
+    for key in (hip.TUNE_ORDER, hip.TUNE_WAVES_A):
+        with pytest.raises(hip.TempoError) as e:
+            ctx.tune(prec, key, -2)
+        assert e.value.code == hip.E_ARG
+    for key in (hip.TUNE_SED_WAVE, hip.TUNE_BLOCK_A, hip.TUNE_FUSED, hip.TUNE_CCN_LDS):
+        with pytest.raises(hip.TempoError) as e:
+            ctx.tune(prec, key, -1)
+        assert e.value.code == hip.E_ARG
