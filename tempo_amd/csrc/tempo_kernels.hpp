@@ -366,17 +366,6 @@ __device__ __forceinline__ ClearAir<R> clear_air_tendencies(const ConstView<S_t<
   return q;
 }
 
-// The number tendency that the level-local physics left a one-moment cloud at a
-// point without PF_TC.  It is stored (none without condensation, or where this
-// ended at saturation; what it activated or evaporated of the floor elsewhere),
-// except in clear air, where it follows from the state.
-template <class R>
-__device__ __forceinline__ R cloudless_ncten(const StepArgs<R>& a, int c, int k) {
-  const size_t o = TEMPO_IDX_STATE(a, c, k), s = TEMPO_IDX_SCR(a, c, k);
-  if (!(a.pf[s] & PF_CLEAR)) return R(a.sd[size_t(SD_NCTEN) * a.plane + s]);
-  return -clear_air_tendencies<R>(const_view(a.cst), a.f[F_P][o], load_t(a, o), a.f[F_QV][o], R(a.dt), R(a.odt)).nwfaten;
-}
-
 // the level-local physics of point (c, k), from the initial checks to the
 // fall speeds (src/module_mp_tempo_main.F90:320-588)
 template <class R, class Point>
@@ -412,6 +401,7 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
         const ClearAir<R> q = clear_air_tendencies<R>(C, pres, t1d, qv1d, dt, odt);
         pt.sr()[SR_RHO * plane + s] = q.rho;
         if (k == 0) pt.sr()[SR_TEMP * plane + s] = q.temp;
+        if (!has_nc) pt.sd()[SD_NCTEN * plane + s] = Sd_t<R>(-q.nwfaten);
         pt.pf()[s] = PF_CLEAR;
         return;
       }
@@ -607,8 +597,7 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
   const bool tg = all || moves(L.qgten) || moves(L.ngten) || moves(L.qbten);
   const bool ts = all || moves(L.qsten);
   const bool ti = all || moves(L.qiten) || moves(L.niten);
-  // (without prognostic cloud number its tendency counts only with a cloud, and
-  // is stored at every point: a cloud may settle there)
+  // (without prognostic cloud number its tendency counts only with a cloud)
   const bool tc = all || L.l_qc || moves(L.qcten) || (has_nc && moves(L.ncten));
   pf |= (tr ? PF_TR : 0u) | (tg ? PF_TG : 0u) | (ts ? PF_TS : 0u) | (ti ? PF_TI : 0u) | (tc ? PF_TC : 0u);
   using D = Sd_t<R>;

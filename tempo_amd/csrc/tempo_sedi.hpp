@@ -1053,7 +1053,7 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
           for (int j = 0; j < CH; ++j) {
             const bool fed = wv::above(v1, j) != X(0.0);
             const int k = j * 64 + wv::lane();
-            if (fed && k < kt && !(a.pf[TEMPO_IDX_SCR(a, c, k)] & PF_TC)) tn[j] = X(cloudless_ncten(a, c, k));
+            if (fed && k < kt && !(a.pf[TEMPO_IDX_SCR(a, c, k)] & PF_TC)) tn[j] = X(sd[SD_NCTEN * plane + TEMPO_IDX_SCR(a, c, k)]);
           }
         }
       }

@@ -219,18 +219,20 @@ enum ScrD {
 };
 // Per point flag bits.  PF_Q*: the species is present after the level-local
 // physics (its mass, number and speed planes hold the point); PF_T*: its
-// tendency planes hold the point, else its tendencies are zero; PF_CLEAR: a
-// point of clear air, whose temperature, vapour and tendencies are those of
-// clear_air_tendencies and only its density (and lowest-level temperature)
-// is stored.
+// tendency planes hold the point, else its tendencies are zero (but for a
+// one-moment cloud's number tendency, which every point has stored: cloud may
+// settle into a level without any); PF_CLEAR: a point of clear air, whose
+// temperature, vapour and tendencies are those of clear_air_tendencies and
+// only its density (and lowest-level temperature) is stored besides.
 //
 // Most points of an atmosphere hold no hydrometeor, or few species.  Instead
 // of writing all 37 scratch planes at every point and reading them back, a
 // plane's 32-byte sector (8 columns of one level) is moved only where one of
 // its columns needs it.  With the clear-air path: 100,000 x 90 2.30 -> 2.20
 // ms a step, 131,072 uneven columns 4.22 -> 3.61, 262,144 x 90 7.0 -> 6.4;
-// 1,024 x 60, where latency counts, 64 -> 66 us.  Kernels that read the planes directly (one lane per column, derivative
-// steps) have every point stored (StepArgs::sparse = 0).
+// 1,024 x 60, where latency counts, 64 -> 66 us.  Kernels that read the planes
+// directly (one lane per column, derivative steps) have every point stored
+// (StepArgs::sparse = 0).
 enum : unsigned {
   PF_QR = 1u, PF_QG = 2u, PF_QS = 4u, PF_QI = 8u, PF_QC = 16u, PF_SNOWMIX = 32u,
   PF_TR = 64u, PF_TG = 128u, PF_TS = 256u, PF_TI = 512u, PF_TC = 1024u, PF_CLEAR = 2048u,
