@@ -386,8 +386,9 @@ __device__ __forceinline__ int wave_fill(const X (&mass)[CH], const R (&raw1)[CH
 
 // one flux-form substep of one field (:1516-1559) in the chunks up to the
 // highest non-zero speed (at the top level above it, which the reference
-// always updates, the flux is zero); returns the surface precipitation
-// increment (0 when the caller does not accumulate it)
+// always updates, the flux is zero, and only a mass below the limit changes);
+// returns the surface precipitation increment (0 when the caller does not
+// accumulate it)
 template <int CH, class X>
 __device__ __forceinline__ X wave_sediment(const SedCol<CH, X>& g, X (&xr)[CH], const X (&vt)[CH], X (&xten)[CH],
                                            double limit, int steps, int ktop, int chunks, double dt, bool precip) {
@@ -971,6 +972,9 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
       for (int j = 0; j < CH; ++j) {
         V v = raw[j];
         if (pfl[j] & PF_SNOWMIX) {
+          // the top level, which rain's sedimentation always updates, holds at
+          // least r1, also in a chunk above the highest mass, left out there
+          if (CH > 1 && !kSemi && (any & PF_QR) && j * 64 + wv::lane() == g.nzc - 1 && !(rr[j] > kR1)) rr[j] = X(kR1);
           const V sr_ = V(xs[j] / (xs[j] + rr[j]));
           v = v * sr_ + (V(1.0) - sr_) * V(vr[j]);
         }

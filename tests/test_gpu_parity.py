@@ -1557,3 +1557,37 @@ def test_gpu_launch_choices_can_be_restored(hip, dtype):
         with pytest.raises(hip.TempoError) as e:
             ctx.tune(prec, key, -1)
         assert e.value.code == hip.E_ARG
+
+
+def test_gpu_rain_below_presence_at_the_top_level(hip):
+    """rain whose mixing ratio is above the presence threshold and whose mass
+    per volume is not, at a warm top level in the last register chunk of the
+    wavefront sedimentation: the top level's mass is raised to the threshold
+    there too, and mixes into the speed of the melting snow (FP64, against one
+    lane per column, bit for bit)"""
+    from tempo_amd import generator as gen
+    ctx = context(hip, dict(aerosolaware=False, hailaware=False))
+    for nz in (64, 66, 130):
+        ncol = 16
+        st = {n: np.zeros((nz, ncol)) for n in ("qc", "qr", "qi", "qs", "qg", "ni", "nr", "w")}
+        st["t"] = np.full((nz, ncol), 250.0)
+        st["t"][-1] = 273.15 + 1e-9
+        st["p"] = np.linspace(8.0e4, 2.35e4, nz)[:, None] + np.zeros(ncol)
+        st["dz"] = np.full((nz, ncol), 100.0)
+        st["qv"] = 0.3 * gen.rslf(st["p"], st["t"])
+        st["qv"][-1] = 1.0001 * gen.rslf(st["p"], st["t"])[-1]
+        st["qs"][-1] = np.linspace(1e-6, 1e-5, ncol)
+        st["qr"][-1] = np.linspace(1.2e-12, 2.8e-12, ncol)
+        st["nr"][-1] = 4e-3
+        got = {}
+        try:
+            for wave in (1, 0):
+                ctx.tune(hip.FP64, hip.TUNE_SED_WAVE, wave)
+                dev = to_dev(st, torch.float64)
+                d = ctx.run(dev, 20.0, 2)
+                got[wave] = {n: v.cpu().numpy() for n, v in {**dev, **d}.items()}
+        finally:
+            ctx.tune(hip.FP64, hip.TUNE_SED_WAVE, 1)
+        assert (got[0]["qs"][-2] > 0.0).all()  # the snow falls
+        for n, v in got[1].items():
+            assert np.array_equal(v, got[0][n], equal_nan=True), (nz, n)
