@@ -188,10 +188,11 @@ __device__ __host__ __forceinline__ double pow_special(double x, double y, doubl
   return odd ? copysign(r, x) : r;
 }
 
-// x^n for n = 1, 2, 3, 4, 5, 7, 8: products carried in double-double (relative
-// error below 2^-100) and rounded once, as pow_cr rounds, at a tenth of its
-// instructions.  Where a product leaves the range in which its low part is
-// exact, the plain product: it overflows or vanishes as the power does.
+// x^n for n = 1, 2, 3, 4, 5, 7, 8: products of the significand carried in
+// double-double (relative error below 2^-100) and rounded once, as pow_cr
+// rounds, at a tenth of its instructions.  The exponent goes in last, so that
+// no product leaves the range in which its low part is exact; 0, infinities and
+// NaN, whose low parts are none, take the plain product.
 template <int n>
 __device__ __host__ __forceinline__ dd pow_whole_dd(double x) {
 #pragma clang fp contract(off)
@@ -210,30 +211,38 @@ __device__ __host__ __forceinline__ dd pow_whole_dd(double x) {
 template <int n>
 __device__ __host__ __forceinline__ double pow_whole(double x) {
 #pragma clang fp contract(off)
+  int e;
+  const double m = frexp(x, &e);
+  const dd d = pow_whole_dd<(n < 0 ? -n : n)>(m);
+  const bool in = fabs(d.hi) > 0.0 && fabs(d.hi) < 2.0;
   if constexpr (n < 0) {
-    const dd d = pow_whole_dd<-n>(x);
     const double q = 1.0 / d.hi;
     const double r = fma(-q, d.hi, 1.0) - q * d.lo;
-    return fabs(d.hi) > 1.0e-250 && fabs(d.hi) < 1.0e250 ? fma(q, r, q) : q;
+    return in ? ldexp(fma(q, r, q), n * e) : q;
   } else {
-    const dd d = pow_whole_dd<n>(x);
-    return fabs(d.hi) > 1.0e-250 && fabs(d.hi) < 1.0e250 ? d.hi + d.lo : d.hi;
+    return in ? ldexp(d.hi + d.lo, n * e) : d.hi;
   }
 }
 
-// x^(n + 1/2), and its inverse: the square root with its residual, times x^n
+// x^(n + 1/2), and its inverse: the square root with its residual, times x^n,
+// of the significand beside an even exponent
 template <int n, bool kInverse = false>
 __device__ __host__ __forceinline__ double pow_half(double x) {
 #pragma clang fp contract(off)
-  const double s = sqrt(x);
-  const double sl = fma(-s, s, x) * double(0.5f / float(s));
-  const dd w = pow_whole_dd<n>(x);
+  int e;
+  double m = frexp(x, &e);
+  const int half = e >> 1;
+  m = ldexp(m, e - 2 * half);  // in [1/2, 2)
+  const double s = sqrt(m);
+  const double sl = fma(-s, s, m) * double(0.5f / float(s));
+  const dd w = pow_whole_dd<n>(m);
   dd p = two_prod(w.hi, s);
   p.lo += fma(w.hi, sl, w.lo * s);
-  const bool in = x > 1.0e-60 && x < 1.0e60;
-  if (!kInverse) return in ? p.hi + p.lo : w.hi * s;
+  const bool in = positive_finite(x);
+  const int shift = half * (2 * n + 1);
+  if (!kInverse) return in ? ldexp(p.hi + p.lo, shift) : w.hi * s;
   const double q = 1.0 / p.hi;
-  return in ? fma(q, fma(-q, p.hi, 1.0) - q * p.lo, q) : 1.0 / (w.hi * s);
+  return in ? ldexp(fma(q, fma(-q, p.hi, 1.0) - q * p.lo, q), -shift) : 1.0 / (w.hi * s);
 }
 
 // x^y for y = the double nearest 1/3 (1/3 - 1.85e-17): the cube root by

@@ -120,3 +120,16 @@ def test_special_arguments(shim):
         for k, e in enumerate(EXPONENTS):
             x = np.array([0.0, inf, 1.0, 1e-300, 1e300, nan])
             np.testing.assert_allclose(shim(10 + k, x, 0.0), np.power(x, e), rtol=1e-15, atol=5e-324)
+
+
+@pytest.mark.parametrize("k", range(len(EXPONENTS)))
+def test_pow_known_exponent_whole_range(shim, k):
+    """arguments from the smallest to the largest for which the power is a
+    normal number"""
+    rng = np.random.default_rng(30 + k)
+    e = EXPONENTS[k]
+    ends = sorted((708.0 / abs(e) if abs(e) > 1 else 708.0, 60.0 * math.log(10.0), 250.0 * math.log(10.0) / abs(e)))
+    lx = np.concatenate([rng.uniform(-ends[-1], ends[-1], N)] + [s * v + rng.uniform(-1, 1, 50) for v in ends[:-1] for s in (-1, 1)])
+    lx = lx[np.abs(lx * e) < 708.0]
+    x = np.exp(np.clip(lx, -708.0, 709.0))
+    check(shim(10 + k, x, 0.0), decimals(lambda v: (v.ln() * Decimal(e)).exp(), x))
