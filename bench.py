@@ -20,7 +20,8 @@ against FP64 report with branch accounting, the forward + adjoint timings
 (16,384 x 64 single step; 12 steps x 262,144 x 90), the step on host
 arrays with its PCIe transfers (tempo_hip_run_host_prec, FP64 and FP32) and
 the reference CPU step timed on this host's cores over a bounded sample of
-the same seeded step (oracle/cpu_baseline.py, run in a child process).
+the same seeded step (oracle/cpu_baseline.py, run in a child process; none
+where the reference build is not present).
 """
 import argparse
 import json
@@ -81,6 +82,18 @@ def cpu_baseline(ctx, cols, workers, repeats):
     cb["cpu_model"] = out["cpu_model"]
     cb["affinity_cores"] = out["affinity_cores"]
     return cb, out
+
+
+def cpu_report(ctx, value, cols, workers, repeats):
+    """The report's entries on the CPU baseline.  Where the reference build is
+    not present (it is compiled from the reference's sources) there is none:
+    the rest of the report stands without it."""
+    from oracle import ref
+    if not ref.available("o2"):
+        return {"cpu_baseline": None, "cpu_baseline_missing": "no reference -O2 build (make -C oracle ref)"}
+    cb, raw = cpu_baseline(ctx, cols, workers, repeats)
+    return {"cpu_baseline": cb, "gpu_over_cpu": round(value / cb["value"], 2),
+            "cpu_baseline_wall_s": round(raw["wall_s"], 3)}
 
 
 def adjoint_timing(steps):
@@ -507,10 +520,7 @@ def main():
     if a.multistep_adjoint:
         out["multistep_adjoint"] = multistep_adjoint(ncol=a.multistep_adjoint)
     if not a.no_cpu_baseline:
-        cb, raw = cpu_baseline(ctx, a.cpu_cols, a.cpu_workers, a.cpu_repeats)
-        out["cpu_baseline"] = cb
-        out["gpu_over_cpu"] = round(value / cb["value"], 2)
-        out["cpu_baseline_wall_s"] = round(raw["wall_s"], 3)
+        out.update(cpu_report(ctx, value, a.cpu_cols, a.cpu_workers, a.cpu_repeats))
     print(json.dumps(out), flush=True)
 
 
