@@ -328,16 +328,6 @@ __device__ __forceinline__ void graupel_fallspeed(const ConstView<S_t<R>>& C, co
 // digits.  A wavefront of clear points takes these few operations instead of
 // the 1,200 instructions that lead to the same result; they are the general
 // path's own, in its order, with its fused multiply-adds (mad).
-__device__ __forceinline__ float mad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ __forceinline__ double mad(double a, double b, double c) {
-#pragma clang fp contract(off)
-  return a * b + c;
-}
-template <class T>
-__device__ __forceinline__ Sig<T> mad(Sig<T> a, Sig<T> b, Sig<T> c) { return mad(a.v, b.v, c.v); }
-template <class T>
-__device__ __forceinline__ Dual<T> mad(Dual<T> a, Dual<T> b, Dual<T> c) { return a * b + c; }
-
 template <class R>
 __device__ __forceinline__ bool clear_air(R pres, R temp, R qv) {
   return qv < R(0.999) * rslf(pres, temp) && (temp >= R(kT0) || qv < R(1.2) * rsif(pres, temp));
@@ -486,8 +476,8 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
   sum_tendencies(C, L, t);
 
   // provisional update and re-checks on copies (:459-526)
-  L.temp = t1d + L.tten * dt;
-  L.qv = mx(R(kMinQv), qv1d + L.qvten * dt);
+  L.temp = mad(L.tten, dt, t1d);
+  L.qv = mx(R(kMinQv), mad(L.qvten, dt, qv1d));
   L.rho = rho_of(C, L.pres, L.temp, L.qv);
   L.nwfaten = L.nwfaten - (t.pna_rca + t.pna_sca + t.pna_gca + t.pni_iha) / L.rho;
   L.nifaten = L.nifaten - (t.pnd_rcd + t.pnd_scd + t.pnd_gcd) / L.rho;
@@ -522,8 +512,8 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
     L.tten = L.tten + L.lvap * L.ocp * t.prw_vcd;
     R x = qc1d, xn = nc1d;
     cloud_check(C, L, x, xn, has_nc, ncv, dt, odt);
-    L.qv = mx(R(kMinQv), qv1d + L.qvten * dt);
-    L.temp = t1d + L.tten * dt;
+    L.qv = mx(R(kMinQv), mad(L.qvten, dt, qv1d));
+    L.temp = mad(L.tten, dt, t1d);
     L.rho = rho_of(C, L.pres, L.temp, L.qv);
     thermo(C, L);
   }
@@ -536,8 +526,8 @@ __device__ __forceinline__ void phase_a_point(const StepArgs<R>& a, int c, int k
     L.tten = L.tten - L.lvap * L.ocp * t.prv_rev;
     R x = qr1d, xn = nr1d;
     rain_check(C, L, x, xn, dt, odt);
-    L.qv = mx(R(kMinQv), qv1d + L.qvten * dt);
-    L.temp = t1d + L.tten * dt;
+    L.qv = mx(R(kMinQv), mad(L.qvten, dt, qv1d));
+    L.temp = mad(L.tten, dt, t1d);
     L.rho = rho_of(C, L.pres, L.temp, L.qv);
     thermo(C, L);
   }
@@ -1421,14 +1411,14 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
       auto put = [&](int f, R v) {
         if (!same_bits(pt.f(f), v)) a.fo[f][o] = v;
       };
-      const R t_new = t1d + tten * dt;
+      const R t_new = mad(tten, dt, t1d);
       if (a.f[F_T])
         put(F_T, t_new);
       else
         put(F_TH, t_new / pt.f(F_PII));
-      put(F_QV, mx(R(kMinQv), (qv1d + qvten * dt)));
-      if (has_nwfa) put(F_NWFA, mx(R(kNwfaDefault), mn(R(kAeroMax), (pt.f(F_NWFA) + nwfaten * dt))));
-      if (has_nifa) put(F_NIFA, mx(R(kNifaDefault), mn(R(kAeroMax), (pt.f(F_NIFA) + nifaten * dt))));
+      put(F_QV, mx(R(kMinQv), mad(qvten, dt, qv1d)));
+      if (has_nwfa) put(F_NWFA, mx(R(kNwfaDefault), mn(R(kAeroMax), mad(nwfaten, dt, pt.f(F_NWFA)))));
+      if (has_nifa) put(F_NIFA, mx(R(kNifaDefault), mn(R(kAeroMax), mad(nifaten, dt, pt.f(F_NIFA)))));
       if (a.d3[D3_NC_MIX]) a.d3[D3_NC_MIX][d3] = R(0);
       if (a.d3[D3_MVD_R]) a.d3[D3_MVD_R][d3] = a.fl.mvd_r ? R(kD0R) : R(0);
       if (a.d3[D3_MVD_G]) a.d3[D3_MVD_G][d3] = a.fl.mvd_g ? R(kD0G) : R(0);
@@ -1488,11 +1478,11 @@ __device__ __forceinline__ void phase_c_point(const StepArgs<R>& a, int c, int k
 
   if (!a.fl.turn_off_micro) freeze_cloud_melt_ice(C, L, qc1d, qi1d, ni1d, nc1d, has_nc, ncv, lvap, ocp, dt, odt);
   // final update (:738-748)
-  const R t_new = pt.t() + L.tten * dt;
-  const R qv_new = mx(R(kMinQv), (pt.f(F_QV) + L.qvten * dt));
+  const R t_new = mad(L.tten, dt, pt.t());
+  const R qv_new = mx(R(kMinQv), mad(L.qvten, dt, pt.f(F_QV)));
   L.rho = rho_of(C, L.pres, L.temp, L.qv);
-  auto nwfa_new = [&]() { return mx(R(kNwfaDefault), mn(R(kAeroMax), (pt.f(F_NWFA) + L.nwfaten * dt))); };
-  auto nifa_new = [&]() { return mx(R(kNifaDefault), mn(R(kAeroMax), (pt.f(F_NIFA) + L.nifaten * dt))); };
+  auto nwfa_new = [&]() { return mx(R(kNwfaDefault), mn(R(kAeroMax), mad(L.nwfaten, dt, pt.f(F_NWFA)))); };
+  auto nifa_new = [&]() { return mx(R(kNifaDefault), mn(R(kAeroMax), mad(L.nifaten, dt, pt.f(F_NIFA)))); };
   if constexpr (!Point::kAdjoint) {
     if (has_nwfa) a.fo[F_NWFA][o] = nwfa_new();
     if (has_nifa) a.fo[F_NIFA][o] = nifa_new();

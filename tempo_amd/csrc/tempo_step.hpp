@@ -438,6 +438,19 @@ struct Tend {
   R pna_rca, pna_sca, pna_gca, pnd_rcd, pnd_scd, pnd_gcd;
 };
 
+// a * b + c where the clear-air path repeats the general one: one rounding in
+// FP32, two in FP64, whatever the compiler fuses elsewhere, so that a point's
+// result is the same on either path
+__device__ __forceinline__ float mad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double mad(double a, double b, double c) {
+#pragma clang fp contract(off)
+  return a * b + c;
+}
+template <class T>
+__device__ __forceinline__ Sig<T> mad(Sig<T> a, Sig<T> b, Sig<T> c) { return mad(a.v, b.v, c.v); }
+template <class T>
+__device__ __forceinline__ Dual<T> mad(Dual<T> a, Dual<T> b, Dual<T> c) { return a * b + c; }
+
 template <class R>
 __device__ __forceinline__ R rho_of(const ConstView<S_t<R>>& C, R pres, R temp, R qv) {
   return C.u.roverrv * pres / (R(kRdry) * temp * (qv + C.u.roverrv));
@@ -536,9 +549,9 @@ __device__ __forceinline__ void thermo(const ConstView<S_t<R>>& C, Lvl<R>& L) {
     L.visco = (R(1.718) + R(0.0049) * tempc) * R(1.0e-5);
   else
     L.visco = (R(1.718) + R(0.0049) * tempc - R(1.2e-5) * tempc * tempc) * R(1.0e-5);
-  L.ocp = R(1.0) / (R(kCp) * (R(1.0) + R(0.887) * L.qv));
+  L.ocp = R(1.0) / (R(kCp) * mad(R(0.887), L.qv, R(1.0)));
   L.vsc2 = msqrt(L.rho / L.visco);
-  L.lvap = R(kLvap0) + R(2106.0 - 4218.0) * tempc;
+  L.lvap = mad(R(2106.0 - 4218.0), tempc, R(kLvap0));
   L.tcond = (R(5.69) + R(0.0168) * tempc) * R(1.0e-5) * R(418.936);
   L.lvt2 = L.lvap * L.lvap * L.ocp * C.u.orv * otemp * otemp;
 }
