@@ -118,11 +118,11 @@ struct Radar {
   double sbins[kRadarBins], dsbins[kRadarBins];  // snow diameters 100 um .. 2 cm and widths
   double gbins[kRadarBins], dgbins[kRadarBins];  // graupel diameters 100 um .. 5 cm and widths
   double simpson[kRadarBins];                    // Simpson weights of the bins (:226-233)
-  double ocmg[kNrhg], ocms, obms;                // oamg^obmg, oams^obms, 1/bm_s
+  double ocmg[kNrhg], ocms;                      // oamg^obmg, oams^obms
   // the first (ice-water) Maxwell-Garnett mixing's operands: m_w^2, m_i^2
-  // and its two shape factors, fixed by the 10-cm indices of water and ice at
+  // and its shape factor, fixed by the 10-cm indices of water and ice at
   // 0 C (complex_water_ray, complex_ice_maetzler, :144-201)
-  double m1_re, m1_im, m3_re, m3_im, b2_re, b2_im, b3_re, b3_im;
+  double m1_re, m1_im, m3_re, m3_im, b3_re, b3_im;
   double k_w;  // |(m_w^2 - 1)/(m_w^2 + 2)|^2
 };
 

@@ -97,19 +97,16 @@ void build_radar(const Const<double>& c, Radar& r) {
     w[n + 2] += 1.0 / 3.0;
   }
   for (int n = 0; n < kRadarBins; ++n) r.simpson[n] = w[n];
-  // obms, ocms = oams**obms, ocmg = oamg**obmg (src/module_mp_tempo_params.F90:468-473)
-  r.obms = 1.0 / kBmS;
-  r.ocms = std::pow(c.oams, r.obms);
+  // ocms = oams**obms, ocmg = oamg**obmg (src/module_mp_tempo_params.F90:468-473)
+  r.ocms = std::pow(c.oams, 1.0 / kBmS);
   for (int m = 0; m < kNrhg; ++m) r.ocmg[m] = std::pow(1.0 / c.am_g[m], c.obmg);
-  // the first Maxwell-Garnett mixing: m1t = m_w^2, m2t = m_air^2 = 1, m3t = m_i^2
-  const cxd m_w = water_ray(0.10, 0.0), m_i = ice_maetzler(0.10, 0.0), m_air(1.0, 0.0);
-  const cxd m1t = cx_mul(m_w, m_w), m2t = cx_mul(m_air, m_air), m3t = cx_mul(m_i, m_i);
+  // the first Maxwell-Garnett mixing: m1t = m_w^2, m3t = m_i^2
+  const cxd m_w = water_ray(0.10, 0.0), m_i = ice_maetzler(0.10, 0.0);
+  const cxd m1t = cx_mul(m_w, m_w), m3t = cx_mul(m_i, m_i);
   const cxd two(2.0, 0.0), one(1.0, 0.0);
-  const cxd beta2 = cx_mul(cx_div(cx_mul(two, m1t), m2t - m1t), cx_mul(cx_div(m2t, m2t - m1t), std::log(cx_div(m2t, m1t))) - one);
   const cxd beta3 = cx_mul(cx_div(cx_mul(two, m1t), m3t - m1t), cx_mul(cx_div(m3t, m3t - m1t), std::log(cx_div(m3t, m1t))) - one);
   r.m1_re = m1t.real(); r.m1_im = m1t.imag();
   r.m3_re = m3t.real(); r.m3_im = m3t.imag();
-  r.b2_re = beta2.real(); r.b2_im = beta2.imag();
   r.b3_re = beta3.real(); r.b3_im = beta3.imag();
   const double kw = std::abs(cx_div(m1t - one, m1t + cxd(2.0, 0.0)));
   r.k_w = kw * kw;

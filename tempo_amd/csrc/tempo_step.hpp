@@ -373,8 +373,9 @@ struct DualGeom {
 
 // launch shape of one step (host-side choice, see tempo_hip_tune)
 struct LaunchCfg {
-  int sed_wave = 1;   // sedimentation: 1 = one wavefront per column (nz <= 128), 0 = one lane per column,
-                      // 2 = the wavefront kernel issuing every staging pass (check form)
+  int sed_wave = 1;   // sedimentation: 1 = one wavefront per column (flux form nz <= 256, semi-Lagrangian and
+                      // tangents nz <= 128), 0 = one lane per column, 2 = the wavefront kernel issuing every
+                      // staging pass (check form, flux form nz <= 128)
   int order = -1;     // point grouping within blocks: bit 0 phase A, bit 1 final update (-1: point_order)
   int block_a = 256;  // threads per block of the level-local kernels (64, 128 or 256)
   int block_c = 256;
