@@ -668,14 +668,14 @@ __global__ void __launch_bounds__(256) k_dual_pack_n(DualBatch<T> b, DualGeom g)
   const T* t = b.t[blockIdx.z];
   b.d[blockIdx.z][p.e] = Dual<T>(b.v[blockIdx.z][p.o], t ? t[p.o] : T(0));
 }
-// duals into values and tangents (either may be NULL); zeros at the levels a
-// column does not have (nlev, may be NULL), where the step sets no diagnostics
-template <class T>
+// duals into values and tangents (either may be NULL); with kDepth, zeros at the
+// levels a column does not have, where the step sets no diagnostics
+template <class T, bool kDepth>
 __global__ void __launch_bounds__(256) k_dual_unpack_n(DualBatch<T> b, DualGeom g, const int* __restrict__ nlev) {
   const PlanePoint p = plane_point(g);
   if (!p.in) return;
-  const bool none = nlev && int(blockIdx.y) >= nlev[blockIdx.x * 256u + threadIdx.x];
-  const Dual<T> x = none ? Dual<T>(T(0), T(0)) : b.d[blockIdx.z][p.e];
+  Dual<T> x = b.d[blockIdx.z][p.e];
+  if (kDepth && int(blockIdx.y) >= nlev[blockIdx.x * 256u + threadIdx.x]) x = Dual<T>(T(0), T(0));
   if (b.v[blockIdx.z]) b.v[blockIdx.z][p.o] = x.v;
   if (b.t[blockIdx.z]) b.t[blockIdx.z][p.o] = x.d;
 }
@@ -701,7 +701,8 @@ hipError_t launch_dual_pack_n(const DualBatch<T>& b, int n, const DualGeom& g, h
 }
 template <class T>
 hipError_t launch_dual_unpack_n(const DualBatch<T>& b, int n, const DualGeom& g, const int* nlev, hipStream_t s) {
-  return launch_batch(k_dual_unpack_n<T>, b, n, g, s, nlev);
+  return nlev ? launch_batch(k_dual_unpack_n<T, true>, b, n, g, s, nlev)
+              : launch_batch(k_dual_unpack_n<T, false>, b, n, g, s, nlev);
 }
 
 }  // namespace tempo
