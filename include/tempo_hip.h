@@ -272,8 +272,11 @@ int tempo_hip_tlm(tempo_hip_ctx *ctx, const tempo_hip_fields *f, const tempo_hip
  * entries ignored).  Writes dL/d(input) of t, qv, qc, qr, qi, qs, qg, nc,
  * nr, ni, nwfa, nifa, ng and qb into the matching entries of xbar (NULL
  * entries are skipped and cost nothing), with the branches frozen as in
- * tempo_hip_tlm; p, w, dz enter as constants.  Working memory (about 2.5 kB
- * per column-level) is allocated on first use.  Returns
+ * tempo_hip_tlm; p, w, dz enter as constants.  Working memory is allocated
+ * on first use of a size and kept until tempo_hip_finalize: about 1.4 kB per
+ * column-level in FP32 and 1.9 kB in FP64 (2.2 and 2.8 kB above 128 levels),
+ * and below 2^21 column-levels 0.64 kB (0.95 kB) per column-level and entry
+ * of xbar more, at most 1.33 GB (1.99 GB).  Returns
  * TEMPO_HIP_E_UNSUPPORTED for a context with semi_sedi_flag or
  * refl10cm_from_melting_flag. */
 int tempo_hip_adjoint(tempo_hip_ctx *ctx, const tempo_hip_fields *f, const tempo_hip_fields *ybar,

@@ -589,21 +589,16 @@ __global__ void __launch_bounds__(64 * kScrW) k_adj_sed_wave(StepArgs<D> a, AdjA
   }
 }
 
-// All tangent passes and S^T of one adjoint step.  a: dual step arguments
-// over the working state copy (whose fields point into `work_state`);
-// `inputs` is the packed input state.  snap_a / snap_b receive the working
-// state and scratch after phase A and after phase B of a tangent-free run,
-// so that the later passes restart from them instead of recomputing.
-// scratch snapshots of the adjoint: working-precision and FP64 planes after
-// phase A (used for nz > 128 only), and the post-sedimentation tendency
-// values (NULL where nothing overwrites them)
+// Copies an adjoint step needs: the working-precision and FP64 scratch planes
+// after phase A (used for nz > 128 only), and the post-sedimentation tendency
+// values (NULL where nothing overwrites them).
 struct AdjSnap {
   void* sr_a;  // sr_bytes
   void* sd_a;  // sd_bytes
   void* sd_b;  // sd_bytes (holds 10 FP64 planes of the post-sedimentation tendencies)
 };
 
-// The passes of one adjoint.  The state is out of place: a.f holds the
+// The passes of one adjoint: all tangent passes and S^T.  The state is out of place: a.f holds the
 // packed inputs (duals, zero tangents: the passes seed what they read), a.fa
 // the state after the initial checks (phase A's output); no pass stores a new
 // state.
@@ -624,9 +619,8 @@ hipError_t adjoint_passes(const StepArgs<D>& a, AdjArgs g, Dual<double>* vtbuf, 
 
   // tangent-free forward.  Its sedimentation on the values, one wavefront
   // per column (the tangents are zero in this pass), writes only the ten
-  // tendency planes, which S^T does not read and every later reader finds
-  // rewritten by a local pass's phase A (it writes all planes of each live
-  // point it runs), so the scratch after A needs no snapshot.  The
+  // tendency planes, which S^T does not read and whose values the later passes
+  // want as they are, so the scratch after A needs no snapshot.  The
   // lane-per-column form (nz > 128) uses state planes as work space: the
   // scratch after A is snapshotted and restored before S^T.
   const bool wave_b = a.nz <= kSedLevels;

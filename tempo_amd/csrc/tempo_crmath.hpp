@@ -31,9 +31,9 @@
 // for special arguments, each call site took several kilobytes and the FP64
 // level physics 757 KB of code, which a compute unit's 64 KB instruction
 // cache cannot hold: a single column waited 213 us in that kernel, most of
-// it for instructions.  In this form it is 205 KB; a step of one column of 60
-// levels takes 186 instead of 335 us, of 25,000 x 90 2.12 instead of
-// 3.33 ms.  Special arguments (0, negative, infinite, NaN, 1) are a short
+// it for instructions.  In this form it is 205 KB: by this alone a step of one
+// column of 60 levels took 186 instead of 335 us, of 25,000 x 90 2.12 instead
+// of 3.33 ms.  Special arguments (0, negative, infinite, NaN, 1) are a short
 // block of selects, results near overflow or in the subnormal range come
 // from the final scaling.
 #pragma once

@@ -1102,12 +1102,12 @@ __device__ __forceinline__ void phase_b_group(const StepArgs<R>& a, int c0, void
   if (a.d2[D2_HAIL_COL]) a.d2[D2_HAIL_COL][d2] = R(0);
 }
 
-// waves per SIMD by chunks: one chunk fits 8 without spills, two are held to
-// 6, three and four take what their registers allow.  A spill is a
-// scratch-memory access in every stage and dominates soon: two chunks held to
-// 8 waves (128 B of spills) take 1.20 ms at 100,000 x 90 against 0.50 at 6
-// (52 B) and 0.42 with precipitation sums and substep records kept in LDS
-// and 32-bit plane offsets (12 B); at 5 waves 0.49 before that.
+// Waves per SIMD by chunks, as many as the registers allow next to no spills:
+// one chunk is held to 7 (50 VGPRs in FP32, none spilled, where 8 run), two to 6
+// (80 VGPRs, 20 B spilled), three and four take what they need (110, 138).  A
+// spill is a scratch-memory access in every stage and dominates soon: two
+// chunks held to 8 waves (128 B of spills) took 1.20 ms at 100,000 x 90 against
+// 0.50 at 6 (52 B then) and 0.49 at 5; now 0.40 at 6.
 // Against one lane per column the wavefront form takes, for the whole step,
 // 0.33 instead of 2.93 ms at 8,191 x 160 (FP32; one lane per column is 128
 // wavefronts on 256 CUs).
