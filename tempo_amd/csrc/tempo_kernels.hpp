@@ -794,7 +794,7 @@ __device__ void semi_sediment(const StepArgs<R>& a, int c, int nzc, W_t<R>* xr, 
   arr(WI, 0) = V(0);
   arr(WI, 1) = W(0.5) * (V(1) + V(0));
   for (int k = 2; k < nz - 1; ++k) arr(WI, k) = fa1 * (V(k) + V(k - 1)) - fa2 * (V(k + 1) + V(k - 2));
-  arr(WI, nz - 1) = W(0.5) * (V(nz - 1) + V(nz - 2));
+  if (nz > 1) arr(WI, nz - 1) = W(0.5) * (V(nz - 1) + V(nz - 2));  // a single level has none below it
   arr(WI, nz) = V(nz);
   for (int k = 1; k < nz; ++k)
     if (V(k) == W(0.0)) {

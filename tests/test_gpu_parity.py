@@ -1591,3 +1591,39 @@ def test_gpu_rain_below_presence_at_the_top_level(hip):
         assert (got[0]["qs"][-2] > 0.0).all()  # the snow falls
         for n, v in got[1].items():
             assert np.array_equal(v, got[0][n], equal_nan=True), (nz, n)
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "fp64"])
+def test_gpu_semi_lagrangian_one_level_columns(hip, dtype):
+    """semi-Lagrangian sedimentation of columns of one and two active levels
+    beside deeper ones: the wavefront form against one lane per column bit for
+    bit, and each shallow column as it is alone (nothing below its only level
+    is read)"""
+    from tempo_amd import generator as gen
+    ctx = context(hip, dict(aerosolaware=True, hailaware=True, semi_sedi=True))
+    prec, td = (hip.FP32, torch.float32) if dtype == "fp32" else (hip.FP64, torch.float64)
+    ncol = 24
+    st, m = gen.generate("multistep", ncol=ncol, col0=321)
+    st["qr"][:3] = np.linspace(1e-6, 1e-3, 3 * ncol).reshape(3, ncol)
+    st["nr"][:3] = 1e4
+    st["qg"][:3] = 1e-4
+    st["ng"][:3], st["qb"][:3] = 1e3, 1e-4 / 400.0
+    nlev = np.where(np.arange(ncol) % 3 == 0, 1, np.where(np.arange(ncol) % 3 == 1, 2, 60)).astype(np.int32)
+
+    def run(cols):
+        dev = {k: torch.tensor(np.ascontiguousarray(v[:, cols]), dtype=td, device="cuda") for k, v in st.items()}
+        d = ctx.run(dev, m["dt"], 2, nlev=torch.tensor(nlev[cols], device="cuda"))
+        return {k: v.cpu().numpy() for k, v in {**dev, **d}.items()}
+    got = {}
+    try:
+        for wave in (1, 0):
+            ctx.tune(prec, hip.TUNE_SED_WAVE, wave)
+            got[wave] = run(np.arange(ncol))
+            for c in (0, 1, 3, 21):
+                for k, v in run(np.array([c])).items():
+                    assert np.array_equal(v[..., 0], got[wave][k][..., c]), (wave, c, k)
+    finally:
+        ctx.tune(prec, hip.TUNE_SED_WAVE, 1)
+    assert (got[1]["rain_precip"][nlev == 1] > 0.0).all()
+    for k, v in got[1].items():
+        assert np.array_equal(v, got[0][k], equal_nan=True), k
